@@ -31,6 +31,7 @@ ARCH = "gfx950"
 UNITS = [
     ("mg_api.hip", "mg_api", []),
     ("swiglu_inst.hip", "swiglu_inst", []),
+    ("block_inst.hip", "block_inst", []),
     ("rmsnorm_fwd_inst.hip", "rmsnorm_fwd_f32", ["-DMG_DTYPE=0"]),
     ("rmsnorm_fwd_inst.hip", "rmsnorm_fwd_f16", ["-DMG_DTYPE=1"]),
     ("rmsnorm_fwd_inst.hip", "rmsnorm_fwd_bf16", ["-DMG_DTYPE=2"]),

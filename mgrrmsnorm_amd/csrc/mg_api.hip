@@ -2,6 +2,7 @@
 // Validation happens before any HIP call so that argument errors are reported on hosts
 // without a GPU.
 #include "megagemm_hip.h"
+#include "megagemm_hip_block.h"
 #include "megagemm_hip_tuning.h"
 #include "mg_launch.hpp"
 #include "mg_device.hpp"
@@ -657,6 +658,38 @@ int mg_swiglu_bwd(void* dgu, const void* dh, const void* gu, int64_t M, int64_t 
         launch_swiglu_bwd(dtype, mode, swiglu_unroll(1, 4), xcd_group_or(kXcdGroupStreaming), dgu, dh, gu, (long)M, (long)H, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip("mg_swiglu_bwd: launch", e);
     return MG_OK;
+}
+
+static int block_projection(const char* fn, bool paired, void* out, const void* x, const void* w, int64_t tokens,
+                            int64_t K, int64_t N, int dtype, void* stream) {
+    static_assert(MG_BLOCK_MAX_TOKENS == kSkinnyMaxTokens, "header and kernel agree");
+    if (dtype != MG_F16 && dtype != MG_BF16)
+        return fail(MG_ERR_UNSUPPORTED, "%s: dtype must be 1 (fp16) or 2 (bf16), got %d", fn, dtype);
+    if (tokens < 1 || tokens > kSkinnyMaxTokens)
+        return fail(MG_ERR_UNSUPPORTED, "%s: tokens must be in [1, %d] (got %lld)", fn, kSkinnyMaxTokens, (long long)tokens);
+    if (K < 8 || K % 8 != 0 || K >= (1LL << 30) || N < 1 || N >= (1LL << 30))
+        return fail(MG_ERR_UNSUPPORTED, "%s: the inner size must be a multiple of 8 and both sizes in [1, 2^30) (got %lld, %lld)",
+                    fn, (long long)K, (long long)N);
+    if (out == nullptr || x == nullptr || w == nullptr) return fail(MG_ERR_INVALID_ARG, "%s: a pointer is NULL", fn);
+    if (!aligned(out, 2) || !aligned(x, 16) || !aligned(w, 16))
+        return fail(MG_ERR_INVALID_ARG, "%s: inputs must be 16-byte aligned", fn);
+    int cus = 0;
+    const int rc = cu_count(&cus);
+    if (rc != MG_OK) return rc;
+    const SkinnyArgs a = {out, x, w, (int)tokens, (int)K, (int)N, cus};
+    const hipError_t e = launch_skinny_gemm(dtype, paired, a, (hipStream_t)stream);
+    if (e != hipSuccess) return fail_hip(fn, e);
+    return MG_OK;
+}
+
+int mg_block_gate_up(void* h, const void* x, const void* w12, int64_t tokens, int64_t d_model, int64_t hidden,
+                     int dtype, void* stream) {
+    return block_projection("mg_block_gate_up", true, h, x, w12, tokens, d_model, hidden, dtype, stream);
+}
+
+int mg_block_down(void* out, const void* h, const void* w3, int64_t tokens, int64_t d_model, int64_t hidden,
+                  int dtype, void* stream) {
+    return block_projection("mg_block_down", false, out, h, w3, tokens, hidden, d_model, dtype, stream);
 }
 
 }  // extern "C"

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "megagemm_hip.h"
+#include "megagemm_hip_block.h"
 
 namespace {
 
@@ -247,6 +248,36 @@ Tensor swiglu(const Tensor& w12_out, int64_t hidden_dim) {
     return swiglu_forward(fused.view({-1, 2 * hidden_dim}), hidden_dim).view(shape);
 }
 
+// w3(silu(gate) * up) with [gate | up] = w12(x) where nothing is to be differentiated and the call is
+// one of those mg_block_gate_up and mg_block_down take; an undefined tensor (None) where it is not, and
+// the caller then goes through the projections and the activation one by one.
+Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
+    const Tensor none;
+    const auto type = x.scalar_type();
+    if (!x.is_cuda() || (type != at::kHalf && type != at::kBFloat16) || x.dim() < 1 || w12.dim() != 2 || w3.dim() != 2)
+        return none;
+    const int64_t d_model = w3.size(0), hidden = w3.size(1);
+    if (d_model < 1 || x.size(-1) != d_model || w12.size(0) != 2 * hidden || w12.size(1) != d_model) return none;
+    const int64_t tokens = x.numel() / d_model;
+    if (tokens < 1 || tokens > MG_BLOCK_MAX_TOKENS || d_model % 8 != 0 || hidden % 8 != 0 || hidden < 8) return none;
+    if (w12.scalar_type() != type || w3.scalar_type() != type || w12.device() != x.device() || w3.device() != x.device() ||
+        !w12.is_contiguous() || !w3.is_contiguous())
+        return none;
+    if (torch::GradMode::is_enabled() && (x.requires_grad() || w12.requires_grad() || w3.requires_grad())) return none;
+    const Tensor xc = x.contiguous();
+    const auto off = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; };
+    if (off(xc) || off(w12) || off(w3)) return none;
+    const int code = dtype_code(type);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    auto h = torch::empty({tokens, hidden}, xc.options());
+    auto out = torch::empty_like(xc);
+    void* stream = current_stream();
+    int rc = mg_block_gate_up(h.data_ptr(), xc.data_ptr(), w12.data_ptr(), tokens, d_model, hidden, code, stream);
+    if (rc == MG_OK) rc = mg_block_down(out.data_ptr(), h.data_ptr(), w3.data_ptr(), tokens, d_model, hidden, code, stream);
+    TORCH_CHECK(rc == MG_OK, "SwiGLU block failed (code ", rc, "): ", mg_last_error());
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -267,6 +298,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("grad_out"), py::arg("gate_up"), py::arg("hidden_dim"));
     m.def("rmsnorm", &rmsnorm, "differentiable RMSNorm over the last dimension", py::arg("input"), py::arg("weight"),
           py::arg("epsilon") = 1e-5);
+    m.def("swiglu_block", &swiglu_block, "the whole SwiGLU block for a few rows, not differentiable; None where it does not apply",
+          py::arg("x"), py::arg("w12"), py::arg("w3"));
     m.def("swiglu", &swiglu, "differentiable silu(gate) * up over the last dimension", py::arg("w12_out"),
           py::arg("hidden_dim"));
 }

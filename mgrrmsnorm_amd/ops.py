@@ -142,3 +142,11 @@ def swiglu(w12_out: torch.Tensor, hidden_dim: int) -> torch.Tensor:
         raise RuntimeError(f"last dimension must be 2*hidden_dim = {2 * hidden_dim}, got {tuple(w12_out.shape)}")
     fused = w12_out if w12_out.is_contiguous() else w12_out.contiguous()
     return swiglu_forward(fused.view(-1, 2 * hidden_dim), hidden_dim).view(*fused.shape[:-1], hidden_dim)
+
+
+def swiglu_block(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
+    """w3(silu(gate) * up) with [gate | up] = w12(x), for the few rows of a decoding step and with
+    nothing to differentiate; None when the call is not of that kind (or the extension is not
+    built) and has to go through the projections and `swiglu`."""
+    ext = _extension()
+    return ext.swiglu_block(x, w12, w3) if ext is not None else None

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _module
 from torch.autograd.function import once_differentiable
 
 from . import ops
@@ -43,6 +44,26 @@ class MegaGemmFunction(torch.autograd.Function):
         return grad.view(fused.shape), None
 
 
+def _plain_weight(linear):
+    """The weight of a projection that is exactly `x @ weight.T`: a bias-free nn.Linear that nobody
+    has hooked, replaced, parametrised or wrapped; else None."""
+    if (type(linear) is not nn.Linear or linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
+            or linear._backward_pre_hooks or "forward" in linear.__dict__):
+        return None
+    parameters = linear._parameters
+    weight = parameters.get("weight")
+    return weight if type(weight) is nn.Parameter and parameters.get("bias") is None else None
+
+
+def _calls_observed():
+    """Something wants to see the projections as torch operations: autocast, a dispatch or function
+    mode, the compiler, or a global module hook."""
+    return (torch.is_autocast_enabled() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0 or torch.compiler.is_compiling()
+            or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
+            or _module._global_backward_pre_hooks)
+
+
 class MegaGemmTriton(nn.Module):
     """SwiGLU feed-forward block: w3(silu(w1 x) * (w2 x)) with w1 and w2 fused into w12.
 
@@ -63,6 +84,14 @@ class MegaGemmTriton(nn.Module):
         self.w3 = nn.Linear(self.hidden, d_model, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # a decoding step: projections and activation in two kernels that read the weights once,
+        # while the projections are the plain ones this module made
+        if type(x) is torch.Tensor and not _calls_observed():
+            w12, w3 = _plain_weight(self._modules.get("w12")), _plain_weight(self._modules.get("w3"))
+            if w12 is not None and w3 is not None and w3.size(-1) == self.hidden:
+                out = ops.swiglu_block(x, w12, w3)
+                if out is not None:
+                    return out
         # the activation's autograd node lives in the compiled extension when that is built
         # (else MegaGemmFunction); with nothing to differentiate it is the bare kernel
         return self.w3(ops.swiglu(self.w12(x), self.hidden))

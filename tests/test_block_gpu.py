@@ -1,0 +1,100 @@
+"""The SwiGLU block as one operator (megagemm_hip_block.h): a decoding step through MegaGemmTriton
+against the same formula in float64, at the sizes where the split over workgroups, waves and
+16-row tiles has edges, and the calls that have to keep going through the projections."""
+import pytest
+import torch
+
+from mgrrmsnorm_amd import MegaGemmTriton, ops
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16}
+HALF_ULP = {"bf16": 2.0 ** -9, "fp16": 2.0 ** -12}   # largest relative error of one rounding (bf16: 8 bits, fp16: 11)
+
+
+def _case(tokens, d_model, hidden, dtype, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    n = lambda *s: torch.randn(s, generator=g, device="cuda")
+    dt = DTYPES[dtype]
+    return n(tokens, d_model).to(dt), (n(2 * hidden, d_model) * d_model ** -0.5).to(dt), (n(d_model, hidden) * hidden ** -0.5).to(dt)
+
+
+def _within(out, x, w12, w3, dtype):
+    """Every element within what one rounding of h, one of the result and two fp32 sums can do."""
+    xd, ad, bd = x.double(), w12.double(), w3.double()
+    gate, up = (xd @ ad.t()).chunk(2, -1)
+    h = torch.nn.functional.silu(gate) * up
+    ref = h @ bd.t()
+    u, e = HALF_ULP[dtype], 2.0 ** -24
+    tiny = 2.0 ** -25 if dtype == "fp16" else 0.0                       # half a subnormal step of fp16
+    # error of gate and up from an fp32 sum of d_model products, carried through silu'(g) <= 1.1
+    ag, au = (xd.abs() @ ad.abs().t()).chunk(2, -1)
+    k = (x.size(-1) + 8) * e
+    dh = k * (1.1 * ag * up.abs() + au * gate.abs()) + 8 * e * h.abs() + u * h.abs() + tiny
+    bound = (dh + (w3.size(1) + 8) * e * h.abs()) @ bd.abs().t() * (1 + u) + u * ref.abs() + tiny
+    worst = ((out.double() - ref).abs() - bound).max().item()
+    assert worst <= 0.0, f"beyond the error bound by {worst}"
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("tokens,d_model,hidden", [
+    (1, 8, 8), (3, 40, 24), (16, 64, 72), (15, 72, 1000), (2, 520, 264), (16, 1152, 3072),
+    (8, 4096, 6912),      # three and a half tiles of columns per workgroup, one of the second projection
+    (5, 64, 9000),        # more columns per workgroup than four tiles hold
+    (7, 17000, 128),      # the same in the second projection
+    (9, 8192, 2048),      # two tiles of the second projection per workgroup
+])
+def test_decode_block_against_float64(tokens, d_model, hidden, dtype):
+    x, w12, w3 = _case(tokens, d_model, hidden, dtype)
+    out = ops.swiglu_block(x, w12, w3)
+    assert out is not None and out.shape == x.shape and out.dtype == x.dtype
+    _within(out, x, w12, w3, dtype)
+    assert torch.equal(out, ops.swiglu_block(x, w12, w3))   # fixed summation order
+
+
+def test_rows_do_not_depend_on_each_other():
+    x, w12, w3 = _case(16, 256, 512, "bf16")
+    out = ops.swiglu_block(x, w12, w3)
+    for t in (1, 5):
+        assert torch.equal(ops.swiglu_block(x[:t].contiguous(), w12, w3), out[:t])
+    x[3] = float("nan")
+    bad = ops.swiglu_block(x, w12, w3)
+    keep = [t for t in range(16) if t != 3]
+    assert torch.isnan(bad[3]).all() and torch.equal(bad[keep], out[keep])
+
+
+def test_module_takes_it_and_steps_aside():
+    module = MegaGemmTriton(256).cuda().to(torch.bfloat16)
+    x = torch.randn(2, 3, 256, device="cuda", dtype=torch.bfloat16)
+    w12, w3 = module.w12.weight, module.w3.weight
+    with torch.no_grad():
+        fused = module(x)
+        assert torch.equal(fused, ops.swiglu_block(x, w12, w3)) and fused.shape == x.shape
+        seen = []
+        handle = module.w12.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+        hooked = module(x)
+        handle.remove()
+        assert seen == [(2, 3, 2 * module.hidden)]
+        assert (hooked - fused).abs().max() <= 2.0 ** -6 * fused.abs().max()   # h and [gate | up] rounded on the way
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert module(x).dtype == torch.float16
+    y = module(x)                                       # gradients wanted: the differentiable path
+    assert y.requires_grad
+    y.sum().backward()
+    assert w12.grad is not None and w3.grad is not None
+
+
+@pytest.mark.parametrize("change", ["tokens", "dtype", "width", "alignment", "layout"])
+def test_calls_it_does_not_take(change):
+    x, w12, w3 = _case(4, 64, 64, "bf16")
+    if change == "tokens":
+        x = x.repeat(5, 1)
+    elif change == "dtype":
+        x, w12, w3 = x.float(), w12.float(), w3.float()
+    elif change == "width":
+        x, w12, w3 = _case(4, 60, 64, "bf16")
+    elif change == "alignment":
+        w3 = torch.empty(64 * 64 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(64, 64).copy_(w3)
+    else:
+        w12 = w12.t().contiguous().t()
+    assert ops.swiglu_block(x, w12, w3) is None
