@@ -50,6 +50,14 @@ SIGNATURES = {
     "mg_rmsnorm_bwd_timeline": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _i64, _i64, _vp, _vp]),
 }
 
+# the entry points of include/megagemm_hip_fused.h
+FUSED_SIGNATURES = {
+    "mg_rmsnorm_bwd_small_fits": (_int, [_i64, _i64, _int]),
+    "mg_rmsnorm_bwd_small": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _vp]),
+    "mg_block_gate_up": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
+    "mg_block_down": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
+}
+
 
 def load() -> ctypes.CDLL:
     """Load the library once per process; raise RuntimeError when it has not been built."""
@@ -67,7 +75,7 @@ def load() -> ctypes.CDLL:
             lib = ctypes.CDLL(str(LIB_PATH))
         except OSError as exc:  # e.g. libamdhip64.so not found
             raise RuntimeError(f"cannot load {LIB_PATH}: {exc}") from exc
-        for name, (restype, argtypes) in SIGNATURES.items():
+        for name, (restype, argtypes) in {**SIGNATURES, **FUSED_SIGNATURES}.items():
             fn = getattr(lib, name)
             fn.restype = restype
             fn.argtypes = argtypes

@@ -2,7 +2,7 @@
 // Validation happens before any HIP call so that argument errors are reported on hosts
 // without a GPU.
 #include "megagemm_hip.h"
-#include "megagemm_hip_block.h"
+#include "megagemm_hip_fused.h"
 #include "megagemm_hip_tuning.h"
 #include "mg_launch.hpp"
 #include "mg_device.hpp"
@@ -657,6 +657,43 @@ int mg_swiglu_bwd(void* dgu, const void* dh, const void* gu, int64_t M, int64_t 
     hipError_t e =
         launch_swiglu_bwd(dtype, mode, swiglu_unroll(1, 4), xcd_group_or(kXcdGroupStreaming), dgu, dh, gu, (long)M, (long)H, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip("mg_swiglu_bwd: launch", e);
+    return MG_OK;
+}
+
+// What rmsnorm_bwd_small can hold at all; mg_rmsnorm_bwd_small_fits says where it is also faster.
+static bool bwd_small_holds(int64_t rows, int64_t cols, int es) {
+    return rows >= 1 && cols >= 1 && cols * es <= 2048 * kVec && rows <= (1LL << 20) && rows * cols * es < (1LL << 31);
+}
+
+// Up to 1024 rows: a line of columns is then eight rows per thread of its workgroup (bf16, one launch
+// against two: 1024 x 768 6.7 / 8.6 us, 1024 x 4096 9.5 / 10.4, 1024 x 16384 26.7 / 35.6; 1536 x 4096 14.6 / 13.6).  fp32
+// reads twice the bytes for as many columns: beyond 512 rows only up to 8 MiB per tensor (1024 x 2048 9.4 /
+// 9.7, 512 x 8191 18.7 / 22.2; 768 x 4096 13.1 / 13.0, 1024 x 4096 16.2 / 14.0).
+int mg_rmsnorm_bwd_small_fits(int64_t rows, int64_t cols, int dtype) {
+    const int es = esize_of(dtype);
+    return es != 0 && bwd_small_holds(rows, cols, es) && rows <= 1024 &&
+           (es == 2 || rows <= 512 || rows * cols * es <= (8LL << 20));
+}
+
+int mg_rmsnorm_bwd_small(void* dx, float* dw_f32, void* dw_cast, const void* dy, const void* x, const void* w,
+                         const float* inv_rms, int64_t rows, int64_t cols, int dtype, void* stream) {
+    const int rc = check_rmsnorm_dims("mg_rmsnorm_bwd_small", rows, cols, dtype);
+    if (rc != MG_OK) return rc;
+    const int es = esize_of(dtype);
+    if (!bwd_small_holds(rows, cols, es))
+        return fail(MG_ERR_UNSUPPORTED, "mg_rmsnorm_bwd_small: %lld x %lld %s is not a shape for it", (long long)rows,
+                    (long long)cols, dtype_name(dtype));
+    if (dx == nullptr || dy == nullptr || x == nullptr || w == nullptr || inv_rms == nullptr)
+        return fail(MG_ERR_INVALID_ARG, "mg_rmsnorm_bwd_small: dx, dy, x, w and inv_rms must not be NULL");
+    if (!aligned(dx, es) || !aligned(dy, es) || !aligned(x, es) || !aligned(w, es) || !aligned(inv_rms, 4) ||
+        !aligned(dw_f32, 4) || !aligned(dw_cast, es))
+        return fail(MG_ERR_INVALID_ARG, "mg_rmsnorm_bwd_small: a pointer is not aligned to its element size");
+    const BwdSmallArgs a = {dx, dw_f32, dw_cast, dy, x, w, inv_rms, (int)rows, (int)cols};
+    hipStream_t s = (hipStream_t)stream;
+    const hipError_t e = by_dtype(
+        dtype, [&] { return launch_rmsnorm_bwd_small<float>(a, s); },
+        [&] { return launch_rmsnorm_bwd_small<half_t>(a, s); }, [&] { return launch_rmsnorm_bwd_small<bf16_t>(a, s); });
+    if (e != hipSuccess) return fail_hip("mg_rmsnorm_bwd_small: launch", e);
     return MG_OK;
 }
 

@@ -192,6 +192,13 @@ struct BwdArgs {
 template <typename T> hipError_t launch_rmsnorm_fwd(const RowCfg& cfg, bool generic, const FwdArgs& a, hipStream_t s);
 template <typename T> hipError_t launch_rmsnorm_bwd(const RowCfg& cfg, bool generic, const BwdArgs& a, hipStream_t s);
 
+// The one-launch backward of few rows (rmsnorm_bwd_small.hpp).
+struct BwdSmallArgs {
+    void* dx; float* dw_f32; void* dw_cast; const void* dy; const void* x; const void* w; const float* inv_rms;
+    int rows, cols;
+};
+template <typename T> hipError_t launch_rmsnorm_bwd_small(const BwdSmallArgs& a, hipStream_t s);
+
 hipError_t launch_dw_reduce(float* dw_f32, void* dw_cast, int cast_dtype, const float* part, int P, int ld,
                             int cols, hipStream_t s);
 hipError_t launch_fill_zero(float* p, long n, hipStream_t s);

@@ -3,6 +3,7 @@
 #include <atomic>
 
 #include "mg_launch.hpp"
+#include "rmsnorm_bwd_small.hpp"
 #include "rmsnorm_kernels.hpp"
 
 #ifndef MG_DTYPE
@@ -227,6 +228,22 @@ hipError_t launch_rmsnorm_bwd<elem_t>(const RowCfg& cfg, bool generic, const Bwd
     if (cfg.block == 512) return by_tpr<512>(cfg.tpr, cfg.items, a, s);
     if (cfg.block == 256 && cfg.tpr == 256) return by_items<256, 256>(cfg.items, a, s);
     return hipErrorInvalidValue;
+}
+
+template <>
+hipError_t launch_rmsnorm_bwd_small<elem_t>(const BwdSmallArgs& a, hipStream_t s) {
+    const long nvec = ((long)a.cols * (long)sizeof(elem_t) + kVec - 1) / kVec;
+    if (nvec > 2048 || (long)a.rows * a.cols * (long)sizeof(elem_t) >= (1L << 31)) return hipErrorInvalidValue;
+    int wpr = 1;
+    while (wpr < 16 && wpr * kWave < nvec) wpr *= 2;
+    const int rows_per_wg = 16 / wpr;
+    const int row_wgs = (a.rows + rows_per_wg - 1) / rows_per_wg;
+    const bool want_dw = a.dw_f32 != nullptr || a.dw_cast != nullptr;
+    const int col_wgs = want_dw ? (int)((nvec + 7) / 8) : 0;
+    auto kernel = nvec > 1024 ? rmsnorm_bwd_small<elem_t, 2> : rmsnorm_bwd_small<elem_t, 1>;
+    return launch(kernel, dim3((unsigned)(row_wgs + col_wgs)), dim3(kSmallBlock), 0, s, (elem_t*)a.dx, a.dw_f32,
+                  (elem_t*)a.dw_cast, (const elem_t*)a.dy, (const elem_t*)a.x, (const elem_t*)a.w, a.inv_rms, a.rows,
+                  a.cols, 1.0f / (float)a.cols, wpr, row_wgs);
 }
 
 }  // namespace mg

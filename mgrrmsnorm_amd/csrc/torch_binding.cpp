@@ -22,7 +22,7 @@
 #include <vector>
 
 #include "megagemm_hip.h"
-#include "megagemm_hip_block.h"
+#include "megagemm_hip_fused.h"
 
 namespace {
 
@@ -85,24 +85,32 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor& grad_output, cons
                 "inv_rms must be a float32 vector with one entry per row");
     const int code = dtype_code(input.scalar_type());
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    int64_t num_partials = 0, ld = 0;
-    TORCH_CHECK(mg_rmsnorm_bwd_workspace(rows, cols, code, &num_partials, &ld) == MG_OK,
-                "RMSNorm backward (workspace query) failed: ", mg_last_error());
     const auto f32 = input.options().dtype(torch::kFloat32);
     auto grad_input = torch::empty_like(input);
-    auto partial = torch::empty({num_partials, ld}, f32);
     void* stream = current_stream();
-    int rc = mg_rmsnorm_bwd(grad_input.data_ptr(), partial.data_ptr<float>(), grad_output.data_ptr(),
-                            input.data_ptr(), weight.data_ptr(), inv_rms.data_ptr<float>(), rows, cols, code,
-                            num_partials, ld, stream);
-    TORCH_CHECK(rc == MG_OK, "RMSNorm backward failed (code ", rc, "): ", mg_last_error());
     Tensor dw_f32, dw_cast;
     if (need_weight_grad) {
         if (want_f32 || code == MG_F32) dw_f32 = torch::empty({cols}, f32);
         dw_cast = code == MG_F32 ? dw_f32 : torch::empty_like(weight);   // weight dtype, as binding.cpp:90
-        rc = mg_rmsnorm_dw_reduce(dw_f32.defined() ? dw_f32.data_ptr<float>() : nullptr,
-                                  code == MG_F32 ? nullptr : dw_cast.data_ptr(), code, partial.data_ptr<float>(),
-                                  num_partials, ld, cols, stream);
+    }
+    float* const to_f32 = dw_f32.defined() ? dw_f32.data_ptr<float>() : nullptr;
+    void* const to_cast = need_weight_grad && code != MG_F32 ? dw_cast.data_ptr() : nullptr;
+    if (mg_rmsnorm_bwd_small_fits(rows, cols, code)) {   // few rows: one launch, no workspace
+        const int rc = mg_rmsnorm_bwd_small(grad_input.data_ptr(), to_f32, to_cast, grad_output.data_ptr(), input.data_ptr(),
+                                            weight.data_ptr(), inv_rms.data_ptr<float>(), rows, cols, code, stream);
+        TORCH_CHECK(rc == MG_OK, "RMSNorm backward failed (code ", rc, "): ", mg_last_error());
+        return {grad_input, dw_f32, dw_cast};
+    }
+    int64_t num_partials = 0, ld = 0;
+    TORCH_CHECK(mg_rmsnorm_bwd_workspace(rows, cols, code, &num_partials, &ld) == MG_OK,
+                "RMSNorm backward (workspace query) failed: ", mg_last_error());
+    auto partial = torch::empty({num_partials, ld}, f32);
+    int rc = mg_rmsnorm_bwd(grad_input.data_ptr(), partial.data_ptr<float>(), grad_output.data_ptr(),
+                            input.data_ptr(), weight.data_ptr(), inv_rms.data_ptr<float>(), rows, cols, code,
+                            num_partials, ld, stream);
+    TORCH_CHECK(rc == MG_OK, "RMSNorm backward failed (code ", rc, "): ", mg_last_error());
+    if (need_weight_grad) {
+        rc = mg_rmsnorm_dw_reduce(to_f32, to_cast, code, partial.data_ptr<float>(), num_partials, ld, cols, stream);
         TORCH_CHECK(rc == MG_OK, "RMSNorm backward (dW reduction) failed (code ", rc, "): ", mg_last_error());
     }
     return {grad_input, dw_f32, dw_cast};

@@ -121,13 +121,20 @@ def rmsnorm_backward_f32(grad_output: torch.Tensor, input: torch.Tensor, weight:
     dev = input.device
     with _lib.device_of(dev):
         stream = _lib.stream_ptr(dev)
-        n_part, ld = _bwd_workspace(lib, dev, rows, cols, code)
         grad_input = torch.empty_like(input)
-        partial = torch.empty((n_part, ld), dtype=torch.float32, device=dev)
         dw_f32 = dw_cast = None
         if need_weight_grad:
             dw_f32 = torch.empty((cols,), dtype=torch.float32, device=dev)
             dw_cast = dw_f32 if code == _lib.MG_F32 else torch.empty_like(weight)
+        if lib.mg_rmsnorm_bwd_small_fits(rows, cols, code):    # few rows: one launch, no workspace
+            rc = lib.mg_rmsnorm_bwd_small(grad_input.data_ptr(), None if dw_f32 is None else dw_f32.data_ptr(),
+                                          None if dw_cast is dw_f32 else dw_cast.data_ptr(), grad_output.data_ptr(),
+                                          input.data_ptr(), weight.data_ptr(), inv_rms.data_ptr(), rows, cols, code, stream)
+            if rc != 0:
+                _lib.check(rc, "RMSNorm backward")
+            return grad_input, dw_f32, dw_cast
+        n_part, ld = _bwd_workspace(lib, dev, rows, cols, code)
+        partial = torch.empty((n_part, ld), dtype=torch.float32, device=dev)
         rc = lib.mg_rmsnorm_bwd(grad_input.data_ptr(), partial.data_ptr(), grad_output.data_ptr(),
                                 input.data_ptr(), weight.data_ptr(), inv_rms.data_ptr(), rows, cols, code,
                                 n_part, ld, stream)

@@ -1,4 +1,4 @@
-"""The SwiGLU block as one operator (megagemm_hip_block.h): a decoding step through MegaGemmTriton
+"""The SwiGLU block as one operator (megagemm_hip_fused.h): a decoding step through MegaGemmTriton
 against the same formula in float64, at the sizes where the split over workgroups, waves and
 16-row tiles has edges, and the calls that have to keep going through the projections."""
 import pytest
