@@ -331,7 +331,8 @@ int mg_rmsnorm_fwd(void* y, float* inv_rms, const void* x, const void* w, int64_
     bool generic = opt_force_generic.load() != 0;
     if (!generic && !choose_fwd_lines(row_bytes, aligned(y, 8), &cfg))
         generic = !choose_fwd(row_bytes, &cfg) && !choose_streaming(row_bytes, &cfg);
-    const FwdArgs a = {y, inv_rms, x, w, (long)rows, (int)cols, eps, xcd_group_or(kXcdGroupStreaming)};
+    const FwdArgs a = {y, inv_rms, x, w, (long)rows, (int)cols, eps, xcd_group_or(kXcdGroupStreaming),
+                       keep_input((long)rows * row_bytes)};
     hipStream_t s = (hipStream_t)stream;
     hipError_t e = by_dtype(
         dtype, [&] { return launch_rmsnorm_fwd<float>(cfg, generic, a, s); },

@@ -37,7 +37,8 @@ template <int NW> struct Words { u32 v[NW]; };
 // Cache policy of a buffer access (the instruction's nt bit).  kStream marks data that is
 // touched once (activations and their gradients): measured on MI355X, non-temporal loads
 // stream about 8 % faster than default ones at sizes beyond the caches and non-temporal
-// stores about 20 % faster at tens of MiB.  kKeep is for what every row re-reads (weights).
+// stores about 20 % faster at tens of MiB.  kKeep is for what every row re-reads (weights), and for a
+// forward input small enough to be in the memory-side cache still when it is read again (keep_input).
 constexpr int kKeep = 0;
 constexpr int kStream = 2;
 

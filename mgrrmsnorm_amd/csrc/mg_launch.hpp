@@ -172,10 +172,22 @@ constexpr int narrow_default_tpr(long row_bytes, bool backward) {
     return nvec <= 32 ? 8 : (nvec <= 64 ? 16 : (nvec <= 128 && row_bytes % 128 == 0 ? 32 : 0));
 }
 
+// Whether the forward pass reads its input (`bytes` of it) with the default cache policy rather
+// than non-temporally.  The input is read again -- by the backward pass, and x by the residual
+// addition too -- and up to half of the 256 MiB memory-side cache it is then still there.
+// bf16, forward + backward on tensors never used before, default / non-temporal policy (us):
+// RMSNorm 4096 columns x 4096 rows (32 MiB) 32.3 / 34.3, 8192 rows 54.0 / 55.9, 16384 rows (128 MiB)
+// 99.3 / 101.2, 24576 rows (192 MiB) 169.8 / 163.1; 262144 x 80 39.8 / 42.9; SwiGLU 8192 x 2*4096
+// (128 MiB) 74.8 / 79.5, 8192 x 2*11008 (344 MiB) 249 / 220.  The same inputs in turn, 16384 x 4096:
+// 104.7 / 111.8.  Beyond half the cache the input pushes out lines that still have to be written back.
+constexpr long kKeepInputBytes = 128L << 20;
+constexpr bool keep_input(long bytes) { return bytes <= kKeepInputBytes; }
+
 struct FwdArgs {
     void* y; float* inv_rms; const void* x; const void* w;
     long rows; int cols; float eps;
     int xcd_group;  // see xcd_remap(); 0 = workgroup ids used as they come
+    bool keep_x;    // x may stay in the caches (see keep_input)
 };
 struct BwdArgs {
     void* dx; float* dw_part; int ld; const void* dy; const void* x; const void* w; const float* inv_rms;

@@ -25,7 +25,7 @@ hipError_t run(const FwdArgs& a, hipStream_t s) {
     const long grid = (a.rows + RPB - 1) / RPB;
     return launch(rmsnorm_fwd_rows<elem_t, VEC, TPR, ITEMS>, dim3((unsigned)grid), dim3(BLOCK), 0, s,
             (elem_t*)a.y, a.inv_rms, (const elem_t*)a.x, (const elem_t*)a.w, a.rows, a.cols, a.eps,
-        1.0f / (float)a.cols, a.xcd_group);
+        1.0f / (float)a.cols, a.xcd_group, a.keep_x);
 }
 
 template <int VEC, int TPR>
@@ -66,20 +66,26 @@ hipError_t lines_by_items(int items, const FwdArgs& a, hipStream_t s) {
     }
 }
 
-template <int TPR, int ITEMS, bool RAGGED>
-hipError_t run_narrow(const FwdArgs& a, hipStream_t s) {
+template <int TPR, int ITEMS, bool RAGGED, int X_POL>
+hipError_t run_narrow_as(const FwdArgs& a, hipStream_t s) {
     constexpr int RPB = 256 / TPR;
     const long grid = (a.rows + RPB - 1) / RPB;
-    return launch(rmsnorm_fwd_narrow<elem_t, TPR, ITEMS, RAGGED>, dim3((unsigned)grid), dim3(256), 0, s,
+    return launch(rmsnorm_fwd_narrow<elem_t, TPR, ITEMS, RAGGED, X_POL>, dim3((unsigned)grid), dim3(256), 0, s,
             (elem_t*)a.y, a.inv_rms, (const elem_t*)a.x, (const elem_t*)a.w, a.rows, a.cols, a.eps,
         1.0f / (float)a.cols, a.xcd_group);
 }
 
-template <int TPR, int G, bool RAGGED, int POL>
+template <int TPR, int ITEMS, bool RAGGED>
+hipError_t run_narrow(const FwdArgs& a, hipStream_t s) {
+    if (RAGGED || a.keep_x) return run_narrow_as<TPR, ITEMS, RAGGED, kKeep>(a, s);
+    return run_narrow_as<TPR, ITEMS, RAGGED, kNarrowPolicy<RAGGED>>(a, s);
+}
+
+template <int TPR, int G, bool RAGGED, int POL, int X_POL>
 hipError_t run_groups(const FwdArgs& a, hipStream_t s) {
     constexpr int RPB = 4 * G * (kWave / TPR);
     const long grid = (a.rows + RPB - 1) / RPB;
-    return launch(rmsnorm_fwd_groups<elem_t, TPR, G, RAGGED, POL>, dim3((unsigned)grid), dim3(256), 0, s,
+    return launch(rmsnorm_fwd_groups<elem_t, TPR, G, RAGGED, POL, X_POL>, dim3((unsigned)grid), dim3(256), 0, s,
             (elem_t*)a.y, a.inv_rms, (const elem_t*)a.x, (const elem_t*)a.w, a.rows, a.cols, a.eps,
         1.0f / (float)a.cols, a.xcd_group);
 }
@@ -89,7 +95,8 @@ hipError_t run_groups(const FwdArgs& a, hipStream_t s) {
 template <int TPR, int G>
 hipError_t groups_by_pitch(const FwdArgs& a, hipStream_t s) {
     const bool ragged = ((long)a.cols * (long)sizeof(elem_t)) % kVec != 0;
-    return ragged ? run_groups<TPR, G, true, kKeep>(a, s) : run_groups<TPR, G, false, kStream>(a, s);
+    if (ragged) return run_groups<TPR, G, true, kKeep, kKeep>(a, s);
+    return a.keep_x ? run_groups<TPR, G, false, kStream, kKeep>(a, s) : run_groups<TPR, G, false, kStream, kStream>(a, s);
 }
 
 template <int TPR>

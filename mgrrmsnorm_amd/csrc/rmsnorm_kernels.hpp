@@ -40,7 +40,8 @@ constexpr u32 kOutOfRange = 0xFFFFFFF0u;
 template <typename T, int VEC, int TPR, int ITEMS>
 __global__ void __launch_bounds__((TPR > 256 ? TPR : 256))
 rmsnorm_fwd_rows(T* __restrict__ y, float* __restrict__ inv_rms, const T* __restrict__ x,
-                 const T* __restrict__ w, long rows, int cols, float eps, float inv_cols, int xcd_group) {
+                 const T* __restrict__ w, long rows, int cols, float eps, float inv_cols, int xcd_group,
+                 bool keep_x) {
     constexpr int BLOCK = TPR > 256 ? TPR : 256;
     constexpr int RPB = BLOCK / TPR;
     constexpr int WPR = TPR / kWave;
@@ -63,7 +64,8 @@ rmsnorm_fwd_rows(T* __restrict__ y, float* __restrict__ inv_rms, const T* __rest
     Words<NW> xv[ITEMS];
     Words<NW> wv[ITEMS];
     u32 x_tail, w_tail;
-    request_row<NW, ITEMS, TPR, kStream>(xv, x_tail, rx, lir, tail);
+    if (keep_x) request_row<NW, ITEMS, TPR, kKeep>(xv, x_tail, rx, lir, tail);   // uniform over the launch
+    else request_row<NW, ITEMS, TPR, kStream>(xv, x_tail, rx, lir, tail);
     request_row<NW, ITEMS, TPR, kKeep>(wv, w_tail, rw, lir, tail);
     patch_row_tail<NW, ITEMS>(xv, x_tail, lir, tail);
     patch_row_tail<NW, ITEMS>(wv, w_tail, lir, tail);
@@ -254,7 +256,7 @@ __device__ __forceinline__ NarrowLane<TPR, ITEMS> narrow_lane(int sub, int lir, 
     return p;
 }
 
-template <typename T, int TPR, int ITEMS, bool RAGGED>
+template <typename T, int TPR, int ITEMS, bool RAGGED, int X_POL>
 __global__ void __launch_bounds__(256)
 rmsnorm_fwd_narrow(T* __restrict__ y, float* __restrict__ inv_rms, const T* __restrict__ x,
                    const T* __restrict__ w, long rows, int cols, float eps, float inv_cols, int xcd_group) {
@@ -280,12 +282,12 @@ rmsnorm_fwd_narrow(T* __restrict__ y, float* __restrict__ inv_rms, const T* __re
     Words<4> xv[ITEMS], wv[ITEMS];
     u32 x_tail = 0, w_tail = 0;
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) xv[i] = buf_load<4, POL>(rx, p.off[i]);
+    for (int i = 0; i < ITEMS; ++i) xv[i] = buf_load<4, X_POL>(rx, p.off[i]);
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) wv[i] = buf_load<4, kKeep>(rw, p.woff[i]);
     if constexpr (RAGGED) {
         if (p.owns_tail) {
-            x_tail = load_b16<POL>(rx, (u32)sub * row_bytes + p.tail_off);
+            x_tail = load_b16<X_POL>(rx, (u32)sub * row_bytes + p.tail_off);
             w_tail = load_b16<kKeep>(rw, p.tail_off);
         }
 #pragma unroll
@@ -322,14 +324,15 @@ rmsnorm_fwd_narrow(T* __restrict__ y, float* __restrict__ inv_rms, const T* __re
 // Every load or store instruction of a wave then covers one contiguous piece of memory (the
 // idle lanes of a row map to nothing), whatever the row pitch -- the layout for pitches that
 // are not multiples of 128 bytes, where the several-vectors-per-lane layout above writes
-// cache lines in pieces.  Ragged rows as above; POL = cache policy of the activations.
+// cache lines in pieces.  Ragged rows as above; POL = cache policy of the activations,
+// X_POL that of the forward input.
 template <int TPR>
 __device__ __forceinline__ float lanes_sum(float v) {
     if constexpr (TPR == kWave) return wave_sum(v);
     else return group_sum<TPR>(v);
 }
 
-template <typename T, int TPR, int G, bool RAGGED, int POL>
+template <typename T, int TPR, int G, bool RAGGED, int POL, int X_POL>
 __global__ void __launch_bounds__(256)
 rmsnorm_fwd_groups(T* __restrict__ y, float* __restrict__ inv_rms, const T* __restrict__ x,
                    const T* __restrict__ w, long rows, int cols, float eps, float inv_cols, int xcd_group) {
@@ -364,7 +367,7 @@ rmsnorm_fwd_groups(T* __restrict__ y, float* __restrict__ inv_rms, const T* __re
     Words<4> xv[G];
     u32 x_tail[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) xv[g] = buf_load<4, POL>(rx, off[g]);
+    for (int g = 0; g < G; ++g) xv[g] = buf_load<4, X_POL>(rx, off[g]);
     Words<4> wv = buf_load<4, kKeep>(rw, mine ? pos : kOutOfRange);
     if constexpr (RAGGED) {
         u32 w_tail = 0;
@@ -372,7 +375,7 @@ rmsnorm_fwd_groups(T* __restrict__ y, float* __restrict__ inv_rms, const T* __re
         for (int g = 0; g < G; ++g) x_tail[g] = 0;
         if (owns_tail) {
 #pragma unroll
-            for (int g = 0; g < G; ++g) x_tail[g] = load_b16<POL>(rx, (u32)(g * RPG + sub) * row_bytes + tail_off);
+            for (int g = 0; g < G; ++g) x_tail[g] = load_b16<X_POL>(rx, (u32)(g * RPG + sub) * row_bytes + tail_off);
             w_tail = load_b16<kKeep>(rw, tail_off);
         }
         trim_row_vector(wv, rem, w_tail);

@@ -104,8 +104,8 @@ hipError_t fwd_vec(int xg, void* h, const void* gu, long M, long H, hipStream_t 
         const long m = (M - r0) < rows_per_launch ? (M - r0) : rows_per_launch;
         const uint32_t total = (uint32_t)(m * nvr);
         const unsigned grid = (unsigned)((total + 256u * UNROLL - 1) / (256u * UNROLL));
-        hipError_t e = launch(swiglu_fwd_vec<T, UNROLL>, dim3(grid), dim3(256), 0, s,
-            (T*)h + r0 * H, (const T*)gu + r0 * 2 * H, total, fd, xg);
+        hipError_t e = launch(keep_input(2 * M * H * (long)sizeof(T)) ? swiglu_fwd_vec<T, UNROLL, true> : swiglu_fwd_vec<T, UNROLL, false>,
+                              dim3(grid), dim3(256), 0, s, (T*)h + r0 * H, (const T*)gu + r0 * 2 * H, total, fd, xg);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

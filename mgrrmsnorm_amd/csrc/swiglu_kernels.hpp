@@ -13,13 +13,21 @@ __device__ __forceinline__ Words<4> gload4(const void* p) {
     u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
     Words<4> o; o.v[0] = t.x; o.v[1] = t.y; o.v[2] = t.z; o.v[3] = t.w; return o;
 }
+// The same, with the default cache policy for an input that is read again (see keep_input).  A
+// template: the two sides of a run-time branch are one load to the compiler, without the hint.
+template <bool KEEP>
+__device__ __forceinline__ Words<4> gload4_input(const void* p) {
+    if constexpr (!KEEP) return gload4(p);
+    u32x4 t = *reinterpret_cast<const u32x4*>(p);
+    Words<4> o; o.v[0] = t.x; o.v[1] = t.y; o.v[2] = t.z; o.v[3] = t.w; return o;
+}
 __device__ __forceinline__ void gstore4(void* p, const Words<4>& w) {
     u32x4 t = {w.v[0], w.v[1], w.v[2], w.v[3]};
     __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
 }
 
 // total = M * nvr vectors, nvr = H * sizeof(T) / 16 vectors per half row.
-template <typename T, int UNROLL>
+template <typename T, int UNROLL, bool KEEP>
 __global__ void __launch_bounds__(256)
 swiglu_fwd_vec(T* __restrict__ h, const T* __restrict__ gu, uint32_t total, FastDiv nvr, int xcd_group) {
     constexpr int EPV = 16 / (int)sizeof(T);
@@ -37,8 +45,8 @@ swiglu_fwd_vec(T* __restrict__ h, const T* __restrict__ gu, uint32_t total, Fast
             const uint32_t row = fastdiv(v, nvr);
             const uint32_t col = v - row * nvr.d;
             const uint64_t gi = (uint64_t)row * (2ull * nvr.d) + col;
-            g[k] = gload4(in + gi * 16);
-            u[k] = gload4(in + (gi + nvr.d) * 16);
+            g[k] = gload4_input<KEEP>(in + gi * 16);
+            u[k] = gload4_input<KEEP>(in + (gi + nvr.d) * 16);
         }
     }
 #pragma unroll
