@@ -28,7 +28,7 @@ int mg_rmsnorm_bwd_small(void* dx, float* dw_f32, void* dw_cast, const void* dy,
                          const float* inv_rms, int64_t rows, int64_t cols, int dtype, void* stream);
 
 /* Most rows (tokens) the two entry points below take. */
-#define MG_BLOCK_MAX_TOKENS 16
+#define MG_BLOCK_MAX_TOKENS 64
 
 /*
  * h[t, n] = silu(g) * u with g = sum_k x[t, k] * w12[n, k], u = sum_k x[t, k] * w12[hidden + n, k]:

@@ -232,7 +232,7 @@ hipError_t launch_swiglu_bwd(int dtype, int mode, int unroll, int xcd_group, voi
 
 // Projections of the SwiGLU block with few rows (skinny_gemm.hpp): out [tokens, N], x [tokens, K],
 // w [N, K] or, paired, [2 N, K] with the activation folded in.  `cus` = compute units of the device.
-constexpr int kSkinnyMaxTokens = 16;
+constexpr int kSkinnyMaxTokens = 64;
 struct SkinnyArgs { void* out; const void* x; const void* w; int tokens, K, N, cus; };
 hipError_t launch_skinny_gemm(int dtype, bool paired, const SkinnyArgs& a, hipStream_t s);
 

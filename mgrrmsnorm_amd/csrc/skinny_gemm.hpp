@@ -1,5 +1,5 @@
 // The two projections of the SwiGLU block for a decoding step: out[t, n] = sum_k x[t, k] * w[n, k]
-// with at most 16 rows t, and the same with silu(gate) * up folded into the first of them.
+// with at most 64 rows t, and the same with silu(gate) * up folded into the first of them.
 #pragma once
 #include "mg_device.hpp"
 
@@ -32,12 +32,15 @@ __device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c, half_t
 //    the activations at once: 24.9 against 22.0 us).  Weights with the default cache policy: a
 //    fragment is half a 128-byte line of each row, and with non-temporal loads the other half is
 //    fetched again (25.6 us).
+//  - NT tiles of 16 tokens share every weight fragment.  A ring of three to six register buffers instead
+//    of two, with buffer loads, is slower (8 tokens 40.6 against 35.2 us for the block): it is not
+//    latency that the loop waits for, and lanes of absent tokens, free when masked off, cost with them.
 // 113 MB of gate and up weights in 22.0 us = 5.1 TB/s, 57 MB of the second projection (one tile per
 // workgroup) in 13.0 us = 4.4 TB/s at 8 tokens; the library products they replace took 28.0 + 24.3
 // and the activation between them 4.0.
-//   needs: 1 <= tokens <= 16; K a multiple of 8; 16-byte aligned x and w
+//   needs: 1 <= tokens <= 16 * NT; K a multiple of 8; 16-byte aligned x and w
 //   grid <= N workgroups of WAVES * 64 threads; PAIRED: w holds N gate rows, then N up rows
-template <typename T, int MB, int WAVES, int U, bool PAIRED>
+template <typename T, int MB, int NT, int WAVES, int U, bool PAIRED>
 __global__ void __launch_bounds__(WAVES * kWave)
 skinny_gemm(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ w, int tokens, int K, int N) {
     constexpr int TC = PAIRED ? 8 : 16;   // output columns per 16-row tile of weights
@@ -52,8 +55,13 @@ skinny_gemm(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ 
     const int lo = (int)((long)blockIdx.x * N / gridDim.x);
     const int hi = (int)((long)(blockIdx.x + 1) * N / gridDim.x);
 
-    const bool x_mine = r < tokens;
-    const T* xp = x + (x_mine ? (long)r * K : 0L) + g * 8;
+    const T* xp[NT];                      // rows r, r + 16, ... of the activations
+    bool x_mine[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        x_mine[t] = t * 16 + r < tokens;
+        xp[t] = x + (x_mine[t] ? (long)(t * 16 + r) * K : 0L) + g * 8;
+    }
     const int chunks = K / CHUNK;
     const int n = chunks > wave ? (chunks - wave + WAVES - 1) / WAVES : 0;   // chunks wave, wave + WAVES, ...
     const int skew = n > 0 ? (int)(blockIdx.x / 8u * 5u) % n : 0;            // / 8: the XCDs have an L2 each
@@ -68,11 +76,13 @@ skinny_gemm(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ 
             const long row = (w_mine[m] ? col : lo) + (PAIRED && r >= 8 ? (long)N : 0L);
             wp[m] = w + row * K + g * 8;
         }
-        f32x4 acc[MB];
+        f32x4 acc[MB][NT];
 #pragma unroll
-        for (int m = 0; m < MB; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-        struct Fragments { u32x4 w[MB][U]; u32x4 x[U]; };
+        struct Fragments { u32x4 w[MB][U]; u32x4 x[NT][U]; };
         auto load = [&](Fragments& f, int i) {
             int j = i + skew;
             if (j >= n) j -= n;
@@ -87,17 +97,22 @@ skinny_gemm(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ 
                 }
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) f.x[u] = u32x4{0, 0, 0, 0};
-            if (x_mine) {
+            for (int t = 0; t < NT; ++t) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) f.x[u] = *reinterpret_cast<const u32x4*>(xp + k + u * 32);
+                for (int u = 0; u < U; ++u) f.x[t][u] = u32x4{0, 0, 0, 0};
+                if (x_mine[t]) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) f.x[t][u] = *reinterpret_cast<const u32x4*>(xp[t] + k + u * 32);
+                }
             }
         };
         auto use = [&](const Fragments& f) {
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int m = 0; m < MB; ++m) acc[m] = mfma_16x16x32(f.w[m][u], f.x[u], acc[m], T());
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[m][t] = mfma_16x16x32(f.w[m][u], f.x[t][u], acc[m][t], T());
         };
         Fragments f0, f1;
         if (n > 0) load(f0, 0);
@@ -112,31 +127,40 @@ skinny_gemm(T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ 
         // the rest of K in steps of 32, the last one possibly short (zeros on both sides)
         for (int k = chunks * CHUNK + wave * 32; k < K; k += WAVES * 32) {
             const bool in = k + g * 8 < K;
-            u32x4 xv = {0, 0, 0, 0};
-            if (in && x_mine) xv = *reinterpret_cast<const u32x4*>(xp + k);
+            u32x4 xv[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                xv[t] = u32x4{0, 0, 0, 0};
+                if (in && x_mine[t]) xv[t] = *reinterpret_cast<const u32x4*>(xp[t] + k);
+            }
 #pragma unroll
             for (int m = 0; m < MB; ++m) {
                 u32x4 wv = {0, 0, 0, 0};
                 if (in && w_mine[m]) wv = *reinterpret_cast<const u32x4*>(wp[m] + k);
-                acc[m] = mfma_16x16x32(wv, xv, acc[m], T());
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[m][t] = mfma_16x16x32(wv, xv[t], acc[m][t], T());
             }
         }
 
-        if (n0 != lo) __syncthreads();    // the sums of the previous columns have been read
+        // the waves' sums, one tile of 16 tokens after the other through the same LDS
 #pragma unroll
-        for (int m = 0; m < MB; ++m) *reinterpret_cast<f32x4*>(&part[wave][m][r * PITCH + g * 4]) = acc[m];
-        __syncthreads();
-        for (int i = tid; i < 16 * COLS; i += WAVES * kWave) {
-            const int c = i % COLS, t = i / COLS;
-            const int at = t * PITCH + c % TC;
-            float s = 0.0f, up = 0.0f;
+        for (int tt = 0; tt < NT; ++tt) {
+            if (tt > 0 || n0 != lo) __syncthreads();   // the previous sums have been read
 #pragma unroll
-            for (int q = 0; q < WAVES; ++q) {
-                s += part[q][c / TC][at];
-                if constexpr (PAIRED) up += part[q][c / TC][at + 8];
+            for (int m = 0; m < MB; ++m) *reinterpret_cast<f32x4*>(&part[wave][m][r * PITCH + g * 4]) = acc[m][tt];
+            __syncthreads();
+            for (int i = tid; i < 16 * COLS; i += WAVES * kWave) {
+                const int c = i % COLS, t = i / COLS;
+                const int at = t * PITCH + c % TC;
+                float s = 0.0f, up = 0.0f;
+#pragma unroll
+                for (int q = 0; q < WAVES; ++q) {
+                    s += part[q][c / TC][at];
+                    if constexpr (PAIRED) up += part[q][c / TC][at + 8];
+                }
+                if constexpr (PAIRED) s = (s * fast_sigmoid(s)) * up;
+                if (tt * 16 + t < tokens && n0 + c < hi) Elem<T>::store1(out + (long)(tt * 16 + t) * N + n0 + c, s);
             }
-            if constexpr (PAIRED) s = (s * fast_sigmoid(s)) * up;
-            if (t < tokens && n0 + c < hi) Elem<T>::store1(out + (long)t * N + n0 + c, s);
         }
     }
 }

@@ -256,6 +256,18 @@ Tensor swiglu(const Tensor& w12_out, int64_t hidden_dim) {
     return swiglu_forward(fused.view({-1, 2 * hidden_dim}), hidden_dim).view(shape);
 }
 
+// Where the two kernels of mg_block_gate_up and mg_block_down are the faster way: every further tile of
+// 16 tokens has each workgroup read that much more of the activations (4096, hidden 6912: 16 tokens 38 us,
+// 64 74 us), while the library's products take about as long for 17 tokens as for 64.  These / projections
+// and activation, us of GPU time in a replayed graph, and of eager calls, which are bound by the host
+// with three operators (47 us): 24 tokens 44.4 / 46.5 and 44 / 48 (170 MB of weights), 38.5 / 41.2 and 38 / 47
+// (130 MB); 32 tokens 48.2 / 46.5 and 48 / 48 (170 MB), 42.5 / 38.4 and 42 / 48 (130 MB), 21.1 / 21.8 and 21 / 46
+// (44 MB); 64 tokens 32.0 / 24.5 and 32 / 46 (44 MB), 24.7 / 23.5 and 24 / 47 (24 MB), 18.4 / 19.9 and 18 / 47 (11 MB).
+bool block_in_two_kernels(int64_t tokens, int64_t weight_bytes) {
+    if (tokens < 1 || tokens > MG_BLOCK_MAX_TOKENS) return false;
+    return tokens <= 24 || weight_bytes <= ((tokens <= 32 ? 64LL : 24LL) << 20);
+}
+
 // w3(silu(gate) * up) with [gate | up] = w12(x) where nothing is to be differentiated and the call is
 // one of those mg_block_gate_up and mg_block_down take; an undefined tensor (None) where it is not, and
 // the caller then goes through the projections and the activation one by one.
@@ -267,7 +279,7 @@ Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     const int64_t d_model = w3.size(0), hidden = w3.size(1);
     if (d_model < 1 || x.size(-1) != d_model || w12.size(0) != 2 * hidden || w12.size(1) != d_model) return none;
     const int64_t tokens = x.numel() / d_model;
-    if (tokens < 1 || tokens > MG_BLOCK_MAX_TOKENS || d_model % 8 != 0 || hidden % 8 != 0 || hidden < 8) return none;
+    if (!block_in_two_kernels(tokens, 2 * 3 * d_model * hidden) || d_model % 8 != 0 || hidden % 8 != 0 || hidden < 8) return none;
     if (w12.scalar_type() != type || w3.scalar_type() != type || w12.device() != x.device() || w3.device() != x.device() ||
         !w12.is_contiguous() || !w3.is_contiguous())
         return none;

@@ -43,6 +43,7 @@ def _within(out, x, w12, w3, dtype):
     (5, 64, 9000),        # more columns per workgroup than four tiles hold
     (7, 17000, 128),      # the same in the second projection
     (9, 8192, 2048),      # two tiles of the second projection per workgroup
+    (17, 40, 24), (24, 4096, 6912), (32, 1152, 3072), (33, 264, 9000), (48, 520, 264), (49, 9000, 72), (64, 1024, 3072),   # tiles of tokens
 ])
 def test_decode_block_against_float64(tokens, d_model, hidden, dtype):
     x, w12, w3 = _case(tokens, d_model, hidden, dtype)
@@ -84,11 +85,13 @@ def test_module_takes_it_and_steps_aside():
     assert w12.grad is not None and w3.grad is not None
 
 
-@pytest.mark.parametrize("change", ["tokens", "dtype", "width", "alignment", "layout"])
+@pytest.mark.parametrize("change", ["tokens", "size", "dtype", "width", "alignment", "layout"])
 def test_calls_it_does_not_take(change):
     x, w12, w3 = _case(4, 64, 64, "bf16")
     if change == "tokens":
-        x = x.repeat(5, 1)
+        x = x.repeat(17, 1)
+    elif change == "size":
+        x, w12, w3 = _case(25, 4096, 6912, "bf16")   # the library is as fast from here on
     elif change == "dtype":
         x, w12, w3 = x.float(), w12.float(), w3.float()
     elif change == "width":
