@@ -51,6 +51,14 @@ void check_pair(const Tensor& input, const Tensor& weight) {
     TORCH_CHECK(weight.device() == input.device(), "input and weight must be on the same device");
 }
 
+// A contiguous tensor like a contiguous `t`: what empty_like gives, without the extra dispatch.
+Tensor empty_as(const Tensor& t) { return at::empty(t.sizes(), t.options()); }
+
+// `t` as a matrix of rows of `cols` elements: itself when it already is one (a view costs a dispatch,
+// and forward + backward of a layer would make four).
+Tensor as_rows(const Tensor& t, int64_t cols) { return t.dim() == 2 && t.size(1) == cols ? t : t.view({-1, cols}); }
+Tensor as_shape(const Tensor& t, at::IntArrayRef shape) { return t.sizes() == shape ? t : t.view(shape); }
+
 void* current_stream() { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 
 std::vector<Tensor> rmsnorm_forward(const Tensor& input, const Tensor& weight, double epsilon) {
@@ -61,8 +69,8 @@ std::vector<Tensor> rmsnorm_forward(const Tensor& input, const Tensor& weight, d
     TORCH_CHECK(cols >= 1, "hidden size must be >= 1");
     const int code = dtype_code(input.scalar_type());
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
-    auto output = torch::empty_like(input);
-    auto inv_rms = torch::empty({rows}, input.options().dtype(torch::kFloat32));
+    auto output = empty_as(input);
+    auto inv_rms = at::empty({rows}, input.options().dtype(torch::kFloat32));
     const int rc = mg_rmsnorm_fwd(output.data_ptr(), inv_rms.data_ptr<float>(), input.data_ptr(), weight.data_ptr(),
                                   rows, cols, (float)epsilon, code, current_stream());
     TORCH_CHECK(rc == MG_OK, "RMSNorm forward failed (code ", rc, "): ", mg_last_error());
@@ -86,12 +94,12 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor& grad_output, cons
     const int code = dtype_code(input.scalar_type());
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(input.device());
     const auto f32 = input.options().dtype(torch::kFloat32);
-    auto grad_input = torch::empty_like(input);
+    auto grad_input = empty_as(input);
     void* stream = current_stream();
     Tensor dw_f32, dw_cast;
     if (need_weight_grad) {
-        if (want_f32 || code == MG_F32) dw_f32 = torch::empty({cols}, f32);
-        dw_cast = code == MG_F32 ? dw_f32 : torch::empty_like(weight);   // weight dtype, as binding.cpp:90
+        if (want_f32 || code == MG_F32) dw_f32 = at::empty({cols}, f32);
+        dw_cast = code == MG_F32 ? dw_f32 : empty_as(weight);   // weight dtype, as binding.cpp:90
     }
     float* const to_f32 = dw_f32.defined() ? dw_f32.data_ptr<float>() : nullptr;
     void* const to_cast = need_weight_grad && code != MG_F32 ? dw_cast.data_ptr() : nullptr;
@@ -104,7 +112,7 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor& grad_output, cons
     int64_t num_partials = 0, ld = 0;
     TORCH_CHECK(mg_rmsnorm_bwd_workspace(rows, cols, code, &num_partials, &ld) == MG_OK,
                 "RMSNorm backward (workspace query) failed: ", mg_last_error());
-    auto partial = torch::empty({num_partials, ld}, f32);
+    auto partial = at::empty({num_partials, ld}, f32);
     int rc = mg_rmsnorm_bwd(grad_input.data_ptr(), partial.data_ptr<float>(), grad_output.data_ptr(),
                             input.data_ptr(), weight.data_ptr(), inv_rms.data_ptr<float>(), rows, cols, code,
                             num_partials, ld, stream);
@@ -135,7 +143,7 @@ Tensor swiglu_forward(const Tensor& gate_up, int64_t hidden_dim) {
     const int code = dtype_code(gate_up.scalar_type());
     const int64_t M = gate_up.size(0);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(gate_up.device());
-    auto out = torch::empty({M, hidden_dim}, gate_up.options());
+    auto out = at::empty({M, hidden_dim}, gate_up.options());
     const int rc = mg_swiglu_fwd(out.data_ptr(), gate_up.data_ptr(), M, hidden_dim, code, current_stream());
     TORCH_CHECK(rc == MG_OK, "SwiGLU forward failed (code ", rc, "): ", mg_last_error());
     return out;
@@ -152,7 +160,7 @@ Tensor swiglu_backward(const Tensor& grad_out, const Tensor& gate_up, int64_t hi
                 "grad_output must be [M, hidden_dim] with the dtype of the forward input");
     const int code = dtype_code(gate_up.scalar_type());
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(gate_up.device());
-    auto grad_in = torch::empty_like(gate_up);
+    auto grad_in = empty_as(gate_up);
     const int rc = mg_swiglu_bwd(grad_in.data_ptr(), grad_out.data_ptr(), gate_up.data_ptr(), M, hidden_dim, code,
                                  current_stream());
     TORCH_CHECK(rc == MG_OK, "SwiGLU backward failed (code ", rc, "): ", mg_last_error());
@@ -171,13 +179,11 @@ struct RMSNormNode : public torch::autograd::Function<RMSNormNode> {
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& input, const Tensor& weight,
                           double epsilon) {
         TORCH_CHECK(input.dim() >= 1, "RMSNorm needs at least one dimension");
-        const auto shape = input.sizes().vec();
-        auto x2d = input.contiguous().view({-1, shape.back()});
+        auto x2d = as_rows(input.contiguous(), input.size(-1));
         auto w = weight.contiguous();
         auto out = rmsnorm_forward(x2d, w, epsilon);
         ctx->save_for_backward({x2d, w, out[1]});
-        ctx->saved_data["shape"] = shape;
-        return out[0].view(shape);
+        return as_shape(out[0], input.sizes());
     }
 
     static torch::autograd::tensor_list backward(torch::autograd::AutogradContext* ctx,
@@ -186,10 +192,10 @@ struct RMSNormNode : public torch::autograd::Function<RMSNormNode> {
         torch::NoGradGuard no_grad;
         const auto saved = ctx->get_saved_variables();
         const Tensor &x2d = saved[0], &w = saved[1], &inv_rms = saved[2];
-        auto dy = grads[0].contiguous().view(x2d.sizes());
+        auto dy = as_shape(grads[0].contiguous(), x2d.sizes());
         if (dy.scalar_type() != x2d.scalar_type()) dy = dy.to(x2d.scalar_type());
         auto r = backward_impl(dy, x2d, w, inv_rms, ctx->needs_input_grad(1), false);
-        return {std::get<0>(r).view(ctx->saved_data["shape"].toIntVector()), std::get<2>(r), Tensor()};
+        return {as_shape(std::get<0>(r), grads[0].sizes()), std::get<2>(r), Tensor()};   // y has the shape of x
     }
 };
 
@@ -199,10 +205,9 @@ struct SwigluNode : public torch::autograd::Function<SwigluNode> {
                     2 * hidden_dim, ", got ", w12_out.dim() >= 1 ? w12_out.size(-1) : 0);
         auto fused = w12_out.contiguous();
         ctx->save_for_backward({fused});
-        ctx->saved_data["hidden_dim"] = hidden_dim;
         auto shape = fused.sizes().vec();
         shape.back() = hidden_dim;
-        return swiglu_forward(fused.view({-1, 2 * hidden_dim}), hidden_dim).view(shape);
+        return as_shape(swiglu_forward(as_rows(fused, 2 * hidden_dim), hidden_dim), shape);
     }
 
     static torch::autograd::tensor_list backward(torch::autograd::AutogradContext* ctx,
@@ -211,11 +216,11 @@ struct SwigluNode : public torch::autograd::Function<SwigluNode> {
         torch::NoGradGuard no_grad;
         const auto saved = ctx->get_saved_variables();
         const Tensor& fused = saved[0];
-        const int64_t hidden_dim = ctx->saved_data["hidden_dim"].toInt();
-        auto dh = grads[0].contiguous().view({-1, hidden_dim});
+        const int64_t hidden_dim = fused.size(-1) / 2;
+        auto dh = as_rows(grads[0].contiguous(), hidden_dim);
         if (dh.scalar_type() != fused.scalar_type()) dh = dh.to(fused.scalar_type());
-        auto grad = swiglu_backward(dh, fused.view({-1, 2 * hidden_dim}), hidden_dim);
-        return {grad.view(fused.sizes()), Tensor()};
+        auto grad = swiglu_backward(dh, as_rows(fused, 2 * hidden_dim), hidden_dim);
+        return {as_shape(grad, fused.sizes()), Tensor()};
     }
 };
 
@@ -238,7 +243,7 @@ Tensor rmsnorm(const Tensor& input, const Tensor& weight, double epsilon) {
     const int code = dtype_code(x.scalar_type());
     const int64_t rows = x.numel() / cols;
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    auto output = torch::empty_like(x);
+    auto output = empty_as(x);
     const int rc = mg_rmsnorm_fwd(output.data_ptr(), nullptr, x.data_ptr(), w.data_ptr(), rows, cols, (float)epsilon,
                                   code, current_stream());
     TORCH_CHECK(rc == MG_OK, "RMSNorm forward failed (code ", rc, "): ", mg_last_error());
@@ -253,7 +258,7 @@ Tensor swiglu(const Tensor& w12_out, int64_t hidden_dim) {
     auto fused = w12_out.contiguous();
     auto shape = fused.sizes().vec();
     shape.back() = hidden_dim;
-    return swiglu_forward(fused.view({-1, 2 * hidden_dim}), hidden_dim).view(shape);
+    return as_shape(swiglu_forward(as_rows(fused, 2 * hidden_dim), hidden_dim), shape);
 }
 
 // Where the two kernels of mg_block_gate_up and mg_block_down are the faster way: every further tile of
@@ -289,8 +294,8 @@ Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     if (off(xc) || off(w12) || off(w3)) return none;
     const int code = dtype_code(type);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    auto h = torch::empty({tokens, hidden}, xc.options());
-    auto out = torch::empty_like(xc);
+    auto h = at::empty({tokens, hidden}, xc.options());
+    auto out = empty_as(xc);
     void* stream = current_stream();
     int rc = mg_block_gate_up(h.data_ptr(), xc.data_ptr(), w12.data_ptr(), tokens, d_model, hidden, code, stream);
     if (rc == MG_OK) rc = mg_block_down(out.data_ptr(), h.data_ptr(), w3.data_ptr(), tokens, d_model, hidden, code, stream);
