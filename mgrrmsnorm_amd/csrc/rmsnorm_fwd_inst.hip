@@ -23,9 +23,10 @@ hipError_t run(const FwdArgs& a, hipStream_t s) {
     constexpr int BLOCK = TPR > 256 ? TPR : 256;
     constexpr int RPB = BLOCK / TPR;
     const long grid = (a.rows + RPB - 1) / RPB;
-    return launch(rmsnorm_fwd_rows<elem_t, VEC, TPR, ITEMS>, dim3((unsigned)grid), dim3(BLOCK), 0, s,
+    const auto kernel = a.keep_x ? rmsnorm_fwd_rows<elem_t, VEC, TPR, ITEMS, kKeep> : rmsnorm_fwd_rows<elem_t, VEC, TPR, ITEMS, kStream>;
+    return launch(kernel, dim3((unsigned)grid), dim3(BLOCK), 0, s,
             (elem_t*)a.y, a.inv_rms, (const elem_t*)a.x, (const elem_t*)a.w, a.rows, a.cols, a.eps,
-        1.0f / (float)a.cols, a.xcd_group, a.keep_x);
+        1.0f / (float)a.cols, a.xcd_group);
 }
 
 template <int VEC, int TPR>

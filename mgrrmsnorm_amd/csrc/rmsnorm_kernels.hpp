@@ -37,11 +37,10 @@ constexpr u32 kOutOfRange = 0xFFFFFFF0u;
 //   grid  = ceil(rows / RPB) workgroups, RPB = BLOCK / TPR rows per workgroup
 //   block = BLOCK = max(TPR, 256) threads
 // =================================================================================
-template <typename T, int VEC, int TPR, int ITEMS>
+template <typename T, int VEC, int TPR, int ITEMS, int X_POL>
 __global__ void __launch_bounds__((TPR > 256 ? TPR : 256))
 rmsnorm_fwd_rows(T* __restrict__ y, float* __restrict__ inv_rms, const T* __restrict__ x,
-                 const T* __restrict__ w, long rows, int cols, float eps, float inv_cols, int xcd_group,
-                 bool keep_x) {
+                 const T* __restrict__ w, long rows, int cols, float eps, float inv_cols, int xcd_group) {
     constexpr int BLOCK = TPR > 256 ? TPR : 256;
     constexpr int RPB = BLOCK / TPR;
     constexpr int WPR = TPR / kWave;
@@ -64,8 +63,7 @@ rmsnorm_fwd_rows(T* __restrict__ y, float* __restrict__ inv_rms, const T* __rest
     Words<NW> xv[ITEMS];
     Words<NW> wv[ITEMS];
     u32 x_tail, w_tail;
-    if (keep_x) request_row<NW, ITEMS, TPR, kKeep>(xv, x_tail, rx, lir, tail);   // uniform over the launch
-    else request_row<NW, ITEMS, TPR, kStream>(xv, x_tail, rx, lir, tail);
+    request_row<NW, ITEMS, TPR, X_POL>(xv, x_tail, rx, lir, tail);
     request_row<NW, ITEMS, TPR, kKeep>(wv, w_tail, rw, lir, tail);
     patch_row_tail<NW, ITEMS>(xv, x_tail, lir, tail);
     patch_row_tail<NW, ITEMS>(wv, w_tail, lir, tail);
