@@ -171,3 +171,29 @@ def test_binding_choice_can_be_forced_to_ctypes():
     assert outs[""].splitlines()[0] in ("extension", "ctypes")      # extension once it is built
     for text in outs.values():
         assert "must be a CUDA tensor" in text
+
+
+def test_rmsnorm_uses_the_weight_attribute(monkeypatch):
+    """`self.weight` decides, however it comes about: the parameter, a tensor set over it in the
+    instance (what tensor-swapping wrappers do), or a subclass that answers the attribute itself."""
+    from mgrrmsnorm_amd import RMSNorm, ops
+
+    monkeypatch.setattr(ops, "rmsnorm", lambda x, weight, eps: weight)
+    x = torch.zeros(2, 4)
+    norm = RMSNorm(4)
+    assert norm(x) is norm.weight
+    shadow = torch.full((4,), 3.0)
+    norm.__dict__["weight"] = shadow
+    assert norm(x) is shadow
+
+    class Scaled(RMSNorm):
+        def __getattribute__(self, name):
+            value = super().__getattribute__(name)
+            return value * 2 if name == "weight" else value
+
+    assert torch.equal(Scaled(4)(x), torch.full((4,), 2.0))
+
+    moved = RMSNorm(4)              # no parameter at all any more: a plain attribute in its place
+    del moved.weight
+    moved.weight = shadow
+    assert moved(x) is shadow
