@@ -187,8 +187,8 @@ def test_rmsnorm_uses_the_weight_attribute(monkeypatch):
     assert norm(x) is shadow
 
     class Scaled(RMSNorm):
-        def __getattribute__(self, name):
-            value = super().__getattribute__(name)
+        def __getattr__(self, name):      # where nn.Module answers for its parameters
+            value = super().__getattr__(name)
             return value * 2 if name == "weight" else value
 
     assert torch.equal(Scaled(4)(x), torch.full((4,), 2.0))
