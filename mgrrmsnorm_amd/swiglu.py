@@ -13,7 +13,8 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
-from torch.nn.modules import module as _module
+import torch.nn.functional as F
+from torch.nn.modules import linear as _linear, module as _module
 from torch.autograd.function import once_differentiable
 
 from . import ops
@@ -45,11 +46,33 @@ class MegaGemmFunction(torch.autograd.Function):
         return grad.view(fused.shape), None
 
 
+def _defined_in(module, function):
+    """`function` if it is `module`'s own, else None: replaced before this package was imported."""
+    code = getattr(function, "__code__", None)
+    return function if code is not None and code.co_filename == module.__file__ else None
+
+
+# What a projection's call consists of, to notice when any part of it has been replaced.
+_Linear = nn.Linear
+_LINEAR_FORWARD = _defined_in(_linear, nn.Linear.forward)
+_MODULE_CALL = _defined_in(_module, nn.Module.__call__)
+_CALL_IMPL = _defined_in(_module, nn.Module._call_impl)
+_SWIGLU = _defined_in(ops, ops.swiglu)
+_SET_ON_AN_INSTANCE = frozenset(("forward", "weight", "bias", "_compiled_call_impl", "_call_impl", "_wrapped_call_impl"))
+
+
+def _calls_replaced():
+    """nn.Linear, the calling of modules, the linear operator or the activation is not the original:
+    its replacement has to be called in a decoding step as everywhere else."""
+    return (_Linear.forward is not _LINEAR_FORWARD or _Linear.__call__ is not _MODULE_CALL
+            or _Linear._call_impl is not _CALL_IMPL or F.linear is not torch._C._nn.linear or ops.swiglu is not _SWIGLU)
+
+
 def _plain_weight(linear):
     """The weight of a projection that is exactly `x @ weight.T`: a bias-free nn.Linear that nobody
-    has hooked, replaced, parametrised or wrapped; else None."""
-    if (type(linear) is not nn.Linear or linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
-            or linear._backward_pre_hooks or "forward" in linear.__dict__):
+    has hooked, replaced, parametrised, compiled or wrapped; else None."""
+    if (type(linear) is not _Linear or linear._forward_hooks or linear._forward_pre_hooks or linear._backward_hooks
+            or linear._backward_pre_hooks or not _SET_ON_AN_INSTANCE.isdisjoint(linear.__dict__)):
         return None
     parameters = linear._parameters
     weight = parameters.get("weight")
@@ -87,9 +110,9 @@ class MegaGemmTriton(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # a decoding step: projections and activation in two kernels that read the weights once,
         # while the projections are the plain ones this module made
-        if type(x) is torch.Tensor and not _calls_observed():
-            w12, w3 = _plain_weight(self._modules.get("w12")), _plain_weight(self._modules.get("w3"))
-            if w12 is not None and w3 is not None and w3.size(-1) == self.hidden:
+        if type(x) is torch.Tensor and not _calls_observed() and not _calls_replaced():
+            w12, w3 = _plain_weight(self.w12), _plain_weight(self.w3)
+            if w12 is not None and w3 is not None and w3.dim() == 2 and w3.size(1) == self.hidden:
                 out = ops.swiglu_block(x, w12, w3)
                 if out is not None:
                     return out
