@@ -80,10 +80,10 @@ def _plain_weight(linear):
 
 
 def _calls_observed():
-    """Something wants to see the projections as torch operations: autocast, a dispatch or function
-    mode, the compiler, or a global module hook."""
-    return (torch.is_autocast_enabled() or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._len_torch_function_stack() > 0 or torch.compiler.is_compiling()
+    """Something wants to see the projections as torch operations: the compiler (asked first, because it
+    cannot trace the other questions), autocast, a dispatch or function mode, or a global module hook."""
+    return (torch.compiler.is_compiling() or torch.is_autocast_enabled() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0
             or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
             or _module._global_backward_pre_hooks)
 

@@ -130,3 +130,15 @@ def test_parameters_swapped_for_one_call(handed_over):
     values = {name: p.detach() * 2 for name, p in m.named_parameters()}
     seen = handed_over(lambda x: torch.func.functional_call(m, values, (x,)))
     assert seen is None
+
+
+def test_the_block_compiles_as_one_graph(monkeypatch):
+    """With an activation that can be traced, the module is one graph: the question whether a
+    compiler is looking comes before anything that the compiler itself cannot trace."""
+    monkeypatch.setattr(ops, "swiglu", lambda x, hidden: F.silu(x[..., :hidden]) * x[..., hidden:])
+    m = _module()
+    x = torch.randn(2, 16)
+    torch._dynamo.reset()
+    with torch.no_grad():
+        compiled = torch.compile(m, backend="eager", fullgraph=True)
+        assert torch.equal(compiled(x), m(x))
