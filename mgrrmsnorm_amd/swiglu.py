@@ -81,9 +81,9 @@ def _plain_weight(linear):
 
 def _calls_observed():
     """Something wants to see the projections as torch operations: the compiler (asked first, because it
-    cannot trace the other questions), autocast, a dispatch or function mode, or a global module hook."""
-    return (torch.compiler.is_compiling() or torch.is_autocast_enabled() or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._len_torch_function_stack() > 0
+    cannot trace the other questions), a trace, autocast, a dispatch or function mode, or a global module hook."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled()
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
             or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
             or _module._global_backward_pre_hooks)
 

@@ -142,3 +142,9 @@ def test_the_block_compiles_as_one_graph(monkeypatch):
     with torch.no_grad():
         compiled = torch.compile(m, backend="eager", fullgraph=True)
         assert torch.equal(compiled(x), m(x))
+
+
+def test_a_trace_records_the_projections(handed_over):
+    m = _module()
+    assert handed_over(lambda x: torch.jit.trace(m, x, check_trace=False)) is None
+    assert handed_over(m) is not None
