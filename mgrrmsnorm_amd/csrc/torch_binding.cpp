@@ -281,6 +281,10 @@ Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     const auto type = x.scalar_type();
     if (!x.is_cuda() || (type != at::kHalf && type != at::kBFloat16) || x.dim() < 1 || w12.dim() != 2 || w3.dim() != 2)
         return none;
+    // Sparse coordinate tensors are for the products (weights of that kind are not contiguous, below).
+    // Compressed ones raise where they are asked whether they are contiguous, and should: torch's
+    // product of 16-bit ones ends the process on ROCm 7 instead of raising.
+    if (x.is_sparse()) return none;
     const int64_t d_model = w3.size(0), hidden = w3.size(1);
     if (d_model < 1 || x.size(-1) != d_model || w12.size(0) != 2 * hidden || w12.size(1) != d_model) return none;
     const int64_t tokens = x.numel() / d_model;

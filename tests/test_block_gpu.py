@@ -101,3 +101,16 @@ def test_calls_it_does_not_take(change):
     else:
         w12 = w12.t().contiguous().t()
     assert ops.swiglu_block(x, w12, w3) is None
+
+
+@pytest.mark.parametrize("operand", [0, 1, 2])
+def test_sparse_operands(operand):
+    """Coordinate tensors are left to the projections; compressed ones raise here.  Neither is taken on
+    to torch's products: those of 16-bit compressed weights end the process instead of raising."""
+    operands = list(_case(4, 64, 64, "bf16"))
+    dense = operands[operand]
+    operands[operand] = dense.to_sparse()
+    assert ops.swiglu_block(*operands) is None
+    operands[operand] = dense.to_sparse_csr()
+    with pytest.raises(RuntimeError, match="contiguous"):
+        ops.swiglu_block(*operands)
