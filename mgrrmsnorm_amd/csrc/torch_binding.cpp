@@ -18,6 +18,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
 #include <tuple>
 #include <vector>
 
@@ -261,16 +262,25 @@ Tensor swiglu(const Tensor& w12_out, int64_t hidden_dim) {
     return as_shape(swiglu_forward(as_rows(fused, 2 * hidden_dim), hidden_dim), shape);
 }
 
-// Where the two kernels of mg_block_gate_up and mg_block_down are the faster way: every further tile of
-// 16 tokens has each workgroup read that much more of the activations (4096, hidden 6912: 16 tokens 38 us,
-// 64 74 us), while the library's products take about as long for 17 tokens as for 64.  These / projections
-// and activation, us of GPU time in a replayed graph, and of eager calls, which are bound by the host
-// with three operators (47 us): 24 tokens 44.4 / 46.5 and 44 / 48 (170 MB of weights), 38.5 / 41.2 and 38 / 47
-// (130 MB); 32 tokens 48.2 / 46.5 and 48 / 48 (170 MB), 42.5 / 38.4 and 42 / 48 (130 MB), 21.1 / 21.8 and 21 / 46
-// (44 MB); 64 tokens 32.0 / 24.5 and 32 / 46 (44 MB), 24.7 / 23.5 and 24 / 47 (24 MB), 18.4 / 19.9 and 18 / 47 (11 MB).
-bool block_in_two_kernels(int64_t tokens, int64_t weight_bytes) {
+// Where the two kernels of mg_block_gate_up and mg_block_down take no more GPU time than the projections
+// and the activation between them; eager calls, which three operators keep at 47 us on the host, then win
+// by more.  Each further tile of 16 tokens has every workgroup read that much more of the activations, and so
+// does each pass that a wide projection takes, while the library's products take about as long for 17
+// tokens as for 64.  GPU time in a replayed graph, us, these / projections and activation; d_model x hidden,
+// MiB of weights; weights read from memory, and the same three layers in turn (what fits the cache):
+//   16 tokens, every size measured (1 MiB to 2.3 GiB): 2048 x 3584 16.6 / 29.1, 4096 x 6912 38.8 / 54.6, 8192 x 28672
+//     253 / 267, 12288 x 32768 412 / 428; the one loss is 8192 x 1024 with cached weights (21.1 / 23.7, 21.9 / 20.3);
+//   32 tokens: 2048 x 3584 (42) 22.5 / 26.8, 22.2 / 22.9; 1280 x 5120 (38) 24.0 / 27.2, 24.1 / 24.3; beyond, 1792 x 4864
+//     (50) 26.5 / 28.7, 26.2 / 25.5, 3072 x 8192 (144) 48.1 / 41.3 and at 17 tokens already 41.0 / 39.8, 5120 x
+//     13824 (405) 108 / 92; wider than four to one, 1024 x 8192 (48) 32.2 / 30.3;
+//   64 tokens: 768 x 2048 (9) 18.9 / 23.3, 19.3 / 19.3; 1024 x 1360 (8) 15.5 / 24.1, 15.7 / 20.1; beyond, 1024 x 2304 (14)
+//     fp16 21.9 / 22.5, 22.6 / 19.0, 1536 x 2560 (22) 25.6 / 27.0, 25.8 / 22.3; wider than three to one, 576 x 2304
+//     (8) fp16 19.6 / 19.1, 19.9 / 16.4.
+bool block_in_two_kernels(int64_t tokens, int64_t d_model, int64_t hidden) {
     if (tokens < 1 || tokens > MG_BLOCK_MAX_TOKENS) return false;
-    return tokens <= 24 || weight_bytes <= ((tokens <= 32 ? 64LL : 24LL) << 20);
+    if (tokens <= 16) return true;
+    const int64_t wide = std::max(d_model, hidden), narrow = std::min(d_model, hidden), bytes = 2 * 3 * d_model * hidden;
+    return tokens <= 32 ? bytes <= (42LL << 20) && wide <= 4 * narrow : bytes <= (9LL << 20) && wide <= 3 * narrow;
 }
 
 // w3(silu(gate) * up) with [gate | up] = w12(x) where nothing is to be differentiated and the call is
@@ -288,7 +298,7 @@ Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     const int64_t d_model = w3.size(0), hidden = w3.size(1);
     if (d_model < 1 || x.size(-1) != d_model || w12.size(0) != 2 * hidden || w12.size(1) != d_model) return none;
     const int64_t tokens = x.numel() / d_model;
-    if (!block_in_two_kernels(tokens, 2 * 3 * d_model * hidden) || d_model % 8 != 0 || hidden % 8 != 0 || hidden < 8) return none;
+    if (!block_in_two_kernels(tokens, d_model, hidden) || d_model % 8 != 0 || hidden % 8 != 0 || hidden < 8) return none;
     if (w12.scalar_type() != type || w3.scalar_type() != type || w12.device() != x.device() || w3.device() != x.device() ||
         !w12.is_contiguous() || !w3.is_contiguous())
         return none;

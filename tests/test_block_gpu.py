@@ -4,6 +4,7 @@ against the same formula in float64, at the sizes where the split over workgroup
 import pytest
 import torch
 
+import gpu_util as U
 from mgrrmsnorm_amd import MegaGemmTriton, ops
 
 pytestmark = pytest.mark.gpu
@@ -36,6 +37,21 @@ def _within(out, x, w12, w3, dtype):
     assert worst <= 0.0, f"beyond the error bound by {worst}"
 
 
+def _two_kernels(x, w12, w3, dtype):
+    """The block through the C entry points, which take up to 64 tokens of any size."""
+    tokens, d_model, hidden = x.size(0), x.size(1), w3.size(1)
+    h, out = torch.empty(tokens, hidden, device="cuda", dtype=x.dtype), torch.empty_like(x)
+    U.check(U.lib().mg_block_gate_up(h.data_ptr(), x.data_ptr(), w12.data_ptr(), tokens, d_model, hidden, U.CODES[dtype], U.stream()))
+    U.check(U.lib().mg_block_down(out.data_ptr(), h.data_ptr(), w3.data_ptr(), tokens, d_model, hidden, U.CODES[dtype], U.stream()))
+    return out
+
+
+def _taken(tokens, d_model, hidden):
+    """The operator's rule: tokens, MiB of weights, and how far the two widths lie apart."""
+    mib, apart = 6 * d_model * hidden / 2 ** 20, max(d_model, hidden) / min(d_model, hidden)
+    return tokens <= 16 or (tokens <= 32 and mib <= 42 and apart <= 4) or (tokens <= 64 and mib <= 9 and apart <= 3)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("tokens,d_model,hidden", [
     (1, 8, 8), (3, 40, 24), (16, 64, 72), (15, 72, 1000), (2, 520, 264), (16, 1152, 3072),
@@ -47,10 +63,26 @@ def _within(out, x, w12, w3, dtype):
 ])
 def test_decode_block_against_float64(tokens, d_model, hidden, dtype):
     x, w12, w3 = _case(tokens, d_model, hidden, dtype)
-    out = ops.swiglu_block(x, w12, w3)
-    assert out is not None and out.shape == x.shape and out.dtype == x.dtype
+    out = _two_kernels(x, w12, w3, dtype)
     _within(out, x, w12, w3, dtype)
-    assert torch.equal(out, ops.swiglu_block(x, w12, w3))   # fixed summation order
+    assert torch.equal(out, _two_kernels(x, w12, w3, dtype))   # fixed summation order
+    block = ops.swiglu_block(x, w12, w3)
+    assert (block is not None) == _taken(tokens, d_model, hidden)
+    if block is not None:
+        assert block.shape == x.shape and block.dtype == x.dtype and torch.equal(block, out)
+
+
+@pytest.mark.parametrize("tokens,d_model,hidden,taken", [
+    (16, 8192, 14336, True), (17, 2048, 3584, True), (17, 2048, 3592, False), (32, 2048, 3584, True),
+    (24, 4096, 6912, False), (17, 1024, 4096, True), (17, 1024, 4104, False), (17, 4104, 1024, False),
+    (33, 768, 2048, True), (33, 768, 2056, False), (64, 768, 2048, True), (64, 1024, 3072, False),
+    (33, 512, 1536, True), (33, 512, 1544, False), (64, 1544, 512, False),
+])
+def test_where_the_block_takes_the_two_kernels(tokens, d_model, hidden, taken):
+    """Beyond these lines the library's products are at least as fast on the GPU (see block_in_two_kernels)."""
+    assert _taken(tokens, d_model, hidden) == taken
+    x, w12, w3 = (torch.zeros(s, device="cuda", dtype=torch.bfloat16) for s in ((tokens, d_model), (2 * hidden, d_model), (d_model, hidden)))
+    assert (ops.swiglu_block(x, w12, w3) is not None) == taken
 
 
 def test_rows_do_not_depend_on_each_other():
