@@ -283,6 +283,15 @@ bool block_in_two_kernels(int64_t tokens, int64_t d_model, int64_t hidden) {
     return tokens <= 32 ? bytes <= (42LL << 20) && wide <= 4 * narrow : bytes <= (9LL << 20) && wide <= 3 * narrow;
 }
 
+// Whether a block of this hidden width may take `x` to swiglu_block at all, from x alone: asked first, so that
+// the calls it is not for go on without the questions about modes and projections (2 us of 48).
+bool swiglu_block_fits(const Tensor& x, int64_t hidden) {
+    const auto type = x.scalar_type();
+    if ((type != at::kHalf && type != at::kBFloat16) || !x.is_cuda() || x.dim() < 1 || x.size(-1) < 1) return false;
+    if (x.requires_grad() && torch::GradMode::is_enabled()) return false;
+    return block_in_two_kernels(x.numel() / x.size(-1), x.size(-1), hidden);
+}
+
 // w3(silu(gate) * up) with [gate | up] = w12(x) where nothing is to be differentiated and the call is
 // one of those mg_block_gate_up and mg_block_down take; an undefined tensor (None) where it is not, and
 // the caller then goes through the projections and the activation one by one.
@@ -339,6 +348,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("epsilon") = 1e-5);
     m.def("swiglu_block", &swiglu_block, "the whole SwiGLU block for a few rows, not differentiable; None where it does not apply",
           py::arg("x"), py::arg("w12"), py::arg("w3"));
+    m.def("swiglu_block_fits", &swiglu_block_fits, "whether the size and type of x are for swiglu_block", py::arg("x"),
+          py::arg("hidden_dim"));
     m.def("swiglu", &swiglu, "differentiable silu(gate) * up over the last dimension", py::arg("w12_out"),
           py::arg("hidden_dim"));
 }

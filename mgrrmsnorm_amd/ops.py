@@ -144,6 +144,12 @@ def swiglu(w12_out: torch.Tensor, hidden_dim: int) -> torch.Tensor:
     return swiglu_forward(fused.view(-1, 2 * hidden_dim), hidden_dim).view(*fused.shape[:-1], hidden_dim)
 
 
+def swiglu_block_fits(x: torch.Tensor, hidden_dim: int) -> bool:
+    """Whether `x` alone -- its size, type and device -- could be for `swiglu_block`."""
+    ext = _extension()
+    return ext is not None and ext.swiglu_block_fits(x, hidden_dim)
+
+
 def swiglu_block(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
     """w3(silu(gate) * up) with [gate | up] = w12(x), for the few rows of a decoding step and with
     nothing to differentiate; None when the call is not of that kind (or the extension is not

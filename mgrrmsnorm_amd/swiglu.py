@@ -80,9 +80,9 @@ def _plain_weight(linear):
 
 
 def _calls_observed():
-    """Something wants to see the projections as torch operations: the compiler (asked first, because it
-    cannot trace the other questions), a trace, autocast, a dispatch or function mode, or a global module hook."""
-    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_autocast_enabled()
+    """Something wants to see the projections as torch operations: a trace, autocast, a dispatch or function
+    mode, or a global module hook."""
+    return (torch.jit.is_tracing() or torch.is_autocast_enabled()
             or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
             or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
             or _module._global_backward_pre_hooks)
@@ -109,8 +109,10 @@ class MegaGemmTriton(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # a decoding step: projections and activation in two kernels that read the weights once,
-        # while the projections are the plain ones this module made
-        if type(x) is torch.Tensor and not _calls_observed() and not _calls_replaced():
+        # while the projections are the plain ones this module made (the compiler is asked about
+        # first, because it cannot trace the other questions; then the size, which most calls end at)
+        if (not torch.compiler.is_compiling() and type(x) is torch.Tensor and ops.swiglu_block_fits(x, self.hidden)
+                and not _calls_observed() and not _calls_replaced()):
             w12, w3 = _plain_weight(self.w12), _plain_weight(self.w3)
             if w12 is not None and w3 is not None and w3.dim() == 2 and w3.size(1) == self.hidden:
                 out = ops.swiglu_block(x, w12, w3)

@@ -14,6 +14,7 @@ def handed_over(monkeypatch):
     """Calls the module and returns the (w12, w3) it handed to ops.swiglu_block, or None if it went
     through the projections."""
     calls = []
+    monkeypatch.setattr(ops, "swiglu_block_fits", lambda x, hidden: True, raising=False)
     monkeypatch.setattr(ops, "swiglu_block", lambda x, w12, w3: calls.append((w12, w3)))
 
     def call(module, x=None):
@@ -142,6 +143,17 @@ def test_the_block_compiles_as_one_graph(monkeypatch):
     with torch.no_grad():
         compiled = torch.compile(m, backend="eager", fullgraph=True)
         assert torch.equal(compiled(x), m(x))
+
+
+def test_calls_of_other_sizes_end_at_the_size(monkeypatch):
+    """A call that is not for the two kernels is not held up by questions about modes and projections."""
+    from mgrrmsnorm_amd import swiglu
+
+    asked = []
+    monkeypatch.setattr(swiglu, "_calls_observed", lambda: asked.append(1))
+    with pytest.raises(RuntimeError):           # a tensor of the CPU
+        _module()(torch.zeros(65, 16))
+    assert not asked
 
 
 def test_a_trace_records_the_projections(handed_over):
