@@ -180,7 +180,9 @@ struct RMSNormNode : public torch::autograd::Function<RMSNormNode> {
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& input, const Tensor& weight,
                           double epsilon) {
         TORCH_CHECK(input.dim() >= 1, "RMSNorm needs at least one dimension");
-        auto x2d = as_rows(input.contiguous(), input.size(-1));
+        // a view even of what is a matrix already: it keeps the data it was made of when a caller gives
+        // `input` other data (`x.data = ...`) before the backward pass
+        auto x2d = input.contiguous().view({-1, input.size(-1)});
         auto w = weight.contiguous();
         auto out = rmsnorm_forward(x2d, w, epsilon);
         ctx->save_for_backward({x2d, w, out[1]});

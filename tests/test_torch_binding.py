@@ -147,6 +147,29 @@ def test_cpp_autograd_nodes_match_python_functions(binding, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(40, 64), (2, 20, 64)])
+def test_input_given_other_data_before_the_backward_pass(binding, shape):
+    """`x.data = ...` after the forward pass leaves the saved input as it was, in every shape and as
+    with the Python function."""
+    from mgrrmsnorm_amd import RMSNormFunction
+
+    first, other, dy = (torch.randn(shape, device="cuda") for _ in range(3))
+    w = torch.randn(64, device="cuda")
+
+    def grads(fn, swap):
+        x, wa = first.clone().requires_grad_(True), w.clone().requires_grad_(True)
+        y = fn(x, wa)
+        if swap:
+            x.data = other
+        y.backward(dy)
+        return x.grad, wa.grad
+
+    for fn in (lambda a, b: binding.rmsnorm(a, b, 1e-6), lambda a, b: RMSNormFunction.apply(a, b, 1e-6)):
+        for a, b in zip(grads(fn, True), grads(fn, False)):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
 def test_cpp_autograd_nodes_refuse_a_second_derivative(binding):
     x = torch.randn((4, 64), device="cuda", requires_grad=True)
     w = torch.ones(64, device="cuda", requires_grad=True)
