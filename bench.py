@@ -10,8 +10,9 @@ RMSNorm forward + backward (three launches: forward, backward pass 1, dW reducti
 algorithmic bytes per step / wall time per step over exactly K steps (the median of five
 such readings; all five are in `readings_us_per_step`).
 
-Buffers rotate over several independent sets whose total size exceeds the 256 MB
-Infinity Cache, so consecutive steps do not find their inputs cached.
+Buffers rotate over independent sets: so many that the forward inputs alone, which the kernels
+leave in the 256 MiB Infinity Cache where they are small, exceed it four times.  No step finds its
+inputs cached by an earlier one; its backward pass may find what its own forward pass left.
 
 Everything runs on the default stream while it is the process's only stream; the HIP-graph
 reading of the default `--launch best` comes last, because capturing a graph creates a stream
@@ -42,6 +43,14 @@ ESIZE = {"fp32": 4, "fp16": 2, "bf16": 2}
 CODE = {"fp32": 0, "fp16": 1, "bf16": 2}
 TORCH = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}
 INFINITY_CACHE_BYTES = 256 << 20
+KEPT_INPUT_BYTES = 128 << 20     # forward inputs of up to this size are read so that they may stay in that cache
+
+
+def buffer_sets(input_bytes, set_bytes):
+    """How many sets of buffers exceed the cache four times: counted by the forward input where that may
+    stay in the cache (everything else is read and written past it), else by all tensors of a set."""
+    counted = input_bytes if input_bytes <= KEPT_INPUT_BYTES else set_bytes
+    return max(2, -(-4 * INFINITY_CACHE_BYTES // counted))
 
 
 def log(*a):
@@ -59,8 +68,7 @@ class RmsNormWorkload:
         self.fwd_bytes = 2 * rows * cols * e + cols * e
         self.bwd_bytes = 3 * rows * cols * e + cols * e + 4 * cols
         self.step_bytes = self.fwd_bytes + (self.bwd_bytes if backward else 0)
-        per_set = (4 if backward else 2) * rows * cols * e
-        self.nsets = nsets if nsets > 0 else max(2, -(-4 * INFINITY_CACHE_BYTES // per_set))
+        self.nsets = nsets if nsets > 0 else buffer_sets(rows * cols * e, (4 if backward else 2) * rows * cols * e)
         td = TORCH[dtype]
         g = torch.Generator(device="cuda").manual_seed(seed)
         self.w = (1 + 0.02 * torch.randn(cols, generator=g, device="cuda")).to(td)
@@ -145,8 +153,7 @@ class SwigluWorkload:
         e = ESIZE[dtype]
         self.fwd_bytes, self.bwd_bytes = 3 * M * H * e, 5 * M * H * e
         self.step_bytes = self.fwd_bytes + self.bwd_bytes
-        per_set = 6 * M * H * e
-        self.nsets = nsets if nsets > 0 else max(2, -(-4 * INFINITY_CACHE_BYTES // per_set))
+        self.nsets = nsets if nsets > 0 else buffer_sets(2 * M * H * e, 6 * M * H * e)
         td = TORCH[dtype]
         g = torch.Generator(device="cuda").manual_seed(seed)
         self.sets = []
@@ -364,7 +371,7 @@ def time_module_surface(rows, cols, dtype, iters=300, repeats=6):
     td = TORCH[dtype]
     e = ESIZE[dtype]
     norm = megagemm.RMSNorm(cols, 1e-6).cuda().to(td)
-    nsets = max(2, -(-4 * INFINITY_CACHE_BYTES // (4 * rows * cols * e)))
+    nsets = buffer_sets(rows * cols * e, 4 * rows * cols * e)
     g = torch.Generator(device="cuda").manual_seed(7)
     xs = [torch.randn((rows, cols), generator=g, device="cuda").to(td).requires_grad_(True) for _ in range(nsets)]
     dys = [torch.randn((rows, cols), generator=g, device="cuda").to(td) for _ in range(nsets)]
@@ -659,8 +666,9 @@ def main():
                          "'second-stream' enqueues them one by one with the dW reduction on a second stream "
                          "(measured on request only: it is slower)")
     ap.add_argument("--buffer-sets", type=int, default=0,
-                    help="input/output buffer sets the steps rotate over; 0 = enough to exceed four times the "
-                         "256 MiB Infinity Cache (the reported configuration), 1 = everything stays cache resident")
+                    help="input/output buffer sets the steps rotate over; 0 = so many that the forward inputs alone exceed "
+                         "the 256 MiB Infinity Cache four times (the reported configuration), 1 = everything stays "
+                         "cache resident")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--option", action="append", default=[], metavar="KEY=VALUE",
                     help="tuning override passed to mg_set_option before anything is timed (repeatable)")

@@ -69,6 +69,21 @@ def test_algorithmic_bytes_are_reads_plus_writes_of_every_tensor():
     assert bench.HBM_PEAK_GBPS == 8000.0
 
 
+def test_buffer_sets_count_what_may_stay_in_the_cache():
+    """Forward inputs of up to 128 MiB may stay in the 256 MiB cache, so they alone have to exceed it
+    four times; the kernels' line and the benchmark's are the same."""
+    import bench
+
+    mib = 1 << 20
+    assert bench.buffer_sets(32 * mib, 128 * mib) == 32        # the headline: 4096 x 4096 bf16, forward + backward
+    assert bench.buffer_sets(32 * mib, 64 * mib) == 32         # forward alone
+    assert bench.buffer_sets(128 * mib, 512 * mib) == 8
+    assert bench.buffer_sets(128 * mib + 1, 512 * mib) == 2
+    assert bench.buffer_sets(2048 * mib, 8192 * mib) == 2
+    line = re.search(r"kKeepInputBytes = (\d+)L << 20", (ROOT / "mgrrmsnorm_amd" / "csrc" / "mg_launch.hpp").read_text())
+    assert bench.KEPT_INPUT_BYTES == int(line.group(1)) << 20
+
+
 def test_profiles_carry_the_hash_of_the_sources_they_were_taken_with():
     import bench
 
