@@ -15,7 +15,9 @@ extern "C" {
 #endif
 
 /*
- * 1 if mg_rmsnorm_bwd_small takes this shape (and is the faster way there), else 0.
+ * 1 if mg_rmsnorm_bwd_small takes this shape (and is the faster way there), else 0.  0 as well while any
+ * mg_set_option override is in force that mg_rmsnorm_bwd follows ("force_generic", "bwd_*", "narrow_groups",
+ * "xcd_group"), so that a caller who asks first gets the backward pass the override is about.
  */
 int mg_rmsnorm_bwd_small_fits(int64_t rows, int64_t cols, int dtype);
 

@@ -19,7 +19,8 @@ extern "C" {
 
 /*
  * Reports the launch shape mg_rmsnorm_fwd (backward == 0) or mg_rmsnorm_bwd (backward != 0)
- * takes for rows of `cols` elements; no counterpart in
+ * takes for rows of `cols` elements (mg_rmsnorm_bwd_small, which the torch bindings call instead where
+ * mg_rmsnorm_bwd_small_fits says so, is another kernel); no counterpart in
  * the reference (whose launchers always use 256 threads per row, src/rmsnorm_kernel.cu:530).
  * Host-only: needs no device.  *generic = 1 means the element-wise kernels (one 256-thread
  * workgroup per row, *vectors_per_thread = 0).  *generic = 0 with *vectors_per_thread = 0
@@ -108,7 +109,9 @@ int mg_rmsnorm_bwd_timeline(void* dx, float* dw_partial, const void* dy, const v
  * 0 = never, the default; a "fwd_tpr" / "fwd_items" override switches it off as well), "swiglu_unroll",
  * "force_generic" (1 = always take the one-element-per-thread kernels, which nothing selects by itself), "xcd_group" (consecutive workgroups
  * handled by one die at a time, 0 = off, -1 = automatic), "swiglu_max_units" (vectors or
- * elements one SwiGLU launch may cover before the input is split by rows; 0 = 2^31).  Returns MG_ERR_INVALID_ARG for
+ * elements one SwiGLU launch may cover before the input is split by rows; 0 = 2^31).  While an option that
+ * mg_rmsnorm_bwd follows is set, mg_rmsnorm_bwd_small_fits answers 0 and the torch bindings take the two calls
+ * for every number of rows.  Returns MG_ERR_INVALID_ARG for
  * an unknown key.  Values that do not fit a given problem are ignored for that call.
  */
 int mg_set_option(const char* key, int value);

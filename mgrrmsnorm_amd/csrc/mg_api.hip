@@ -35,6 +35,14 @@ std::atomic<int> opt_fwd_tpr{0}, opt_fwd_items{0}, opt_bwd_tpr{0}, opt_bwd_wg_pe
     opt_swiglu_unroll{0}, opt_force_generic{0}, opt_bwd_block{0}, opt_xcd_group{-1}, opt_bwd_prefetch{-1}, opt_groups{-1}, opt_bwd_lds{-1}, opt_bwd_ring{-1}, opt_bwd_partials{0}, opt_bwd_partial_policy{0},
     opt_fwd_lines{0};
 
+// Whether any option is in force that the two-call backward pass follows: the one-launch kernel of few rows
+// has none of these to set, so the calls they are meant for stay with the two calls.
+bool bwd_overridden() {
+    return opt_force_generic.load() != 0 || opt_bwd_tpr.load() != 0 || opt_bwd_block.load() != 0 || opt_bwd_wg_per_cu.load() != 0 ||
+           opt_bwd_partials.load() != 0 || opt_bwd_partial_policy.load() != 0 || opt_bwd_prefetch.load() != -1 ||
+           opt_groups.load() != -1 || opt_bwd_lds.load() != -1 || opt_bwd_ring.load() != -1 || opt_xcd_group.load() != -1;
+}
+
 // Consecutive logical workgroups one die handles at a time in the one-shot streaming
 // kernels (see xcd_remap); the "xcd_group" option overrides it (0 switches the remap off).
 constexpr int kXcdGroupStreaming = 32;
@@ -673,7 +681,7 @@ static bool bwd_small_holds(int64_t rows, int64_t cols, int es) {
 int mg_rmsnorm_bwd_small_fits(int64_t rows, int64_t cols, int dtype) {
     const int es = esize_of(dtype);
     return es != 0 && bwd_small_holds(rows, cols, es) && rows <= 1024 &&
-           (es == 2 || rows <= 512 || rows * cols * es <= (8LL << 20));
+           (es == 2 || rows <= 512 || rows * cols * es <= (8LL << 20)) && !bwd_overridden();
 }
 
 int mg_rmsnorm_bwd_small(void* dx, float* dw_f32, void* dw_cast, const void* dy, const void* x, const void* w,

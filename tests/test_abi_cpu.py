@@ -272,6 +272,31 @@ def test_set_option(lib):
         assert lib.mg_set_option(key, -1) == 0
 
 
+@pytest.mark.parametrize("key,value,default", [
+    ("force_generic", 1, 0), ("bwd_tpr", 256, 0), ("bwd_block", 1024, 0), ("bwd_wg_per_cu", 2, 0), ("bwd_partials", 7, 0),
+    ("bwd_partial_policy", 1, 0), ("bwd_prefetch", 0, -1), ("narrow_groups", 0, -1), ("bwd_lds", 0, -1), ("bwd_ring", 0, -1),
+    ("xcd_group", 0, -1)])
+def test_an_override_of_the_backward_pass_keeps_few_rows_with_it(lib, key, value, default):
+    """The one-launch backward of few rows steps aside while an option is set that it does not have."""
+    fits = lambda: lib.mg_rmsnorm_bwd_small_fits(64, 4096, 2)
+    assert fits() == 1
+    try:
+        assert lib.mg_set_option(key.encode(), value) == 0
+        assert fits() == 0
+    finally:
+        assert lib.mg_set_option(key.encode(), default) == 0
+    assert fits() == 1
+
+
+def test_options_of_the_forward_pass_leave_it(lib):
+    for key, value, default in (("fwd_tpr", 256, 0), ("fwd_items", 2, 0), ("fwd_lines", 1, 0), ("swiglu_unroll", 2, 0)):
+        try:
+            assert lib.mg_set_option(key.encode(), value) == 0
+            assert lib.mg_rmsnorm_bwd_small_fits(64, 4096, 2) == 1
+        finally:
+            assert lib.mg_set_option(key.encode(), default) == 0
+
+
 def test_option_generation_counts_successful_changes_only(lib):
     g0 = lib.mg_option_generation()
     assert lib.mg_set_option(b"no_such_key", 1) == -1

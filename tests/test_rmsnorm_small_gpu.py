@@ -69,3 +69,26 @@ def test_which_shapes_take_it():
     assert fits(1, 1, 2) and fits(1024, 16384, 2) and fits(512, 8192, 0) and fits(1024, 2048, 0)
     assert not fits(0, 64, 2) and not fits(1025, 64, 2) and not fits(1, 16385, 2) and not fits(513, 8192, 0)
     assert not fits(4, 64, 7)
+
+
+@pytest.mark.parametrize("option", [("force_generic", 1, 0), ("bwd_partials", 7, 0)])
+def test_overrides_reach_few_rows_through_both_bindings(option):
+    """With an override set, backward of few rows through the bindings is what the two C calls give."""
+    from mgrrmsnorm_amd import ops, ops_ctypes
+
+    rows, cols, dtype = 200, 1000, "bf16"
+    x, dy, w = U.rmsnorm_inputs(rows, cols, dtype, seed=3)
+    xd, gd, wd = x.cuda(), dy.cuda(), w.cuda()
+    key, value, default = option
+    y, s = ops.rmsnorm_forward(xd, wd, EPS)
+    alone = ops.rmsnorm_backward_f32(gd, xd, wd, s)[1]
+    try:
+        U.check(U.lib().mg_set_option(key.encode(), value))
+        dx, dw, cast, _ = U.rmsnorm_bwd(gd, xd, wd, s, dtype)
+        for module in (ops, ops_ctypes):
+            got = module.rmsnorm_backward_f32(gd, xd, wd, s)
+            assert torch.equal(got[0], dx) and torch.equal(got[1], dw) and torch.equal(got[2], cast)
+    finally:
+        U.check(U.lib().mg_set_option(key.encode(), default))
+    assert not torch.equal(dw, alone)          # another summation order: the override did reach the sums
+    assert torch.equal(ops.rmsnorm_backward_f32(gd, xd, wd, s)[1], alone)
