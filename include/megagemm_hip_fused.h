@@ -25,6 +25,8 @@ int mg_rmsnorm_bwd_small_fits(int64_t rows, int64_t cols, int dtype);
  * RMSNorm backward as mg_rmsnorm_bwd followed by mg_rmsnorm_dw_reduce, without a workspace: dx and
  * the finished dW (in fp32, in `dtype`, both, or -- both NULL -- neither).  Summation order of dW is
  * fixed, but not that of the two-call path.  Shapes it does not take: MG_ERR_UNSUPPORTED.
+ * No output may overlap an input: unlike in the two calls, dx is written while x and dy of the same rows are
+ * still read for dW, and dW while w and inv_rms are read for dx.  Such a call is refused (MG_ERR_INVALID_ARG).
  */
 int mg_rmsnorm_bwd_small(void* dx, float* dw_f32, void* dw_cast, const void* dy, const void* x, const void* w,
                          const float* inv_rms, int64_t rows, int64_t cols, int dtype, void* stream);
@@ -37,7 +39,7 @@ int mg_rmsnorm_bwd_small(void* dx, float* dw_f32, void* dw_cast, const void* dy,
  * first projection and activation in one pass, g and u kept in fp32.
  *   h   [tokens, hidden], x [tokens, d_model], w12 [2 * hidden, d_model]
  *   dtype  MG_F16 or MG_BF16; 1 <= tokens <= MG_BLOCK_MAX_TOKENS; d_model a multiple of 8;
- *   x and w12 16-byte aligned.  Anything else: MG_ERR_UNSUPPORTED or MG_ERR_INVALID_ARG.
+ *   x and w12 16-byte aligned; h overlaps neither.  Anything else: MG_ERR_UNSUPPORTED or MG_ERR_INVALID_ARG.
  */
 int mg_block_gate_up(void* h, const void* x, const void* w12, int64_t tokens, int64_t d_model, int64_t hidden,
                      int dtype, void* stream);

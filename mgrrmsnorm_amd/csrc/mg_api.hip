@@ -669,6 +669,11 @@ int mg_swiglu_bwd(void* dgu, const void* dh, const void* gu, int64_t M, int64_t 
     return MG_OK;
 }
 
+static bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const uintptr_t p = (uintptr_t)a, q = (uintptr_t)b;
+    return a != nullptr && b != nullptr && p < q + (uintptr_t)b_bytes && q < p + (uintptr_t)a_bytes;
+}
+
 // What rmsnorm_bwd_small can hold at all; mg_rmsnorm_bwd_small_fits says where it is also faster.
 static bool bwd_small_holds(int64_t rows, int64_t cols, int es) {
     return rows >= 1 && cols >= 1 && cols * es <= 2048 * kVec && rows <= (1LL << 20) && rows * cols * es < (1LL << 31);
@@ -697,6 +702,11 @@ int mg_rmsnorm_bwd_small(void* dx, float* dw_f32, void* dw_cast, const void* dy,
     if (!aligned(dx, es) || !aligned(dy, es) || !aligned(x, es) || !aligned(w, es) || !aligned(inv_rms, 4) ||
         !aligned(dw_f32, 4) || !aligned(dw_cast, es))
         return fail(MG_ERR_INVALID_ARG, "mg_rmsnorm_bwd_small: a pointer is not aligned to its element size");
+    // its workgroups write dx and dW while others still read the same rows for the other of the two
+    const struct { const void* p; int64_t bytes; } in[] = {{dy, rows * cols * es}, {x, rows * cols * es}, {w, cols * es}, {inv_rms, rows * 4}};
+    for (const auto& i : in)
+        if (overlap(dx, rows * cols * es, i.p, i.bytes) || overlap(dw_f32, cols * 4, i.p, i.bytes) || overlap(dw_cast, cols * es, i.p, i.bytes))
+            return fail(MG_ERR_INVALID_ARG, "mg_rmsnorm_bwd_small: an output overlaps an input");
     const BwdSmallArgs a = {dx, dw_f32, dw_cast, dy, x, w, inv_rms, (int)rows, (int)cols};
     hipStream_t s = (hipStream_t)stream;
     const hipError_t e = by_dtype(
@@ -719,6 +729,8 @@ static int block_projection(const char* fn, bool paired, void* out, const void* 
     if (out == nullptr || x == nullptr || w == nullptr) return fail(MG_ERR_INVALID_ARG, "%s: a pointer is NULL", fn);
     if (!aligned(out, 2) || !aligned(x, 16) || !aligned(w, 16))
         return fail(MG_ERR_INVALID_ARG, "%s: inputs must be 16-byte aligned", fn);
+    if (overlap(out, tokens * N * 2, x, tokens * K * 2) || overlap(out, tokens * N * 2, w, (paired ? 2 : 1) * N * K * 2))
+        return fail(MG_ERR_INVALID_ARG, "%s: the output overlaps an input", fn);
     int cus = 0;
     const int rc = cu_count(&cus);
     if (rc != MG_OK) return rc;

@@ -136,6 +136,21 @@ def test_swiglu_rejects_bad_arguments(lib):
     assert lib.mg_swiglu_bwd(None, None, None, 0, 8, 1, None) == 0
 
 
+def test_one_launch_entry_points_refuse_outputs_over_inputs(lib):
+    """Their workgroups write while others still read: dx = dy and the like would race."""
+    f = lib.mg_rmsnorm_bwd_small
+    rows, cols, n = 4, 64, 4 * 64 * 2                    # bf16: dx, dy and x are n bytes each
+    at = dict(dx=0x10000, dw=0x20000, cast=0x30000, dy=0x40000, x=0x50000, w=0x60000, s=0x70000)
+    call = lambda **kw: f(*({**at, **kw}[k] for k in ("dx", "dw", "cast", "dy", "x", "w", "s")), rows, cols, 2, None)
+    for over in (dict(dx=at["dy"]), dict(dx=at["x"]), dict(dx=at["x"] + n - 2), dict(dx=at["x"] - n + 2), dict(dx=at["w"]),
+                 dict(dw=at["s"]), dict(dw=at["x"]), dict(cast=at["w"]), dict(cast=at["dy"] + n - 2)):
+        assert call(**over) == -1 and "overlaps" in _err(lib), over
+    tokens, d, h = 4, 64, 128
+    assert lib.mg_block_gate_up(at["x"], at["x"], at["w"], tokens, d, h, 2, None) == -1 and "overlaps" in _err(lib)
+    assert lib.mg_block_gate_up(at["w"] + 2 * h * d * 2 - 2, at["x"], at["w"], tokens, d, h, 2, None) == -1 and "overlaps" in _err(lib)
+    assert lib.mg_block_down(at["x"] + tokens * h * 2 - 2, at["x"], at["w"], tokens, d, h, 2, None) == -1 and "overlaps" in _err(lib)
+
+
 def test_copy_bytes_rejects_bad_arguments(lib):
     assert lib.mg_copy_bytes(FAKE, FAKE, 24, None) == -1 and "multiple of 16" in _err(lib)
     assert lib.mg_copy_bytes(FAKE, FAKE + 4, 32, None) == -1 and "aligned" in _err(lib)
