@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define MG_ABI_VERSION 2
+#define MG_ABI_VERSION 3
 
 /* element types; the reference encodes these in function-name suffixes
  * (_fp32/_fp16/_bf16, src/rmsnorm_kernel.h:9-67) */

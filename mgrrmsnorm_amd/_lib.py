@@ -18,7 +18,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libmegagemm_hip.so"
-ABI_VERSION = 2
+ABI_VERSION = 3
 
 MG_F32, MG_F16, MG_BF16 = 0, 1, 2
 _DTYPE_CODE = {torch.float32: MG_F32, torch.float16: MG_F16, torch.bfloat16: MG_BF16}
@@ -75,11 +75,15 @@ def load() -> ctypes.CDLL:
             lib = ctypes.CDLL(str(LIB_PATH))
         except OSError as exc:  # e.g. libamdhip64.so not found
             raise RuntimeError(f"cannot load {LIB_PATH}: {exc}") from exc
-        for name, (restype, argtypes) in {**SIGNATURES, **FUSED_SIGNATURES}.items():
-            fn = getattr(lib, name)
-            fn.restype = restype
-            fn.argtypes = argtypes
-        got = lib.mg_abi_version()
+        try:
+            got = lib.mg_abi_version()      # before anything that another version may not have
+            if got == ABI_VERSION:
+                for name, (restype, argtypes) in {**SIGNATURES, **FUSED_SIGNATURES}.items():
+                    fn = getattr(lib, name)
+                    fn.restype = restype
+                    fn.argtypes = argtypes
+        except AttributeError as exc:
+            raise RuntimeError(f"{LIB_PATH} lacks an entry point of this package ({exc}); rebuild it") from exc
         if got != ABI_VERSION:
             raise RuntimeError(f"{LIB_PATH} has ABI version {got}, this package needs {ABI_VERSION}; rebuild it")
         _lib = lib

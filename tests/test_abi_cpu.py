@@ -66,9 +66,23 @@ def test_header_compiles_as_c_and_cxx(tmp_path):
 def test_abi_version(lib):
     from mgrrmsnorm_amd import _lib
 
-    assert lib.mg_abi_version() == _lib.ABI_VERSION == 2
+    assert lib.mg_abi_version() == _lib.ABI_VERSION == 3
     text = HEADER.read_text()
-    assert re.search(r"#define\s+MG_ABI_VERSION\s+2\b", text)
+    assert re.search(r"#define\s+MG_ABI_VERSION\s+3\b", text)
+
+
+@pytest.mark.parametrize("version,message", [(2, "has ABI version 2"), (3, "lacks an entry point")])
+def test_a_library_of_other_sources_is_refused_with_a_message(tmp_path, monkeypatch, version, message):
+    """An older library lacks entry points: its version is read before they are looked up."""
+    from mgrrmsnorm_amd import _lib
+
+    src, old = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text(f"int mg_abi_version(void) {{ return {version}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(old)], check=True)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", old)
+    with pytest.raises(RuntimeError, match=f"{message}.*rebuild it"):
+        _lib.load()
 
 
 def _err(lib):
