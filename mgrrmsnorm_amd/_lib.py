@@ -30,7 +30,7 @@ _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
 
-# name -> (restype, argtypes); mirrors include/megagemm_hip.h and megagemm_hip_tuning.h one to one
+# name -> (restype, argtypes); mirrors include/megagemm_hip.h, megagemm_hip_tuning.h and megagemm_hip_fused.h one to one
 SIGNATURES = {
     "mg_abi_version": (_int, []),
     "mg_last_error": (ctypes.c_char_p, []),
@@ -48,10 +48,6 @@ SIGNATURES = {
     "mg_row_probe": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     "mg_rmsnorm_launch_info": (_int, [_int, _i64, _int] + [ctypes.POINTER(_int)] * 4),
     "mg_rmsnorm_bwd_timeline": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _i64, _i64, _vp, _vp]),
-}
-
-# the entry points of include/megagemm_hip_fused.h
-FUSED_SIGNATURES = {
     "mg_rmsnorm_bwd_small_fits": (_int, [_i64, _i64, _int]),
     "mg_rmsnorm_bwd_small": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _vp]),
     "mg_block_gate_up": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
@@ -78,7 +74,7 @@ def load() -> ctypes.CDLL:
         try:
             got = lib.mg_abi_version()      # before anything that another version may not have
             if got == ABI_VERSION:
-                for name, (restype, argtypes) in {**SIGNATURES, **FUSED_SIGNATURES}.items():
+                for name, (restype, argtypes) in SIGNATURES.items():
                     fn = getattr(lib, name)
                     fn.restype = restype
                     fn.argtypes = argtypes

@@ -24,6 +24,7 @@ def lib():
 
 
 TUNING_HEADER = ROOT / "include" / "megagemm_hip_tuning.h"
+FUSED_HEADER = ROOT / "include" / "megagemm_hip_fused.h"
 
 
 def _declared_in(header):
@@ -32,7 +33,7 @@ def _declared_in(header):
 
 
 def _declared_functions():
-    return sorted(_declared_in(HEADER) + _declared_in(TUNING_HEADER))
+    return sorted(_declared_in(HEADER) + _declared_in(TUNING_HEADER) + _declared_in(FUSED_HEADER))
 
 
 def test_header_declares_the_expected_entry_points():
@@ -43,6 +44,9 @@ def test_header_declares_the_expected_entry_points():
     assert _declared_in(TUNING_HEADER) == sorted([
         "mg_set_option", "mg_option_generation", "mg_copy_bytes", "mg_stream_probe", "mg_row_probe",
         "mg_rmsnorm_launch_info", "mg_rmsnorm_bwd_timeline"])
+    # one launch for what takes several
+    assert _declared_in(FUSED_HEADER) == sorted([
+        "mg_rmsnorm_bwd_small_fits", "mg_rmsnorm_bwd_small", "mg_block_gate_up", "mg_block_down"])
 
 
 def test_library_exports_every_declared_symbol(lib):
@@ -56,7 +60,7 @@ def test_library_exports_every_declared_symbol(lib):
 
 def test_header_compiles_as_c_and_cxx(tmp_path):
     src = tmp_path / "t.c"
-    src.write_text('#include "megagemm_hip.h"\n#include "megagemm_hip_tuning.h"\nint main(void){return MG_ABI_VERSION - 1;}\n')
+    src.write_text('#include "megagemm_hip.h"\n#include "megagemm_hip_tuning.h"\n#include "megagemm_hip_fused.h"\nint main(void){return MG_ABI_VERSION - 1;}\n')
     subprocess.run(["gcc", "-std=c99", "-Wall", "-Werror", f"-I{HEADER.parent}", "-c", str(src), "-o",
                     str(tmp_path / "t.o")], check=True)
     subprocess.run(["g++", "-x", "c++", "-Wall", "-Werror", f"-I{HEADER.parent}", "-c", str(src), "-o",
@@ -148,6 +152,38 @@ def test_swiglu_rejects_bad_arguments(lib):
     assert lib.mg_swiglu_bwd(FAKE, None, FAKE, 4, 8, 2, None) == -1
     assert lib.mg_swiglu_bwd(FAKE, FAKE + 2, FAKE, 4, 8, 0, None) == -1 and "aligned" in _err(lib)
     assert lib.mg_swiglu_bwd(None, None, None, 0, 8, 1, None) == 0
+
+
+def test_bwd_small_rejects_bad_arguments(lib):
+    f = lib.mg_rmsnorm_bwd_small
+    far = [0x1000000 * (i + 1) for i in range(7)]        # dx, dw_f32, dw_cast, dy, x, w, inv_rms: never dereferenced
+    assert f(*far, 4, 64, 7, None) == -1 and "dtype" in _err(lib)
+    assert f(*far, -1, 64, 2, None) == -1 and "rows" in _err(lib)
+    assert f(*far, 4, 0, 2, None) == -1 and "cols" in _err(lib)
+    for shape in ((0, 64, 2), (4, 16385, 2), (4, 8193, 0), ((1 << 20) + 1, 8, 2), (1 << 20, 1024, 2)):
+        assert f(*far, *shape, None) == -2 and "not a shape" in _err(lib)
+        assert not lib.mg_rmsnorm_bwd_small_fits(*shape)
+    for i in (0, 3, 4, 5, 6):                            # either dW may be NULL, nothing else
+        assert f(*[None if j == i else p for j, p in enumerate(far)], 4, 64, 2, None) == -1 and "NULL" in _err(lib)
+    for i in range(7):
+        assert f(*[p + 1 if j == i else p for j, p in enumerate(far)], 4, 64, 2, None) == -1 and "aligned" in _err(lib)
+
+
+@pytest.mark.parametrize("name", ["mg_block_gate_up", "mg_block_down"])
+def test_block_projections_reject_bad_arguments(lib, name):
+    f = getattr(lib, name)
+    out, x, w = 0x10000, 0x20000, 0x40000
+    inner = lambda k, n: (k, n) if name == "mg_block_gate_up" else (n, k)     # (d_model, hidden) from the inner and outer size
+    assert f(out, x, w, 4, 64, 64, 0, None) == -2 and "dtype" in _err(lib)
+    assert f(out, x, w, 4, 64, 64, 7, None) == -2 and "dtype" in _err(lib)
+    for tokens in (0, -1, 65):
+        assert f(out, x, w, tokens, 64, 64, 2, None) == -2 and "tokens" in _err(lib)
+    for sizes in ((0, 64), (4, 64), (60, 64), (1 << 30, 64), (64, 0), (64, 1 << 30)):
+        assert f(out, x, w, 4, *inner(*sizes), 2, None) == -2 and "inner size" in _err(lib)
+    for pointers in ((None, x, w), (out, None, w), (out, x, None)):
+        assert f(*pointers, 4, 64, 64, 2, None) == -1 and "NULL" in _err(lib)
+    for pointers in ((out + 1, x, w), (out, x + 8, w), (out, x, w + 2)):
+        assert f(*pointers, 4, 64, 64, 2, None) == -1 and "aligned" in _err(lib)
 
 
 def test_one_launch_entry_points_refuse_outputs_over_inputs(lib):

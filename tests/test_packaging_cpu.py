@@ -48,7 +48,8 @@ def test_build_hip_produces_a_loadable_extension(built):
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
     assert mod.abi_version() == _lib.ABI_VERSION
-    for name in ("rmsnorm_forward", "rmsnorm_backward", "swiglu_forward", "swiglu_backward", "rmsnorm", "swiglu"):
+    for name in ("rmsnorm_forward", "rmsnorm_backward", "swiglu_forward", "swiglu_backward", "rmsnorm", "swiglu",
+                 "swiglu_block", "swiglu_block_fits"):
         assert callable(getattr(mod, name))
     with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
         mod.rmsnorm_forward(torch.ones(2, 8), torch.ones(8), 1e-6)
@@ -88,9 +89,9 @@ def test_pip_install_builds_and_ships_everything(installed):
     lib = ctypes.CDLL(str(lib_path))
     lib.mg_abi_version.restype = ctypes.c_int
     assert lib.mg_abi_version() == _lib.ABI_VERSION
-    for name in ("mg_api.hip", "rmsnorm_kernels.hpp", "torch_binding.cpp"):
+    for name in ("mg_api.hip", "rmsnorm_kernels.hpp", "skinny_gemm.hpp", "rmsnorm_bwd_small.hpp", "torch_binding.cpp"):
         assert (pkg / "csrc" / name).exists(), f"csrc/{name} did not ship"
-    for name in ("megagemm_hip.h", "megagemm_hip_tuning.h"):
+    for name in ("megagemm_hip.h", "megagemm_hip_tuning.h", "megagemm_hip_fused.h"):
         assert (site / "include" / name).exists(), f"include/{name} did not ship"
     assert (site / "megagemm" / "__init__.py").exists() and (site / "rmsnorm_cuda_ops.py").exists()
     # the installed copy imports on its own and finds its library next to itself
