@@ -18,8 +18,16 @@ CODES = {"fp32": 0, "fp16": 1, "bf16": 2}
 FP32_ULP = compare.FP32_ULP
 
 
+# rows on either side of the line where the bindings' backward goes from one launch to two
+BOTH_BACKWARDS = (300, 1100)
+
+
 def lib():
     return _lib.load()
+
+
+def takes_one_launch(rows, cols, dtype):
+    return bool(lib().mg_rmsnorm_bwd_small_fits(rows, cols, CODES[dtype]))
 
 
 def stream():

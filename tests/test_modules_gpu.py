@@ -8,6 +8,7 @@ import torch
 import torch.nn.functional as F
 
 import gpu_util as U
+from gpu_util import BOTH_BACKWARDS
 
 pytestmark = pytest.mark.gpu
 
@@ -231,7 +232,8 @@ def test_state_dict_round_trip_between_module_names():
     assert torch.equal(n1(x), n2(x))
 
 
-def test_module_forward_backward_under_graph_capture():
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
+def test_module_forward_backward_under_graph_capture(rows):
     """The nn.Module path (allocation through torch's caching allocator, launches through the
     C ABI) captured into one HIP graph: replays, separated by eager work, reproduce the eager
     gradients.  This is the way to run small shapes without paying the Python round trip."""
@@ -240,9 +242,9 @@ def test_module_forward_backward_under_graph_capture():
     torch.manual_seed(3)
     C, H = 2048, 1024
     norm = RMSNorm(C, 1e-6).cuda().to(torch.bfloat16)
-    x = torch.randn(256, C, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    x = torch.randn(rows, C, device="cuda", dtype=torch.bfloat16, requires_grad=True)
     proj = torch.randn(C, 2 * H, device="cuda", dtype=torch.bfloat16) * 0.05
-    g = torch.randn(256, H, device="cuda", dtype=torch.bfloat16)
+    g = torch.randn(rows, H, device="cuda", dtype=torch.bfloat16)
 
     def step():
         x.grad = None
@@ -275,7 +277,8 @@ def test_module_forward_backward_under_graph_capture():
         assert torch.equal(norm.weight.grad, want[2]), f"replay {i}: dW"
 
 
-def test_concurrent_calls_from_several_threads():
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
+def test_concurrent_calls_from_several_threads(rows):
     """The library is re-entrant: four threads, each on its own stream, run forward+backward
     at the same time and each gets the answer a lone call gives."""
     import threading
@@ -285,7 +288,7 @@ def test_concurrent_calls_from_several_threads():
     torch.manual_seed(11)
     C = 2048
     w = (1 + 0.02 * torch.randn(C, device="cuda")).to(torch.bfloat16)
-    xs = [torch.randn(300 + 17 * i, C, device="cuda").to(torch.bfloat16) for i in range(4)]
+    xs = [torch.randn(rows + 17 * i, C, device="cuda").to(torch.bfloat16) for i in range(4)]
     gs = [torch.randn_like(x) for x in xs]
     want = []
     for x, g in zip(xs, gs):
@@ -352,11 +355,12 @@ def test_inference_path_equals_autograd_path():
     assert xg.grad is not None
 
 
-def test_frozen_weight_skips_the_dw_reduction():
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
+def test_frozen_weight_skips_the_dw_reduction(rows):
     from mgrrmsnorm_amd import RMSNorm
 
     norm = RMSNorm(512, 1e-6).cuda()
-    x = torch.randn(40, 512, device="cuda", requires_grad=True)
+    x = torch.randn(rows, 512, device="cuda", requires_grad=True)
     norm(x).sum().backward()
     want = x.grad.clone()
     assert norm.weight.grad is not None
@@ -367,7 +371,8 @@ def test_frozen_weight_skips_the_dw_reduction():
     assert norm.weight.grad is None and torch.equal(x.grad, want)
 
 
-def test_backward_on_the_calling_thread_gives_the_same_bits():
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
+def test_backward_on_the_calling_thread_gives_the_same_bits(rows):
     """torch.autograd.set_multithreading_enabled(False) makes the engine run the backward pass
     on the calling thread instead of its device worker; the nodes must not care."""
     from mgrrmsnorm_amd import MegaGemmTriton, RMSNorm
@@ -375,7 +380,7 @@ def test_backward_on_the_calling_thread_gives_the_same_bits():
     torch.manual_seed(11)
     norm = RMSNorm(2048, 1e-6).cuda().to(torch.bfloat16)
     mlp = MegaGemmTriton(2048).cuda().to(torch.bfloat16)
-    x = torch.randn(5, 33, 2048, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(4, rows // 4, 2048, device="cuda", dtype=torch.bfloat16)
     dy = torch.randn_like(x)
 
     def grads():

@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 import torch
 
+from gpu_util import BOTH_BACKWARDS, takes_one_launch
+
 
 @pytest.fixture(scope="module")
 def binding():
@@ -56,12 +58,14 @@ def test_stale_extension_is_refused():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
 @pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
-def test_binding_matches_oracle_and_ctypes_path(binding, dtype):
+def test_binding_matches_oracle_and_ctypes_path(binding, dtype, rows):
     import gpu_util as U
     from mgrrmsnorm_amd import ops_ctypes
 
-    rows, cols, eps = 300, 4096, 1e-6
+    cols, eps = 4096, 1e-6
+    assert takes_one_launch(rows, cols, dtype) == (rows == BOTH_BACKWARDS[0])
     x, dy, w = U.rmsnorm_inputs(rows, cols, dtype, seed=5)
     y_ref, s_ref, dx_ref, dw_ref, floor = U.rmsnorm_reference(x, dy, w, eps, dtype)
     xd, dyd, wd = x.cuda(), dy.cuda(), w.cuda()
@@ -80,6 +84,8 @@ def test_binding_matches_oracle_and_ctypes_path(binding, dtype):
     y2, s2 = ops_ctypes.rmsnorm_forward(xd, wd, eps)
     dx2, dw2 = ops_ctypes.rmsnorm_backward(dyd, xd, wd, s2)
     assert torch.equal(y, y2) and torch.equal(s, s2) and torch.equal(dx, dx2) and torch.equal(dw, dw2)
+    dx5, none3, none4 = ops_ctypes.rmsnorm_backward_f32(dyd, xd, wd, s2, need_weight_grad=False)
+    assert none3 is None and none4 is None and torch.equal(dx5, dx)
 
 
 @pytest.mark.gpu
@@ -101,16 +107,17 @@ def test_swiglu_binding_matches_oracle_and_ctypes_path(binding, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_cpp_autograd_nodes_match_python_functions(binding, dtype):
+def test_cpp_autograd_nodes_match_python_functions(binding, dtype, rows):
     """binding.rmsnorm / binding.swiglu (autograd nodes in C++) against RMSNormFunction /
     MegaGemmFunction (Python autograd.Functions over the same kernels): identical bits."""
     from mgrrmsnorm_amd import MegaGemmFunction, RMSNormFunction
 
     g = torch.Generator().manual_seed(9)
-    x = torch.randn((3, 50, 768), generator=g).to(dtype).cuda()
+    x = torch.randn((2, rows // 2, 768), generator=g).to(dtype).cuda()
     w = (1 + 0.02 * torch.randn(768, generator=g)).to(dtype).cuda()
-    dy = torch.randn((3, 50, 768), generator=g).to(dtype).cuda()
+    dy = torch.randn((2, rows // 2, 768), generator=g).to(dtype).cuda()
     outs = []
     for fn in (lambda a, b: binding.rmsnorm(a, b, 1e-6), lambda a, b: RMSNormFunction.apply(a, b, 1e-6)):
         xa, wa = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
@@ -198,7 +205,8 @@ def test_binding_checks_shapes_on_the_gpu(binding):
 
 
 @pytest.mark.gpu
-def test_modules_give_the_same_bits_through_either_binding(binding, monkeypatch):
+@pytest.mark.parametrize("rows", BOTH_BACKWARDS)
+def test_modules_give_the_same_bits_through_either_binding(binding, monkeypatch, rows):
     """megagemm.RMSNorm / MegaGemmTriton through the compiled extension (C++ autograd nodes)
     and through the ctypes binding (Python autograd.Functions): same outputs and gradients."""
     import megagemm
@@ -207,8 +215,8 @@ def test_modules_give_the_same_bits_through_either_binding(binding, monkeypatch)
     torch.manual_seed(3)
     norm = megagemm.RMSNorm(1024, 1e-6).cuda().to(torch.bfloat16)
     mlp = megagemm.MegaGemmTriton(1024).cuda().to(torch.bfloat16)
-    x = torch.randn(4, 40, 1024, device="cuda", dtype=torch.bfloat16)
-    g = torch.randn(4, 40, 1024, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(4, rows // 4, 1024, device="cuda", dtype=torch.bfloat16)
+    g = torch.randn(4, rows // 4, 1024, device="cuda", dtype=torch.bfloat16)
 
     def run():
         for p in list(norm.parameters()) + list(mlp.parameters()):
