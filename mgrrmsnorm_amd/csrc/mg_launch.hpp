@@ -189,7 +189,11 @@ struct FwdArgs {
     void* y; float* inv_rms; const void* x; const void* w;
     long rows; int cols; float eps;
     int xcd_group;  // see xcd_remap(); 0 = workgroup ids used as they come
-    bool keep_x;    // x may stay in the caches (see keep_input)
+    // x may stay in the caches (see keep_input).  Followed by rmsnorm_fwd_rows, and by the narrow and group
+    // layouts at pitches that are multiples of 16 bytes; at other pitches those always read x with the
+    // default policy.  Rows streamed twice read it so the first time and non-temporally the second; the
+    // layout on the lines of the output ("fwd_lines") always reads it non-temporally.
+    bool keep_x;
 };
 struct BwdArgs {
     void* dx; float* dw_part; int ld; const void* dy; const void* x; const void* w; const float* inv_rms;

@@ -16,9 +16,10 @@ namespace mg {
 //     lane, 16 / wpr rows per workgroup;
 //   the others, one per 128-byte line of columns: dW; 8 lanes side by side hold the line of a row,
 //     128 rows at a time, kRowsInFlight (4: with 8 the workgroup has a compute unit to itself and
-//     512 x 4096 takes 7.8 us) of them per thread requested before the first is used; the sums of a wave's 8 rows are added by lane exchanges, those of the 16 waves through LDS, both in
-//     a fixed order.
-// Rows need no alignment beyond an element's (see RowTail).
+//     512 x 4096 takes 7.8 us) of them per thread requested before the first is used; the sums of a
+//     wave's 8 rows are added by lane exchanges, those of the 16 waves through LDS, both in a fixed order.
+// Rows need no alignment beyond an element's (see RowTail).  Outputs overlap no input (checked on the host):
+// a row's dx is written while other workgroups read the row for dW.
 //   block = 1024 threads; rows * cols * sizeof(T) < 2^31; ITEMS * 64 * wpr vectors hold a row
 constexpr int kSmallBlock = 1024;
 constexpr int kRowsInFlight = 4;

@@ -146,3 +146,38 @@ def test_sparse_operands(operand):
     operands[operand] = dense.to_sparse_csr()
     with pytest.raises(RuntimeError, match="contiguous"):
         ops.swiglu_block(*operands)
+
+
+def test_the_block_under_graph_capture_and_on_other_streams():
+    """A decoding step captured into a graph, and issued from four threads on streams of their own."""
+    import threading
+
+    module = MegaGemmTriton(512).cuda().to(torch.bfloat16)
+    xs = [torch.randn(8, 512, device="cuda", dtype=torch.bfloat16) for _ in range(4)]
+    with torch.no_grad():
+        want = [module(x) for x in xs]
+        assert torch.equal(want[0], ops.swiglu_block(xs[0], module.w12.weight, module.w3.weight))
+        static, graph = xs[0].clone(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            out = module(static)
+        for x, y in zip(xs, want):
+            static.copy_(x)
+            torch.zeros(1024, device="cuda").add_(1)       # eager work between replays
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, y)
+    got = [None] * 4
+
+    def work(i):
+        with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                got[i] = module(xs[i])
+            torch.cuda.current_stream().synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -1,5 +1,5 @@
-"""The forward kernels read inputs of up to 128 MiB with another cache policy than larger ones:
-the same rows give the same bits on both sides of that line."""
+"""Most forward kernels read inputs of up to 128 MiB with another cache policy than larger ones, which
+are other instances of the kernel: the same rows give the same bits on both sides of that line."""
 import pytest
 import torch
 
@@ -13,8 +13,17 @@ def _copies(block, rows):
     return block.repeat((rows + block.size(0) - 1) // block.size(0), 1)[:rows].contiguous()
 
 
-# one shape of each family of forward kernels: rows, several vectors per lane, row groups, two reads
-@pytest.mark.parametrize("cols,dtype", [(4096, BF16), (8191, F16), (1024, F16), (80, BF16), (64, F32), (100, BF16), (70000, BF16)])
+# by family of forward kernels, with shapes on different numbers of lanes
+FOLLOW_THE_LINE = [
+    (4096, BF16), (8191, F16), (1032, BF16), (2048, F32), (16384, BF16),     # a row over 64 ... 1024 threads
+    (1024, F16), (512, BF16), (256, F16),                                    # several vectors per lane, 32, 16 and 8 lanes
+    (80, BF16), (64, F32), (264, BF16), (24, F16), (8, BF16),                # row groups, 16, 16, 64, 4 and 1 lanes
+]
+# ... and those that read every input alike, where only the rows' independence of their number is tested
+READ_ALIKE = [(100, BF16), (129, F16), (70000, BF16)]                        # ragged groups and lanes; rows read twice
+
+
+@pytest.mark.parametrize("cols,dtype", FOLLOW_THE_LINE + READ_ALIKE)
 def test_rmsnorm_forward_on_both_sides_of_the_line(cols, dtype):
     from mgrrmsnorm_amd import ops
 
@@ -29,6 +38,7 @@ def test_rmsnorm_forward_on_both_sides_of_the_line(cols, dtype):
         assert torch.equal(yy, _copies(y, rows)) and torch.equal(ss, _copies(s[:, None], rows)[:, 0])
 
 
+# aligned half rows follow the line; ragged ones (2731) are read alike
 @pytest.mark.parametrize("hidden,dtype", [(4096, BF16), (1000, F32), (2731, F16)])
 def test_swiglu_forward_on_both_sides_of_the_line(hidden, dtype):
     from mgrrmsnorm_amd import ops
