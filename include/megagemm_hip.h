@@ -62,7 +62,8 @@ const char* mg_last_error(void);
  *
  *   s[r]    = 1 / sqrt(mean_c(x[r,c]^2) + eps)        (fp32 accumulation)
  *   y[r,c]  = (x[r,c] * s[r]) * w[c]                  (fp32, rounded once, to nearest even)
- *   inv_rms[r] = s[r]                                 (fp32; pointer may be NULL)
+ *   inv_rms[r] = s[r]                                 (fp32; pointer may be NULL: no backward pass follows, and
+ *                                                      x is then read past the caches at every size)
  *
  * x, y: [rows, cols] of `dtype`; w: [cols] of the same dtype.  Any cols >= 1 is accepted
  * (the reference requires cols % 4 == 0 for fp32 and cols % 2 == 0 otherwise and skips a

@@ -2,7 +2,8 @@
  * megagemm_hip_fused.h -- entry points that do in one launch what takes several through
  * megagemm_hip.h, for the calls whose time is launches and latency: RMSNorm backward of a few rows,
  * and the two projections of the SwiGLU block (reference: megagemm/swiglu.py:165-172, two
- * torch.matmul around the Triton activation) in a decoding step of a small batch.
+ * torch.matmul around the Triton activation) in a decoding step of a small batch -- and the activation
+ * where no backward pass follows.
  * Conventions as in megagemm_hip.h.
  */
 #ifndef MEGAGEMM_HIP_FUSED_H
@@ -50,6 +51,12 @@ int mg_block_gate_up(void* h, const void* x, const void* w12, int64_t tokens, in
  */
 int mg_block_down(void* out, const void* h, const void* w3, int64_t tokens, int64_t d_model, int64_t hidden,
                   int dtype, void* stream);
+
+/*
+ * mg_swiglu_fwd for an input that no backward pass will read again: the same results; gu is read past the
+ * memory-side cache and leaves the room in it to others (mg_swiglu_fwd keeps up to 128 MiB of it there).
+ */
+int mg_swiglu_fwd_only(void* h, const void* gu, int64_t M, int64_t H, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -50,6 +50,7 @@ SIGNATURES = {
     "mg_rmsnorm_bwd_timeline": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _i64, _i64, _vp, _vp]),
     "mg_rmsnorm_bwd_small_fits": (_int, [_i64, _i64, _int]),
     "mg_rmsnorm_bwd_small": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _vp]),
+    "mg_swiglu_fwd_only": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "mg_block_gate_up": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "mg_block_down": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
 }

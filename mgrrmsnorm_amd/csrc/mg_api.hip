@@ -340,7 +340,7 @@ int mg_rmsnorm_fwd(void* y, float* inv_rms, const void* x, const void* w, int64_
     if (!generic && !choose_fwd_lines(row_bytes, aligned(y, 8), &cfg))
         generic = !choose_fwd(row_bytes, &cfg) && !choose_streaming(row_bytes, &cfg);
     const FwdArgs a = {y, inv_rms, x, w, (long)rows, (int)cols, eps, xcd_group_or(kXcdGroupStreaming),
-                       keep_input((long)rows * row_bytes)};
+                       keep_input((long)rows * row_bytes, inv_rms != nullptr)};   // inv_rms is for a backward pass
     hipStream_t s = (hipStream_t)stream;
     hipError_t e = by_dtype(
         dtype, [&] { return launch_rmsnorm_fwd<float>(cfg, generic, a, s); },
@@ -639,18 +639,27 @@ static int swiglu_unroll(int dflt, int maxv) {
     return dflt;
 }
 
-int mg_swiglu_fwd(void* h, const void* gu, int64_t M, int64_t H, int dtype, void* stream) {
-    int rc = check_swiglu("mg_swiglu_fwd", M, H, dtype);
+static int swiglu_fwd(const char* fn, bool read_again, void* h, const void* gu, int64_t M, int64_t H, int dtype, void* stream) {
+    int rc = check_swiglu(fn, M, H, dtype);
     if (rc != MG_OK) return rc;
     if (M == 0) return MG_OK;
-    if (h == nullptr || gu == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_swiglu_fwd: h and gu must not be NULL");
+    if (h == nullptr || gu == nullptr) return fail(MG_ERR_INVALID_ARG, "%s: h and gu must not be NULL", fn);
     const int es = esize_of(dtype);
     if (!aligned(h, es) || !aligned(gu, es))
-        return fail(MG_ERR_INVALID_ARG, "mg_swiglu_fwd: a pointer is not aligned to its element size");
+        return fail(MG_ERR_INVALID_ARG, "%s: a pointer is not aligned to its element size", fn);
     const int mode = swiglu_mode(H * es, aligned(h, 16) && aligned(gu, 16));
-    hipError_t e = launch_swiglu_fwd(dtype, mode, swiglu_unroll(1, 8), xcd_group_or(kXcdGroupStreaming), h, gu, (long)M, (long)H, (hipStream_t)stream);
-    if (e != hipSuccess) return fail_hip("mg_swiglu_fwd: launch", e);
+    hipError_t e = launch_swiglu_fwd(dtype, mode, swiglu_unroll(1, 8), xcd_group_or(kXcdGroupStreaming), read_again, h, gu, (long)M,
+                                     (long)H, (hipStream_t)stream);
+    if (e != hipSuccess) return fail_hip(fn, e);
     return MG_OK;
+}
+
+int mg_swiglu_fwd(void* h, const void* gu, int64_t M, int64_t H, int dtype, void* stream) {
+    return swiglu_fwd("mg_swiglu_fwd", true, h, gu, M, H, dtype, stream);
+}
+
+int mg_swiglu_fwd_only(void* h, const void* gu, int64_t M, int64_t H, int dtype, void* stream) {
+    return swiglu_fwd("mg_swiglu_fwd_only", false, h, gu, M, H, dtype, stream);
 }
 
 int mg_swiglu_bwd(void* dgu, const void* dh, const void* gu, int64_t M, int64_t H, int dtype, void* stream) {

@@ -173,17 +173,20 @@ constexpr int narrow_default_tpr(long row_bytes, bool backward) {
 }
 
 // Whether the forward pass reads its input (`bytes` of it) with the default cache policy rather
-// than non-temporally.  The input is read again -- by the backward pass, and x by the residual
-// addition too -- and up to half of the 256 MiB memory-side cache it is then still there.
+// than non-temporally: where a backward pass follows and reads it again, up to half of the 256 MiB
+// memory-side cache, in which it is then still there.
 // bf16, forward + backward on tensors never used before, default / non-temporal policy (us):
 // RMSNorm 4096 columns x 4096 rows (32 MiB) 32.3 / 34.3, 8192 rows 54.0 / 55.9, 16384 rows (128 MiB)
 // 99.3 / 101.2, 24576 rows (192 MiB) 169.8 / 163.1; 262144 x 80 39.8 / 42.9; SwiGLU 8192 x 2*4096
 // (128 MiB) 74.8 / 79.5, 8192 x 2*11008 (344 MiB) 249 / 220.  The same inputs in turn, 16384 x 4096:
 // 104.7 / 111.8.  Beyond half the cache the input pushes out lines that still have to be written back.
+// Where none follows it only keeps room from others.  Forward alone, new tensors: SwiGLU 4096 x 2*4096 17.9 / 17.4,
+// 8192 x 2*4096 33.6 / 32.1, RMSNorm 65536 x 768 33.8 / 33.2, 4096 x 4096 13.2 either way; the addition that wrote the
+// input and the forward pass together: RMSNorm 4096 x 4096 29.3 / 27.8, 65536 x 768 79 / 75, SwiGLU 4096 x 2*4096 50 / 47.6.
 // Ragged half rows of SwiGLU are not asked: the same inputs in turn, 8192 x 2*2731 fp16, take 75.6 / 65.6.
 // A template argument of the kernels: a branch at run time costs larger inputs 0.1-0.6 %.
 constexpr long kKeepInputBytes = 128L << 20;
-constexpr bool keep_input(long bytes) { return bytes <= kKeepInputBytes; }
+constexpr bool keep_input(long bytes, bool read_again) { return read_again && bytes <= kKeepInputBytes; }
 
 struct FwdArgs {
     void* y; float* inv_rms; const void* x; const void* w;
@@ -231,7 +234,7 @@ hipError_t launch_row_probe(void* dst, const void* a, const void* b, long rows, 
 // split by rows, as are inputs above the "swiglu_max_units" option.
 constexpr int kSwigluElementwise = 0, kSwigluAligned = 1, kSwigluRagged = 2;
 void set_swiglu_max_units(long units);
-hipError_t launch_swiglu_fwd(int dtype, int mode, int unroll, int xcd_group, void* h, const void* gu, long M, long H,
+hipError_t launch_swiglu_fwd(int dtype, int mode, int unroll, int xcd_group, bool read_again, void* h, const void* gu, long M, long H,
                              hipStream_t s);
 hipError_t launch_swiglu_bwd(int dtype, int mode, int unroll, int xcd_group, void* dgu, const void* dh, const void* gu,
                              long M, long H, hipStream_t s);

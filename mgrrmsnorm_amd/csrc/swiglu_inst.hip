@@ -96,7 +96,7 @@ long rows_per_launch_for(long units_per_row) {
 }
 
 template <typename T, int UNROLL>
-hipError_t fwd_vec(int xg, void* h, const void* gu, long M, long H, hipStream_t s) {
+hipError_t fwd_vec(int xg, bool read_again, void* h, const void* gu, long M, long H, hipStream_t s) {
     const long nvr = H * (long)sizeof(T) / 16;
     const long rows_per_launch = rows_per_launch_for(nvr);
     const FastDiv fd = make_fastdiv((uint32_t)nvr);
@@ -104,8 +104,8 @@ hipError_t fwd_vec(int xg, void* h, const void* gu, long M, long H, hipStream_t 
         const long m = (M - r0) < rows_per_launch ? (M - r0) : rows_per_launch;
         const uint32_t total = (uint32_t)(m * nvr);
         const unsigned grid = (unsigned)((total + 256u * UNROLL - 1) / (256u * UNROLL));
-        hipError_t e = launch(keep_input(2 * M * H * (long)sizeof(T)) ? swiglu_fwd_vec<T, UNROLL, true> : swiglu_fwd_vec<T, UNROLL, false>,
-                              dim3(grid), dim3(256), 0, s, (T*)h + r0 * H, (const T*)gu + r0 * 2 * H, total, fd, xg);
+        const auto kernel = keep_input(2 * M * H * (long)sizeof(T), read_again) ? swiglu_fwd_vec<T, UNROLL, true> : swiglu_fwd_vec<T, UNROLL, false>;
+        hipError_t e = launch(kernel, dim3(grid), dim3(256), 0, s, (T*)h + r0 * H, (const T*)gu + r0 * 2 * H, total, fd, xg);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -197,14 +197,14 @@ hipError_t bwd_gen(void* dgu, const void* dh, const void* gu, long M, long H, hi
 }
 
 template <typename T>
-hipError_t fwd_t(int mode, int unroll, int xg, void* h, const void* gu, long M, long H, hipStream_t s) {
+hipError_t fwd_t(int mode, int unroll, int xg, bool read_again, void* h, const void* gu, long M, long H, hipStream_t s) {
     if (mode == kSwigluElementwise) return fwd_gen<T>(h, gu, M, H, s);
     if (mode == kSwigluRagged) return fwd_ragged<T>(xg, h, gu, M, H, s);
     switch (unroll) {
-        case 1: return fwd_vec<T, 1>(xg, h, gu, M, H, s);
-        case 2: return fwd_vec<T, 2>(xg, h, gu, M, H, s);
-        case 4: return fwd_vec<T, 4>(xg, h, gu, M, H, s);
-        case 8: return fwd_vec<T, 8>(xg, h, gu, M, H, s);
+        case 1: return fwd_vec<T, 1>(xg, read_again, h, gu, M, H, s);
+        case 2: return fwd_vec<T, 2>(xg, read_again, h, gu, M, H, s);
+        case 4: return fwd_vec<T, 4>(xg, read_again, h, gu, M, H, s);
+        case 8: return fwd_vec<T, 8>(xg, read_again, h, gu, M, H, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -228,12 +228,12 @@ void set_swiglu_max_units(long units) {
     g_max_units.store(units >= 1 && units <= kMaxUnitsPerLaunchDefault ? units : kMaxUnitsPerLaunchDefault);
 }
 
-hipError_t launch_swiglu_fwd(int dtype, int mode, int unroll, int xg, void* h, const void* gu, long M, long H,
+hipError_t launch_swiglu_fwd(int dtype, int mode, int unroll, int xg, bool read_again, void* h, const void* gu, long M, long H,
                              hipStream_t s) {
     switch (dtype) {
-        case MG_F32: return fwd_t<float>(mode, unroll, xg, h, gu, M, H, s);
-        case MG_F16: return fwd_t<half_t>(mode, unroll, xg, h, gu, M, H, s);
-        case MG_BF16: return fwd_t<bf16_t>(mode, unroll, xg, h, gu, M, H, s);
+        case MG_F32: return fwd_t<float>(mode, unroll, xg, read_again, h, gu, M, H, s);
+        case MG_F16: return fwd_t<half_t>(mode, unroll, xg, read_again, h, gu, M, H, s);
+        case MG_BF16: return fwd_t<bf16_t>(mode, unroll, xg, read_again, h, gu, M, H, s);
         default: return hipErrorInvalidValue;
     }
 }

@@ -137,7 +137,8 @@ std::vector<Tensor> rmsnorm_backward(const Tensor& grad_output, const Tensor& in
     return {std::get<0>(r), std::get<2>(r)};
 }
 
-Tensor swiglu_forward(const Tensor& gate_up, int64_t hidden_dim) {
+// `backward_follows`: gate_up will be read again
+Tensor swiglu_forward_impl(const Tensor& gate_up, int64_t hidden_dim, bool backward_follows) {
     check_input(gate_up, "w12_out");
     TORCH_CHECK(gate_up.dim() == 2 && gate_up.size(1) == 2 * hidden_dim, "expected a [M, ", 2 * hidden_dim,
                 "] matrix, got ", gate_up.sizes());
@@ -145,10 +146,13 @@ Tensor swiglu_forward(const Tensor& gate_up, int64_t hidden_dim) {
     const int64_t M = gate_up.size(0);
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(gate_up.device());
     auto out = at::empty({M, hidden_dim}, gate_up.options());
-    const int rc = mg_swiglu_fwd(out.data_ptr(), gate_up.data_ptr(), M, hidden_dim, code, current_stream());
+    const auto forward = backward_follows ? mg_swiglu_fwd : mg_swiglu_fwd_only;
+    const int rc = forward(out.data_ptr(), gate_up.data_ptr(), M, hidden_dim, code, current_stream());
     TORCH_CHECK(rc == MG_OK, "SwiGLU forward failed (code ", rc, "): ", mg_last_error());
     return out;
 }
+
+Tensor swiglu_forward(const Tensor& gate_up, int64_t hidden_dim) { return swiglu_forward_impl(gate_up, hidden_dim, true); }
 
 Tensor swiglu_backward(const Tensor& grad_out, const Tensor& gate_up, int64_t hidden_dim) {
     check_input(grad_out, "grad_output");
@@ -261,7 +265,7 @@ Tensor swiglu(const Tensor& w12_out, int64_t hidden_dim) {
     auto fused = w12_out.contiguous();
     auto shape = fused.sizes().vec();
     shape.back() = hidden_dim;
-    return as_shape(swiglu_forward(as_rows(fused, 2 * hidden_dim), hidden_dim), shape);
+    return as_shape(swiglu_forward_impl(as_rows(fused, 2 * hidden_dim), hidden_dim, false), shape);
 }
 
 // Where the two kernels of mg_block_gate_up and mg_block_down take no more GPU time than the projections

@@ -117,6 +117,7 @@ def rmsnorm(input: torch.Tensor, weight: torch.Tensor, epsilon: float = 1e-5) ->
     ext = _extension()
     if ext is not None:
         return ext.rmsnorm(input, weight, epsilon)     # autograd node in C++
+    from . import ops_ctypes
     from .rmsnorm import RMSNormFunction
 
     if torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad):
@@ -126,7 +127,7 @@ def rmsnorm(input: torch.Tensor, weight: torch.Tensor, epsilon: float = 1e-5) ->
         raise RuntimeError("RMSNorm needs at least one dimension")
     x2d = (input if input.is_contiguous() else input.contiguous()).view(-1, shape[-1])
     w = weight if weight.is_contiguous() else weight.contiguous()
-    return rmsnorm_forward(x2d, w, epsilon)[0].view(shape)
+    return ops_ctypes.rmsnorm_output(x2d, w, epsilon).view(shape)
 
 
 def swiglu(w12_out: torch.Tensor, hidden_dim: int) -> torch.Tensor:
@@ -134,6 +135,7 @@ def swiglu(w12_out: torch.Tensor, hidden_dim: int) -> torch.Tensor:
     ext = _extension()
     if ext is not None:
         return ext.swiglu(w12_out, hidden_dim)         # autograd node in C++
+    from . import ops_ctypes
     from .swiglu import MegaGemmFunction
 
     if torch.is_grad_enabled() and w12_out.requires_grad:
@@ -141,7 +143,7 @@ def swiglu(w12_out: torch.Tensor, hidden_dim: int) -> torch.Tensor:
     if w12_out.dim() < 1 or w12_out.size(-1) != 2 * hidden_dim:
         raise RuntimeError(f"last dimension must be 2*hidden_dim = {2 * hidden_dim}, got {tuple(w12_out.shape)}")
     fused = w12_out if w12_out.is_contiguous() else w12_out.contiguous()
-    return swiglu_forward(fused.view(-1, 2 * hidden_dim), hidden_dim).view(*fused.shape[:-1], hidden_dim)
+    return ops_ctypes.swiglu_output(fused.view(-1, 2 * hidden_dim), hidden_dim).view(*fused.shape[:-1], hidden_dim)
 
 
 def swiglu_block_fits(x: torch.Tensor, hidden_dim: int) -> bool:

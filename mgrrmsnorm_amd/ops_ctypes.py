@@ -49,6 +49,15 @@ def _check_pair(input: torch.Tensor, weight: torch.Tensor) -> None:
 
 def rmsnorm_forward(input: torch.Tensor, weight: torch.Tensor, epsilon: float):
     """y = x * rsqrt(mean(x^2) + eps) * w.  Returns [output, inv_rms]."""
+    return _rmsnorm_forward(input, weight, epsilon, True)
+
+
+def rmsnorm_output(input: torch.Tensor, weight: torch.Tensor, epsilon: float):
+    """The output of rmsnorm_forward alone, where no backward pass follows."""
+    return _rmsnorm_forward(input, weight, epsilon, False)[0]
+
+
+def _rmsnorm_forward(input, weight, epsilon, backward_follows):
     if not (input.is_cuda and weight.is_cuda and input.is_contiguous() and weight.is_contiguous()):
         for t, n in ((input, "input"), (weight, "weight")):
             _require_gpu(t, n)
@@ -64,9 +73,9 @@ def rmsnorm_forward(input: torch.Tensor, weight: torch.Tensor, epsilon: float):
     dev = input.device
     with _lib.device_of(dev):
         output = torch.empty_like(input)
-        inv_rms = torch.empty((rows,), dtype=torch.float32, device=dev)
-        rc = lib.mg_rmsnorm_fwd(output.data_ptr(), inv_rms.data_ptr(), input.data_ptr(), weight.data_ptr(),
-                                rows, cols, epsilon, code, _lib.stream_ptr(dev))
+        inv_rms = torch.empty((rows,), dtype=torch.float32, device=dev) if backward_follows else None
+        rc = lib.mg_rmsnorm_fwd(output.data_ptr(), None if inv_rms is None else inv_rms.data_ptr(), input.data_ptr(),
+                                weight.data_ptr(), rows, cols, epsilon, code, _lib.stream_ptr(dev))
     if rc != 0:
         _lib.check(rc, "RMSNorm forward")
     return [output, inv_rms]
@@ -158,6 +167,15 @@ def rmsnorm_backward(grad_output: torch.Tensor, input: torch.Tensor, weight: tor
 
 def swiglu_forward(gate_up: torch.Tensor, hidden_dim: int) -> torch.Tensor:
     """gate_up: [M, 2*hidden_dim] = [gate | up] per row -> [M, hidden_dim]."""
+    return _swiglu_forward(gate_up, hidden_dim, True)
+
+
+def swiglu_output(gate_up: torch.Tensor, hidden_dim: int) -> torch.Tensor:
+    """swiglu_forward where no backward pass follows."""
+    return _swiglu_forward(gate_up, hidden_dim, False)
+
+
+def _swiglu_forward(gate_up, hidden_dim, backward_follows):
     _require_gpu(gate_up, "w12_out")
     _require_contiguous(gate_up, "w12_out")
     if gate_up.dim() != 2 or gate_up.size(1) != 2 * hidden_dim:
@@ -167,8 +185,8 @@ def swiglu_forward(gate_up: torch.Tensor, hidden_dim: int) -> torch.Tensor:
     lib = _lib.load()
     with _lib.device_of(gate_up.device):
         out = torch.empty((M, hidden_dim), dtype=gate_up.dtype, device=gate_up.device)
-        rc = lib.mg_swiglu_fwd(out.data_ptr(), gate_up.data_ptr(), M, hidden_dim, code,
-                               _lib.stream_ptr(gate_up.device))
+        forward = lib.mg_swiglu_fwd if backward_follows else lib.mg_swiglu_fwd_only
+        rc = forward(out.data_ptr(), gate_up.data_ptr(), M, hidden_dim, code, _lib.stream_ptr(gate_up.device))
     _lib.check(rc, "SwiGLU forward")
     return out
 

@@ -46,7 +46,7 @@ def test_header_declares_the_expected_entry_points():
         "mg_rmsnorm_launch_info", "mg_rmsnorm_bwd_timeline"])
     # one launch for what takes several
     assert _declared_in(FUSED_HEADER) == sorted([
-        "mg_rmsnorm_bwd_small_fits", "mg_rmsnorm_bwd_small", "mg_block_gate_up", "mg_block_down"])
+        "mg_rmsnorm_bwd_small_fits", "mg_rmsnorm_bwd_small", "mg_block_gate_up", "mg_block_down", "mg_swiglu_fwd_only"])
 
 
 def test_library_exports_every_declared_symbol(lib):
@@ -199,6 +199,16 @@ def test_one_launch_entry_points_refuse_outputs_over_inputs(lib):
     assert lib.mg_block_gate_up(at["x"], at["x"], at["w"], tokens, d, h, 2, None) == -1 and "overlaps" in _err(lib)
     assert lib.mg_block_gate_up(at["w"] + 2 * h * d * 2 - 2, at["x"], at["w"], tokens, d, h, 2, None) == -1 and "overlaps" in _err(lib)
     assert lib.mg_block_down(at["x"] + tokens * h * 2 - 2, at["x"], at["w"], tokens, d, h, 2, None) == -1 and "overlaps" in _err(lib)
+
+
+def test_swiglu_fwd_only_rejects_what_swiglu_fwd_rejects(lib):
+    f = lib.mg_swiglu_fwd_only
+    assert f(FAKE, FAKE, 4, 0, 2, None) == -1 and "mg_swiglu_fwd_only: H" in _err(lib)
+    assert f(FAKE, FAKE, -1, 8, 2, None) == -1 and f(FAKE, FAKE, 4, 8, 4, None) == -1
+    assert f(None, FAKE, 4, 8, 2, None) == -1 and "mg_swiglu_fwd_only" in _err(lib)
+    assert f(FAKE, FAKE + 1, 4, 8, 2, None) == -1 and "aligned" in _err(lib)
+    assert f(FAKE, FAKE, 4, 1 << 30, 2, None) == -2 and f(FAKE, FAKE, 1 << 39, 4, 2, None) == -2
+    assert f(None, None, 0, 8, 2, None) == 0
 
 
 def test_copy_bytes_rejects_bad_arguments(lib):

@@ -49,3 +49,41 @@ def test_swiglu_forward_on_both_sides_of_the_line(hidden, dtype):
     h = ops.swiglu_forward(block, hidden)
     for rows in (at, at + 1):
         assert torch.equal(ops.swiglu_forward(_copies(block, rows), hidden), _copies(h, rows))
+
+
+def _kernels(fn):
+    """Names of this library's forward kernels that `fn` launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events() if "rmsnorm_fwd" in e.name or "swiglu_fwd" in e.name]
+
+
+@pytest.mark.parametrize("backend", ["extension", "ctypes"])
+@pytest.mark.parametrize("path", ["rmsnorm", "swiglu"])
+def test_inputs_are_kept_only_for_a_backward_pass(monkeypatch, backend, path):
+    """Without a gradient to compute, an input of any size is read as a large one is."""
+    import mgrrmsnorm_amd
+    from mgrrmsnorm_amd import ops
+
+    assert ops.backend() == "extension"
+    if backend == "ctypes":
+        monkeypatch.setattr(ops, "_binding", None)
+    cols = 1024
+    norm = mgrrmsnorm_amd.RMSNorm(cols).cuda().to(BF16)
+    call = norm if path == "rmsnorm" else lambda x: ops.swiglu(x, cols // 2)
+    small, large = (torch.zeros(rows, cols, device="cuda", dtype=BF16) for rows in (512, LINE // (cols * 2) + 1))
+
+    def name(x, grad):
+        with torch.set_grad_enabled(grad):
+            got = _kernels(lambda: call(x.requires_grad_(grad)))
+        assert len(got) == 1, got
+        return got[0]
+
+    streamed = name(large, True)
+    assert name(small, True) != streamed
+    assert name(small, False) == streamed and name(large, False) == streamed
