@@ -32,6 +32,8 @@ UNITS = [
     ("mg_api.hip", "mg_api", []),
     ("swiglu_inst.hip", "swiglu_inst", []),
     ("block_inst.hip", "block_inst", []),
+    ("mlp_inst.hip", "mlp_f16", ["-DMG_DTYPE=1"]),
+    ("mlp_inst.hip", "mlp_bf16", ["-DMG_DTYPE=2"]),
     ("rmsnorm_fwd_inst.hip", "rmsnorm_fwd_f32", ["-DMG_DTYPE=0"]),
     ("rmsnorm_fwd_inst.hip", "rmsnorm_fwd_f16", ["-DMG_DTYPE=1"]),
     ("rmsnorm_fwd_inst.hip", "rmsnorm_fwd_bf16", ["-DMG_DTYPE=2"]),

@@ -55,6 +55,14 @@ SIGNATURES = {
     "mg_block_down": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
 }
 
+# the same for include/megagemm_hip_mlp.h
+MLP_SIGNATURES = {
+    "mg_mlp_fits": (_int, [_i64, _i64, _i64, _int]),
+    "mg_mlp_preferred": (_int, [_i64, _i64, _i64, _int]),
+    "mg_mlp_fwd": (_int, [_vp] * 6 + [_i64, _i64, _i64, _int, _vp]),
+    "mg_mlp_bwd": (_int, [_vp] * 10 + [_i64, _i64, _i64, _int, _vp]),
+}
+
 
 def load() -> ctypes.CDLL:
     """Load the library once per process; raise RuntimeError when it has not been built."""
@@ -75,7 +83,7 @@ def load() -> ctypes.CDLL:
         try:
             got = lib.mg_abi_version()      # before anything that another version may not have
             if got == ABI_VERSION:
-                for name, (restype, argtypes) in SIGNATURES.items():
+                for name, (restype, argtypes) in [*SIGNATURES.items(), *MLP_SIGNATURES.items()]:
                     fn = getattr(lib, name)
                     fn.restype = restype
                     fn.argtypes = argtypes

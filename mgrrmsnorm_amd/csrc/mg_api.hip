@@ -3,6 +3,7 @@
 // without a GPU.
 #include "megagemm_hip.h"
 #include "megagemm_hip_fused.h"
+#include "megagemm_hip_mlp.h"
 #include "megagemm_hip_tuning.h"
 #include "mg_launch.hpp"
 #include "mg_device.hpp"
@@ -757,6 +758,104 @@ int mg_block_gate_up(void* h, const void* x, const void* w12, int64_t tokens, in
 int mg_block_down(void* out, const void* h, const void* w3, int64_t tokens, int64_t d_model, int64_t hidden,
                   int dtype, void* stream) {
     return block_projection("mg_block_down", false, out, h, w3, tokens, hidden, d_model, dtype, stream);
+}
+
+// The kernels address every tensor with 32-bit byte offsets that have to stay apart from kNowhere, tiles reaching past
+// the end included.
+int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
+    if (dtype != MG_F16 && dtype != MG_BF16) return 0;
+    if (tokens < 1 || d_model < 64 || hidden < 64 || d_model % 64 != 0 || hidden % 64 != 0) return 0;
+    if (tokens > (1LL << 24) || d_model > 65536 || hidden > 65536) return 0;
+    const int64_t most = (1LL << 31) - 1;
+    return tokens * d_model * 2 <= most && tokens * hidden * 4 <= most && hidden * d_model * 4 <= most;
+}
+
+// Where forward + backward and forward alone both take no more time than the library's products with the activation
+// between them, GPU time in a replayed graph and eager (library / these, us, bf16, d_model x hidden, forward + backward; forward).
+// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162.6 / 47.2.
+//   256 tokens and more: 512 x 1024, 300 60.7 / 49.0; 21.2 / 17.0; 2048 x 3584, 300 142.6 / 108.3; 43.4 / 37.9, 1024 213.6 / 169.4;
+//     64.2 / 56.8, 4096 560 / 496; 166 / 156; 2048 x 5504, 300 203.9 / 197.4; 53.2 / 50.6; beyond 128 MiB of weights,
+//     4096 x 11008, 300 567 / 488; 133 / 151;
+//   fewer: 512 x 1024, 80 46.8 / 43.0; 17.8 / 16.3; beyond 4 MiB, 1024 x 2816, 80 76.3 / 80.2; 19.6 / 24.6.
+int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
+    if (tokens <= MG_BLOCK_MAX_TOKENS || !mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
+    return tokens <= 4096 && 6 * d_model * hidden <= (tokens >= 256 ? 128LL << 20 : 4LL << 20);
+}
+
+namespace {
+
+struct MlpTensor { const char* name; const void* p; int64_t bytes; };
+
+int check_mlp(const char* fn, int64_t tokens, int64_t d_model, int64_t hidden, int dtype, const MlpTensor* out, int outs,
+              const MlpTensor* in, int ins) {
+    if (!mg_mlp_fits(tokens, d_model, hidden, dtype))
+        return fail(MG_ERR_UNSUPPORTED, "%s: %lld tokens of %lld x %lld with dtype %d is not for it (fp16 or bf16, widths multiples of 64, "
+                    "tensors below 2 GiB)", fn, (long long)tokens, (long long)d_model, (long long)hidden, dtype);
+    for (int i = 0; i < ins; ++i)
+        if (in[i].p == nullptr) return fail(MG_ERR_INVALID_ARG, "%s: %s must not be NULL", fn, in[i].name);
+    for (int i = 0; i < ins + outs; ++i) {
+        const MlpTensor& t = i < ins ? in[i] : out[i - ins];
+        if (!aligned(t.p, 16)) return fail(MG_ERR_INVALID_ARG, "%s: %s is not 16-byte aligned", fn, t.name);
+    }
+    for (int i = 0; i < outs; ++i) {
+        for (int k = 0; k < ins; ++k)
+            if (overlap(out[i].p, out[i].bytes, in[k].p, in[k].bytes))
+                return fail(MG_ERR_INVALID_ARG, "%s: %s overlaps %s", fn, out[i].name, in[k].name);
+        for (int k = 0; k < i; ++k)
+            if (overlap(out[i].p, out[i].bytes, out[k].p, out[k].bytes))
+                return fail(MG_ERR_INVALID_ARG, "%s: %s overlaps %s", fn, out[i].name, out[k].name);
+    }
+    return MG_OK;
+}
+
+int run_mlp(const char* fn, int dtype, MlpWhat what, MlpArgs a, hipStream_t s) {
+    const int rc = cu_count(&a.cus);
+    if (rc != MG_OK) return rc;
+    const hipError_t e = dtype == MG_F16 ? launch_mlp<half_t>(what, a, s) : launch_mlp<bf16_t>(what, a, s);
+    return e == hipSuccess ? MG_OK : fail_hip(fn, e);
+}
+
+}  // namespace
+
+int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12, const void* w3, int64_t tokens,
+               int64_t d_model, int64_t hidden, int dtype, void* stream) {
+    const int64_t td = tokens * d_model * 2, th = tokens * hidden * 2, w = d_model * hidden * 2;
+    const MlpTensor in[] = {{"x", x, td}, {"w12", w12, 2 * w}, {"w3", w3, w}}, outs[] = {{"out", out, td}, {"h", h, th}, {"gate_up", gate_up, 2 * th}};
+    int rc = check_mlp("mg_mlp_fwd", tokens, d_model, hidden, dtype, outs, 3, in, 3);
+    if (rc != MG_OK) return rc;
+    if (out == nullptr || h == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_fwd: out and h must not be NULL");
+    const int t = (int)tokens, d = (int)d_model, n = (int)hidden;
+    hipStream_t s = (hipStream_t)stream;
+    rc = run_mlp("mg_mlp_fwd", dtype, MlpWhat::gate_up, {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d, t, n, d, 0}, s);
+    if (rc != MG_OK) return rc;
+    return run_mlp("mg_mlp_fwd", dtype, MlpWhat::down, {out, nullptr, nullptr, h, (uint32_t)th, n, w3, (uint32_t)w, n, t, d, n, 0}, s);
+}
+
+int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy, const void* x, const void* w12, const void* w3,
+               const void* gate_up, const void* h, int64_t tokens, int64_t d_model, int64_t hidden, int dtype, void* stream) {
+    const int64_t td = tokens * d_model * 2, th = tokens * hidden * 2, w = d_model * hidden * 2;
+    const MlpTensor in[] = {{"dy", dy, td}, {"x", x, td}, {"w12", w12, 2 * w}, {"w3", w3, w}, {"gate_up", gate_up, 2 * th}, {"h", h, th}};
+    const MlpTensor outs[] = {{"dx", dx, td}, {"dw12", dw12, 2 * w}, {"dw3", dw3, w}, {"d_gate_up", d_gate_up, 2 * th}};
+    int rc = check_mlp("mg_mlp_bwd", tokens, d_model, hidden, dtype, outs, 4, in, 6);
+    if (rc != MG_OK) return rc;
+    if (d_gate_up == nullptr && (dx != nullptr || dw12 != nullptr))
+        return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
+    const int t = (int)tokens, d = (int)d_model, n = (int)hidden;
+    hipStream_t s = (hipStream_t)stream;
+    if (dw3 != nullptr) {
+        rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::weight_grad, {dw3, nullptr, nullptr, dy, (uint32_t)td, d, h, (uint32_t)th, n, d, n, t, 0}, s);
+        if (rc != MG_OK) return rc;
+    }
+    if (dx == nullptr && dw12 == nullptr) return MG_OK;
+    rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::activation_bwd,
+                 {d_gate_up, nullptr, gate_up, dy, (uint32_t)td, d, w3, (uint32_t)w, n, t, n, d, 0}, s);
+    if (rc == MG_OK && dw12 != nullptr)
+        rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::weight_grad,
+                     {dw12, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, x, (uint32_t)td, d, 2 * n, d, t, 0}, s);
+    if (rc == MG_OK && dx != nullptr)
+        rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::input_grad,
+                     {dx, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, w12, (uint32_t)(2 * w), d, t, d, 2 * n, 0}, s);
+    return rc;
 }
 
 }  // extern "C"

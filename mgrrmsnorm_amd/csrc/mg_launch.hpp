@@ -245,4 +245,16 @@ constexpr int kSkinnyMaxTokens = 64;
 struct SkinnyArgs { void* out; const void* x; const void* w; int tokens, K, N, cus; };
 hipError_t launch_skinny_gemm(int dtype, bool paired, const SkinnyArgs& a, hipStream_t s);
 
+// Products of the whole SwiGLU block (mlp_gemm.hpp): out [M, N] from a and b, each `*_bytes` long with `*_ld` elements
+// per line.  gate_up: b holds N gate rows, then N up rows; out may be NULL, second gets the activation.  activation_bwd: `in` is
+// [gate | up].  weight_grad: a is [K, M], b [K, N], any K; otherwise a is [M, K] with K a multiple of 64.
+enum class MlpWhat { gate_up, down, activation_bwd, input_grad, weight_grad };
+struct MlpArgs {
+    void* out; void* second; const void* in;
+    const void* a; uint32_t a_bytes; int a_ld;
+    const void* b; uint32_t b_bytes; int b_ld;
+    int M, N, K, cus;
+};
+template <typename T> hipError_t launch_mlp(MlpWhat what, const MlpArgs& a, hipStream_t s);
+
 }  // namespace mg

@@ -24,6 +24,7 @@
 
 #include "megagemm_hip.h"
 #include "megagemm_hip_fused.h"
+#include "megagemm_hip_mlp.h"
 
 namespace {
 
@@ -332,6 +333,112 @@ Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     return out;
 }
 
+// ---- the whole block on this package's own products ----
+// A dense tensor of a GPU that nothing else wants to see the operations of: no transform of torch.func, no
+// tangent, no lazy conjugate or negative, no subclass.
+bool plain_dense(const Tensor& t) {
+    constexpr c10::DispatchKeySet others({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
+                                          c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
+                                          c10::DispatchKey::ZeroTensor, c10::DispatchKey::NestedTensor});
+    return t.layout() == at::kStrided && t.is_cuda() && !t.key_set().has_any(others) && !t._fw_grad(0).defined();
+}
+
+// Saved tensors that somebody packs (checkpointing, offloading) and torch.func's transforms are for the
+// projections, whose tensors these have always been.
+bool calls_transformed() {
+    return at::SavedTensorDefaultHooks::get_hooks(false).has_value() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+Tensor mlp_forward(const Tensor& x, const Tensor& w12, const Tensor& w3, Tensor* gate_up, Tensor* h) {
+    const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = x.numel() / d_model;
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    if (gate_up != nullptr) *gate_up = at::empty({tokens, 2 * hidden}, x.options());
+    *h = at::empty({tokens, hidden}, x.options());
+    auto out = empty_as(x);
+    const int rc = mg_mlp_fwd(out.data_ptr(), h->data_ptr(), gate_up != nullptr ? gate_up->data_ptr() : nullptr, x.data_ptr(),
+                              w12.data_ptr(), w3.data_ptr(), tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
+    TORCH_CHECK(rc == MG_OK, "SwiGLU block forward failed (code ", rc, "): ", mg_last_error());
+    return out;
+}
+
+Tensor swiglu_projections(const Tensor& x, const Tensor& w12, const Tensor& w3) {
+    return at::linear(swiglu(at::linear(x, w12), w3.size(1)), w3);
+}
+
+struct MlpNode : public torch::autograd::Function<MlpNode> {
+    static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w12, const Tensor& w3) {
+        // Aliases even of what is contiguous: they keep the data they were made of when a caller gives an operand other
+        // data before the backward pass.  The operands themselves are for a backward pass that records its own graph.
+        const Tensor xd = x.contiguous().detach(), ad = w12.detach(), bd = w3.detach();
+        Tensor gate_up, h;
+        const Tensor out = mlp_forward(xd, ad, bd, &gate_up, &h);
+        ctx->save_for_backward({xd, ad, bd, gate_up, h, x, w12, w3});
+        return out;
+    }
+
+    static torch::autograd::tensor_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::tensor_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const bool want[] = {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2)};
+        torch::autograd::tensor_list out(3);
+        if (torch::GradMode::is_enabled()) {   // create_graph: through operations that record it (or refuse, as the activation does)
+            torch::autograd::variable_list wanted;
+            for (int i = 0; i < 3; ++i)
+                if (want[i]) wanted.push_back(saved[5 + i]);
+            const auto y = swiglu_projections(saved[5], saved[6], saved[7]);
+            const auto g = torch::autograd::grad({y}, wanted, {grads[0].to(y.scalar_type())}, true, true, true);
+            for (int i = 0, k = 0; i < 3; ++i)
+                if (want[i]) out[i] = g[k++];
+            return out;
+        }
+        const Tensor &x = saved[0], &w12 = saved[1], &w3 = saved[2], &gate_up = saved[3], &h = saved[4];
+        const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = x.numel() / d_model;
+        const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+        auto dy = grads[0].contiguous();
+        if (dy.scalar_type() != x.scalar_type()) dy = dy.to(x.scalar_type());
+        if (reinterpret_cast<uintptr_t>(dy.data_ptr()) % 16 != 0) dy = dy.clone();
+        Tensor d_gate_up;
+        if (want[0] || want[1]) d_gate_up = empty_as(gate_up);
+        for (int i = 0; i < 3; ++i)
+            if (want[i]) out[i] = empty_as(saved[i]);
+        const auto at = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
+        const int rc = mg_mlp_bwd(at(out[0]), at(out[1]), at(out[2]), at(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
+                                  gate_up.data_ptr(), h.data_ptr(), tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
+        TORCH_CHECK(rc == MG_OK, "SwiGLU block backward failed (code ", rc, "): ", mg_last_error());
+        return out;
+    }
+};
+
+// Whether a block of this hidden width may take `x` to swiglu_mlp at all, from x alone.
+bool swiglu_mlp_fits(const Tensor& x, int64_t hidden) {
+    const auto type = x.scalar_type();
+    if ((type != at::kHalf && type != at::kBFloat16) || !x.is_cuda() || x.dim() < 1 || x.size(-1) < 1) return false;
+    return mg_mlp_preferred(x.numel() / x.size(-1), x.size(-1), hidden, dtype_code(type)) == 1;
+}
+
+// w3(silu(gate) * up) with [gate | up] = w12(x), differentiable, in this package's own products; an undefined tensor
+// (None) where the call is not one of theirs, and the caller then goes through the projections and the activation.
+Tensor swiglu_mlp(const Tensor& x, const Tensor& w12, const Tensor& w3) {
+    const Tensor none;
+    const auto type = x.scalar_type();
+    if ((type != at::kHalf && type != at::kBFloat16) || x.dim() < 1 || w12.dim() != 2 || w3.dim() != 2) return none;
+    if (!plain_dense(x) || !plain_dense(w12) || !plain_dense(w3) || calls_transformed()) return none;
+    const int64_t d_model = w3.size(0), hidden = w3.size(1);
+    if (d_model < 1 || x.size(-1) != d_model || w12.size(0) != 2 * hidden || w12.size(1) != d_model) return none;
+    if (w12.scalar_type() != type || w3.scalar_type() != type || w12.device() != x.device() || w3.device() != x.device() ||
+        !w12.is_contiguous() || !w3.is_contiguous())
+        return none;
+    if (mg_mlp_preferred(x.numel() / d_model, d_model, hidden, dtype_code(type)) != 1) return none;
+    const auto off = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; };
+    if (off(w12) || off(w3) || (x.is_contiguous() && off(x))) return none;   // a copy of x is aligned
+    if (torch::GradMode::is_enabled() && (x.requires_grad() || w12.requires_grad() || w3.requires_grad())) {
+        if (!x.requires_grad() && !w12.requires_grad()) return none;   // only w3 learns: nothing of the activation has to be kept
+        return MlpNode::apply(x, w12, w3);
+    }
+    Tensor h;
+    return mlp_forward(x.contiguous(), w12, w3, nullptr, &h);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -356,6 +463,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("x"), py::arg("w12"), py::arg("w3"));
     m.def("swiglu_block_fits", &swiglu_block_fits, "whether the size and type of x are for swiglu_block", py::arg("x"),
           py::arg("hidden_dim"));
+    m.def("swiglu_mlp", &swiglu_mlp, "the whole SwiGLU block, differentiable, on the package's own products; None where it does not apply",
+          py::arg("x"), py::arg("w12"), py::arg("w3"));
+    m.def("swiglu_mlp_fits", &swiglu_mlp_fits, "whether the size and type of x are for swiglu_mlp", py::arg("x"), py::arg("hidden_dim"));
     m.def("swiglu", &swiglu, "differentiable silu(gate) * up over the last dimension", py::arg("w12_out"),
           py::arg("hidden_dim"));
 }

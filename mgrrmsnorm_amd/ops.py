@@ -158,3 +158,25 @@ def swiglu_block(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
     built) and has to go through the projections and `swiglu`."""
     ext = _extension()
     return ext.swiglu_block(x, w12, w3) if ext is not None else None
+
+
+def swiglu_mlp_fits(x: torch.Tensor, hidden_dim: int) -> bool:
+    """Whether `x` alone -- its size, type and device -- could be for `swiglu_mlp`."""
+    ext = _extension()
+    if ext is not None:
+        return ext.swiglu_mlp_fits(x, hidden_dim)
+    from . import ops_ctypes
+
+    return ops_ctypes.swiglu_mlp_fits(x, hidden_dim)
+
+
+def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
+    """Differentiable w3(silu(gate) * up) with [gate | up] = w12(x) on this package's own matrix products,
+    for more rows than a decoding step has; None when the call is not of that kind and has to go
+    through the projections and `swiglu`."""
+    ext = _extension()
+    if ext is not None:
+        return ext.swiglu_mlp(x, w12, w3)              # autograd node in C++
+    from . import ops_ctypes
+
+    return ops_ctypes.swiglu_mlp(x, w12, w3)

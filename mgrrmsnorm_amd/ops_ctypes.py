@@ -209,3 +209,94 @@ def swiglu_backward(grad_out: torch.Tensor, gate_up: torch.Tensor, hidden_dim: i
                                _lib.stream_ptr(gate_up.device))
     _lib.check(rc, "SwiGLU backward")
     return grad_in
+
+
+# ---- the whole SwiGLU block on the library's own products (megagemm_hip_mlp.h) ----
+
+_MLP_CODES = {torch.float16: 1, torch.bfloat16: 2}
+
+
+def swiglu_mlp_fits(x: torch.Tensor, hidden_dim: int) -> bool:
+    code = _MLP_CODES.get(x.dtype)
+    if code is None or not x.is_cuda or x.dim() < 1 or x.size(-1) < 1:
+        return False
+    return _lib.load().mg_mlp_preferred(x.numel() // x.size(-1), x.size(-1), hidden_dim, code) == 1
+
+
+def _plain_dense(t: torch.Tensor) -> bool:
+    """A dense tensor of a GPU that nothing else wants to see the operations of."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout is torch.strided and t.is_cuda and not t.is_nested
+            and not t.is_conj() and not t.is_neg() and not t._is_zerotensor()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
+
+
+def _pointer(t) -> int | None:
+    return None if t is None else t.data_ptr()
+
+
+def _mlp_forward(x, w12, w3, keep_gate_up):
+    d_model, hidden = w3.shape
+    tokens = x.numel() // d_model
+    with _lib.device_of(x.device):
+        gate_up = x.new_empty(tokens, 2 * hidden) if keep_gate_up else None
+        h = x.new_empty(tokens, hidden)
+        out = torch.empty_like(x)
+        rc = _lib.load().mg_mlp_fwd(out.data_ptr(), h.data_ptr(), _pointer(gate_up), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
+                                    tokens, d_model, hidden, _MLP_CODES[x.dtype], _lib.stream_ptr(x.device))
+    _lib.check(rc, "SwiGLU block forward")
+    return out, gate_up, h
+
+
+class _MlpFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w12, w3):
+        # aliases even of what is contiguous: they keep the data they were made of when a caller gives an operand
+        # other data before the backward pass; the operands themselves are for one that records its own graph
+        xd, ad, bd = x.contiguous().detach(), w12.detach(), w3.detach()
+        out, gate_up, h = _mlp_forward(xd, ad, bd, True)
+        ctx.save_for_backward(xd, ad, bd, gate_up, h, x, w12, w3)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        x, w12, w3, gate_up, h, *operands = ctx.saved_tensors
+        want = ctx.needs_input_grad
+        if torch.is_grad_enabled():      # create_graph: through operations that record it (or refuse, as the activation does)
+            from . import ops
+
+            linear = torch.nn.functional.linear
+            y = linear(ops.swiglu(linear(operands[0], operands[1]), w3.size(1)), operands[2])
+            grads = iter(torch.autograd.grad(y, [t for t, w in zip(operands, want) if w], grad_output.to(y.dtype),
+                                             retain_graph=True, create_graph=True, allow_unused=True))
+            return tuple(next(grads) if w else None for w in want)
+        d_model, hidden = w3.shape
+        dy = grad_output.contiguous().to(x.dtype)
+        if dy.data_ptr() % 16 != 0:
+            dy = dy.clone()
+        with _lib.device_of(x.device):
+            grads = [torch.empty_like(t) if w else None for t, w in zip((x, w12, w3), want)]
+            d_gate_up = torch.empty_like(gate_up) if want[0] or want[1] else None
+            rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
+                                        gate_up.data_ptr(), h.data_ptr(), x.numel() // d_model, d_model, hidden, _MLP_CODES[x.dtype],
+                                        _lib.stream_ptr(x.device))
+        _lib.check(rc, "SwiGLU block backward")
+        return tuple(grads)
+
+
+def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
+    """ops.swiglu_mlp; the same calls are taken as in csrc/torch_binding.cpp."""
+    if x.dtype not in _MLP_CODES or x.dim() < 1 or w12.dim() != 2 or w3.dim() != 2 or not all(map(_plain_dense, (x, w12, w3))):
+        return None
+    if torch._C._autograd._top_saved_tensors_default_hooks(False) is not None or torch._C._functorch.peek_interpreter_stack() is not None:
+        return None
+    d_model, hidden = w3.shape
+    if d_model < 1 or x.size(-1) != d_model or w12.shape != (2 * hidden, d_model):
+        return None
+    if any(w.dtype != x.dtype or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16 != 0 for w in (w12, w3)):
+        return None
+    if not swiglu_mlp_fits(x, hidden) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or w12.requires_grad or w3.requires_grad):
+        return _MlpFunction.apply(x, w12, w3) if x.requires_grad or w12.requires_grad else None
+    return _mlp_forward(x.contiguous(), w12, w3, False)[0]

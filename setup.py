@@ -73,6 +73,6 @@ setup(
     packages=["mgrrmsnorm_amd", "megagemm"],
     py_modules=["rmsnorm_cuda_ops"],
     package_data={"mgrrmsnorm_amd": ["libmegagemm_hip.so", "_binding*.so", "csrc/*.hip", "csrc/*.hpp", "csrc/*.cpp"]},
-    data_files=[("include", ["include/megagemm_hip.h", "include/megagemm_hip_tuning.h", "include/megagemm_hip_fused.h"])],
+    data_files=[("include", ["include/megagemm_hip.h", "include/megagemm_hip_tuning.h", "include/megagemm_hip_fused.h", "include/megagemm_hip_mlp.h"])],
     cmdclass={"build_hip": BuildHip, "build_py": BuildPyWithHip, "develop": DevelopWithHip},
 )

@@ -1,0 +1,83 @@
+"""What of the block's own products can be checked without a GPU: the sizes and arguments the C entry points take,
+and the calls MegaGemmTriton hands to them."""
+import pytest
+import torch
+
+from mgrrmsnorm_amd import _lib, ops
+from test_block_route_cpu import CHANGES, REPLACED, _module
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _lib.load()
+
+
+@pytest.mark.parametrize("tokens,d_model,hidden,dtype,fits", [
+    (1, 64, 64, 1, 1), (0, 64, 64, 1, 0), (1, 64, 64, 0, 0), (5, 96, 64, 2, 0), (5, 64, 96, 2, 0), (5, 65536, 8128, 2, 1), (5, 65536, 8192, 2, 0),
+    (5, 65600, 64, 2, 0), (5, 16384, 32704, 2, 1), (5, 16384, 32768, 2, 0), (1 << 24, 64, 64, 2, 0), (8191, 64, 65536, 2, 1), (8192, 64, 65536, 2, 0),
+])
+def test_sizes(lib, tokens, d_model, hidden, dtype, fits):
+    assert lib.mg_mlp_fits(tokens, d_model, hidden, dtype) == fits
+    assert lib.mg_mlp_preferred(tokens, d_model, hidden, dtype) <= fits
+
+
+def test_bad_arguments_are_refused(lib):
+    t, d, h = 100, 64, 128
+    error = lambda: lib.mg_last_error().decode()
+    p = {n: 0x10000000 * (i + 1) for i, n in enumerate(("out", "h", "gu", "x", "w12", "w3", "dx", "dw12", "dw3", "dgu", "dy"))}
+
+    def fwd(sizes=(t, d, h), dtype=2, **other):
+        q = {**p, **other}
+        return lib.mg_mlp_fwd(*(q[n] for n in ("out", "h", "gu", "x", "w12", "w3")), *sizes, dtype, None)
+
+    def bwd(**other):
+        q = {**p, **other}
+        return lib.mg_mlp_bwd(*(q[n] for n in ("dx", "dw12", "dw3", "dgu", "dy", "x", "w12", "w3", "gu", "h")), t, d, h, 2, None)
+
+    assert fwd((t, d, 96)) == -2 and fwd(dtype=0) == -2 and fwd((0, d, h)) == -2
+    for name in ("out", "h", "x", "w12", "w3"):
+        assert fwd(**{name: None}) == -1 and "NULL" in error()
+    for name in ("dy", "x", "w12", "w3", "gu", "h", "dgu"):
+        assert bwd(**{name: None}) == -1
+    for call, name in ((fwd, "x"), (fwd, "gu"), (bwd, "dw3"), (bwd, "h")):
+        assert call(**{name: p[name] + 8}) == -1 and "aligned" in error()
+    for call, a, b in ((fwd, "out", "x"), (fwd, "h", "gu"), (fwd, "gu", "w12"), (bwd, "dgu", "gu"), (bwd, "dx", "dy"), (bwd, "dw3", "dw12")):
+        assert call(**{a: p[b]}) == -1 and "overlaps" in error()
+
+
+@pytest.fixture
+def handed_over(monkeypatch):
+    """Calls the module and returns the (w12, w3) it handed to ops.swiglu_mlp, or None."""
+    calls = []
+    monkeypatch.setattr(ops, "swiglu_block_fits", lambda x, hidden: False)
+    monkeypatch.setattr(ops, "swiglu_mlp_fits", lambda x, hidden: True)
+    monkeypatch.setattr(ops, "swiglu_mlp", lambda x, w12, w3: calls.append((w12, w3)))
+
+    def call(module):
+        calls.clear()
+        try:
+            module(torch.zeros(2, 16))
+        except RuntimeError:       # past the hand-over: no GPU, or a stand-in of another shape
+            pass
+        return calls[0] if calls else None
+    return call
+
+
+def test_a_module_as_made_is_handed_over(handed_over):
+    m = _module()
+    w12, w3 = handed_over(m)
+    assert w12 is m.w12.weight and w3 is m.w3.weight
+
+
+@pytest.mark.parametrize("change", CHANGES)
+def test_a_changed_projection_is_called(handed_over, change):
+    m = _module()
+    CHANGES[change](m)
+    assert handed_over(m) is None
+
+
+@pytest.mark.parametrize("what", REPLACED)
+def test_a_replaced_function_is_called(handed_over, monkeypatch, what):
+    owner, name, value = REPLACED[what]
+    monkeypatch.setattr(owner, name, value)
+    assert handed_over(_module()) is None

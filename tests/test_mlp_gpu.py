@@ -1,0 +1,264 @@
+"""The SwiGLU block on the package's own matrix products (megagemm_hip_mlp.h): every output against the same
+formula in float64 at the edges of the tiles, and what the module does around it."""
+import pytest
+import torch
+
+import gpu_util as U
+from mgrrmsnorm_amd import MegaGemmTriton, ops
+from test_block_gpu import _case, _within
+
+pytestmark = pytest.mark.gpu
+
+# largest relative error of rounding to p significant bits, 2^-p: bf16 has 8 of them, fp16 11
+ROUNDING = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}
+
+
+def _call(name, tensors, sizes, dtype):
+    U.check(getattr(U.lib(), name)(*[t if t is None else t.data_ptr() for t in tensors], *sizes, U.CODES[dtype], U.stream()))
+
+
+def _guarded(shape, dtype):
+    """An output between two canaries."""
+    n = shape[0] * shape[1]
+    flat = torch.full((n + 512,), 7.0, device="cuda", dtype=dtype)
+    return flat[256:256 + n].view(shape), flat
+
+
+def _intact(*flats):
+    for f in flats:
+        assert (f[:256] == 7).all() and (f[-256:] == 7).all()
+
+
+def _bounded(got, ref, terms, count, dtype, extra=0.0):
+    """One rounding of the result and an fp32 sum of `count` products whose absolute values add up to `terms`."""
+    u, tiny = ROUNDING[dtype], 2.0 ** -25 if dtype == "fp16" else 0.0
+    bound = ((count + 8) * 2.0 ** -24 * terms + extra) * (1 + u) + u * ref.abs() + tiny
+    worst = ((got.double() - ref).abs() - bound).max().item()
+    assert worst <= 0.0, f"beyond the error bound by {worst}"
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("tokens,d_model,hidden", [
+    (1, 64, 64), (65, 64, 192), (127, 192, 64), (128, 128, 128), (129, 128, 256), (257, 320, 448), (300, 704, 1088),
+    (1000, 512, 1344), (1024, 2048, 3584), (513, 1536, 4096), (2047, 1024, 2816), (96, 4096, 6912), (640, 3136, 8384),
+])
+def test_products_against_float64(tokens, d_model, hidden, dtype):
+    x, w12, w3 = _case(tokens, d_model, hidden, dtype)
+    dy = torch.randn(tokens, d_model, device="cuda", generator=torch.Generator("cuda").manual_seed(5)).to(x.dtype)
+    sizes, dt = (tokens, d_model, hidden), x.dtype
+
+    def run():
+        (out, c0), (h, c1), (gu, c2) = (_guarded(s, dt) for s in ((tokens, d_model), (tokens, hidden), (tokens, 2 * hidden)))
+        _call("mg_mlp_fwd", (out, h, gu, x, w12, w3), sizes, dtype)
+        (dx, c3), (da, c4), (db, c5), (dgu, c6) = (_guarded(s, dt) for s in (
+            (tokens, d_model), (2 * hidden, d_model), (d_model, hidden), (tokens, 2 * hidden)))
+        _call("mg_mlp_bwd", (dx, da, db, dgu, dy, x, w12, w3, gu, h), sizes, dtype)
+        _intact(c0, c1, c2, c3, c4, c5, c6)
+        return out, h, gu, dx, da, db, dgu
+
+    out, h, gu, dx, da, db, dgu = first = run()
+    assert all(torch.equal(a, b) for a, b in zip(first, run()))          # fixed summation order
+    _within(out, x, w12, w3, dtype)
+    xd, ad, bd, yd, hd, gd = (t.double() for t in (x, w12, w3, dy, h, gu))
+    _bounded(gu, xd @ ad.t(), xd.abs() @ ad.abs().t(), d_model, dtype)
+    _bounded(out, hd @ bd.t(), hd.abs() @ bd.abs().t(), hidden, dtype)
+    _bounded(db, yd.t() @ hd, yd.abs().t() @ hd.abs(), tokens, dtype)
+    # the activation's backward from the stored gate and up, and the error of the sum it starts from
+    gate, up = gd.chunk(2, -1)
+    dh, terms = yd @ bd, yd.abs() @ bd.abs()
+    s = torch.sigmoid(gate)
+    slope = s * (1 + gate * (1 - s))
+    wiggle = 24 * 2.0 ** -24 * dh.abs()                                  # of the activation's own arithmetic
+    parts = (1 + gate.abs()) * s
+    for got, factor, size in ((dgu[:, :hidden], up * slope, up.abs() * parts), (dgu[:, hidden:], gate * s, gate.abs() * s)):
+        _bounded(got, dh * factor, terms * size, d_model, dtype, wiggle * size)
+    dd = dgu.double()
+    _bounded(dx, dd @ ad, dd.abs() @ ad.abs(), 2 * hidden, dtype)
+    _bounded(da, dd.t() @ xd, dd.abs().t() @ xd.abs(), tokens, dtype)
+    # each gradient alone, and no [gate | up] kept
+    again = torch.empty_like(out)
+    _call("mg_mlp_fwd", (again, torch.empty_like(h), None, x, w12, w3), sizes, dtype)
+    assert torch.equal(again, out)
+    work = torch.empty_like(dgu)
+    for i, want in enumerate((dx, da, db)):
+        alone = [None, None, None]
+        alone[i] = torch.empty_like(want)
+        _call("mg_mlp_bwd", (*alone, None if i == 2 else work, dy, x, w12, w3, gu, h), sizes, dtype)
+        assert torch.equal(alone[i], want)
+
+
+def test_what_is_not_finite_stays_in_its_row_and_column():
+    x, w12, w3 = _case(200, 256, 512, "bf16")
+    dy = torch.randn_like(x)
+    sizes = (200, 256, 512)
+
+    def run(x):
+        out, h, gu = torch.empty_like(x), x.new_empty(200, 512), x.new_empty(200, 1024)
+        _call("mg_mlp_fwd", (out, h, gu, x, w12, w3), sizes, "bf16")
+        dx, dgu = torch.empty_like(x), torch.empty_like(gu)
+        _call("mg_mlp_bwd", (dx, None, None, dgu, dy, x, w12, w3, gu, h), sizes, "bf16")
+        return out, dx
+
+    want = run(x)
+    bad = x.clone()
+    bad[77] = float("nan")
+    bad[199, 3] = float("inf")
+    keep = [i for i in range(200) if i not in (77, 199)]
+    for a, b in zip(run(bad), want):
+        assert torch.isnan(a[77]).all() and not torch.isfinite(a[199]).any() and torch.equal(a[keep], b[keep])
+
+
+def _module(d_model=512, hidden=1024, dtype=torch.bfloat16, seed=0):
+    torch.manual_seed(seed)
+    module = MegaGemmTriton(d_model, multiple_of=64, hidden_multiple=hidden / d_model).cuda().to(dtype)
+    assert module.hidden == hidden
+    return module
+
+
+def _grads(module, x, dy, call=None):
+    for p in module.parameters():
+        p.grad = None
+    x = x.detach().clone().requires_grad_()
+    y = (call or module)(x)
+    y.backward(dy)
+    return [y.detach(), x.grad, module.w12.weight.grad, module.w3.weight.grad]
+
+
+def _through_projections(module):
+    return lambda x: module.w3(ops.swiglu(module.w12(x), module.hidden))
+
+
+def _close(got, want):
+    for a, b in zip(got, want):      # [gate | up] and the gradient of h rounded on one way and not on the other
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert (a.float() - b.float()).norm() <= 2.0 ** -6 * b.float().norm()
+
+
+def _takes(module, x):
+    return ops.swiglu_mlp(x, module.w12.weight, module.w3.weight) is not None
+
+
+@pytest.mark.parametrize("binding", ["extension", "ctypes"])
+@pytest.mark.parametrize("shape", [(300, 512), (3, 100, 512), (2, 5, 33, 512)])
+def test_module_takes_it(shape, binding, monkeypatch):
+    if binding == "ctypes":
+        monkeypatch.setattr(ops, "_binding", None)
+        monkeypatch.setattr(ops, "_resolved", True)
+    module = _module()
+    x, dy = (torch.randn(shape, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    got = _grads(module, x, dy)
+    _close(got, _grads(module, x, dy, _through_projections(module)))
+    with torch.no_grad():
+        assert torch.equal(module(x), got[0]) and torch.equal(ops.swiglu_mlp(x, module.w12.weight, module.w3.weight), got[0])
+    # operands and gradients of other layouts
+    xt = x.transpose(0, 1).contiguous().transpose(0, 1)
+    assert all(torch.equal(a, b) for a, b in zip(_grads(module, x, dy), _grads(module, x, dy.transpose(0, 1).contiguous().transpose(0, 1))))
+    assert torch.equal(module(xt), got[0])
+    # the same in place: y is not a view of anything saved
+    xa = x.clone().requires_grad_()
+    y = module(xa)
+    y.mul_(2).backward(dy / 2)
+    assert torch.equal(xa.grad, got[1])
+    # parts of the gradients, a second backward pass, other data under the operands in between
+    xa = x.clone().requires_grad_()
+    y = module(xa)
+    xa.data = torch.zeros_like(x)
+    w = module.w3.weight
+    keep, w.data = w.data, torch.zeros_like(w.data)
+    for t, want in ((xa, got[1]), (module.w12.weight, got[2]), (w, got[3])):
+        assert torch.equal(torch.autograd.grad(y, t, dy, retain_graph=True)[0], want)
+    w.data = keep
+    for name in ("w12", "w3"):
+        frozen = getattr(module, name).weight.requires_grad_(False)
+        part = _grads(module, x, dy)
+        frozen.requires_grad_()
+        assert [g is None for g in part] == [False, False, name == "w12", name == "w3"]
+        assert all(g is None or torch.equal(g, want) for g, want in zip(part, got))
+    xa = x.clone().requires_grad_()
+    y = module(xa)
+    with torch.no_grad():
+        xa.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward(dy)
+
+
+@pytest.mark.parametrize("binding", ["extension", "ctypes"])
+def test_what_goes_through_the_projections(binding, monkeypatch):
+    if binding == "ctypes":
+        monkeypatch.setattr(ops, "_binding", None)
+        monkeypatch.setattr(ops, "_resolved", True)
+    module = _module()
+    w12, w3 = module.w12.weight, module.w3.weight
+    x = torch.randn(300, 512, device="cuda", dtype=torch.bfloat16)
+    assert _takes(module, x)
+    for y in (x[:64], x.float(), x[:, :511], torch.randn(300 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(300, 512)):
+        assert ops.swiglu_mlp(y, w12, w3) is None
+    assert ops.swiglu_mlp(x, w12.t().contiguous().t(), w3) is None and ops.swiglu_mlp(x, w12.half(), w3) is None
+    assert ops.swiglu_mlp(x.to_sparse(), w12, w3) is None and ops.swiglu_mlp(x.cpu(), w12, w3) is None
+    assert ops.swiglu_mlp(x, w12.detach()[:, :448].contiguous(), w3.detach()[:448].contiguous()) is None
+    odd = torch.zeros(2 * 1000, 512, device="cuda", dtype=torch.bfloat16)
+    assert ops.swiglu_mlp(x, odd, torch.zeros(512, 1000, device="cuda", dtype=torch.bfloat16)) is None
+    # who looks at saved tensors, tangents or transforms sees the projections' ones
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert not _takes(module, x)
+    with torch.autograd.forward_ad.dual_level():
+        assert not _takes(module, torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(_takes(module, t)), t)[1])(x.expand(2, 300, 512))
+    torch.func.grad(lambda t: (seen.append(_takes(module, t)), t.sum())[1])(x)
+    assert seen == [False, False]
+    w12.requires_grad_(False)
+    assert not _takes(module, x) and _takes(module, x.clone().requires_grad_())   # only w3 learns
+    w12.requires_grad_()
+    # a checkpointed block, and a gradient of a gradient, which the activation refuses
+    dy = torch.randn_like(x)
+    got = _grads(module, x, dy, lambda t: torch.utils.checkpoint.checkpoint(module, t, use_reentrant=False))
+    _close(got, _grads(module, x, dy))
+    xa = x.clone().requires_grad_()
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(module(xa).sum(), xa, create_graph=True)[0].sum().backward()
+    for call in (module, _through_projections(module)):       # past the activation it can be had
+        g = torch.autograd.grad(call(x), w3, dy, create_graph=True)[0]
+        second = torch.autograd.grad(g.float().square().sum(), w12)[0]
+        assert torch.isfinite(second).all() and second.abs().max() > 0
+
+
+def test_the_block_under_graph_capture_and_on_other_streams():
+    import threading
+
+    module = _module()
+    module.requires_grad_(False)
+    xs = [torch.randn(300, 512, device="cuda", dtype=torch.bfloat16) for _ in range(4)]
+    dy = torch.randn_like(xs[0])
+
+    def step(x):
+        x.requires_grad_()
+        y = module(x)
+        return y.detach(), torch.autograd.grad(y, x, dy)[0]
+
+    want = [step(x.clone()) for x in xs]
+    static, graph = xs[0].clone(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = step(static)
+    for x, y in zip(xs, want):
+        with torch.no_grad():
+            static.copy_(x)
+        torch.zeros(1024, device="cuda").add_(1)       # eager work between replays
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, y))
+    got = [None] * 4
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(10):
+                got[i] = step(xs[i].clone())
+            torch.cuda.current_stream().synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(torch.equal(a, b) for g, w in zip(got, want) for a, b in zip(g, w))
