@@ -1,7 +1,8 @@
 /*
  * megagemm_hip_mlp.h -- the whole SwiGLU block (reference: megagemm/swiglu.py:165-172, two torch.matmul
  * around the Triton activation, and their autograd) on this library's own matrix products, with the activation
- * and its backward inside them: forward in two launches, backward in four.
+ * and its backward inside them: forward in two launches, backward in four, and one more for each
+ * product whose k is split.
  * Conventions as in megagemm_hip.h.  x, out, dy, dx [tokens, d_model]; w12 [2 * hidden, d_model], gate rows first;
  * w3 [d_model, hidden]; gate_up [tokens, 2 * hidden]; h [tokens, hidden]; all of `dtype`, MG_F16 or MG_BF16.
  */
@@ -27,12 +28,18 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
 
 /*
- * [gate | up] = x * w12^T, h = silu(gate) * up from sums kept in fp32, out = h * w3^T.
- * gate_up may be NULL where no backward pass follows.  Pointers 16-byte aligned; no output overlaps an input or
- * another output.  MG_ERR_UNSUPPORTED for sizes mg_mlp_fits does not take.
+ * Bytes of workspace the two entry points need on the current device, 0 for none: where tokens are few, k is split over
+ * workgroups, whose sums meet there in fp32.
  */
-int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12, const void* w3, int64_t tokens,
-               int64_t d_model, int64_t hidden, int dtype, void* stream);
+int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int64_t* forward_bytes, int64_t* backward_bytes);
+
+/*
+ * [gate | up] = x * w12^T, h = silu(gate) * up from sums kept in fp32, out = h * w3^T.
+ * gate_up may be NULL where no backward pass follows, workspace where none is needed.  Pointers 16-byte aligned; no output
+ * (the workspace is one) overlaps an input or another output.  MG_ERR_UNSUPPORTED for sizes mg_mlp_fits does not take.
+ */
+int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12, const void* w3, void* workspace, int64_t workspace_bytes,
+               int64_t tokens, int64_t d_model, int64_t hidden, int dtype, void* stream);
 
 /*
  * The gradients for dy as the gradient of out: dx, dw12 and dw3, each NULL where not wanted.  gate_up and h as
@@ -40,7 +47,8 @@ int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12
  * Sums in a fixed order: bit-identical from run to run.  Otherwise as mg_mlp_fwd.
  */
 int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy, const void* x, const void* w12, const void* w3,
-               const void* gate_up, const void* h, int64_t tokens, int64_t d_model, int64_t hidden, int dtype, void* stream);
+               const void* gate_up, const void* h, void* workspace, int64_t workspace_bytes, int64_t tokens, int64_t d_model, int64_t hidden,
+               int dtype, void* stream);
 
 #ifdef __cplusplus
 }

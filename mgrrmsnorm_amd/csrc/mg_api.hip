@@ -9,6 +9,7 @@
 #include "mg_device.hpp"
 #include "rmsnorm_kernels.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
@@ -770,16 +771,17 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
     return tokens * d_model * 2 <= most && tokens * hidden * 4 <= most && hidden * d_model * 4 <= most;
 }
 
-// Where forward + backward and forward alone both take no more time than the library's products with the activation
-// between them, GPU time in a replayed graph and eager (library / these, us, bf16, d_model x hidden, forward + backward; forward).
-// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162.6 / 47.2.
-//   256 tokens and more: 512 x 1024, 300 60.7 / 49.0; 21.2 / 17.0; 2048 x 3584, 300 142.6 / 108.3; 43.4 / 37.9, 1024 213.6 / 169.4;
-//     64.2 / 56.8, 4096 560 / 496; 166 / 156; 2048 x 5504, 300 203.9 / 197.4; 53.2 / 50.6; beyond 128 MiB of weights,
-//     4096 x 11008, 300 567 / 488; 133 / 151;
-//   fewer: 512 x 1024, 80 46.8 / 43.0; 17.8 / 16.3; beyond 4 MiB, 1024 x 2816, 80 76.3 / 80.2; 19.6 / 24.6.
+// Where forward + backward takes no more time than with the library's products and the activation between them.  GPU time in
+// replayed graphs (library / these, us, bf16, d_model x hidden, forward + backward; forward):
+//   1024 x 1792: 80 tokens 64.6 / 52.9; 18.7 / 20.5, 1024 97 / 78; 30 / 26.5, 8192 379 / 309; 113 / 93
+//   2048 x 3584: 80 97 / 72; 26.3 / 25.4, 1024 209 / 165; 68 / 58, 8192 1059 / 975; 324 / 336
+//   4096 x 11008: 80 435 / 244; 78 / 65, 320 533 / 440; 141 / 150, 1024 1008 / 885; 318 / 299, 2048 1958 / 1486; 617 / 503
+//   and beyond 128 MiB of weights from 4096 tokens on, 3072 x 8192 1614 / 1708; 498 / 536, 4096 x 6912 1850 / 1750; 548 / 593.
+// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162.6 / 47.2; 47 / 15.  Forward alone goes the same way, so that
+// it gives the same bits; it loses up to 9 % where its tiles just miss a round of the compute units.
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
     if (tokens <= MG_BLOCK_MAX_TOKENS || !mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
-    return tokens <= 4096 && 6 * d_model * hidden <= (tokens >= 256 ? 128LL << 20 : 4LL << 20);
+    return tokens < 4096 || 6 * d_model * hidden <= 128LL << 20;
 }
 
 namespace {
@@ -808,53 +810,101 @@ int check_mlp(const char* fn, int64_t tokens, int64_t d_model, int64_t hidden, i
     return MG_OK;
 }
 
-int run_mlp(const char* fn, int dtype, MlpWhat what, MlpArgs a, hipStream_t s) {
-    const int rc = cu_count(&a.cus);
-    if (rc != MG_OK) return rc;
-    const hipError_t e = dtype == MG_F16 ? launch_mlp<half_t>(what, a, s) : launch_mlp<bf16_t>(what, a, s);
+// The products of one pass, in the order of their launches.
+struct MlpStep { MlpWhat what; bool wanted; int64_t M, N, K; };
+
+int64_t mlp_partial_bytes(const MlpStep* steps, int count, int cus) {
+    int64_t most = 0;
+    for (int i = 0; i < count; ++i) {
+        const MlpPlan p = mlp_plan_for(steps[i].what, steps[i].M, steps[i].N, steps[i].K, cus);
+        if (steps[i].wanted && p.splits > 1) most = std::max(most, (int64_t)p.splits * steps[i].M * steps[i].N * 4);
+    }
+    return most;
+}
+
+int run_mlp(const char* fn, int dtype, const MlpStep& step, MlpArgs a, int cus, void* workspace, hipStream_t s) {
+    a.M = (int)step.M;
+    a.N = (int)step.N;
+    a.K = (int)step.K;
+    a.partial = workspace;
+    const MlpPlan plan = mlp_plan_for(step.what, step.M, step.N, step.K, cus);
+    const hipError_t e = dtype == MG_F16 ? launch_mlp<half_t>(step.what, a, plan, s) : launch_mlp<bf16_t>(step.what, a, plan, s);
     return e == hipSuccess ? MG_OK : fail_hip(fn, e);
+}
+
+struct MlpForward {
+    MlpStep steps[2];
+    MlpForward(int64_t t, int64_t d, int64_t h) : steps{{MlpWhat::gate_up, true, t, h, d}, {MlpWhat::down, true, t, d, h}} {}
+};
+struct MlpBackward {
+    MlpStep steps[4];
+    MlpBackward(int64_t t, int64_t d, int64_t h, bool x, bool w12, bool w3)
+        : steps{{MlpWhat::weight_grad, w3, d, h, t}, {MlpWhat::activation_bwd, x || w12, t, h, d},
+                {MlpWhat::weight_grad, w12, 2 * h, d, t}, {MlpWhat::input_grad, x, t, d, 2 * h}} {}
+};
+
+int check_workspace(const char* fn, const MlpStep* steps, int count, const void* workspace, int64_t workspace_bytes, int* cus) {
+    const int rc = cu_count(cus);
+    if (rc != MG_OK) return rc;
+    const int64_t need = mlp_partial_bytes(steps, count, *cus);
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+        return fail(MG_ERR_INVALID_ARG, "%s: the workspace must hold %lld bytes (mg_mlp_workspace)", fn, (long long)need);
+    return MG_OK;
 }
 
 }  // namespace
 
-int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12, const void* w3, int64_t tokens,
-               int64_t d_model, int64_t hidden, int dtype, void* stream) {
+int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int64_t* forward_bytes, int64_t* backward_bytes) {
+    if (forward_bytes == nullptr || backward_bytes == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_workspace: an output is NULL");
+    if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return fail(MG_ERR_UNSUPPORTED, "mg_mlp_workspace: sizes mg_mlp_fits does not take");
+    int cus = 0;
+    const int rc = cu_count(&cus);
+    if (rc != MG_OK) return rc;
+    *forward_bytes = mlp_partial_bytes(MlpForward(tokens, d_model, hidden).steps, 2, cus);
+    *backward_bytes = mlp_partial_bytes(MlpBackward(tokens, d_model, hidden, true, true, true).steps, 4, cus);
+    return MG_OK;
+}
+
+int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12, const void* w3, void* workspace, int64_t workspace_bytes,
+               int64_t tokens, int64_t d_model, int64_t hidden, int dtype, void* stream) {
     const int64_t td = tokens * d_model * 2, th = tokens * hidden * 2, w = d_model * hidden * 2;
-    const MlpTensor in[] = {{"x", x, td}, {"w12", w12, 2 * w}, {"w3", w3, w}}, outs[] = {{"out", out, td}, {"h", h, th}, {"gate_up", gate_up, 2 * th}};
-    int rc = check_mlp("mg_mlp_fwd", tokens, d_model, hidden, dtype, outs, 3, in, 3);
+    const MlpTensor in[] = {{"x", x, td}, {"w12", w12, 2 * w}, {"w3", w3, w}};
+    const MlpTensor outs[] = {{"out", out, td}, {"h", h, th}, {"gate_up", gate_up, 2 * th}, {"workspace", workspace, workspace_bytes}};
+    int rc = check_mlp("mg_mlp_fwd", tokens, d_model, hidden, dtype, outs, 4, in, 3);
     if (rc != MG_OK) return rc;
     if (out == nullptr || h == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_fwd: out and h must not be NULL");
-    const int t = (int)tokens, d = (int)d_model, n = (int)hidden;
-    hipStream_t s = (hipStream_t)stream;
-    rc = run_mlp("mg_mlp_fwd", dtype, MlpWhat::gate_up, {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d, t, n, d, 0}, s);
+    const MlpForward pass(tokens, d_model, hidden);
+    int cus = 0;
+    rc = check_workspace("mg_mlp_fwd", pass.steps, 2, workspace, workspace_bytes, &cus);
     if (rc != MG_OK) return rc;
-    return run_mlp("mg_mlp_fwd", dtype, MlpWhat::down, {out, nullptr, nullptr, h, (uint32_t)th, n, w3, (uint32_t)w, n, t, d, n, 0}, s);
+    const int d = (int)d_model, n = (int)hidden;
+    hipStream_t s = (hipStream_t)stream;
+    rc = run_mlp("mg_mlp_fwd", dtype, pass.steps[0], {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d}, cus, workspace, s);
+    if (rc != MG_OK) return rc;
+    return run_mlp("mg_mlp_fwd", dtype, pass.steps[1], {out, nullptr, nullptr, h, (uint32_t)th, n, w3, (uint32_t)w, n}, cus, workspace, s);
 }
 
 int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy, const void* x, const void* w12, const void* w3,
-               const void* gate_up, const void* h, int64_t tokens, int64_t d_model, int64_t hidden, int dtype, void* stream) {
+               const void* gate_up, const void* h, void* workspace, int64_t workspace_bytes, int64_t tokens, int64_t d_model, int64_t hidden,
+               int dtype, void* stream) {
     const int64_t td = tokens * d_model * 2, th = tokens * hidden * 2, w = d_model * hidden * 2;
     const MlpTensor in[] = {{"dy", dy, td}, {"x", x, td}, {"w12", w12, 2 * w}, {"w3", w3, w}, {"gate_up", gate_up, 2 * th}, {"h", h, th}};
-    const MlpTensor outs[] = {{"dx", dx, td}, {"dw12", dw12, 2 * w}, {"dw3", dw3, w}, {"d_gate_up", d_gate_up, 2 * th}};
-    int rc = check_mlp("mg_mlp_bwd", tokens, d_model, hidden, dtype, outs, 4, in, 6);
+    const MlpTensor outs[] = {{"dx", dx, td}, {"dw12", dw12, 2 * w}, {"dw3", dw3, w}, {"d_gate_up", d_gate_up, 2 * th}, {"workspace", workspace, workspace_bytes}};
+    int rc = check_mlp("mg_mlp_bwd", tokens, d_model, hidden, dtype, outs, 5, in, 6);
     if (rc != MG_OK) return rc;
-    if (d_gate_up == nullptr && (dx != nullptr || dw12 != nullptr))
-        return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
-    const int t = (int)tokens, d = (int)d_model, n = (int)hidden;
-    hipStream_t s = (hipStream_t)stream;
-    if (dw3 != nullptr) {
-        rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::weight_grad, {dw3, nullptr, nullptr, dy, (uint32_t)td, d, h, (uint32_t)th, n, d, n, t, 0}, s);
-        if (rc != MG_OK) return rc;
-    }
-    if (dx == nullptr && dw12 == nullptr) return MG_OK;
-    rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::activation_bwd,
-                 {d_gate_up, nullptr, gate_up, dy, (uint32_t)td, d, w3, (uint32_t)w, n, t, n, d, 0}, s);
-    if (rc == MG_OK && dw12 != nullptr)
-        rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::weight_grad,
-                     {dw12, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, x, (uint32_t)td, d, 2 * n, d, t, 0}, s);
-    if (rc == MG_OK && dx != nullptr)
-        rc = run_mlp("mg_mlp_bwd", dtype, MlpWhat::input_grad,
-                     {dx, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, w12, (uint32_t)(2 * w), d, t, d, 2 * n, 0}, s);
+    const MlpBackward pass(tokens, d_model, hidden, dx != nullptr, dw12 != nullptr, dw3 != nullptr);
+    if (pass.steps[1].wanted && d_gate_up == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
+    int cus = 0;
+    rc = check_workspace("mg_mlp_bwd", pass.steps, 4, workspace, workspace_bytes, &cus);
+    if (rc != MG_OK) return rc;
+    const int d = (int)d_model, n = (int)hidden;
+    const MlpArgs args[] = {
+        {dw3, nullptr, nullptr, dy, (uint32_t)td, d, h, (uint32_t)th, n},
+        {d_gate_up, nullptr, gate_up, dy, (uint32_t)td, d, w3, (uint32_t)w, n},
+        {dw12, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, x, (uint32_t)td, d},
+        {dx, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, w12, (uint32_t)(2 * w), d}};
+    for (int i = 0; i < 4 && rc == MG_OK; ++i)
+        if (pass.steps[i].wanted) rc = run_mlp("mg_mlp_bwd", dtype, pass.steps[i], args[i], cus, workspace, (hipStream_t)stream);
     return rc;
 }
 

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mlp_plan.hpp"
+
 #include <tuple>
 #include <utility>
 
@@ -248,13 +250,19 @@ hipError_t launch_skinny_gemm(int dtype, bool paired, const SkinnyArgs& a, hipSt
 // Products of the whole SwiGLU block (mlp_gemm.hpp): out [M, N] from a and b, each `*_bytes` long with `*_ld` elements
 // per line.  gate_up: b holds N gate rows, then N up rows; out may be NULL, second gets the activation.  activation_bwd: `in` is
 // [gate | up].  weight_grad: a is [K, M], b [K, N], any K; otherwise a is [M, K] with K a multiple of 64.
+// partial: plan.splits * M * N floats where the plan splits k.
 enum class MlpWhat { gate_up, down, activation_bwd, input_grad, weight_grad };
 struct MlpArgs {
     void* out; void* second; const void* in;
     const void* a; uint32_t a_bytes; int a_ld;
     const void* b; uint32_t b_bytes; int b_ld;
-    int M, N, K, cus;
+    int M, N, K;
+    void* partial;
 };
-template <typename T> hipError_t launch_mlp(MlpWhat what, const MlpArgs& a, hipStream_t s);
+inline MlpPlan mlp_plan_for(MlpWhat what, int64_t M, int64_t N, int64_t K, int cus) {
+    const bool fused = what == MlpWhat::gate_up || what == MlpWhat::activation_bwd;   // the activation needs whole sums
+    return mlp_plan(M, what == MlpWhat::gate_up ? 2 * N : N, K, what == MlpWhat::weight_grad, !fused, cus);
+}
+template <typename T> hipError_t launch_mlp(MlpWhat what, const MlpArgs& a, MlpPlan plan, hipStream_t s);
 
 }  // namespace mg

@@ -112,17 +112,22 @@ __device__ __forceinline__ void step_barrier(const char MG_LDS* a, const char MG
 
 template <class C> struct MlpFragments { u32x4 a[C::FM], b[C::FN]; };
 template <class C> struct MlpSums { f32x4 v[C::FM][C::FN]; };
+// What a wave has of the finished sums: a WKth of its tile's rows, the one after those of the groups before its own.
+template <class C> struct MlpShare { f32x4 v[C::FM / C::WK][C::FN]; };
 
-// One workgroup's product, bound by LDS: of the 1024 cycles that the matrix instructions of a 256 x 128 x 64 step take, its
-// fragments need 1024 (128 bytes a cycle) and its arrival from memory 384, and 1570 are measured with few workgroups,
-// 1630 with the chip full.  So the loop keeps all three going: requests are STAGES steps ahead, fragments one
-// instruction's worth of k, and one barrier a step serves both the arrival and the reuse of a stage.  What loses: reads and
-// multiplications in separate blocks in place of the compiler's own order (33.7 against 31.6 us for 1024 x 7168 outputs,
-// k 2048), s_setprio around the multiplications (35.1), waves of 128 x 64 with the k of a step split over two groups (33.4),
-// four waves of 128 x 64 (49).
-// At 1024 tokens, 2048 x 3584 (bf16, us, these / the library's): gate and up with the activation 30 / 35 + 4, second
-// projection 20.1 / 22.3, gradient of h with the activation's 20 / 27 + 8, of x 38.4 / 53, of w3 18.9 / 25.8, of w12 29.4 / 36.
-//  `sums.v[i][j][q]` of a wave becomes out[m, n] with
+// One workgroup's product, bound by LDS (128 bytes a cycle).  Of the 1024 cycles that the matrix instructions of a
+// 128 x 256 x 64 step take on eight waves of 64 x 64, its fragments need 1024 and its arrival from memory 384; measured 0.66 us.
+// Smaller tiles can have waves as large by sharing a step's k between groups of waves: 128 x 128 on four of 64 x 64 twice over
+// 18.5 us for 1024 x 3584 outputs, k 2048, against 19.8 on eight of 64 x 32 (at 128 x 256 it is no gain in a whole block,
+// where the operands come from memory: 36.3 against 34.1 us for gate and up).  The loop keeps memory, LDS and matrix cores
+// going at once: requests STAGES steps ahead, fragments one instruction's worth of k, and one barrier a step for both the arrival
+// and the reuse of a stage.  What loses (1024 x 7168 outputs, k 2048): reads and multiplications in separate blocks 33.7
+// against 31.6 us, s_setprio around the multiplications 35.1, the same tile on four waves 43 (one wave a SIMD leaves its matrix
+// core waiting); on the whole block, the tiles' k started at different places 184-198 against 179 us; one 4-byte request per
+// line four steps further ahead, 93 -> 100 us for 1024 x 2048, k 7168.
+// At 1024 tokens, 2048 x 3584 (us, these / the library's): gate and up with the activation 34 / 35 + 4, second projection
+// 26 / 25, gradient of h with the activation's 22.5 / 27 + 8, of x 39 / 52, of w3 21 / 26, of w12 34 / 42.
+// `sums.v[i][j][q]` of a wave becomes out[m, n] with
 //   m = m0 + wm * TM + i * 16 + lane % 16,   n = n0 + wn * TN + j * 16 + 4 * (lane / 16) + q
 // (b is the instruction's first operand: a lane then owns four consecutive n and stores 8 bytes).
 template <typename T, class C, bool A_ALONG_K, bool B_ALONG_K, bool PAIRED>
@@ -136,7 +141,6 @@ struct MlpProduct {
     MlpOperand A, B;
     int left;                    // steps not requested yet
     int wave, fa[C::FM], fb[C::FN];
-
     __device__ __forceinline__ void request(char MG_LDS* to) {
         const bool any = left > 0;                       // nothing left: out of range, nothing is read and zeros arrive
         ta.request(to, make_rsrc(A.p, any ? A.bytes : 0u), wave);
@@ -167,24 +171,41 @@ struct MlpProduct {
         step_barrier(first, others, others);
         read(f, first, 0);
     }
-    // One step.  On entry `f` holds its first fragments, read before; on return the next step's.
+    // With one substep a step is one block of instructions: the next fragments' reads between the first half of the
+    // multiplications, the requests between all of them.  Left to itself the compiler issues the reads in a bunch, in front of
+    // the multiplications or behind them (1024 x 3584 outputs, k 2048: 18.9 / 18.5 us, 1024 x 2048, k 3584: 22.2 / 21.5; with two
+    // substeps its own order is as good or better).
+    static __device__ __forceinline__ void interleave() {
+        constexpr int M = C::FM * C::FN, H = M / 2, R = C::FM * (A_ALONG_K ? 1 : 2) + C::FN * (B_ALONG_K ? 1 : 2);
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+            const int reads = i < H ? R * (i + 1) / H - R * i / H : 0, requests = PER_STEP * (i + 1) / M - PER_STEP * i / M;
+#pragma unroll
+            for (int k = 0; k < reads; ++k) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+            for (int k = 0; k < requests; ++k) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+    }
+
+    // One step.  On entry `f` holds its first fragments, read before; on return `next_f` holds the next step's.
+    // With two substeps the two may be the same.
     __device__ __forceinline__ void step(const char MG_LDS* __restrict__ tile, const char MG_LDS* __restrict__ next, char MG_LDS* __restrict__ refill,
-                                         MlpSums<C>& sums, MlpFragments<C>& f) {
+                                         MlpSums<C>& sums, MlpFragments<C>& f, MlpFragments<C>& next_f) {
         MlpFragments<C> g;
         if constexpr (C::SUBSTEPS == 2) {
             read(g, tile, 1);
             multiply(sums, f);
-            f = g;
         }
         wait_requests<PER_STEP * (C::STAGES - 2)>();     // the next step has arrived ...
         step_barrier(tile, next, refill);                // ... for every wave, and every wave has read all of this one
-        read(g, next, 0);
+        read(next_f, next, 0);
         request(refill);
-        multiply(sums, f);
-        f = g;
+        multiply(sums, C::SUBSTEPS == 2 ? g : f);
+        if constexpr (C::SUBSTEPS == 1) interleave();
     }
 
-    __device__ __forceinline__ void run(MlpSums<C>& sums, char MG_LDS* lds, int K, int m0, int n0, int hidden) {
+    __device__ __forceinline__ void run(MlpShare<C>& share, char MG_LDS* lds, int first, int steps, int m0, int n0, int hidden) {
         const int tid = threadIdx.x, lane = tid & (kWave - 1);
         wave = __builtin_amdgcn_readfirstlane(tid / kWave);
         const int wm = wave % C::WM, wn = wave / C::WM % C::WN, kg = wave / (C::WM * C::WN);
@@ -194,44 +215,76 @@ struct MlpProduct {
         for (int i = 0; i < C::FM; ++i) fa[i] = TA::fragment(wm * C::TM + i * 16, lane, kg * C::SUBSTEPS);
 #pragma unroll
         for (int j = 0; j < C::FN; ++j) fb[j] = TB::fragment(wn * C::TN + j * 16, lane, kg * C::SUBSTEPS);
+        MlpSums<C> sums;
 #pragma unroll
         for (int i = 0; i < C::FM; ++i)
 #pragma unroll
             for (int j = 0; j < C::FN; ++j) sums.v[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        const int steps = (K + C::BK - 1) / C::BK;
         left = steps;
-        MlpFragments<C> f;
+        ta.advance((u32)first * TA::step(A.ld));
+        tb.advance((u32)first * TB::step(B.ld));
+        MlpFragments<C> f, g;
         start(lds, lds + C::STAGE, f);
+        const auto after = [](int at) { return at == (C::STAGES - 1) * C::STAGE ? 0 : at + C::STAGE; };
         int at = 0;
+        if constexpr (C::SUBSTEPS == 2) {
 #pragma clang loop unroll(disable)
-        for (int k = 0; k < steps; ++k) {
-            const int next = at == (C::STAGES - 1) * C::STAGE ? 0 : at + C::STAGE;
-            step(lds + at, lds + next, lds + at, sums, f);
-            at = next;
+            for (int k = 0; k < steps; ++k) {
+                const int next = after(at);
+                step(lds + at, lds + next, lds + at, sums, f, f);
+                at = next;
+            }
+        } else {   // two sets of fragments in turn; an odd step at the end multiplies zeros
+#pragma clang loop unroll(disable)
+            for (int k = 0; k < steps; k += 2) {
+                const int next = after(at), over = after(next);
+                step(lds + at, lds + next, lds + at, sums, f, g);
+                step(lds + next, lds + over, lds + next, sums, g, f);
+                at = over;
+            }
         }
         wait_requests<0>();                              // LDS is used again, by this workgroup or the next
         __syncthreads();
-        if constexpr (C::WK > 1) {                       // the groups' sums, in order
-            constexpr int W = C::WM * C::WN, HOLDS = C::STAGES * C::STAGE / (W * kWave * 16);
-            static_assert(HOLDS >= (C::WK - 1) * C::FM * C::FN, "fragments of every wave that LDS holds");
+        if constexpr (C::WK == 1) {
+#pragma unroll
+            for (int i = 0; i < C::FM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::FN; ++j) share.v[i][j] = sums.v[i][j];
+        } else {   // every group hands the others their rows and adds up its own, in the order of the groups
+            constexpr int W = C::WM * C::WN, EACH = C::FM / C::WK, HOLDS = C::STAGES * C::STAGE / (W * kWave * 16);
+            static_assert(C::FM % C::WK == 0 && HOLDS >= (C::WK - 1) * C::FM * C::FN, "fragments of every wave that LDS holds");
             f32x4 MG_LDS* mine = (f32x4 MG_LDS*)lds + wave % W * kWave + lane;
+            // fragment i, j of the rows of group `to`, from group `from`
+            const auto place = [&](int to, int from, int i, int j) -> f32x4 MG_LDS& {
+                return mine[(((to * (C::WK - 1) + from - (from > to ? 1 : 0)) * EACH + i) * C::FN + j) * (W * kWave)];
+            };
 #pragma unroll
-            for (int g = 1; g < C::WK; ++g)
-                if (kg == g) {
+            for (int from = 0; from < C::WK; ++from)
+                if (kg == from) {
 #pragma unroll
-                    for (int i = 0; i < C::FM; ++i)
+                    for (int to = 0; to < C::WK; ++to)
 #pragma unroll
-                        for (int j = 0; j < C::FN; ++j) mine[(((g - 1) * C::FM + i) * C::FN + j) * (W * kWave)] = sums.v[i][j];
+                        for (int i = 0; i < EACH; ++i)
+#pragma unroll
+                            for (int j = 0; j < C::FN; ++j) {
+                                if (to == from) share.v[i][j] = sums.v[to * EACH + i][j];
+                                else place(to, from, i, j) = sums.v[to * EACH + i][j];
+                            }
                 }
             __syncthreads();
-            if (kg == 0) {
 #pragma unroll
-                for (int i = 0; i < C::FM; ++i)
+            for (int to = 0; to < C::WK; ++to)
+                if (kg == to) {
 #pragma unroll
-                    for (int j = 0; j < C::FN; ++j)
+                    for (int i = 0; i < EACH; ++i)
 #pragma unroll
-                        for (int g = 1; g < C::WK; ++g) sums.v[i][j] += mine[(((g - 1) * C::FM + i) * C::FN + j) * (W * kWave)];
-            }
+                        for (int j = 0; j < C::FN; ++j) {
+                            f32x4 s = to == 0 ? share.v[i][j] : place(to, 0, i, j);
+#pragma unroll
+                            for (int from = 1; from < C::WK; ++from) s += from == to ? share.v[i][j] : place(to, from, i, j);
+                            share.v[i][j] = s;
+                        }
+                }
             __syncthreads();
         }
     }
@@ -240,6 +293,7 @@ struct MlpProduct {
 // What becomes of the sums.
 struct MlpOut { void* out; void* second; const void* in; int M, N; };
 constexpr int kMlpStore = 0;     // out [M, N]
+constexpr int kMlpPartial = 3;   // out [splits, M, N] in fp32, for mlp_add
 constexpr int kMlpGateUp = 1;    // N = hidden: out [M, 2 N] = [gate | up] unless NULL, second [M, N] = silu(gate) * up
 constexpr int kMlpActBwd = 2;    // N = hidden: out [M, 2 N] = gradient of `in` [M, 2 N] = [gate | up] for the sums as the gradient of silu(gate) * up
 
@@ -256,14 +310,14 @@ __device__ __forceinline__ void mlp_load8(float* f, rsrc_t r, bool in, u32 at) {
 // eight lanes (four of a 32-column tile) a whole piece of a row: stored straight from the sums, 8 bytes here and there,
 // the results take 9 of 33 us at 7168 x 2048 outputs.  N is a multiple of 8.
 template <typename T, class C, int WHAT>
-__device__ __forceinline__ void mlp_finish(const MlpSums<C>& sums, char MG_LDS* lds, const MlpOut& o, int m0, int n0) {
+__device__ __forceinline__ void mlp_finish(const MlpShare<C>& share, char MG_LDS* lds, const MlpOut& o, int m0, int n0) {
     constexpr bool PAIRED = WHAT == kMlpGateUp;
     constexpr int COLS = PAIRED ? C::TN / 2 : C::TN;     // of the result
     constexpr int LANES = COLS / 8, ROWS = LANES >= 4 ? kWave / LANES : 16, BUFFERS = 2;
-    static_assert(C::WM * C::WN * BUFFERS * 16 * C::TN * 4 <= C::STAGE * C::STAGES, "");
+    static_assert(C::WAVES * BUFFERS * 16 * C::TN * 4 <= C::STAGE * C::STAGES, "");
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int wm = wave % C::WM, wn = wave / C::WM % C::WN;
-    if (wave >= C::WM * C::WN) return;                   // k groups but the first
+    const int wm = wave % C::WM, wn = wave / C::WM % C::WN, kg = wave / (C::WM * C::WN);
+    m0 += wm * C::TM + kg * (C::TM / C::WK);
     const u32 M = (u32)o.M, N = (u32)o.N;
     const rsrc_t out = make_rsrc(o.out, o.out == nullptr ? 0u : M * N * (WHAT == kMlpStore ? 2u : 4u));
     const rsrc_t second = make_rsrc(o.second, PAIRED ? M * N * 2u : 0u);
@@ -271,17 +325,17 @@ __device__ __forceinline__ void mlp_finish(const MlpSums<C>& sums, char MG_LDS* 
     const int row = lane / LANES, unit = lane % LANES * 2;
     const u32 n = (u32)(n0 + wn * COLS + lane % LANES * 8);
     // 16-byte units of a row, permuted by its number: rows of TN floats start in the same bank
-    const auto place = [](int r, int u) { return r * C::TN * 4 + ((u ^ (C::TN == 64 ? r & 15 : (r >> 1) & 7)) << 4); };
-    static_assert(C::TN == 64 || C::TN == 32, "");
+    const auto place = [](int r, int u) { return r * C::TN * 4 + ((u ^ (C::TN >= 64 ? r & 15 : (r >> 1) & 7)) << 4); };
+    static_assert(C::TN == 128 || C::TN == 64 || C::TN == 32, "");
 #pragma unroll
-    for (int i = 0; i < C::FM; ++i) {
+    for (int i = 0; i < C::FM / C::WK; ++i) {
         char MG_LDS* part = lds + (wave * BUFFERS + i % BUFFERS) * (16 * C::TN * 4);
 #pragma unroll
-        for (int j = 0; j < C::FN; ++j) *(f32x4 MG_LDS*)(part + place(lane & 15, j * 4 + (lane >> 4))) = sums.v[i][j];
+        for (int j = 0; j < C::FN; ++j) *(f32x4 MG_LDS*)(part + place(lane & 15, j * 4 + (lane >> 4))) = share.v[i][j];
 #pragma unroll
         for (int r0 = 0; r0 < 16; r0 += ROWS) {
             const int r = r0 + row;
-            const u32 m = (u32)(m0 + wm * C::TM + i * 16 + r);
+            const u32 m = (u32)(m0 + i * 16 + r);
             const bool ok = m < M && n < N && r < 16;
             float f[8];
             const auto get = [&](float* to, int u) {
@@ -291,7 +345,11 @@ __device__ __forceinline__ void mlp_finish(const MlpSums<C>& sums, char MG_LDS* 
             };
             get(f, unit);
             get(f + 4, unit + 1);
-            if constexpr (WHAT == kMlpStore) {
+            if constexpr (WHAT == kMlpPartial) {
+                const u32 at = ok ? (m * N + n) * 4u : kNowhere;
+                buf_store<4>(out, at, pack_vec<float, 4>(f));
+                buf_store<4>(out, ok ? at + 16u : kNowhere, pack_vec<float, 4>(f + 4));
+            } else if constexpr (WHAT == kMlpStore) {
                 mlp_store8<T>(out, ok, m * N + n, f);
             } else if constexpr (PAIRED) {
                 float u[8], h[8];
@@ -319,36 +377,54 @@ __device__ __forceinline__ void mlp_finish(const MlpSums<C>& sums, char MG_LDS* 
     }
 }
 
+// out = the sums of the splits, in their order.  `vectors` of eight elements.
+template <typename T>
+__global__ void __launch_bounds__(256)
+mlp_add(T* __restrict__ out, const float* __restrict__ parts, u32 vectors, int splits) {
+    const u32 v = blockIdx.x * 256u + threadIdx.x;
+    if (v >= vectors) return;
+    const f32x4* at = reinterpret_cast<const f32x4*>(parts) + 2ul * v;
+    f32x4 lo = at[0], hi = at[1];
+    for (int s = 1; s < splits; ++s) {
+        at += 2ul * vectors;
+        lo += at[0];
+        hi += at[1];
+    }
+    const float f[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    const Words<4> w = pack_vec<T, 4>(f);
+    reinterpret_cast<u32x4*>(out)[v] = u32x4{w.v[0], w.v[1], w.v[2], w.v[3]};
+}
+
 // Which tile a workgroup computes.  Workgroups go to the 8 dies round-robin by id: each die gets an equal
-// share of consecutive tiles, counted down columns of at most `high` row tiles, so that what it reads through its own
-// L2 is a block of both operands of about the same height and width.
-__device__ __forceinline__ void mlp_tile(int id, int rows, int cols, int high, int& tm, int& tn) {
-    const int count = rows * cols, die = id % 8, each = count / 8, more = count % 8;
-    const int t = die * each + (die < more ? die : more) + id / 8;
-    const int band = t / (high * cols), first = band * high, in = t - first * cols;
-    const int h = rows - first < high ? rows - first : high;
+// share of consecutive tiles, counted down columns of at most 8 row tiles, so that what it reads through its own
+// L2 is a block of both operands of about the same height and width.  The splits of k follow each other.
+__device__ __forceinline__ void mlp_tile(int id, int rows, int cols, int splits, int& tm, int& tn, int& split) {
+    constexpr int HIGH = 8;
+    const int count = rows * cols * splits, die = id % 8, each = count / 8, more = count % 8;
+    int t = die * each + (die < more ? die : more) + id / 8;
+    split = t / (rows * cols);
+    t -= split * rows * cols;
+    const int band = t / (HIGH * cols), first = band * HIGH, in = t - first * cols;
+    const int h = rows - first < HIGH ? rows - first : HIGH;
     tm = first + in % h;
     tn = in / h;
 }
 
 template <typename T, class C, bool A_ALONG_K, bool B_ALONG_K, int WHAT>
-__device__ __forceinline__ void mlp_product(char MG_LDS* lds, int id, const MlpOperand& A, const MlpOperand& B, const MlpOut& o, int K, int high) {
+__global__ void __launch_bounds__(C::THREADS, C::WAVES / 4)
+mlp_gemm(MlpOperand A, MlpOperand B, MlpOut o, int K, int splits) {
+    __shared__ __attribute__((aligned(1024))) char lds[C::STAGE * C::STAGES];
     constexpr int BN = WHAT == kMlpGateUp ? C::BN / 2 : C::BN;
-    int tm, tn;
-    mlp_tile(id, (o.M + C::BM - 1) / C::BM, (o.N + BN - 1) / BN, high, tm, tn);
-    MlpSums<C> sums;
+    int tm, tn, split;
+    mlp_tile(blockIdx.x, (o.M + C::BM - 1) / C::BM, (o.N + BN - 1) / BN, splits, tm, tn, split);
+    const int steps = (K + C::BK - 1) / C::BK, first = split * steps / splits, last = (split + 1) * steps / splits;
+    MlpShare<C> share;
     MlpProduct<T, C, A_ALONG_K, B_ALONG_K, WHAT == kMlpGateUp> p;
     p.A = A;
     p.B = B;
-    p.run(sums, lds, K, tm * C::BM, tn * BN, o.N);
-    mlp_finish<T, C, WHAT>(sums, lds, o, tm * C::BM, tn * BN);
-}
-
-template <typename T, class C, bool A_ALONG_K, bool B_ALONG_K, int WHAT>
-__global__ void __launch_bounds__(C::THREADS, C::WAVES / 4)
-mlp_gemm(MlpOperand A, MlpOperand B, MlpOut o, int K, int high) {
-    __shared__ __attribute__((aligned(1024))) char lds[C::STAGE * C::STAGES];
-    mlp_product<T, C, A_ALONG_K, B_ALONG_K, WHAT>((char MG_LDS*)lds, blockIdx.x, A, B, o, K, high);
+    p.run(share, (char MG_LDS*)lds, first, last - first, tm * C::BM, tn * BN, o.N);
+    if constexpr (WHAT == kMlpPartial) o.out = (float*)o.out + (size_t)split * o.M * o.N;
+    mlp_finish<T, C, WHAT>(share, (char MG_LDS*)lds, o, tm * C::BM, tn * BN);
 }
 
 }  // namespace mg

@@ -350,14 +350,25 @@ bool calls_transformed() {
            c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
 
+// What mg_mlp_fwd or mg_mlp_bwd needs besides its tensors; undefined where that is nothing.
+Tensor mlp_workspace(const Tensor& x, int64_t tokens, int64_t d_model, int64_t hidden, bool forward) {
+    int64_t bytes[2] = {0, 0};
+    TORCH_CHECK(mg_mlp_workspace(tokens, d_model, hidden, dtype_code(x.scalar_type()), &bytes[0], &bytes[1]) == MG_OK,
+                "SwiGLU block (workspace query) failed: ", mg_last_error());
+    const int64_t need = bytes[forward ? 0 : 1];
+    return need > 0 ? at::empty({need}, x.options().dtype(at::kByte)) : Tensor();
+}
+void* pointer_of(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
 Tensor mlp_forward(const Tensor& x, const Tensor& w12, const Tensor& w3, Tensor* gate_up, Tensor* h) {
     const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = x.numel() / d_model;
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     if (gate_up != nullptr) *gate_up = at::empty({tokens, 2 * hidden}, x.options());
     *h = at::empty({tokens, hidden}, x.options());
     auto out = empty_as(x);
+    const Tensor work = mlp_workspace(x, tokens, d_model, hidden, true);
     const int rc = mg_mlp_fwd(out.data_ptr(), h->data_ptr(), gate_up != nullptr ? gate_up->data_ptr() : nullptr, x.data_ptr(),
-                              w12.data_ptr(), w3.data_ptr(), tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
+                              w12.data_ptr(), w3.data_ptr(), pointer_of(work), work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
     TORCH_CHECK(rc == MG_OK, "SwiGLU block forward failed (code ", rc, "): ", mg_last_error());
     return out;
 }
@@ -401,9 +412,10 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
         if (want[0] || want[1]) d_gate_up = empty_as(gate_up);
         for (int i = 0; i < 3; ++i)
             if (want[i]) out[i] = empty_as(saved[i]);
-        const auto at = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
-        const int rc = mg_mlp_bwd(at(out[0]), at(out[1]), at(out[2]), at(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
-                                  gate_up.data_ptr(), h.data_ptr(), tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
+        const Tensor work = mlp_workspace(x, tokens, d_model, hidden, false);
+        const int rc = mg_mlp_bwd(pointer_of(out[0]), pointer_of(out[1]), pointer_of(out[2]), pointer_of(d_gate_up), dy.data_ptr(), x.data_ptr(),
+                                  w12.data_ptr(), w3.data_ptr(), gate_up.data_ptr(), h.data_ptr(), pointer_of(work),
+                                  work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
         TORCH_CHECK(rc == MG_OK, "SwiGLU block backward failed (code ", rc, "): ", mg_last_error());
         return out;
     }

@@ -235,6 +235,15 @@ def _pointer(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def _mlp_workspace(x, tokens, d_model, hidden, forward):
+    """(tensor or None, its bytes) that mg_mlp_fwd or mg_mlp_bwd needs besides its tensors."""
+    sizes = ctypes.c_int64(0), ctypes.c_int64(0)
+    _lib.check(_lib.load().mg_mlp_workspace(tokens, d_model, hidden, _MLP_CODES[x.dtype], *map(ctypes.byref, sizes)),
+               "SwiGLU block (workspace query)")
+    need = sizes[0 if forward else 1].value
+    return (torch.empty(need, dtype=torch.uint8, device=x.device) if need else None), need
+
+
 def _mlp_forward(x, w12, w3, keep_gate_up):
     d_model, hidden = w3.shape
     tokens = x.numel() // d_model
@@ -242,8 +251,9 @@ def _mlp_forward(x, w12, w3, keep_gate_up):
         gate_up = x.new_empty(tokens, 2 * hidden) if keep_gate_up else None
         h = x.new_empty(tokens, hidden)
         out = torch.empty_like(x)
+        work, size = _mlp_workspace(x, tokens, d_model, hidden, True)
         rc = _lib.load().mg_mlp_fwd(out.data_ptr(), h.data_ptr(), _pointer(gate_up), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
-                                    tokens, d_model, hidden, _MLP_CODES[x.dtype], _lib.stream_ptr(x.device))
+                                    _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype], _lib.stream_ptr(x.device))
     _lib.check(rc, "SwiGLU block forward")
     return out, gate_up, h
 
@@ -277,8 +287,10 @@ class _MlpFunction(torch.autograd.Function):
         with _lib.device_of(x.device):
             grads = [torch.empty_like(t) if w else None for t, w in zip((x, w12, w3), want)]
             d_gate_up = torch.empty_like(gate_up) if want[0] or want[1] else None
+            tokens = x.numel() // d_model
+            work, size = _mlp_workspace(x, tokens, d_model, hidden, False)
             rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
-                                        gate_up.data_ptr(), h.data_ptr(), x.numel() // d_model, d_model, hidden, _MLP_CODES[x.dtype],
+                                        gate_up.data_ptr(), h.data_ptr(), _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype],
                                         _lib.stream_ptr(x.device))
         _lib.check(rc, "SwiGLU block backward")
         return tuple(grads)

@@ -28,11 +28,11 @@ def test_bad_arguments_are_refused(lib):
 
     def fwd(sizes=(t, d, h), dtype=2, **other):
         q = {**p, **other}
-        return lib.mg_mlp_fwd(*(q[n] for n in ("out", "h", "gu", "x", "w12", "w3")), *sizes, dtype, None)
+        return lib.mg_mlp_fwd(*(q[n] for n in ("out", "h", "gu", "x", "w12", "w3")), None, 0, *sizes, dtype, None)
 
     def bwd(**other):
         q = {**p, **other}
-        return lib.mg_mlp_bwd(*(q[n] for n in ("dx", "dw12", "dw3", "dgu", "dy", "x", "w12", "w3", "gu", "h")), t, d, h, 2, None)
+        return lib.mg_mlp_bwd(*(q[n] for n in ("dx", "dw12", "dw3", "dgu", "dy", "x", "w12", "w3", "gu", "h")), None, 0, t, d, h, 2, None)
 
     assert fwd((t, d, 96)) == -2 and fwd(dtype=0) == -2 and fwd((0, d, h)) == -2
     for name in ("out", "h", "x", "w12", "w3"):

@@ -1,5 +1,7 @@
 """The SwiGLU block on the package's own matrix products (megagemm_hip_mlp.h): every output against the same
 formula in float64 at the edges of the tiles, and what the module does around it."""
+import ctypes
+
 import pytest
 import torch
 
@@ -14,7 +16,13 @@ ROUNDING = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}
 
 
 def _call(name, tensors, sizes, dtype):
-    U.check(getattr(U.lib(), name)(*[t if t is None else t.data_ptr() for t in tensors], *sizes, U.CODES[dtype], U.stream()))
+    need = ctypes.c_int64(0), ctypes.c_int64(0)
+    U.check(U.lib().mg_mlp_workspace(*sizes, U.CODES[dtype], *map(ctypes.byref, need)))
+    size = need[name == "mg_mlp_bwd"].value
+    work = torch.full((size + 1024,), 0x7F, device="cuda", dtype=torch.uint8)       # NaN where nothing is written
+    U.check(getattr(U.lib(), name)(*[t if t is None else t.data_ptr() for t in tensors], work.data_ptr() if size else None, size,
+                                   *sizes, U.CODES[dtype], U.stream()))
+    assert (work[size:] == 0x7F).all()
 
 
 def _guarded(shape, dtype):
@@ -41,6 +49,7 @@ def _bounded(got, ref, terms, count, dtype, extra=0.0):
 @pytest.mark.parametrize("tokens,d_model,hidden", [
     (1, 64, 64), (65, 64, 192), (127, 192, 64), (128, 128, 128), (129, 128, 256), (257, 320, 448), (300, 704, 1088),
     (1000, 512, 1344), (1024, 2048, 3584), (513, 1536, 4096), (2047, 1024, 2816), (96, 4096, 6912), (640, 3136, 8384),
+    (127, 1024, 11008), (130, 3136, 8000), (70, 8192, 1088), (200, 704, 2752),   # k in 2 to 8 parts, of 43.5 and 9.5 steps
 ])
 def test_products_against_float64(tokens, d_model, hidden, dtype):
     x, w12, w3 = _case(tokens, d_model, hidden, dtype)
