@@ -22,10 +22,10 @@ extern "C" {
 int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
 
 /*
- * 1 where forward and backward through them also take no more time than library products around mg_swiglu_fwd and
- * mg_swiglu_bwd (0 for sizes they do not take); both bindings ask this.
+ * 1 where they also take no more time than library products around mg_swiglu_fwd and mg_swiglu_bwd (0 for sizes they do not
+ * take): forward and backward, or the forward pass that no backward pass follows.  Both bindings ask this.
  */
-int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
+int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only);
 
 /*
  * Bytes of workspace the two entry points need on the current device, 0 for none: where tokens are few, k is split over

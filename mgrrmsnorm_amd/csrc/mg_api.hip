@@ -771,17 +771,21 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
     return tokens * d_model * 2 <= most && tokens * hidden * 4 <= most && hidden * d_model * 4 <= most;
 }
 
-// Where forward + backward takes no more time than with the library's products and the activation between them.  GPU time in
+// Where they take no more time than the library's products and the activation between them.  GPU time in
 // replayed graphs (library / these, us, bf16, d_model x hidden, forward + backward; forward):
 //   1024 x 1792: 80 tokens 64.6 / 52.9; 18.7 / 20.5, 1024 97 / 78; 30 / 26.5, 8192 379 / 309; 113 / 93
-//   2048 x 3584: 80 97 / 72; 26.3 / 25.4, 1024 209 / 165; 68 / 58, 8192 1059 / 975; 324 / 336
-//   4096 x 11008: 80 435 / 244; 78 / 65, 320 533 / 440; 141 / 150, 1024 1008 / 885; 318 / 299, 2048 1958 / 1486; 617 / 503
-//   and beyond 128 MiB of weights from 4096 tokens on, 3072 x 8192 1614 / 1708; 498 / 536, 4096 x 6912 1850 / 1750; 548 / 593.
-// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162.6 / 47.2; 47 / 15.  Forward alone goes the same way, so that
-// it gives the same bits; it loses up to 9 % where its tiles just miss a round of the compute units.
-int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
-    if (tokens <= MG_BLOCK_MAX_TOKENS || !mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
-    return tokens < 4096 || 6 * d_model * hidden <= 128LL << 20;
+//   2048 x 3584: 8 82 / 66, 80 97 / 72; 26.3 / 25.4, 1024 209 / 165; 68 / 58, 8192 1059 / 975; 324 / 336
+//   4096 x 11008: 8 315 / 222, 32 323 / 226; 62 / 57, 320 533 / 440; 141 / 150, 1024 1008 / 885; 318 / 299, 2048 1958 / 1486; 617 / 503
+//   beyond 128 MiB of weights from 4096 tokens on: 3072 x 8192 1614 / 1708; 498 / 536, 4096 x 6912 1850 / 1750; 548 / 593
+//   below 16 MiB: 1024 x 1792 8 46.2 / 49.7, 17 52.1 / 50.2, 48 tokens 55.8 / 51.5; 17.4 / 20.2, 512 x 896 8 37.2 / 42.8.
+// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162.6 / 47.2; 47 / 15.  Beyond the tokens of a decoding step
+// forward alone goes the same way, so that it gives the same bits; it loses up to 9 % where its tiles just miss a round of the
+// compute units.
+int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only) {
+    if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
+    const int64_t weights = 6 * d_model * hidden;
+    if (tokens <= (forward_only ? MG_BLOCK_MAX_TOKENS : 16)) return weights >= 16LL << 20;
+    return tokens < 4096 || weights <= 128LL << 20;
 }
 
 namespace {

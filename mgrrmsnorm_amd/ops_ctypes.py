@@ -216,11 +216,15 @@ def swiglu_backward(grad_out: torch.Tensor, gate_up: torch.Tensor, hidden_dim: i
 _MLP_CODES = {torch.float16: 1, torch.bfloat16: 2}
 
 
+def _preferred(x, hidden, forward_only):
+    d_model = x.size(-1)
+    return _lib.load().mg_mlp_preferred(x.numel() // d_model, d_model, hidden, _MLP_CODES[x.dtype], int(forward_only)) == 1
+
+
 def swiglu_mlp_fits(x: torch.Tensor, hidden_dim: int) -> bool:
-    code = _MLP_CODES.get(x.dtype)
-    if code is None or not x.is_cuda or x.dim() < 1 or x.size(-1) < 1:
+    if x.dtype not in _MLP_CODES or not x.is_cuda or x.dim() < 1 or x.size(-1) < 1:
         return False
-    return _lib.load().mg_mlp_preferred(x.numel() // x.size(-1), x.size(-1), hidden_dim, code) == 1
+    return _preferred(x, hidden_dim, not torch.is_grad_enabled())
 
 
 def _plain_dense(t: torch.Tensor) -> bool:
@@ -307,8 +311,9 @@ def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
         return None
     if any(w.dtype != x.dtype or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16 != 0 for w in (w12, w3)):
         return None
-    if not swiglu_mlp_fits(x, hidden) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
+    learns = torch.is_grad_enabled() and (x.requires_grad or w12.requires_grad or w3.requires_grad)
+    if not _preferred(x, hidden, not learns) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
         return None
-    if torch.is_grad_enabled() and (x.requires_grad or w12.requires_grad or w3.requires_grad):
+    if learns:
         return _MlpFunction.apply(x, w12, w3) if x.requires_grad or w12.requires_grad else None
     return _mlp_forward(x.contiguous(), w12, w3, False)[0]

@@ -109,14 +109,16 @@ class MegaGemmTriton(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # The whole block at once, while the projections are the plain ones this module made: a decoding step in
-        # two kernels that read the weights once, longer inputs on the package's own matrix products.  The compiler is
+        # two kernels that read the weights once, everything else on the package's own matrix products.  The compiler is
         # asked about first, because it cannot trace the other questions; then the size, which other calls end at.
         if not torch.compiler.is_compiling() and type(x) is torch.Tensor:
             decoding = ops.swiglu_block_fits(x, self.hidden)
             if ((decoding or ops.swiglu_mlp_fits(x, self.hidden)) and not _calls_observed() and not _calls_replaced()):
                 w12, w3 = _plain_weight(self.w12), _plain_weight(self.w3)
                 if w12 is not None and w3 is not None and w3.dim() == 2 and w3.size(1) == self.hidden:
-                    out = (ops.swiglu_block if decoding else ops.swiglu_mlp)(x, w12, w3)
+                    out = ops.swiglu_block(x, w12, w3) if decoding else None
+                    if out is None:
+                        out = ops.swiglu_mlp(x, w12, w3)
                     if out is not None:
                         return out
         # the activation's autograd node lives in the compiled extension when that is built

@@ -47,7 +47,7 @@ def _bounded(got, ref, terms, count, dtype, extra=0.0):
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("tokens,d_model,hidden", [
-    (1, 64, 64), (65, 64, 192), (127, 192, 64), (128, 128, 128), (129, 128, 256), (257, 320, 448), (300, 704, 1088),
+    (1, 64, 64), (17, 1024, 1792), (64, 2048, 5504), (65, 64, 192), (127, 192, 64), (128, 128, 128), (129, 128, 256), (257, 320, 448), (300, 704, 1088),
     (1000, 512, 1344), (1024, 2048, 3584), (513, 1536, 4096), (2047, 1024, 2816), (96, 4096, 6912), (640, 3136, 8384),
     (127, 1024, 11008), (130, 3136, 8000), (70, 8192, 1088), (200, 704, 2752),   # k in 2 to 8 parts, of 43.5 and 9.5 steps
 ])
@@ -199,8 +199,10 @@ def test_what_goes_through_the_projections(binding, monkeypatch):
     module = _module()
     w12, w3 = module.w12.weight, module.w3.weight
     x = torch.randn(300, 512, device="cuda", dtype=torch.bfloat16)
-    assert _takes(module, x)
-    for y in (x[:64], x.float(), x[:, :511], torch.randn(300 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(300, 512)):
+    assert _takes(module, x) and _takes(module, x[:17])
+    with torch.no_grad():
+        assert _takes(module, x[:65]) and not _takes(module, x[:64])
+    for y in (x[:16], x.float(), x[:, :511], torch.randn(300 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(300, 512)):
         assert ops.swiglu_mlp(y, w12, w3) is None
     assert ops.swiglu_mlp(x, w12.t().contiguous().t(), w3) is None and ops.swiglu_mlp(x, w12.half(), w3) is None
     assert ops.swiglu_mlp(x.to_sparse(), w12, w3) is None and ops.swiglu_mlp(x.cpu(), w12, w3) is None
