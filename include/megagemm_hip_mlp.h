@@ -1,7 +1,7 @@
 /*
  * megagemm_hip_mlp.h -- the whole SwiGLU block (reference: megagemm/swiglu.py:165-172, two torch.matmul
  * around the Triton activation, and their autograd) on this library's own matrix products, with the activation
- * and its backward inside them: forward in two launches, backward in four, and one more for each
+ * and its backward inside them: forward in two launches, backward in two, and one more for each
  * product whose k is split.
  * Conventions as in megagemm_hip.h.  x, out, dy, dx [tokens, d_model]; w12 [2 * hidden, d_model], gate rows first;
  * w3 [d_model, hidden]; gate_up [tokens, 2 * hidden]; h [tokens, hidden]; all of `dtype`, MG_F16 or MG_BF16.
@@ -27,11 +27,17 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
  */
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only);
 
+/* What a workspace is for: the forward pass, or a backward pass that wants the sum of these. */
+#define MG_MLP_FORWARD 0
+#define MG_MLP_DX 1
+#define MG_MLP_DW12 2
+#define MG_MLP_DW3 4
+
 /*
- * Bytes of workspace the two entry points need on the current device, 0 for none: where tokens are few, k is split over
- * workgroups, whose sums meet there in fp32.
+ * Bytes of workspace a pass needs on the current device, 0 for none: where tokens are few, k is split over workgroups,
+ * whose sums meet there in fp32.
  */
-int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int64_t* forward_bytes, int64_t* backward_bytes);
+int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int pass, int64_t* bytes);
 
 /*
  * [gate | up] = x * w12^T, h = silu(gate) * up from sums kept in fp32, out = h * w3^T.

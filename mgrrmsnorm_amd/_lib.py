@@ -59,7 +59,7 @@ SIGNATURES = {
 MLP_SIGNATURES = {
     "mg_mlp_fits": (_int, [_i64, _i64, _i64, _int]),
     "mg_mlp_preferred": (_int, [_i64, _i64, _i64, _int, _int]),
-    "mg_mlp_workspace": (_int, [_i64, _i64, _i64, _int, ctypes.POINTER(_i64), ctypes.POINTER(_i64)]),
+    "mg_mlp_workspace": (_int, [_i64, _i64, _i64, _int, _int, ctypes.POINTER(_i64)]),
     "mg_mlp_fwd": (_int, [_vp] * 7 + [_i64] * 4 + [_int, _vp]),
     "mg_mlp_bwd": (_int, [_vp] * 11 + [_i64] * 4 + [_int, _vp]),
 }

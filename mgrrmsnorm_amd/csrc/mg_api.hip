@@ -814,43 +814,39 @@ int check_mlp(const char* fn, int64_t tokens, int64_t d_model, int64_t hidden, i
     return MG_OK;
 }
 
-// The products of one pass, in the order of their launches.
-struct MlpStep { MlpWhat what; bool wanted; int64_t M, N, K; };
-
-int64_t mlp_partial_bytes(const MlpStep* steps, int count, int cus) {
-    int64_t most = 0;
-    for (int i = 0; i < count; ++i) {
-        const MlpPlan p = mlp_plan_for(steps[i].what, steps[i].M, steps[i].N, steps[i].K, cus);
-        if (steps[i].wanted && p.splits > 1) most = std::max(most, (int64_t)p.splits * steps[i].M * steps[i].N * 4);
-    }
-    return most;
-}
-
-int run_mlp(const char* fn, int dtype, const MlpStep& step, MlpArgs a, int cus, void* workspace, hipStream_t s) {
-    a.M = (int)step.M;
-    a.N = (int)step.N;
-    a.K = (int)step.K;
-    a.partial = workspace;
-    const MlpPlan plan = mlp_plan_for(step.what, step.M, step.N, step.K, cus);
-    const hipError_t e = dtype == MG_F16 ? launch_mlp<half_t>(step.what, a, plan, s) : launch_mlp<bf16_t>(step.what, a, plan, s);
-    return e == hipSuccess ? MG_OK : fail_hip(fn, e);
-}
+int64_t partial_bytes(MlpPlan p, int64_t M, int64_t N) { return p.splits > 1 ? p.splits * M * N * 4 : 0; }
 
 struct MlpForward {
-    MlpStep steps[2];
-    MlpForward(int64_t t, int64_t d, int64_t h) : steps{{MlpWhat::gate_up, true, t, h, d}, {MlpWhat::down, true, t, d, h}} {}
-};
-struct MlpBackward {
-    MlpStep steps[4];
-    MlpBackward(int64_t t, int64_t d, int64_t h, bool x, bool w12, bool w3)
-        : steps{{MlpWhat::weight_grad, w3, d, h, t}, {MlpWhat::activation_bwd, x || w12, t, h, d},
-                {MlpWhat::weight_grad, w12, 2 * h, d, t}, {MlpWhat::input_grad, x, t, d, 2 * h}} {}
+    MlpPlan gate_up, down;
+    int64_t workspace;
+    MlpForward(int64_t t, int64_t d, int64_t h, int cus)
+        : gate_up(mlp_plan(mlp_size(MlpWhat::gate_up, t, h, d), cus)), down(mlp_plan(mlp_size(MlpWhat::down, t, d, h), cus)),
+          workspace(partial_bytes(down, t, d)) {}
 };
 
-int check_workspace(const char* fn, const MlpStep* steps, int count, const void* workspace, int64_t workspace_bytes, int* cus) {
-    const int rc = cu_count(cus);
-    if (rc != MG_OK) return rc;
-    const int64_t need = mlp_partial_bytes(steps, count, *cus);
+// Two launches: the gradients of w3 and, through the activation, of [gate | up]; then those of w12 and x.
+struct MlpBackward {
+    MlpPlan w3{-1, 1}, act{-1, 1}, w12{-1, 1}, x{-1, 1};
+    int64_t workspace[2], at[2];   // bytes of each launch, and where its second product's begin
+    MlpBackward(int64_t t, int64_t d, int64_t h, bool want_x, bool want_12, bool want_3, int cus) {
+        const MlpSize s3 = mlp_size(MlpWhat::weight_grad, d, h, t), sa = mlp_size(MlpWhat::activation_bwd, t, h, d);
+        const MlpSize s12 = mlp_size(MlpWhat::weight_grad, 2 * h, d, t), sx = mlp_size(MlpWhat::input_grad, t, d, 2 * h);
+        const bool want_a = want_x || want_12;
+        if (want_3 && want_a) mlp_plan_pair(s3, sa, cus, &w3, &act);
+        else if (want_3) w3 = mlp_plan(s3, cus);
+        else if (want_a) act = mlp_plan(sa, cus);
+        if (want_12 && want_x) mlp_plan_pair(s12, sx, cus, &w12, &x);
+        else if (want_12) w12 = mlp_plan(s12, cus);
+        else if (want_x) x = mlp_plan(sx, cus);
+        at[0] = partial_bytes(w3, d, h);
+        workspace[0] = at[0];
+        at[1] = partial_bytes(w12, 2 * h, d);
+        workspace[1] = at[1] + partial_bytes(x, t, d);
+    }
+    int64_t needs() const { return std::max(workspace[0], workspace[1]); }
+};
+
+int check_workspace(const char* fn, int64_t need, const void* workspace, int64_t workspace_bytes) {
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MG_ERR_INVALID_ARG, "%s: the workspace must hold %lld bytes (mg_mlp_workspace)", fn, (long long)need);
     return MG_OK;
@@ -858,14 +854,16 @@ int check_workspace(const char* fn, const MlpStep* steps, int count, const void*
 
 }  // namespace
 
-int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int64_t* forward_bytes, int64_t* backward_bytes) {
-    if (forward_bytes == nullptr || backward_bytes == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_workspace: an output is NULL");
+int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int pass, int64_t* bytes) {
+    if (bytes == nullptr || pass < 0 || pass > (MG_MLP_DX | MG_MLP_DW12 | MG_MLP_DW3))
+        return fail(MG_ERR_INVALID_ARG, "mg_mlp_workspace: bytes must not be NULL, and pass a sum of MG_MLP_ constants");
     if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return fail(MG_ERR_UNSUPPORTED, "mg_mlp_workspace: sizes mg_mlp_fits does not take");
     int cus = 0;
     const int rc = cu_count(&cus);
     if (rc != MG_OK) return rc;
-    *forward_bytes = mlp_partial_bytes(MlpForward(tokens, d_model, hidden).steps, 2, cus);
-    *backward_bytes = mlp_partial_bytes(MlpBackward(tokens, d_model, hidden, true, true, true).steps, 4, cus);
+    *bytes = pass == MG_MLP_FORWARD
+                 ? MlpForward(tokens, d_model, hidden, cus).workspace
+                 : MlpBackward(tokens, d_model, hidden, pass & MG_MLP_DX, pass & MG_MLP_DW12, pass & MG_MLP_DW3, cus).needs();
     return MG_OK;
 }
 
@@ -877,15 +875,21 @@ int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12
     int rc = check_mlp("mg_mlp_fwd", tokens, d_model, hidden, dtype, outs, 4, in, 3);
     if (rc != MG_OK) return rc;
     if (out == nullptr || h == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_fwd: out and h must not be NULL");
-    const MlpForward pass(tokens, d_model, hidden);
     int cus = 0;
-    rc = check_workspace("mg_mlp_fwd", pass.steps, 2, workspace, workspace_bytes, &cus);
+    rc = cu_count(&cus);
     if (rc != MG_OK) return rc;
-    const int d = (int)d_model, n = (int)hidden;
+    const MlpForward pass(tokens, d_model, hidden, cus);
+    rc = check_workspace("mg_mlp_fwd", pass.workspace, workspace, workspace_bytes);
+    if (rc != MG_OK) return rc;
+    const int t = (int)tokens, d = (int)d_model, n = (int)hidden;
     hipStream_t s = (hipStream_t)stream;
-    rc = run_mlp("mg_mlp_fwd", dtype, pass.steps[0], {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d}, cus, workspace, s);
+    const auto run = [&](MlpWhat what, const MlpArgs& a, MlpPlan p) {
+        const hipError_t e = dtype == MG_F16 ? launch_mlp_forward<half_t>(what, a, p, s) : launch_mlp_forward<bf16_t>(what, a, p, s);
+        return e == hipSuccess ? MG_OK : fail_hip("mg_mlp_fwd", e);
+    };
+    rc = run(MlpWhat::gate_up, {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d, t, n, d, nullptr}, pass.gate_up);
     if (rc != MG_OK) return rc;
-    return run_mlp("mg_mlp_fwd", dtype, pass.steps[1], {out, nullptr, nullptr, h, (uint32_t)th, n, w3, (uint32_t)w, n}, cus, workspace, s);
+    return run(MlpWhat::down, {out, nullptr, nullptr, h, (uint32_t)th, n, w3, (uint32_t)w, n, t, d, n, workspace}, pass.down);
 }
 
 int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy, const void* x, const void* w12, const void* w3,
@@ -896,20 +900,32 @@ int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy,
     const MlpTensor outs[] = {{"dx", dx, td}, {"dw12", dw12, 2 * w}, {"dw3", dw3, w}, {"d_gate_up", d_gate_up, 2 * th}, {"workspace", workspace, workspace_bytes}};
     int rc = check_mlp("mg_mlp_bwd", tokens, d_model, hidden, dtype, outs, 5, in, 6);
     if (rc != MG_OK) return rc;
-    const MlpBackward pass(tokens, d_model, hidden, dx != nullptr, dw12 != nullptr, dw3 != nullptr);
-    if (pass.steps[1].wanted && d_gate_up == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
+    const bool want_x = dx != nullptr, want_12 = dw12 != nullptr, want_3 = dw3 != nullptr;
+    if ((want_x || want_12) && d_gate_up == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
     int cus = 0;
-    rc = check_workspace("mg_mlp_bwd", pass.steps, 4, workspace, workspace_bytes, &cus);
+    rc = cu_count(&cus);
     if (rc != MG_OK) return rc;
-    const int d = (int)d_model, n = (int)hidden;
-    const MlpArgs args[] = {
-        {dw3, nullptr, nullptr, dy, (uint32_t)td, d, h, (uint32_t)th, n},
-        {d_gate_up, nullptr, gate_up, dy, (uint32_t)td, d, w3, (uint32_t)w, n},
-        {dw12, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, x, (uint32_t)td, d},
-        {dx, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, w12, (uint32_t)(2 * w), d}};
-    for (int i = 0; i < 4 && rc == MG_OK; ++i)
-        if (pass.steps[i].wanted) rc = run_mlp("mg_mlp_bwd", dtype, pass.steps[i], args[i], cus, workspace, (hipStream_t)stream);
-    return rc;
+    const MlpBackward pass(tokens, d_model, hidden, want_x, want_12, want_3, cus);
+    rc = check_workspace("mg_mlp_bwd", pass.needs(), workspace, workspace_bytes);
+    if (rc != MG_OK) return rc;
+    const int t = (int)tokens, d = (int)d_model, n = (int)hidden;
+    char* const work = (char*)workspace;
+    const MlpTask w3_grad = {MlpWhat::weight_grad, {dw3, nullptr, nullptr, dy, (uint32_t)td, d, h, (uint32_t)th, n, d, n, t, work}, pass.w3};
+    const MlpTask act = {MlpWhat::activation_bwd, {d_gate_up, nullptr, gate_up, dy, (uint32_t)td, d, w3, (uint32_t)w, n, t, n, d, nullptr}, pass.act};
+    const MlpTask w12_grad = {MlpWhat::weight_grad,
+                              {dw12, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, x, (uint32_t)td, d, 2 * n, d, t, work}, pass.w12};
+    const MlpTask x_grad = {MlpWhat::input_grad,
+                            {dx, nullptr, nullptr, d_gate_up, (uint32_t)(2 * th), 2 * n, w12, (uint32_t)(2 * w), d, t, d, 2 * n, work + pass.at[1]}, pass.x};
+    const auto run = [&](const MlpTask& p, bool want_p, const MlpTask& q, bool want_q) {
+        if (!want_p && !want_q) return (int)MG_OK;
+        const MlpTask tasks[] = {want_p ? p : q, q};
+        const int count = want_p && want_q ? 2 : 1;
+        const hipError_t e = dtype == MG_F16 ? launch_mlp_backward<half_t>(tasks, count, (hipStream_t)stream)
+                                             : launch_mlp_backward<bf16_t>(tasks, count, (hipStream_t)stream);
+        return e == hipSuccess ? (int)MG_OK : fail_hip("mg_mlp_bwd", e);
+    };
+    rc = run(w3_grad, want_3, act, want_x || want_12);
+    return rc == MG_OK ? run(w12_grad, want_12, x_grad, want_x) : rc;
 }
 
 }  // extern "C"

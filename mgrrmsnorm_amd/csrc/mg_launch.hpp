@@ -259,10 +259,13 @@ struct MlpArgs {
     int M, N, K;
     void* partial;
 };
-inline MlpPlan mlp_plan_for(MlpWhat what, int64_t M, int64_t N, int64_t K, int cus) {
+inline MlpSize mlp_size(MlpWhat what, int64_t M, int64_t N, int64_t K) {
     const bool fused = what == MlpWhat::gate_up || what == MlpWhat::activation_bwd;   // the activation needs whole sums
-    return mlp_plan(M, what == MlpWhat::gate_up ? 2 * N : N, K, what == MlpWhat::weight_grad, !fused, cus);
+    return {M, what == MlpWhat::gate_up ? 2 * N : N, K, what == MlpWhat::weight_grad, !fused};
 }
-template <typename T> hipError_t launch_mlp(MlpWhat what, const MlpArgs& a, MlpPlan plan, hipStream_t s);
+struct MlpTask { MlpWhat what; MlpArgs args; MlpPlan plan; };
+template <typename T> hipError_t launch_mlp_forward(MlpWhat what, const MlpArgs& a, MlpPlan plan, hipStream_t s);
+// One or two products that do not need each other, in one launch.
+template <typename T> hipError_t launch_mlp_backward(const MlpTask* tasks, int count, hipStream_t s);
 
 }  // namespace mg

@@ -410,21 +410,30 @@ __device__ __forceinline__ void mlp_tile(int id, int rows, int cols, int splits,
     tn = in / h;
 }
 
+// One product: out from a [M, K] and b [N, K], in `tiles` workgroups (those of all its splits).
+struct MlpJob { MlpOperand A, B; MlpOut o; int K, splits, shape; u32 tiles; };
+
 template <typename T, class C, bool A_ALONG_K, bool B_ALONG_K, int WHAT>
-__global__ void __launch_bounds__(C::THREADS, C::WAVES / 4)
-mlp_gemm(MlpOperand A, MlpOperand B, MlpOut o, int K, int splits) {
-    __shared__ __attribute__((aligned(1024))) char lds[C::STAGE * C::STAGES];
+__device__ __forceinline__ void mlp_job(const MlpJob& job, u32 id, char MG_LDS* lds) {
     constexpr int BN = WHAT == kMlpGateUp ? C::BN / 2 : C::BN;
+    MlpOut o = job.o;
     int tm, tn, split;
-    mlp_tile(blockIdx.x, (o.M + C::BM - 1) / C::BM, (o.N + BN - 1) / BN, splits, tm, tn, split);
-    const int steps = (K + C::BK - 1) / C::BK, first = split * steps / splits, last = (split + 1) * steps / splits;
+    mlp_tile((int)id, (o.M + C::BM - 1) / C::BM, (o.N + BN - 1) / BN, job.splits, tm, tn, split);
+    const int steps = (job.K + C::BK - 1) / C::BK, first = split * steps / job.splits, last = (split + 1) * steps / job.splits;
     MlpShare<C> share;
     MlpProduct<T, C, A_ALONG_K, B_ALONG_K, WHAT == kMlpGateUp> p;
-    p.A = A;
-    p.B = B;
-    p.run(share, (char MG_LDS*)lds, first, last - first, tm * C::BM, tn * BN, o.N);
+    p.A = job.A;
+    p.B = job.B;
+    p.run(share, lds, first, last - first, tm * C::BM, tn * BN, o.N);
     if constexpr (WHAT == kMlpPartial) o.out = (float*)o.out + (size_t)split * o.M * o.N;
-    mlp_finish<T, C, WHAT>(share, (char MG_LDS*)lds, o, tm * C::BM, tn * BN);
+    mlp_finish<T, C, WHAT>(share, lds, o, tm * C::BM, tn * BN);
+}
+
+template <typename T, class C, bool A_ALONG_K, bool B_ALONG_K, int WHAT>
+__global__ void __launch_bounds__(C::THREADS, C::WAVES / 4)
+mlp_gemm(MlpJob job) {
+    __shared__ __attribute__((aligned(1024))) char lds[C::STAGE * C::STAGES];
+    mlp_job<T, C, A_ALONG_K, B_ALONG_K, WHAT>(job, blockIdx.x, (char MG_LDS*)lds);
 }
 
 }  // namespace mg

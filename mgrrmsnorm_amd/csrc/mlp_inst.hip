@@ -24,47 +24,111 @@ template <int I, class C> constexpr bool is_shape() {
 }
 static_assert(is_shape<0, Huge>() && is_shape<1, Large>() && is_shape<2, Medium>() && is_shape<3, Small>(), "the plan's tiles");
 
-template <class C, bool A_ALONG_K, bool B_ALONG_K, int WHAT>
-hipError_t run(const MlpArgs& a, int splits, hipStream_t s) {
-    constexpr int BN = WHAT == kMlpGateUp ? C::BN / 2 : C::BN;
-    const unsigned rows = (a.M + C::BM - 1) / C::BM, cols = (a.N + BN - 1) / BN;
-    const MlpOperand A = {a.a, a.a_bytes, a.a_ld}, B = {a.b, a.b_bytes, a.b_ld};
-    const MlpOut o = {WHAT == kMlpPartial ? a.partial : a.out, a.second, a.in, a.M, a.N};
-    return launch(mlp_gemm<T, C, A_ALONG_K, B_ALONG_K, WHAT>, dim3(rows * cols * splits), dim3(C::THREADS), 0, s, A, B, o, a.K, splits);
+template <int SHAPE> struct ShapeOf;
+template <> struct ShapeOf<0> { using type = Huge; };
+template <> struct ShapeOf<1> { using type = Large; };
+template <> struct ShapeOf<2> { using type = Medium; };
+template <> struct ShapeOf<3> { using type = Small; };
+
+MlpJob job_of(const MlpArgs& a, MlpPlan p, bool paired) {
+    const MlpShape& s = kMlpShapes[p.shape];
+    const int bn = paired ? s.bn / 2 : s.bn;
+    const u32 tiles = (u32)((a.M + s.bm - 1) / s.bm) * (u32)((a.N + bn - 1) / bn) * (u32)p.splits;
+    return {{a.a, a.a_bytes, a.a_ld}, {a.b, a.b_bytes, a.b_ld}, {p.splits > 1 ? a.partial : a.out, a.second, a.in, a.M, a.N}, a.K, p.splits, p.shape, tiles};
 }
 
-template <bool A_ALONG_K, bool B_ALONG_K, int WHAT>
-hipError_t by_shape(const MlpArgs& a, MlpPlan p, hipStream_t s) {
-    switch (p.shape) {
-        case 0: return run<Huge, A_ALONG_K, B_ALONG_K, WHAT>(a, p.splits, s);
-        case 1: return run<Large, A_ALONG_K, B_ALONG_K, WHAT>(a, p.splits, s);
-        case 2: return run<Medium, A_ALONG_K, B_ALONG_K, WHAT>(a, p.splits, s);
-        case 3: return run<Small, A_ALONG_K, B_ALONG_K, WHAT>(a, p.splits, s);
+// ---- forward: one product a launch, each the other's input ----
+template <int SHAPE, int WHAT>
+hipError_t run(const MlpJob& job, hipStream_t s) {
+    using C = typename ShapeOf<SHAPE>::type;
+    return launch(mlp_gemm<T, C, true, true, WHAT>, dim3(job.tiles), dim3(C::THREADS), 0, s, job);
+}
+template <int WHAT>
+hipError_t by_shape(const MlpJob& job, hipStream_t s) {
+    switch (job.shape) {
+        case 0: return run<0, WHAT>(job, s);
+        case 1: return run<1, WHAT>(job, s);
+        case 2: return run<2, WHAT>(job, s);
+        case 3: return run<3, WHAT>(job, s);
         default: return hipErrorInvalidValue;
     }
 }
 
-template <bool A_ALONG_K, bool B_ALONG_K>
-hipError_t maybe_split(const MlpArgs& a, MlpPlan p, hipStream_t s) {
-    if (p.splits == 1) return by_shape<A_ALONG_K, B_ALONG_K, kMlpStore>(a, p, s);
-    const hipError_t e = by_shape<A_ALONG_K, B_ALONG_K, kMlpPartial>(a, p, s);
-    if (e != hipSuccess) return e;
+hipError_t add_parts(const MlpArgs& a, MlpPlan p, hipStream_t s) {
+    if (p.splits == 1) return hipSuccess;
     const unsigned vectors = (unsigned)((long)a.M * a.N / 8);
     return launch(mlp_add<T>, dim3((vectors + 255) / 256), dim3(256), 0, s, (T*)a.out, (const float*)a.partial, vectors, p.splits);
+}
+
+// ---- backward: two products a launch ----
+// Neither needs the other, and each alone leaves compute units idle: at 1024 tokens, 2048 x 3584, 224 tiles for 256 of them and a
+// ramp, a tail and a launch of its own.  There the four launches took 22.4 + 21 and 39.3 + 33.9 us, the two take 36 and
+// 65, and a whole step 156.3 us instead of 168.6; 300 tokens, 512 x 1024 37.8 instead of 47 (eager: launches).  Longer tiles
+// first, whichever product they are of.  Every kind and size of tile is in the one kernel, which all of them suit: 512
+// threads, one workgroup per compute unit.
+enum Kind { kWeightGrad, kInputGrad, kActBwd };
+constexpr int kBackwardLds = 3 * 48 * 1024;
+static_assert(Huge::STAGE * Huge::STAGES <= kBackwardLds && Large::STAGE * Large::STAGES <= kBackwardLds && Medium::STAGE * Medium::STAGES <= kBackwardLds &&
+              Small::STAGE * Small::STAGES <= kBackwardLds && Huge::THREADS == 512 && Large::THREADS == 512 && Medium::THREADS == 512 && Small::THREADS == 512, "");
+
+template <class C>
+__device__ __forceinline__ void any_kind(const MlpJob& job, int kind, u32 id, char MG_LDS* lds) {
+    if (kind == kWeightGrad) {
+        if (job.splits > 1) mlp_job<T, C, false, false, kMlpPartial>(job, id, lds);
+        else mlp_job<T, C, false, false, kMlpStore>(job, id, lds);
+    } else if (kind == kInputGrad) {
+        if (job.splits > 1) mlp_job<T, C, true, false, kMlpPartial>(job, id, lds);
+        else mlp_job<T, C, true, false, kMlpStore>(job, id, lds);
+    } else {
+        mlp_job<T, C, true, false, kMlpActBwd>(job, id, lds);
+    }
+}
+
+// `a_blocks` workgroups for job a, a multiple of 8 so that both keep their tiles' dies
+__global__ void __launch_bounds__(512, 2)
+mlp_backward(MlpJob a, int a_kind, u32 a_blocks, MlpJob b, int b_kind) {
+    __shared__ __attribute__((aligned(1024))) char lds[kBackwardLds];
+    const bool second = blockIdx.x >= a_blocks;
+    const MlpJob& job = second ? b : a;
+    const int kind = second ? b_kind : a_kind;
+    const u32 id = second ? blockIdx.x - a_blocks : blockIdx.x;
+    if (id >= job.tiles) return;
+    switch (job.shape) {
+        case 0: return any_kind<Huge>(job, kind, id, (char MG_LDS*)lds);
+        case 1: return any_kind<Large>(job, kind, id, (char MG_LDS*)lds);
+        case 2: return any_kind<Medium>(job, kind, id, (char MG_LDS*)lds);
+        case 3: return any_kind<Small>(job, kind, id, (char MG_LDS*)lds);
+    }
+}
+
+Kind kind_of(MlpWhat what) {
+    return what == MlpWhat::weight_grad ? kWeightGrad : what == MlpWhat::input_grad ? kInputGrad : kActBwd;
 }
 
 }  // namespace
 
 template <>
-hipError_t launch_mlp<T>(MlpWhat what, const MlpArgs& a, MlpPlan p, hipStream_t s) {
-    switch (what) {
-        case MlpWhat::gate_up: return by_shape<true, true, kMlpGateUp>(a, p, s);
-        case MlpWhat::down: return maybe_split<true, true>(a, p, s);
-        case MlpWhat::activation_bwd: return by_shape<true, false, kMlpActBwd>(a, p, s);
-        case MlpWhat::input_grad: return maybe_split<true, false>(a, p, s);
-        case MlpWhat::weight_grad: return maybe_split<false, false>(a, p, s);
-    }
-    return hipErrorInvalidValue;
+hipError_t launch_mlp_forward<T>(MlpWhat what, const MlpArgs& a, MlpPlan p, hipStream_t s) {
+    const MlpJob job = job_of(a, p, what == MlpWhat::gate_up);
+    if (what == MlpWhat::gate_up) return by_shape<kMlpGateUp>(job, s);
+    if (p.splits == 1) return by_shape<kMlpStore>(job, s);
+    const hipError_t e = by_shape<kMlpPartial>(job, s);
+    return e == hipSuccess ? add_parts(a, p, s) : e;
+}
+
+template <>
+hipError_t launch_mlp_backward<T>(const MlpTask* tasks, int count, hipStream_t s) {
+    if (count < 1 || count > 2) return hipErrorInvalidValue;
+    MlpJob jobs[2] = {job_of(tasks[0].args, tasks[0].plan, false), {}};
+    if (count == 2) jobs[1] = job_of(tasks[1].args, tasks[1].plan, false);
+    const int last = count - 1;
+    const int first = count == 2 && mlp_tile_us(tasks[1].plan, tasks[1].args.K) > mlp_tile_us(tasks[0].plan, tasks[0].args.K) ? 1 : 0;
+    const int second = count == 2 ? 1 - first : 0;
+    const u32 a_blocks = (jobs[first].tiles + 7) / 8 * 8, b_blocks = count == 2 ? jobs[second].tiles : 0;
+    hipError_t e = launch(mlp_backward, dim3(a_blocks + b_blocks), dim3(512), 0, s, jobs[first], (int)kind_of(tasks[first].what), a_blocks,
+                          jobs[second], (int)kind_of(tasks[second].what));
+    for (int i = 0; i <= last && e == hipSuccess; ++i) e = add_parts(tasks[i].args, tasks[i].plan, s);
+    return e;
 }
 
 }  // namespace mg

@@ -6,34 +6,95 @@
 
 namespace mg {
 
-// Time of a launch = 3 us + rounds of one tile per compute unit * (cost of a tile + 64s of k * time of each), fitted to
-// products with 32 to 5500 tiles of each kind (bf16, us, from the largest tile to the smallest): 7168 x 2048
+// Time of a launch = rounds of one tile per compute unit * (cost of a tile + 64s of k * time of each), in blocks whose operands
+// come from memory.  Single products on cached operands (bf16, us, from the largest tile to the smallest): 7168 x 2048
 // outputs, k 1024: 30 / 36 / 45 / 57; 1024 x 7168, k 2048: 46 / 32 / 34.6 / 50; 1024 x 3584, k 2048: 44 / 27 / 19.1 / 26.5;
-// 1024 x 2048, k 3584: 69 / 40 / 24.5 / 21; 4096 x 11008, k 128: 28.6 / 41 / 49 / 93.
+// 1024 x 2048, k 3584: 69 / 40 / 24.5 / 21; 4096 x 11008, k 128: 28.6 / 41 / 49 / 93.  The times fitted to those (1.1, 0.68, 0.36, 0.31)
+// give the medium tile too much in a block: forward + backward of 128 and 320 tokens, 4096 x 11008, 297 and 458 us
+// with them, 265 and 418 with these; 742, 1664 x 4608 151.5 / 144; 1024, 2048 x 3584 159.6 / 157.3.
 struct MlpShape { int bm, bn, bk; float tile_us, k64_us; };
-constexpr MlpShape kMlpShapes[] = {{256, 256, 64, 9.0f, 1.1f}, {128, 256, 64, 4.7f, 0.68f}, {128, 128, 64, 3.7f, 0.36f}, {128, 64, 128, 2.2f, 0.31f}};
+constexpr MlpShape kMlpShapes[] = {{256, 256, 64, 9.0f, 1.3f}, {128, 256, 64, 4.7f, 0.80f}, {128, 128, 64, 3.7f, 0.47f}, {128, 64, 128, 2.2f, 0.34f}};
 
 struct MlpPlan { int shape, splits; };
 
-// A product [M, N] over K; `ragged`: K need not be a multiple of the step (lines beyond the last read as zero); `splittable`:
-// the sums may be finished by a second launch, from an array of fp32 per split.  Few tokens through wide weights leave most
-// compute units without a tile otherwise: 128 tokens, 4096 x 11008, forward + backward 262 us with splits, 566 without.
-inline MlpPlan mlp_plan(int64_t M, int64_t N, int64_t K, bool ragged, bool splittable, int cus) {
+// What is known of a product [M, N] over K: `ragged`, K need not be a multiple of the step (lines beyond the last read as zero);
+// `splittable`, the sums may be finished by a second launch, from an array of fp32 per split.  Few tokens through wide weights
+// leave most compute units without a tile otherwise: 128 tokens, 4096 x 11008, forward + backward 262 us with splits, 566 without.
+struct MlpSize { int64_t M, N, K; bool ragged, splittable; };
+
+// One way to do it: tiles (of all splits), time of one, and what the second launch adds.
+struct MlpWay { MlpPlan plan; int64_t tiles; float tile_us, extra_us; };
+
+inline float mlp_tile_us(MlpPlan p, int64_t K) {
+    const MlpShape& s = kMlpShapes[p.shape];
+    return s.tile_us + s.k64_us * (float)((K + p.splits - 1) / p.splits) / 64.0f;
+}
+
+// Whether shape `i` can do it, and how if its k goes to `splits`.
+inline bool mlp_way(const MlpSize& p, int i, int splits, MlpWay* way) {
+    const MlpShape& s = kMlpShapes[i];
+    if (!p.ragged && p.K % s.bk != 0) return false;
+    if (splits > 1 && (!p.splittable || p.K / splits < 512 || splits * p.M * p.N * 4 > (256LL << 20))) return false;
+    way->plan = {i, splits};
+    way->tiles = ((p.M + s.bm - 1) / s.bm) * ((p.N + s.bn - 1) / s.bn) * splits;
+    way->tile_us = mlp_tile_us(way->plan, p.K);
+    // written and read at 5 TB/s, the launch, and stores that do not overlap
+    way->extra_us = splits > 1 ? 6.0f + (float)(splits * p.M * p.N) * (8.0f / 5e6f) : 0.0f;
+    return true;
+}
+constexpr int kMlpSplits[] = {1, 2, 3, 4, 6, 8};
+
+inline MlpPlan mlp_plan(const MlpSize& p, int cus) {
     MlpPlan best = {-1, 1};
     float least = 0.0f;
-    for (int i = 0; i < 4; ++i) {
-        const MlpShape& s = kMlpShapes[i];
-        if (!ragged && K % s.bk != 0) continue;
-        const int64_t tiles = ((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-        for (const int splits : {1, 2, 3, 4, 6, 8}) {
-            const int64_t k = (K + splits - 1) / splits;
-            if (splits > 1 && (!splittable || k < 512 || splits * M * N * 4 > (256LL << 20))) break;
-            float t = (float)((tiles * splits + cus - 1) / cus) * (s.tile_us + s.k64_us * (float)k / 64.0f);
-            if (splits > 1) t += 8.0f + (float)(splits * M * N) * (8.0f / 5e6f);   // written and read at 5 TB/s, the launch, and stores that do not overlap
-            if (best.shape < 0 || t < least) { best = {i, splits}; least = t; }
+    for (int i = 0; i < 4; ++i)
+        for (const int splits : kMlpSplits) {
+            MlpWay w;
+            if (!mlp_way(p, i, splits, &w)) break;
+            const float t = (float)((w.tiles + cus - 1) / cus) * w.tile_us + w.extra_us;
+            if (best.shape < 0 || t < least) { best = w.plan; least = t; }
         }
-    }
     return best;
+}
+
+// When the last of `a`'s tiles and then `b`'s, each taking the first compute unit that is free, is done.
+inline float mlp_makespan(const MlpWay& a, const MlpWay& b, int cus) {
+    const int64_t full = a.tiles / cus, more = a.tiles % cus;      // `more` units are free a tile later than the others
+    const float early = (float)full * a.tile_us, late = early + a.tile_us;
+    float low = more > 0 ? late : early, high = late + (float)((b.tiles + cus - 1) / cus) * b.tile_us;
+    for (int i = 0; i < 8 && high - low > 0.5f; ++i) {
+        const float t = 0.5f * (low + high);
+        const int64_t done = more * (t > late ? (int64_t)((t - late) / b.tile_us) : 0) + (cus - more) * (int64_t)((t - early) / b.tile_us);
+        if (done >= b.tiles) high = t;
+        else low = t;
+    }
+    return high;
+}
+
+// The plans of two products that share a launch, longer tiles first: for the pair a cheaper tile often beats the one that fills
+// the compute units by itself.
+inline void mlp_plan_pair(const MlpSize& p, const MlpSize& q, int cus, MlpPlan* plan_p, MlpPlan* plan_q) {
+    float least = -1.0f;
+    MlpWay ways[2][24];
+    int count[2] = {0, 0};
+    const MlpSize* sizes[2] = {&p, &q};
+    for (int k = 0; k < 2; ++k)
+        for (int i = 0; i < 4; ++i)
+            for (const int splits : kMlpSplits) {
+                MlpWay w;
+                if (!mlp_way(*sizes[k], i, splits, &w)) break;
+                // of the split ways only those that still leave units free without
+                if (splits > 1 && w.tiles / splits * (splits - 1) > 2 * cus) break;
+                ways[k][count[k]++] = w;
+            }
+    for (int i = 0; i < count[0]; ++i)
+        for (int k = 0; k < count[1]; ++k) {
+            const MlpWay &a = ways[0][i], &b = ways[1][k];
+            const float work = ((float)a.tiles * a.tile_us + (float)b.tiles * b.tile_us) / (float)cus + a.extra_us + b.extra_us;
+            if (least >= 0.0f && work >= least) continue;      // no order can be better
+            const float t = (a.tile_us >= b.tile_us ? mlp_makespan(a, b, cus) : mlp_makespan(b, a, cus)) + a.extra_us + b.extra_us;
+            if (least < 0.0f || t < least) { least = t; *plan_p = a.plan; *plan_q = b.plan; }
+        }
 }
 
 }  // namespace mg

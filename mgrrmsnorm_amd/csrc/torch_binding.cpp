@@ -351,11 +351,10 @@ bool calls_transformed() {
 }
 
 // What mg_mlp_fwd or mg_mlp_bwd needs besides its tensors; undefined where that is nothing.
-Tensor mlp_workspace(const Tensor& x, int64_t tokens, int64_t d_model, int64_t hidden, bool forward) {
-    int64_t bytes[2] = {0, 0};
-    TORCH_CHECK(mg_mlp_workspace(tokens, d_model, hidden, dtype_code(x.scalar_type()), &bytes[0], &bytes[1]) == MG_OK,
+Tensor mlp_workspace(const Tensor& x, int64_t tokens, int64_t d_model, int64_t hidden, int pass) {
+    int64_t need = 0;
+    TORCH_CHECK(mg_mlp_workspace(tokens, d_model, hidden, dtype_code(x.scalar_type()), pass, &need) == MG_OK,
                 "SwiGLU block (workspace query) failed: ", mg_last_error());
-    const int64_t need = bytes[forward ? 0 : 1];
     return need > 0 ? at::empty({need}, x.options().dtype(at::kByte)) : Tensor();
 }
 void* pointer_of(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -366,7 +365,7 @@ Tensor mlp_forward(const Tensor& x, const Tensor& w12, const Tensor& w3, Tensor*
     if (gate_up != nullptr) *gate_up = at::empty({tokens, 2 * hidden}, x.options());
     *h = at::empty({tokens, hidden}, x.options());
     auto out = empty_as(x);
-    const Tensor work = mlp_workspace(x, tokens, d_model, hidden, true);
+    const Tensor work = mlp_workspace(x, tokens, d_model, hidden, MG_MLP_FORWARD);
     const int rc = mg_mlp_fwd(out.data_ptr(), h->data_ptr(), gate_up != nullptr ? gate_up->data_ptr() : nullptr, x.data_ptr(),
                               w12.data_ptr(), w3.data_ptr(), pointer_of(work), work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
     TORCH_CHECK(rc == MG_OK, "SwiGLU block forward failed (code ", rc, "): ", mg_last_error());
@@ -412,7 +411,7 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
         if (want[0] || want[1]) d_gate_up = empty_as(gate_up);
         for (int i = 0; i < 3; ++i)
             if (want[i]) out[i] = empty_as(saved[i]);
-        const Tensor work = mlp_workspace(x, tokens, d_model, hidden, false);
+        const Tensor work = mlp_workspace(x, tokens, d_model, hidden, (want[0] ? MG_MLP_DX : 0) | (want[1] ? MG_MLP_DW12 : 0) | (want[2] ? MG_MLP_DW3 : 0));
         const int rc = mg_mlp_bwd(pointer_of(out[0]), pointer_of(out[1]), pointer_of(out[2]), pointer_of(d_gate_up), dy.data_ptr(), x.data_ptr(),
                                   w12.data_ptr(), w3.data_ptr(), gate_up.data_ptr(), h.data_ptr(), pointer_of(work),
                                   work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());

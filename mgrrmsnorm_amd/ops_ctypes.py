@@ -239,13 +239,14 @@ def _pointer(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _mlp_workspace(x, tokens, d_model, hidden, forward):
-    """(tensor or None, its bytes) that mg_mlp_fwd or mg_mlp_bwd needs besides its tensors."""
-    sizes = ctypes.c_int64(0), ctypes.c_int64(0)
-    _lib.check(_lib.load().mg_mlp_workspace(tokens, d_model, hidden, _MLP_CODES[x.dtype], *map(ctypes.byref, sizes)),
+def _mlp_workspace(x, tokens, d_model, hidden, wanted):
+    """(tensor or None, its bytes) that a pass needs besides its tensors; wanted: nothing for the forward pass,
+    else the gradients of x, w12 and w3 that are."""
+    need = ctypes.c_int64(0)
+    mask = sum(1 << i for i, w in enumerate(wanted) if w)
+    _lib.check(_lib.load().mg_mlp_workspace(tokens, d_model, hidden, _MLP_CODES[x.dtype], mask, ctypes.byref(need)),
                "SwiGLU block (workspace query)")
-    need = sizes[0 if forward else 1].value
-    return (torch.empty(need, dtype=torch.uint8, device=x.device) if need else None), need
+    return (torch.empty(need.value, dtype=torch.uint8, device=x.device) if need.value else None), need.value
 
 
 def _mlp_forward(x, w12, w3, keep_gate_up):
@@ -255,7 +256,7 @@ def _mlp_forward(x, w12, w3, keep_gate_up):
         gate_up = x.new_empty(tokens, 2 * hidden) if keep_gate_up else None
         h = x.new_empty(tokens, hidden)
         out = torch.empty_like(x)
-        work, size = _mlp_workspace(x, tokens, d_model, hidden, True)
+        work, size = _mlp_workspace(x, tokens, d_model, hidden, ())
         rc = _lib.load().mg_mlp_fwd(out.data_ptr(), h.data_ptr(), _pointer(gate_up), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
                                     _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype], _lib.stream_ptr(x.device))
     _lib.check(rc, "SwiGLU block forward")
@@ -292,7 +293,7 @@ class _MlpFunction(torch.autograd.Function):
             grads = [torch.empty_like(t) if w else None for t, w in zip((x, w12, w3), want)]
             d_gate_up = torch.empty_like(gate_up) if want[0] or want[1] else None
             tokens = x.numel() // d_model
-            work, size = _mlp_workspace(x, tokens, d_model, hidden, False)
+            work, size = _mlp_workspace(x, tokens, d_model, hidden, want[:3])
             rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
                                         gate_up.data_ptr(), h.data_ptr(), _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype],
                                         _lib.stream_ptr(x.device))

@@ -16,9 +16,10 @@ ROUNDING = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}
 
 
 def _call(name, tensors, sizes, dtype):
-    need = ctypes.c_int64(0), ctypes.c_int64(0)
-    U.check(U.lib().mg_mlp_workspace(*sizes, U.CODES[dtype], *map(ctypes.byref, need)))
-    size = need[name == "mg_mlp_bwd"].value
+    need = ctypes.c_int64(0)
+    wanted = sum(1 << i for i, t in enumerate(tensors[:3]) if t is not None) if name == "mg_mlp_bwd" else 0
+    U.check(U.lib().mg_mlp_workspace(*sizes, U.CODES[dtype], wanted, ctypes.byref(need)))
+    size = need.value
     work = torch.full((size + 1024,), 0x7F, device="cuda", dtype=torch.uint8)       # NaN where nothing is written
     U.check(getattr(U.lib(), name)(*[t if t is None else t.data_ptr() for t in tensors], work.data_ptr() if size else None, size,
                                    *sizes, U.CODES[dtype], U.stream()))
@@ -89,11 +90,13 @@ def test_products_against_float64(tokens, d_model, hidden, dtype):
     _call("mg_mlp_fwd", (again, torch.empty_like(h), None, x, w12, w3), sizes, dtype)
     assert torch.equal(again, out)
     work = torch.empty_like(dgu)
-    for i, want in enumerate((dx, da, db)):
-        alone = [None, None, None]
+    for i, (want, a, b, count) in enumerate(((dx, dd, ad, 2 * hidden), (da, dd.t(), xd, tokens), (db, yd.t(), hd, tokens))):
+        alone = [None, None, None]                       # in a launch to itself the sums may go another way
         alone[i] = torch.empty_like(want)
         _call("mg_mlp_bwd", (*alone, None if i == 2 else work, dy, x, w12, w3, gu, h), sizes, dtype)
-        assert torch.equal(alone[i], want)
+        dw = work.double() if i < 2 else None
+        a = (dw if i == 0 else dw.t()) if i < 2 else a
+        _bounded(alone[i], a @ b, a.abs() @ b.abs(), count, dtype)
 
 
 def test_what_is_not_finite_stays_in_its_row_and_column():
@@ -174,15 +177,17 @@ def test_module_takes_it(shape, binding, monkeypatch):
     xa.data = torch.zeros_like(x)
     w = module.w3.weight
     keep, w.data = w.data, torch.zeros_like(w.data)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, (xa, module.w12.weight, w), dy, retain_graph=True), got[1:]))
     for t, want in ((xa, got[1]), (module.w12.weight, got[2]), (w, got[3])):
-        assert torch.equal(torch.autograd.grad(y, t, dy, retain_graph=True)[0], want)
+        _close(torch.autograd.grad(y, t, dy, retain_graph=True), [want])
     w.data = keep
     for name in ("w12", "w3"):
         frozen = getattr(module, name).weight.requires_grad_(False)
         part = _grads(module, x, dy)
         frozen.requires_grad_()
         assert [g is None for g in part] == [False, False, name == "w12", name == "w3"]
-        assert all(g is None or torch.equal(g, want) for g, want in zip(part, got))
+        assert torch.equal(part[0], got[0])
+        _close([g for g in part if g is not None], [want for g, want in zip(part, got) if g is not None])
     xa = x.clone().requires_grad_()
     y = module(xa)
     with torch.no_grad():
