@@ -773,19 +773,20 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
 
 // Where they take no more time than the library's products and the activation between them.  GPU time in
 // replayed graphs (library / these, us, bf16, d_model x hidden, forward + backward; forward):
-//   1024 x 1792: 80 tokens 64.6 / 52.9; 18.7 / 20.5, 1024 97 / 78; 30 / 26.5, 8192 379 / 309; 113 / 93
-//   2048 x 3584: 8 82 / 66, 80 97 / 72; 26.3 / 25.4, 1024 209 / 165; 68 / 58, 8192 1059 / 975; 324 / 336
-//   4096 x 11008: 8 315 / 222, 32 323 / 226; 62 / 57, 320 533 / 440; 141 / 150, 1024 1008 / 885; 318 / 299, 2048 1958 / 1486; 617 / 503
-//   beyond 128 MiB of weights from 4096 tokens on: 3072 x 8192 1614 / 1708; 498 / 536, 4096 x 6912 1850 / 1750; 548 / 593
-//   below 16 MiB: 1024 x 1792 8 46.2 / 49.7, 17 52.1 / 50.2, 48 tokens 55.8 / 51.5; 17.4 / 20.2, 512 x 896 8 37.2 / 42.8.
-// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162.6 / 47.2; 47 / 15.  Beyond the tokens of a decoding step
-// forward alone goes the same way, so that it gives the same bits; it loses up to 9 % where its tiles just miss a round of the
+//   512 x 1024: 1 token 34.6 / 31.5, 320 59 / 37; 21.1 / 17.2, 1024 72 / 43; 24.9 / 19.8
+//   1024 x 1792: 8 46.1 / 39.3, 128 69 / 46; 20.9 / 21.5, 1024 99 / 65; 30.8 / 26.8
+//   2048 x 3584: 8 82 / 66, 128 100 / 65; 28.2 / 27.2, 1024 211 / 153; 64 / 57, 4095 562 / 480; 165 / 152
+//   4096 x 11008: 8 315 / 194, 320 530 / 422; 133 / 153, 1024 985 / 811; 312 / 288, 2048 1986 / 1443; 594 / 471
+//   beyond 128 MiB of weights and 2048 tokens: 4096 x 6912 3072 1414 / 1343; 404 / 442, 3072 x 8192 4095 1620 / 1629; 470 / 481
+//   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2, from there on: 1024 x 2816 48 23.0 / 19.3.
+// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162 / 44; 47 / 15.  Beyond the tokens of a decoding step
+// forward alone goes the same way, so that it gives the same bits; it loses up to 14 % where its tiles just miss a round of the
 // compute units.
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only) {
     if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
     const int64_t weights = 6 * d_model * hidden;
-    if (tokens <= (forward_only ? MG_BLOCK_MAX_TOKENS : 16)) return weights >= 16LL << 20;
-    return tokens < 4096 || weights <= 128LL << 20;
+    if (forward_only && tokens <= MG_BLOCK_MAX_TOKENS) return weights >= 16LL << 20;
+    return tokens <= 2048 || weights <= 128LL << 20;
 }
 
 namespace {

@@ -22,8 +22,8 @@ def test_sizes(lib, tokens, d_model, hidden, dtype, fits):
 
 
 @pytest.mark.parametrize("tokens,d_model,hidden,training,alone", [
-    (16, 1024, 1792, 0, 0), (17, 1024, 1792, 1, 0), (64, 1024, 1792, 1, 0), (65, 1024, 1792, 1, 1), (1, 1024, 2816, 1, 1),
-    (4095, 4096, 6912, 1, 1), (4096, 4096, 6912, 0, 0), (4096, 4096, 5440, 1, 1),
+    (1, 64, 64, 1, 0), (16, 1024, 1792, 1, 0), (64, 1024, 1792, 1, 0), (65, 1024, 1792, 1, 1), (1, 1024, 2816, 1, 1),
+    (2048, 4096, 6912, 1, 1), (2049, 4096, 6912, 0, 0), (8192, 4096, 5440, 1, 1),
 ])
 def test_where_they_are_taken(lib, tokens, d_model, hidden, training, alone):
     assert [lib.mg_mlp_preferred(tokens, d_model, hidden, 2, only) for only in (0, 1)] == [training, alone]

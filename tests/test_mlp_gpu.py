@@ -204,10 +204,10 @@ def test_what_goes_through_the_projections(binding, monkeypatch):
     module = _module()
     w12, w3 = module.w12.weight, module.w3.weight
     x = torch.randn(300, 512, device="cuda", dtype=torch.bfloat16)
-    assert _takes(module, x) and _takes(module, x[:17])
+    assert _takes(module, x) and _takes(module, x[:1])
     with torch.no_grad():
         assert _takes(module, x[:65]) and not _takes(module, x[:64])
-    for y in (x[:16], x.float(), x[:, :511], torch.randn(300 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(300, 512)):
+    for y in (x.float(), x[:, :511], torch.randn(300 * 512 + 1, device="cuda", dtype=torch.bfloat16)[1:].view(300, 512)):
         assert ops.swiglu_mlp(y, w12, w3) is None
     assert ops.swiglu_mlp(x, w12.t().contiguous().t(), w3) is None and ops.swiglu_mlp(x, w12.half(), w3) is None
     assert ops.swiglu_mlp(x.to_sparse(), w12, w3) is None and ops.swiglu_mlp(x.cpu(), w12, w3) is None
