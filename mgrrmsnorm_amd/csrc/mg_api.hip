@@ -888,7 +888,8 @@ int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12
         const hipError_t e = dtype == MG_F16 ? launch_mlp_forward<half_t>(what, a, p, s) : launch_mlp_forward<bf16_t>(what, a, p, s);
         return e == hipSuccess ? MG_OK : fail_hip("mg_mlp_fwd", e);
     };
-    rc = run(MlpWhat::gate_up, {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d, t, n, d, nullptr}, pass.gate_up);
+    rc = run(MlpWhat::gate_up, {gate_up, h, nullptr, x, (uint32_t)td, d, w12, (uint32_t)(2 * w), d, t, n, d, nullptr, w3, (uint32_t)w, cus},
+             pass.gate_up);
     if (rc != MG_OK) return rc;
     return run(MlpWhat::down, {out, nullptr, nullptr, h, (uint32_t)th, n, w3, (uint32_t)w, n, t, d, n, workspace}, pass.down);
 }

@@ -258,6 +258,8 @@ struct MlpArgs {
     const void* b; uint32_t b_bytes; int b_ld;
     int M, N, K;
     void* partial;
+    // gate_up: what the next launch reads, for compute units (of `cus`) that have no tile
+    const void* next; uint32_t next_bytes; int cus;
 };
 inline MlpSize mlp_size(MlpWhat what, int64_t M, int64_t N, int64_t K) {
     const bool fused = what == MlpWhat::gate_up || what == MlpWhat::activation_bwd;   // the activation needs whole sums

@@ -429,10 +429,28 @@ __device__ __forceinline__ void mlp_job(const MlpJob& job, u32 id, char MG_LDS* 
     mlp_finish<T, C, WHAT>(share, lds, o, tm * C::BM, tn * BN);
 }
 
+// Workgroups beyond the tiles of a launch read `bytes` from `p` on, which the next launch will want: compute units that have no
+// tile bring it into the memory-side cache meanwhile, eight requests a wave at a time so that the tiles are held up little.
+// Gate and up / second projection, 1024 tokens, 2048 x 3584: 34.5 / 26.7 -> 35.6 / 22.2 us; 1404, 2944 x 5120 81.7 / 51.4 ->
+// 83.5 / 42.0; 300, 2048 x 5504 32.3 / 17.7 -> 34.5 / 14.9.
+struct MlpWarm { const void* p; u32 bytes; };
+template <class C>
+__device__ __forceinline__ void mlp_warm(const MlpWarm& w, u32 id, u32 count, char MG_LDS* lds) {
+    constexpr u32 PIECE = C::THREADS * 16;
+    const rsrc_t r = make_rsrc(w.p, w.bytes);
+    char MG_LDS* to = lds + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * (kWave * 16);
+    for (u32 at = id * PIECE; at < w.bytes; at += count * PIECE) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (MG_LDS void*)to, 16, (int)(at + threadIdx.x * 16), 0, 0, 0);
+        wait_requests<7>();
+    }
+    wait_requests<0>();
+}
+
 template <typename T, class C, bool A_ALONG_K, bool B_ALONG_K, int WHAT>
 __global__ void __launch_bounds__(C::THREADS, C::WAVES / 4)
-mlp_gemm(MlpJob job) {
+mlp_gemm(MlpJob job, MlpWarm warm) {
     __shared__ __attribute__((aligned(1024))) char lds[C::STAGE * C::STAGES];
+    if (WHAT == kMlpGateUp && blockIdx.x >= job.tiles) return mlp_warm<C>(warm, blockIdx.x - job.tiles, gridDim.x - job.tiles, (char MG_LDS*)lds);
     mlp_job<T, C, A_ALONG_K, B_ALONG_K, WHAT>(job, blockIdx.x, (char MG_LDS*)lds);
 }
 

@@ -4,10 +4,11 @@ Keeps the surface of the reference's megagemm/swiglu.py:86-172:
 `MegaGemmFunction.apply(w12_out, hidden_dim)` maps [..., 2*hidden] = [gate | up] to
 [..., hidden] = silu(gate) * up, and `MegaGemmTriton(d_model, multiple_of=256,
 hidden_multiple=5/3)` owns `w12` (d_model -> 2*hidden) and `w3` (hidden -> d_model), both
-bias-free nn.Linear layers that stay on torch.matmul, except for the few rows of a decoding
-step with nothing to differentiate (ops.swiglu_block).  The class keeps its historical name
-for drop-in use; nothing here uses Triton -- the activation, its backward and the decoding step
-are HIP kernels reached through mgrrmsnorm_amd.ops.
+bias-free nn.Linear layers.  In 16 bits the whole block runs on the package's own matrix products
+(ops.swiglu_mlp; a decoding step of a few rows with nothing to differentiate in ops.swiglu_block);
+calls those do not take go through the projections on torch.matmul and the activation.  The class
+keeps its historical name for drop-in use; nothing here uses Triton -- products, activation and
+backward are HIP kernels reached through mgrrmsnorm_amd.ops.
 """
 from __future__ import annotations
 

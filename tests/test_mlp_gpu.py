@@ -162,6 +162,8 @@ def test_module_takes_it(shape, binding, monkeypatch):
     _close(got, _grads(module, x, dy, _through_projections(module)))
     with torch.no_grad():
         assert torch.equal(module(x), got[0]) and torch.equal(ops.swiglu_mlp(x, module.w12.weight, module.w3.weight), got[0])
+    with torch.inference_mode():
+        assert torch.equal(module(x.clone()), got[0]) and module(x[0, ..., :]).shape == x[0].shape
     # operands and gradients of other layouts
     xt = x.transpose(0, 1).contiguous().transpose(0, 1)
     assert all(torch.equal(a, b) for a, b in zip(_grads(module, x, dy), _grads(module, x, dy.transpose(0, 1).contiguous().transpose(0, 1))))
