@@ -372,39 +372,38 @@ Tensor mlp_forward(const Tensor& x, const Tensor& w12, const Tensor& w3, Tensor*
     return out;
 }
 
-Tensor swiglu_projections(const Tensor& x, const Tensor& w12, const Tensor& w3) {
-    return at::linear(swiglu(at::linear(x, w12), w3.size(1)), w3);
-}
-
 struct MlpNode : public torch::autograd::Function<MlpNode> {
-    static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w12, const Tensor& w3) {
-        // Aliases even of what is contiguous: they keep the data they were made of when a caller gives an operand other
-        // data before the backward pass.  The operands themselves are for a backward pass that records its own graph.
+    // [out, h].  h is an output for the gradient of w3 alone: a graph recorded over that one gets through h to x and w12.
+    static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w12, const Tensor& w3) {
+        // Aliases, for the kernels: they keep the data they were made of when a caller gives an operand other data before the
+        // backward pass.  The operands themselves are for a backward pass that records its own graph.
         const Tensor xd = x.contiguous().detach(), ad = w12.detach(), bd = w3.detach();
         Tensor gate_up, h;
         const Tensor out = mlp_forward(xd, ad, bd, &gate_up, &h);
         ctx->save_for_backward({xd, ad, bd, gate_up, h, x, w12, w3});
-        return out;
+        ctx->set_materialize_grads(false);
+        return {out, h};
     }
 
     static torch::autograd::tensor_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::tensor_list grads) {
         const auto saved = ctx->get_saved_variables();
         const bool want[] = {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2)};
         torch::autograd::tensor_list out(3);
-        if (torch::GradMode::is_enabled()) {   // create_graph: through operations that record it (or refuse, as the activation does)
-            torch::autograd::variable_list wanted;
-            for (int i = 0; i < 3; ++i)
-                if (want[i]) wanted.push_back(saved[5 + i]);
-            const auto y = swiglu_projections(saved[5], saved[6], saved[7]);
-            const auto g = torch::autograd::grad({y}, wanted, {grads[0].to(y.scalar_type())}, true, true, true);
-            for (int i = 0, k = 0; i < 3; ++i)
-                if (want[i]) out[i] = g[k++];
-            return out;
+        const bool records = torch::GradMode::is_enabled();
+        if (!records && grads[0].defined() && !grads[1].defined()) {
+            in_kernels(out, grads[0], want, saved);
+        } else {
+            const int operands = records ? 5 : 0;
+            in_operations(out, grads, want, saved[operands], saved[operands + 1], saved[operands + 2], saved[3], saved[4]);
         }
+        return out;
+    }
+
+    static void in_kernels(torch::autograd::tensor_list& out, const Tensor& grad, const bool* want, const torch::autograd::variable_list& saved) {
         const Tensor &x = saved[0], &w12 = saved[1], &w3 = saved[2], &gate_up = saved[3], &h = saved[4];
         const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = x.numel() / d_model;
         const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-        auto dy = grads[0].contiguous();
+        auto dy = grad.contiguous();
         if (dy.scalar_type() != x.scalar_type()) dy = dy.to(x.scalar_type());
         if (reinterpret_cast<uintptr_t>(dy.data_ptr()) % 16 != 0) dy = dy.clone();
         Tensor d_gate_up;
@@ -416,7 +415,29 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
                                   w12.data_ptr(), w3.data_ptr(), gate_up.data_ptr(), h.data_ptr(), pointer_of(work),
                                   work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
         TORCH_CHECK(rc == MG_OK, "SwiGLU block backward failed (code ", rc, "): ", mg_last_error());
-        return out;
+    }
+
+    // What the projections' and the activation's backward passes do, as operations that record a graph where one is wanted and
+    // refuse what those refuse.
+    static void in_operations(torch::autograd::tensor_list& out, const torch::autograd::tensor_list& grads, const bool* want, const Tensor& x,
+                              const Tensor& w12, const Tensor& w3, const Tensor& gate_up, const Tensor& h) {
+        const int64_t d_model = w3.size(0), hidden = w3.size(1);
+        const auto type = gate_up.scalar_type();
+        Tensor dy, dh = grads[1];
+        if (grads[0].defined()) {
+            dy = grads[0].to(type).reshape({-1, d_model});
+            if (want[2]) out[2] = at::mm(dy.t(), h);
+            if (want[0] || want[1]) dh = dh.defined() ? dh + at::mm(dy, w3) : at::mm(dy, w3);
+        }
+        if (!dh.defined() || !(want[0] || want[1])) return;
+        refuse_double_backward(dh, "SwiGLU");
+        Tensor d_gate_up;
+        {
+            torch::NoGradGuard no_grad;
+            d_gate_up = swiglu_backward(dh.to(type).contiguous(), gate_up, hidden);
+        }
+        if (want[0]) out[0] = at::mm(d_gate_up, w12).reshape(x.sizes());
+        if (want[1]) out[1] = at::mm(d_gate_up.t(), x.reshape({-1, d_model}));
     }
 };
 
@@ -445,7 +466,7 @@ Tensor swiglu_mlp(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     if (off(w12) || off(w3) || (x.is_contiguous() && off(x))) return none;   // a copy of x is aligned
     if (learns) {
         if (!x.requires_grad() && !w12.requires_grad()) return none;   // only w3 learns: nothing of the activation has to be kept
-        return MlpNode::apply(x, w12, w3);
+        return MlpNode::apply(x, w12, w3)[0];
     }
     Tensor h;
     return mlp_forward(x.contiguous(), w12, w3, nullptr, &h);

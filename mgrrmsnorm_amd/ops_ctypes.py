@@ -18,6 +18,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 
@@ -264,41 +265,67 @@ def _mlp_forward(x, w12, w3, keep_gate_up):
 
 
 class _MlpFunction(torch.autograd.Function):
+    """(out, h).  h is an output for the gradient of w3 alone: a graph recorded over that one gets through h to x and w12."""
+
     @staticmethod
     def forward(ctx, x, w12, w3):
-        # aliases even of what is contiguous: they keep the data they were made of when a caller gives an operand
-        # other data before the backward pass; the operands themselves are for one that records its own graph
+        # aliases, for the kernels: they keep the data they were made of when a caller gives an operand other data before
+        # the backward pass; the operands themselves are for one that records its own graph
         xd, ad, bd = x.contiguous().detach(), w12.detach(), w3.detach()
         out, gate_up, h = _mlp_forward(xd, ad, bd, True)
         ctx.save_for_backward(xd, ad, bd, gate_up, h, x, w12, w3)
-        return out
+        ctx.set_materialize_grads(False)
+        return out, h
 
     @staticmethod
-    def backward(ctx, grad_output):
-        x, w12, w3, gate_up, h, *operands = ctx.saved_tensors
-        want = ctx.needs_input_grad
-        if torch.is_grad_enabled():      # create_graph: through operations that record it (or refuse, as the activation does)
-            from . import ops
+    def backward(ctx, grad_output, grad_h):
+        saved, want, records = ctx.saved_tensors, ctx.needs_input_grad, torch.is_grad_enabled()
+        if not records and grad_output is not None and grad_h is None:
+            return _mlp_backward(grad_output, want, *saved[:5])
+        return _mlp_backward_in_operations(grad_output, grad_h, want, *(saved[5:] if records else saved[:3]), *saved[3:5])
 
-            linear = torch.nn.functional.linear
-            y = linear(ops.swiglu(linear(operands[0], operands[1]), w3.size(1)), operands[2])
-            grads = iter(torch.autograd.grad(y, [t for t, w in zip(operands, want) if w], grad_output.to(y.dtype),
-                                             retain_graph=True, create_graph=True, allow_unused=True))
-            return tuple(next(grads) if w else None for w in want)
-        d_model, hidden = w3.shape
-        dy = grad_output.contiguous().to(x.dtype)
-        if dy.data_ptr() % 16 != 0:
-            dy = dy.clone()
-        with _lib.device_of(x.device):
-            grads = [torch.empty_like(t) if w else None for t, w in zip((x, w12, w3), want)]
-            d_gate_up = torch.empty_like(gate_up) if want[0] or want[1] else None
-            tokens = x.numel() // d_model
-            work, size = _mlp_workspace(x, tokens, d_model, hidden, want[:3])
-            rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
-                                        gate_up.data_ptr(), h.data_ptr(), _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype],
-                                        _lib.stream_ptr(x.device))
-        _lib.check(rc, "SwiGLU block backward")
-        return tuple(grads)
+
+def _mlp_backward(grad_output, want, x, w12, w3, gate_up, h):
+    d_model, hidden = w3.shape
+    dy = grad_output.contiguous().to(x.dtype)
+    if dy.data_ptr() % 16 != 0:
+        dy = dy.clone()
+    with _lib.device_of(x.device):
+        grads = [torch.empty_like(t) if w else None for t, w in zip((x, w12, w3), want)]
+        d_gate_up = torch.empty_like(gate_up) if want[0] or want[1] else None
+        tokens = x.numel() // d_model
+        work, size = _mlp_workspace(x, tokens, d_model, hidden, want[:3])
+        rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
+                                    gate_up.data_ptr(), h.data_ptr(), _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype],
+                                    _lib.stream_ptr(x.device))
+    _lib.check(rc, "SwiGLU block backward")
+    return tuple(grads)
+
+
+@once_differentiable
+def _activation_backward(gate_up, dh):
+    return swiglu_backward(dh.to(gate_up.dtype).contiguous(), gate_up, dh.size(1)), None
+
+
+def _mlp_backward_in_operations(grad_output, dh, want, x, w12, w3, gate_up, h):
+    """What the projections' and the activation's backward passes do, as operations that record a graph where one is
+    wanted and refuse what those refuse."""
+    d_model = w3.size(0)
+    out = [None, None, None]
+    if grad_output is not None:
+        dy = grad_output.to(gate_up.dtype).reshape(-1, d_model)
+        if want[2]:
+            out[2] = dy.t().mm(h)
+        if want[0] or want[1]:
+            dh = dy.mm(w3) if dh is None else dh + dy.mm(w3)
+    if dh is None or not (want[0] or want[1]):
+        return tuple(out)
+    d_gate_up, _ = _activation_backward(gate_up, dh)
+    if want[0]:
+        out[0] = d_gate_up.mm(w12).reshape(x.shape)
+    if want[1]:
+        out[1] = d_gate_up.t().mm(x.reshape(-1, d_model))
+    return tuple(out)
 
 
 def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
@@ -316,5 +343,5 @@ def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
     if not _preferred(x, hidden, not learns) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
         return None
     if learns:
-        return _MlpFunction.apply(x, w12, w3) if x.requires_grad or w12.requires_grad else None
+        return _MlpFunction.apply(x, w12, w3)[0] if x.requires_grad or w12.requires_grad else None
     return _mlp_forward(x.contiguous(), w12, w3, False)[0]

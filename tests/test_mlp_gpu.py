@@ -280,3 +280,41 @@ def test_the_block_under_graph_capture_and_on_other_streams():
     for t in threads:
         t.join()
     assert all(torch.equal(a, b) for g, w in zip(got, want) for a, b in zip(g, w))
+
+
+@pytest.fixture(params=["extension", "ctypes"])
+def binding(request, monkeypatch):
+    if request.param == "ctypes":
+        monkeypatch.setattr(ops, "_binding", None)
+        monkeypatch.setattr(ops, "_resolved", True)
+    return request.param
+
+
+def _batch(*shape, seed=0):
+    return torch.randn(shape, device="cuda", generator=torch.Generator("cuda").manual_seed(seed)).to(torch.bfloat16)
+
+
+def test_a_recorded_backward_pass_runs_hooks_once(binding):
+    module = _module()
+    module.w3.requires_grad_(False)          # with w3 learning the activation refuses to be recorded
+    w12, x, dy = module.w12.weight, _batch(300, 512).requires_grad_(), _batch(300, 512, seed=1)
+    want = torch.autograd.grad(module(x), (x, w12), dy)
+    calls = []
+    x.register_hook(lambda g: calls.append("x"))
+    w12.register_hook(lambda g: calls.append("w12"))
+    got = torch.autograd.grad(module(x), (x, w12), dy, create_graph=True)
+    assert sorted(calls) == ["w12", "x"]
+    _close(got, want)
+
+
+def test_second_derivatives(binding):
+    """Of the gradient of w3, through the activation to x and w12: as through the projections."""
+    module = _module()
+    w12, w3, dy = module.w12.weight, module.w3.weight, _batch(300, 512, seed=1)
+
+    def second(call):
+        x = _batch(300, 512).requires_grad_()
+        g = torch.autograd.grad(call(x), w3, dy, create_graph=True)[0]
+        return g.detach(), *torch.autograd.grad(g.float().square().sum() / 2, (x, w12))
+
+    _close(second(module), second(_through_projections(module)))
