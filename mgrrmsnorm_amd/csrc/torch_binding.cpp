@@ -18,6 +18,8 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+
 #include <algorithm>
 #include <tuple>
 #include <vector>
@@ -339,7 +341,7 @@ Tensor swiglu_block(const Tensor& x, const Tensor& w12, const Tensor& w3) {
 bool plain_dense(const Tensor& t) {
     constexpr c10::DispatchKeySet others({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
                                           c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
-                                          c10::DispatchKey::ZeroTensor, c10::DispatchKey::NestedTensor});
+                                          c10::DispatchKey::ZeroTensor, c10::DispatchKey::NestedTensor, c10::DispatchKey::Batched});
     return t.layout() == at::kStrided && t.is_cuda() && !t.key_set().has_any(others) && !t._fw_grad(0).defined();
 }
 
@@ -348,6 +350,12 @@ bool plain_dense(const Tensor& t) {
 bool calls_transformed() {
     return at::SavedTensorDefaultHooks::get_hooks(false).has_value() ||
            c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+// Whether a backward pass is for the kernels: one gradient, of which the same holds as of the operands (a batch of them
+// is no such tensor), and no dispatch mode that looks on.
+bool plain_backward(const Tensor& grad) {
+    return grad.defined() && plain_dense(grad) && !c10::impl::TorchDispatchModeTLS::any_modes_set();
 }
 
 // What mg_mlp_fwd or mg_mlp_bwd needs besides its tensors; undefined where that is nothing.
@@ -390,7 +398,7 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
         const bool want[] = {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2)};
         torch::autograd::tensor_list out(3);
         const bool records = torch::GradMode::is_enabled();
-        if (!records && grads[0].defined() && !grads[1].defined()) {
+        if (!records && !grads[1].defined() && plain_backward(grads[0])) {
             in_kernels(out, grads[0], want, saved);
         } else {
             const int operands = records ? 5 : 0;
@@ -417,8 +425,8 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
         TORCH_CHECK(rc == MG_OK, "SwiGLU block backward failed (code ", rc, "): ", mg_last_error());
     }
 
-    // What the projections' and the activation's backward passes do, as operations that record a graph where one is wanted and
-    // refuse what those refuse.
+    // What the projections' and the activation's backward passes do, as operations that record a graph where one is wanted,
+    // take the gradients those take and refuse what those refuse.
     static void in_operations(torch::autograd::tensor_list& out, const torch::autograd::tensor_list& grads, const bool* want, const Tensor& x,
                               const Tensor& w12, const Tensor& w3, const Tensor& gate_up, const Tensor& h) {
         const int64_t d_model = w3.size(0), hidden = w3.size(1);

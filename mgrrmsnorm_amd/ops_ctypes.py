@@ -236,6 +236,13 @@ def _plain_dense(t: torch.Tensor) -> bool:
             and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
 
 
+def _plain_backward(grad) -> bool:
+    """Whether a backward pass is for the kernels: one gradient, of which the same holds as of the operands (a batch of
+    them is no such tensor), and no dispatch mode that looks on."""
+    return (grad is not None and _plain_dense(grad) and not torch._C._functorch.is_legacy_batchedtensor(grad)
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
 def _pointer(t) -> int | None:
     return None if t is None else t.data_ptr()
 
@@ -280,8 +287,9 @@ class _MlpFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output, grad_h):
         saved, want, records = ctx.saved_tensors, ctx.needs_input_grad, torch.is_grad_enabled()
-        if not records and grad_output is not None and grad_h is None:
+        if not records and grad_h is None and _plain_backward(grad_output):
             return _mlp_backward(grad_output, want, *saved[:5])
+        want = [w and _asked_for(node) for w, (node, _) in zip(want, ctx.next_functions)]
         return _mlp_backward_in_operations(grad_output, grad_h, want, *(saved[5:] if records else saved[:3]), *saved[3:5])
 
 
@@ -302,6 +310,15 @@ def _mlp_backward(grad_output, want, x, w12, w3, gate_up, h):
     return tuple(grads)
 
 
+def _asked_for(node) -> bool:
+    """Whether the backward pass under way goes on to `node`: with w3 alone asked for, the activation is not to be reached, which
+    does not take every gradient that a product takes."""
+    try:
+        return torch._C._will_engine_execute_node(node)
+    except RuntimeError:      # a leaf whose gradient torch.autograd.grad returns
+        return True
+
+
 @once_differentiable
 def _activation_backward(gate_up, dh):
     return swiglu_backward(dh.to(gate_up.dtype).contiguous(), gate_up, dh.size(1)), None
@@ -309,7 +326,7 @@ def _activation_backward(gate_up, dh):
 
 def _mlp_backward_in_operations(grad_output, dh, want, x, w12, w3, gate_up, h):
     """What the projections' and the activation's backward passes do, as operations that record a graph where one is
-    wanted and refuse what those refuse."""
+    wanted, take the gradients those take and refuse what those refuse."""
     d_model = w3.size(0)
     out = [None, None, None]
     if grad_output is not None:

@@ -318,3 +318,26 @@ def test_second_derivatives(binding):
         return g.detach(), *torch.autograd.grad(g.float().square().sum() / 2, (x, w12))
 
     _close(second(module), second(_through_projections(module)))
+
+
+def test_gradients_that_are_no_plain_tensors(binding):
+    """A batch of them (is_grads_batched), lazily negated ones, and a dispatch mode that looks on."""
+    module = _module()
+    w3, x, dy = module.w3.weight, _batch(300, 512), _batch(3, 300, 512, seed=1)
+    y = module(x)
+    _close(torch.autograd.grad(y, w3, dy, is_grads_batched=True, retain_graph=True),
+           [torch.stack([torch.autograd.grad(y, w3, d, retain_graph=True)[0] for d in dy])])
+    with pytest.raises(RuntimeError):        # the activation's kernel takes no batch, as ever
+        torch.autograd.grad(y, module.w12.weight, dy, is_grads_batched=True, retain_graph=True)
+    _close(_grads(module, x, torch._neg_view(dy[0]))[1:], _grads(module, x, -dy[0])[1:])
+
+    class Seen(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    seen = []
+    with Seen():
+        got = torch.autograd.grad(y, (module.w12.weight, w3), dy[0], retain_graph=True)
+    assert torch.ops.aten.mm.default in seen
+    _close(got, torch.autograd.grad(y, (module.w12.weight, w3), dy[0]))
