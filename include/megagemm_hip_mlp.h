@@ -50,6 +50,7 @@ int mg_mlp_fwd(void* out, void* h, void* gate_up, const void* x, const void* w12
 /*
  * The gradients for dy as the gradient of out: dx, dw12 and dw3, each NULL where not wanted.  gate_up and h as
  * mg_mlp_fwd left them.  d_gate_up [tokens, 2 * hidden] is written unless dx and dw12 are both NULL (it may then be NULL).
+ * An input that no wanted gradient reads may be NULL: x without dw12, w12 without dx, w3 and gate_up without both, h without dw3.
  * Sums in a fixed order: bit-identical from run to run.  Otherwise as mg_mlp_fwd.
  */
 int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy, const void* x, const void* w12, const void* w3,

@@ -791,7 +791,7 @@ int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype,
 
 namespace {
 
-struct MlpTensor { const char* name; const void* p; int64_t bytes; };
+struct MlpTensor { const char* name; const void* p; int64_t bytes; bool needed = true; };
 
 int check_mlp(const char* fn, int64_t tokens, int64_t d_model, int64_t hidden, int dtype, const MlpTensor* out, int outs,
               const MlpTensor* in, int ins) {
@@ -799,7 +799,7 @@ int check_mlp(const char* fn, int64_t tokens, int64_t d_model, int64_t hidden, i
         return fail(MG_ERR_UNSUPPORTED, "%s: %lld tokens of %lld x %lld with dtype %d is not for it (fp16 or bf16, widths multiples of 64, "
                     "tensors below 2 GiB)", fn, (long long)tokens, (long long)d_model, (long long)hidden, dtype);
     for (int i = 0; i < ins; ++i)
-        if (in[i].p == nullptr) return fail(MG_ERR_INVALID_ARG, "%s: %s must not be NULL", fn, in[i].name);
+        if (in[i].needed && in[i].p == nullptr) return fail(MG_ERR_INVALID_ARG, "%s: %s must not be NULL", fn, in[i].name);
     for (int i = 0; i < ins + outs; ++i) {
         const MlpTensor& t = i < ins ? in[i] : out[i - ins];
         if (!aligned(t.p, 16)) return fail(MG_ERR_INVALID_ARG, "%s: %s is not 16-byte aligned", fn, t.name);
@@ -898,12 +898,13 @@ int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy,
                const void* gate_up, const void* h, void* workspace, int64_t workspace_bytes, int64_t tokens, int64_t d_model, int64_t hidden,
                int dtype, void* stream) {
     const int64_t td = tokens * d_model * 2, th = tokens * hidden * 2, w = d_model * hidden * 2;
-    const MlpTensor in[] = {{"dy", dy, td}, {"x", x, td}, {"w12", w12, 2 * w}, {"w3", w3, w}, {"gate_up", gate_up, 2 * th}, {"h", h, th}};
+    const bool want_x = dx != nullptr, want_12 = dw12 != nullptr, want_3 = dw3 != nullptr, want_a = want_x || want_12;
+    const MlpTensor in[] = {{"dy", dy, td}, {"x", x, td, want_12}, {"w12", w12, 2 * w, want_x}, {"w3", w3, w, want_a},
+                            {"gate_up", gate_up, 2 * th, want_a}, {"h", h, th, want_3}};
     const MlpTensor outs[] = {{"dx", dx, td}, {"dw12", dw12, 2 * w}, {"dw3", dw3, w}, {"d_gate_up", d_gate_up, 2 * th}, {"workspace", workspace, workspace_bytes}};
     int rc = check_mlp("mg_mlp_bwd", tokens, d_model, hidden, dtype, outs, 5, in, 6);
     if (rc != MG_OK) return rc;
-    const bool want_x = dx != nullptr, want_12 = dw12 != nullptr, want_3 = dw3 != nullptr;
-    if ((want_x || want_12) && d_gate_up == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
+    if (want_a && d_gate_up == nullptr) return fail(MG_ERR_INVALID_ARG, "mg_mlp_bwd: dx and dw12 need d_gate_up");
     int cus = 0;
     rc = cu_count(&cus);
     if (rc != MG_OK) return rc;
@@ -926,7 +927,7 @@ int mg_mlp_bwd(void* dx, void* dw12, void* dw3, void* d_gate_up, const void* dy,
                                              : launch_mlp_backward<bf16_t>(tasks, count, (hipStream_t)stream);
         return e == hipSuccess ? (int)MG_OK : fail_hip("mg_mlp_bwd", e);
     };
-    rc = run(w3_grad, want_3, act, want_x || want_12);
+    rc = run(w3_grad, want_3, act, want_a);
     return rc == MG_OK ? run(w12_grad, want_12, x_grad, want_x) : rc;
 }
 

@@ -371,7 +371,9 @@ Tensor mlp_forward(const Tensor& x, const Tensor& w12, const Tensor& w3, Tensor*
     const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = x.numel() / d_model;
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     if (gate_up != nullptr) *gate_up = at::empty({tokens, 2 * hidden}, x.options());
-    *h = at::empty({tokens, hidden}, x.options());
+    auto lead = x.sizes().vec();
+    lead.back() = hidden;
+    *h = at::empty(lead, x.options());
     auto out = empty_as(x);
     const Tensor work = mlp_workspace(x, tokens, d_model, hidden, MG_MLP_FORWARD);
     const int rc = mg_mlp_fwd(out.data_ptr(), h->data_ptr(), gate_up != nullptr ? gate_up->data_ptr() : nullptr, x.data_ptr(),
@@ -381,15 +383,17 @@ Tensor mlp_forward(const Tensor& x, const Tensor& w12, const Tensor& w3, Tensor*
 }
 
 struct MlpNode : public torch::autograd::Function<MlpNode> {
-    // [out, h].  h is an output for the gradient of w3 alone: a graph recorded over that one gets through h to x and w12.
+    // [out], and h where w3 learns: a graph recorded over the gradient of w3 gets through it to x and w12.
+    // What linear layers keep is kept: x (contiguous here) for the gradient of w12, w12 for that of x, w3, h for that of w3.
     static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& x, const Tensor& w12, const Tensor& w3) {
-        // Aliases, for the kernels: they keep the data they were made of when a caller gives an operand other data before the
-        // backward pass.  The operands themselves are for a backward pass that records its own graph.
-        const Tensor xd = x.contiguous().detach(), ad = w12.detach(), bd = w3.detach();
+        // Aliases: they keep the data they were made of when a caller gives an operand other data before the backward pass.
+        const Tensor none;
+        const bool for_x = x.requires_grad(), for_12 = w12.requires_grad(), for_3 = w3.requires_grad();
         Tensor gate_up, h;
-        const Tensor out = mlp_forward(xd, ad, bd, &gate_up, &h);
-        ctx->save_for_backward({xd, ad, bd, gate_up, h, x, w12, w3});
+        const Tensor out = mlp_forward(x, w12, w3, &gate_up, &h);
+        ctx->save_for_backward({for_12 ? x.detach() : none, for_x ? w12.detach() : none, w3.detach(), gate_up, for_3 ? h : none});
         ctx->set_materialize_grads(false);
+        if (!for_3) return {out};
         return {out, h};
     }
 
@@ -398,30 +402,41 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
         const bool want[] = {ctx->needs_input_grad(0), ctx->needs_input_grad(1), ctx->needs_input_grad(2)};
         torch::autograd::tensor_list out(3);
         const bool records = torch::GradMode::is_enabled();
-        if (!records && !grads[1].defined() && plain_backward(grads[0])) {
+        const auto node = records ? torch::autograd::get_current_node() : nullptr;
+        const auto operand = [&](int i) { return records ? connected(saved[i], node->next_edge(i)) : saved[i]; };
+        if (!records && (grads.size() == 1 || !grads[1].defined()) && plain_backward(grads[0])) {
             in_kernels(out, grads[0], want, saved);
         } else {
-            const int operands = records ? 5 : 0;
-            in_operations(out, grads, want, saved[operands], saved[operands + 1], saved[operands + 2], saved[3], saved[4]);
+            in_operations(out, grads, want, operand(0), operand(1), operand(2), saved[3], saved[4]);
         }
         return out;
     }
 
+    // An operand as it was kept, in the graph where the operand was.
+    static Tensor connected(const Tensor& kept, const torch::autograd::Edge& edge) {
+        if (!kept.defined() || !edge.is_valid()) return kept;
+        const Tensor t = kept.detach();
+        torch::autograd::impl::set_gradient_edge(t, edge);
+        return t;
+    }
+
     static void in_kernels(torch::autograd::tensor_list& out, const Tensor& grad, const bool* want, const torch::autograd::variable_list& saved) {
         const Tensor &x = saved[0], &w12 = saved[1], &w3 = saved[2], &gate_up = saved[3], &h = saved[4];
-        const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = x.numel() / d_model;
-        const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+        const auto type = gate_up.scalar_type();
+        const int64_t d_model = w3.size(0), hidden = w3.size(1), tokens = gate_up.size(0);
+        const c10::hip::HIPGuardMasqueradingAsCUDA guard(gate_up.device());
         auto dy = grad.contiguous();
-        if (dy.scalar_type() != x.scalar_type()) dy = dy.to(x.scalar_type());
+        if (dy.scalar_type() != type) dy = dy.to(type);
         if (reinterpret_cast<uintptr_t>(dy.data_ptr()) % 16 != 0) dy = dy.clone();
         Tensor d_gate_up;
         if (want[0] || want[1]) d_gate_up = empty_as(gate_up);
-        for (int i = 0; i < 3; ++i)
-            if (want[i]) out[i] = empty_as(saved[i]);
-        const Tensor work = mlp_workspace(x, tokens, d_model, hidden, (want[0] ? MG_MLP_DX : 0) | (want[1] ? MG_MLP_DW12 : 0) | (want[2] ? MG_MLP_DW3 : 0));
-        const int rc = mg_mlp_bwd(pointer_of(out[0]), pointer_of(out[1]), pointer_of(out[2]), pointer_of(d_gate_up), dy.data_ptr(), x.data_ptr(),
-                                  w12.data_ptr(), w3.data_ptr(), gate_up.data_ptr(), h.data_ptr(), pointer_of(work),
-                                  work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(x.scalar_type()), current_stream());
+        if (want[0]) out[0] = empty_as(dy);
+        if (want[1]) out[1] = at::empty({2 * hidden, d_model}, dy.options());
+        if (want[2]) out[2] = at::empty({d_model, hidden}, dy.options());
+        const Tensor work = mlp_workspace(gate_up, tokens, d_model, hidden, (want[0] ? MG_MLP_DX : 0) | (want[1] ? MG_MLP_DW12 : 0) | (want[2] ? MG_MLP_DW3 : 0));
+        const int rc = mg_mlp_bwd(pointer_of(out[0]), pointer_of(out[1]), pointer_of(out[2]), pointer_of(d_gate_up), dy.data_ptr(), pointer_of(x),
+                                  pointer_of(w12), w3.data_ptr(), gate_up.data_ptr(), pointer_of(h), pointer_of(work),
+                                  work.defined() ? work.numel() : 0, tokens, d_model, hidden, dtype_code(type), current_stream());
         TORCH_CHECK(rc == MG_OK, "SwiGLU block backward failed (code ", rc, "): ", mg_last_error());
     }
 
@@ -431,10 +446,11 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
                               const Tensor& w12, const Tensor& w3, const Tensor& gate_up, const Tensor& h) {
         const int64_t d_model = w3.size(0), hidden = w3.size(1);
         const auto type = gate_up.scalar_type();
-        Tensor dy, dh = grads[1];
+        const bool through_h = grads.size() == 2 && grads[1].defined();
+        Tensor dy, dh = through_h ? grads[1].reshape({-1, hidden}) : Tensor();
         if (grads[0].defined()) {
             dy = grads[0].to(type).reshape({-1, d_model});
-            if (want[2]) out[2] = at::mm(dy.t(), h);
+            if (want[2]) out[2] = at::mm(dy.t(), h.reshape({-1, hidden}));
             if (want[0] || want[1]) dh = dh.defined() ? dh + at::mm(dy, w3) : at::mm(dy, w3);
         }
         if (!dh.defined() || !(want[0] || want[1])) return;
@@ -444,7 +460,11 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
             torch::NoGradGuard no_grad;
             d_gate_up = swiglu_backward(dh.to(type).contiguous(), gate_up, hidden);
         }
-        if (want[0]) out[0] = at::mm(d_gate_up, w12).reshape(x.sizes());
+        if (want[0]) {
+            auto shape = (through_h ? grads[1] : grads[0]).sizes().vec();
+            shape.back() = d_model;
+            out[0] = at::mm(d_gate_up, w12).reshape(shape);
+        }
         if (want[1]) out[1] = at::mm(d_gate_up.t(), x.reshape({-1, d_model}));
     }
 };
@@ -474,7 +494,7 @@ Tensor swiglu_mlp(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     if (off(w12) || off(w3) || (x.is_contiguous() && off(x))) return none;   // a copy of x is aligned
     if (learns) {
         if (!x.requires_grad() && !w12.requires_grad()) return none;   // only w3 learns: nothing of the activation has to be kept
-        return MlpNode::apply(x, w12, w3)[0];
+        return MlpNode::apply(x.contiguous(), w12, w3)[0];
     }
     Tensor h;
     return mlp_forward(x.contiguous(), w12, w3, nullptr, &h);

@@ -262,7 +262,7 @@ def _mlp_forward(x, w12, w3, keep_gate_up):
     tokens = x.numel() // d_model
     with _lib.device_of(x.device):
         gate_up = x.new_empty(tokens, 2 * hidden) if keep_gate_up else None
-        h = x.new_empty(tokens, hidden)
+        h = x.new_empty(*x.shape[:-1], hidden)
         out = torch.empty_like(x)
         work, size = _mlp_workspace(x, tokens, d_model, hidden, ())
         rc = _lib.load().mg_mlp_fwd(out.data_ptr(), h.data_ptr(), _pointer(gate_up), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
@@ -272,15 +272,20 @@ def _mlp_forward(x, w12, w3, keep_gate_up):
 
 
 class _MlpFunction(torch.autograd.Function):
-    """(out, h).  h is an output for the gradient of w3 alone: a graph recorded over that one gets through h to x and w12."""
+    """(out, h or None): h is an output where w3 learns, as a graph recorded over the gradient of w3 gets through it to x and
+    w12.  What linear layers keep is kept: x (contiguous here) for the gradient of w12, w12 for that of x, w3, h for that of w3."""
 
     @staticmethod
     def forward(ctx, x, w12, w3):
+        for_x, for_12, for_3 = ctx.needs_input_grad
         # aliases, for the kernels: they keep the data they were made of when a caller gives an operand other data before
         # the backward pass; the operands themselves are for one that records its own graph
-        xd, ad, bd = x.contiguous().detach(), w12.detach(), w3.detach()
+        xd, ad, bd = x.detach(), w12.detach(), w3.detach()
         out, gate_up, h = _mlp_forward(xd, ad, bd, True)
-        ctx.save_for_backward(xd, ad, bd, gate_up, h, x, w12, w3)
+        if not for_3:
+            h = None
+        ctx.save_for_backward(xd if for_12 else None, ad if for_x else None, bd, gate_up, h,
+                              x if for_12 else None, w12 if for_x else None, w3)
         ctx.set_materialize_grads(False)
         return out, h
 
@@ -295,17 +300,18 @@ class _MlpFunction(torch.autograd.Function):
 
 def _mlp_backward(grad_output, want, x, w12, w3, gate_up, h):
     d_model, hidden = w3.shape
-    dy = grad_output.contiguous().to(x.dtype)
+    tokens = gate_up.size(0)
+    dy = grad_output.contiguous().to(gate_up.dtype)
     if dy.data_ptr() % 16 != 0:
         dy = dy.clone()
-    with _lib.device_of(x.device):
-        grads = [torch.empty_like(t) if w else None for t, w in zip((x, w12, w3), want)]
+    with _lib.device_of(dy.device):
+        shapes = (dy.shape, (2 * hidden, d_model), (d_model, hidden))
+        grads = [dy.new_empty(s) if w else None for s, w in zip(shapes, want)]
         d_gate_up = torch.empty_like(gate_up) if want[0] or want[1] else None
-        tokens = x.numel() // d_model
-        work, size = _mlp_workspace(x, tokens, d_model, hidden, want[:3])
-        rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), x.data_ptr(), w12.data_ptr(), w3.data_ptr(),
-                                    gate_up.data_ptr(), h.data_ptr(), _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[x.dtype],
-                                    _lib.stream_ptr(x.device))
+        work, size = _mlp_workspace(dy, tokens, d_model, hidden, want[:3])
+        rc = _lib.load().mg_mlp_bwd(*map(_pointer, grads), _pointer(d_gate_up), dy.data_ptr(), _pointer(x), _pointer(w12), w3.data_ptr(),
+                                    gate_up.data_ptr(), _pointer(h), _pointer(work), size, tokens, d_model, hidden, _MLP_CODES[dy.dtype],
+                                    _lib.stream_ptr(dy.device))
     _lib.check(rc, "SwiGLU block backward")
     return tuple(grads)
 
@@ -327,19 +333,22 @@ def _activation_backward(gate_up, dh):
 def _mlp_backward_in_operations(grad_output, dh, want, x, w12, w3, gate_up, h):
     """What the projections' and the activation's backward passes do, as operations that record a graph where one is
     wanted, take the gradients those take and refuse what those refuse."""
-    d_model = w3.size(0)
+    d_model, hidden = w3.shape
     out = [None, None, None]
+    lead = (grad_output if dh is None else dh).shape[:-1]
+    if dh is not None:
+        dh = dh.reshape(-1, hidden)
     if grad_output is not None:
         dy = grad_output.to(gate_up.dtype).reshape(-1, d_model)
         if want[2]:
-            out[2] = dy.t().mm(h)
+            out[2] = dy.t().mm(h.reshape(-1, hidden))
         if want[0] or want[1]:
             dh = dy.mm(w3) if dh is None else dh + dy.mm(w3)
     if dh is None or not (want[0] or want[1]):
         return tuple(out)
     d_gate_up, _ = _activation_backward(gate_up, dh)
     if want[0]:
-        out[0] = d_gate_up.mm(w12).reshape(x.shape)
+        out[0] = d_gate_up.mm(w12).reshape(*lead, d_model)
     if want[1]:
         out[1] = d_gate_up.t().mm(x.reshape(-1, d_model))
     return tuple(out)
@@ -360,5 +369,5 @@ def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
     if not _preferred(x, hidden, not learns) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
         return None
     if learns:
-        return _MlpFunction.apply(x, w12, w3)[0] if x.requires_grad or w12.requires_grad else None
+        return _MlpFunction.apply(x.contiguous(), w12, w3)[0] if x.requires_grad or w12.requires_grad else None
     return _mlp_forward(x.contiguous(), w12, w3, False)[0]

@@ -341,3 +341,67 @@ def test_gradients_that_are_no_plain_tensors(binding):
         got = torch.autograd.grad(y, (module.w12.weight, w3), dy[0], retain_graph=True)
     assert torch.ops.aten.mm.default in seen
     _close(got, torch.autograd.grad(y, (module.w12.weight, w3), dy[0]))
+
+
+@pytest.mark.parametrize("learning", ["x", "w12", "x w3", "w12 w3", "x w12", "x w12 w3"])
+def test_nothing_is_kept_that_no_gradient_needs(learning, binding):
+    """x is kept for the gradient of w12, w12 for that of x, h for that of w3, as by the projections: the others
+    may be changed between the passes, and the memory of activations is free."""
+    module = _module()
+    w12, w3 = module.w12.weight.requires_grad_("w12" in learning), module.w3.weight.requires_grad_("w3" in learning)
+    x0, dy = _batch(100, 512).requires_grad_("x" in learning.split()), _batch(100, 512, seed=1)   # tensors below 1 MiB: allocated to size
+    wanted = [t for t in (x0, w12, w3) if t.requires_grad]
+    want = torch.autograd.grad(module(x0), wanted, dy)
+    mib = lambda: torch.cuda.memory_allocated()
+    before = mib()
+    y = module(x0 * 1)
+    elements = 512 + 2 * 1024 + (1024 if "w3" in learning else 0) + (512 if "w12" in learning else 0)
+    assert mib() - before == 100 * elements * 2       # y, [gate | up], h, x
+    x = x0 * 1
+    y = module(x)
+    with torch.no_grad():
+        if "w12" not in learning:
+            x.add_(y)
+        if "x" not in learning.split():
+            w12.mul_(2)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(y, wanted, dy, retain_graph=True), want))
+    for t in [w3] + [x] * ("w12" in learning) + [w12] * ("x" in learning.split()):
+        y = module(x)
+        with torch.no_grad():
+            t.add_(1)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(y, wanted, dy)
+    # a graph over the gradient of w3 reaches whatever learns
+    if "w3" in learning:
+        def second(call):
+            y = call(x0)
+            g = torch.autograd.grad(y, w3, dy, create_graph=True)[0]
+            return torch.autograd.grad(g.float().square().sum() / 2, wanted[:-1])
+
+        _close(second(module), second(_through_projections(module)))
+
+
+def test_x_that_is_not_contiguous_is_kept_once(binding):
+    module, x0 = _module(), _batch(5, 20, 512).requires_grad_()
+    before = torch.cuda.memory_allocated()
+    y = module((x0 * 1).transpose(0, 1))
+    assert torch.cuda.memory_allocated() - before == 100 * (512 + 2 * 1024 + 1024 + 512) * 2 and y.shape == (20, 5, 512)
+
+
+def test_inputs_that_no_wanted_gradient_reads_may_be_null():
+    x, w12, w3 = _case(300, 512, 1024, "bf16")
+    dy, sizes = _batch(300, 512), (300, 512, 1024)
+    out, h, gu = torch.empty_like(x), x.new_empty(300, 1024), x.new_empty(300, 2048)
+    _call("mg_mlp_fwd", (out, h, gu, x, w12, w3), sizes, "bf16")
+    for wanted, unread in ((0, (5, 9)), (1, (6, 9)), (2, (5, 6, 7, 8))):       # dx, dw12, dw3
+        results = []
+        for drop in ((), unread):
+            grads = [torch.empty_like(t) if i == wanted else None for i, t in enumerate((x, w12, w3))]
+            work = None if wanted == 2 else torch.empty_like(gu)
+            tensors = [*grads, work, dy, x, w12, w3, gu, h]
+            _call("mg_mlp_bwd", [None if i in drop else t for i, t in enumerate(tensors)], sizes, "bf16")
+            results.append(grads[wanted])
+        assert torch.equal(*results)
+        for needed in {4, 5, 6, 7, 8, 9} - set(unread):
+            with pytest.raises(Exception, match="must not be NULL"):
+                _call("mg_mlp_bwd", [None if i == needed else t for i, t in enumerate(tensors)], sizes, "bf16")
