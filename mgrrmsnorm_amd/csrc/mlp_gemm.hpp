@@ -102,12 +102,12 @@ __device__ __forceinline__ void wait_requests() {
     static_assert(OUTSTANDING < 64, "the counter's range");
     __builtin_amdgcn_s_waitcnt((OUTSTANDING & 15) | (OUTSTANDING >> 4) << 14 | 7 << 4);
 }
-// A barrier that accesses through these pointers do not cross: the functions below declare that they do not alias
-// (within one step they do not; the compiler would otherwise wait for every request before any LDS read).
-__device__ __forceinline__ void step_barrier(const char MG_LDS* a, const char MG_LDS* b, char MG_LDS* c) {
-    asm volatile("" ::"s"(a), "s"(b), "s"(c) : "memory");
+// A barrier that accesses through these pointers do not cross.  The functions between two of them declare that theirs do not
+// alias, which holds from one barrier to the next (the compiler would otherwise wait for every request before any LDS read).
+__device__ __forceinline__ void step_barrier(const char MG_LDS* a, const char MG_LDS* b) {
+    asm volatile("" ::"s"(a), "s"(b) : "memory");
     __builtin_amdgcn_s_barrier();
-    asm volatile("" ::"s"(a), "s"(b), "s"(c) : "memory");
+    asm volatile("" ::"s"(a), "s"(b) : "memory");
 }
 
 template <class C> struct MlpFragments { u32x4 a[C::FM], b[C::FN]; };
@@ -162,14 +162,15 @@ struct MlpProduct {
             for (int j = 0; j < C::FN; ++j) sums.v[i][j] = mfma_16x16x32(f.b[j], f.a[i], sums.v[i][j], T());
     }
 
-    // The first STAGES steps requested, the first fragments of step 0 read.  `others` = `first` + one stage.
-    __device__ __forceinline__ void start(char MG_LDS* __restrict__ first, char MG_LDS* __restrict__ others, MlpFragments<C>& f) {
+    // The first STAGES steps requested, the fragments of the first read.  `others` = `first` + one stage.
+    __device__ __forceinline__ void start(char MG_LDS* __restrict__ first, char MG_LDS* __restrict__ others, MlpFragments<C>& f, MlpFragments<C>& g) {
         request(first);
 #pragma unroll
         for (int s = 1; s < C::STAGES; ++s) request(others + (s - 1) * C::STAGE);
         wait_requests<PER_STEP * (C::STAGES - 1)>();
-        step_barrier(first, others, others);
+        step_barrier(first, others);
         read(f, first, 0);
+        if constexpr (C::SUBSTEPS == 2) read(g, first, 1);
     }
     // With one substep a step is one block of instructions: the next fragments' reads between the first half of the
     // multiplications, the requests between all of them.  Left to itself the compiler issues the reads in a bunch, in front of
@@ -188,21 +189,31 @@ struct MlpProduct {
         }
     }
 
-    // One step.  On entry `f` holds its first fragments, read before; on return `next_f` holds the next step's.
-    // With two substeps the two may be the same.
-    __device__ __forceinline__ void step(const char MG_LDS* __restrict__ tile, const char MG_LDS* __restrict__ next, char MG_LDS* __restrict__ refill,
-                                         MlpSums<C>& sums, MlpFragments<C>& f, MlpFragments<C>& next_f) {
-        MlpFragments<C> g;
-        if constexpr (C::SUBSTEPS == 2) {
-            read(g, tile, 1);
-            multiply(sums, f);
-        }
-        wait_requests<PER_STEP * (C::STAGES - 2)>();     // the next step has arrived ...
-        step_barrier(tile, next, refill);                // ... for every wave, and every wave has read all of this one
-        read(next_f, next, 0);
+    // Between two barriers the stage that has arrived, `cur`, is read, and the one before it, which every wave has read,
+    // is requested into, `refill`: different stages, so nothing is accessed through both pointers, as they declare.
+    // One substep a step: `next` becomes cur's fragments while those of the stage before are multiplied.
+    __device__ __forceinline__ void one_substep(const char MG_LDS* __restrict__ cur, char MG_LDS* __restrict__ refill, MlpSums<C>& sums,
+                                                const MlpFragments<C>& f, MlpFragments<C>& next) {
+        read(next, cur, 0);
         request(refill);
-        multiply(sums, C::SUBSTEPS == 2 ? g : f);
-        if constexpr (C::SUBSTEPS == 1) interleave();
+        multiply(sums, f);
+        interleave();
+    }
+    // Two: `g` holds the second fragments of the stage before, and cur's on return; cur's first ones are multiplied in here.
+    __device__ __forceinline__ void two_substeps(const char MG_LDS* __restrict__ cur, char MG_LDS* __restrict__ refill, MlpSums<C>& sums,
+                                                 MlpFragments<C>& g) {
+        MlpFragments<C> f;
+        read(f, cur, 0);
+        request(refill);
+        multiply(sums, g);
+        __builtin_amdgcn_sched_barrier(0);   // else `g` is read between the multiplications that still need it: 2048 tokens,
+        read(g, cur, 1);                     // 4096 x 11008, forward + backward 1552 us against 1416
+        multiply(sums, f);
+    }
+    // From one to the next: that has arrived for every wave, and every wave has read all of this one.
+    __device__ __forceinline__ void next_stage(char MG_LDS* now, char MG_LDS* next) const {
+        wait_requests<PER_STEP * (C::STAGES - 2)>();
+        step_barrier(now, next);
     }
 
     __device__ __forceinline__ void run(MlpShare<C>& share, char MG_LDS* lds, int first, int steps, int m0, int n0, int hidden) {
@@ -224,22 +235,27 @@ struct MlpProduct {
         ta.advance((u32)first * TA::step(A.ld));
         tb.advance((u32)first * TB::step(B.ld));
         MlpFragments<C> f, g;
-        start(lds, lds + C::STAGE, f);
+        start(lds, lds + C::STAGE, f, g);
         const auto after = [](int at) { return at == (C::STAGES - 1) * C::STAGE ? 0 : at + C::STAGE; };
         int at = 0;
         if constexpr (C::SUBSTEPS == 2) {
+            multiply(sums, f);
 #pragma clang loop unroll(disable)
-            for (int k = 0; k < steps; ++k) {
+            for (int k = 1; k < steps; ++k) {
                 const int next = after(at);
-                step(lds + at, lds + next, lds + at, sums, f, f);
+                next_stage(lds + at, lds + next);
+                two_substeps(lds + next, lds + at, sums, g);
                 at = next;
             }
+            multiply(sums, g);
         } else {   // two sets of fragments in turn; an odd step at the end multiplies zeros
 #pragma clang loop unroll(disable)
             for (int k = 0; k < steps; k += 2) {
                 const int next = after(at), over = after(next);
-                step(lds + at, lds + next, lds + at, sums, f, g);
-                step(lds + next, lds + over, lds + next, sums, g, f);
+                next_stage(lds + at, lds + next);
+                one_substep(lds + next, lds + at, sums, f, g);
+                next_stage(lds + next, lds + over);
+                one_substep(lds + over, lds + next, sums, g, f);
                 at = over;
             }
         }
