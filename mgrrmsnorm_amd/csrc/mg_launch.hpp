@@ -251,7 +251,6 @@ hipError_t launch_skinny_gemm(int dtype, bool paired, const SkinnyArgs& a, hipSt
 // per line.  gate_up: b holds N gate rows, then N up rows; out may be NULL, second gets the activation.  activation_bwd: `in` is
 // [gate | up].  weight_grad: a is [K, M], b [K, N], any K; otherwise a is [M, K] with K a multiple of 64.
 // partial: plan.splits * M * N floats where the plan splits k.
-enum class MlpWhat { gate_up, down, activation_bwd, input_grad, weight_grad };
 struct MlpArgs {
     void* out; void* second; const void* in;
     const void* a; uint32_t a_bytes; int a_ld;
@@ -261,10 +260,6 @@ struct MlpArgs {
     // gate_up: what the next launch reads, for compute units (of `cus`) that have no tile
     const void* next; uint32_t next_bytes; int cus;
 };
-inline MlpSize mlp_size(MlpWhat what, int64_t M, int64_t N, int64_t K) {
-    const bool fused = what == MlpWhat::gate_up || what == MlpWhat::activation_bwd;   // the activation needs whole sums
-    return {M, what == MlpWhat::gate_up ? 2 * N : N, K, what == MlpWhat::weight_grad, !fused};
-}
 struct MlpTask { MlpWhat what; MlpArgs args; MlpPlan plan; };
 template <typename T> hipError_t launch_mlp_forward(MlpWhat what, const MlpArgs& a, MlpPlan plan, hipStream_t s);
 // One or two products that do not need each other, in one launch.

@@ -1,7 +1,9 @@
-// Which tile a product of the SwiGLU block is cut into, and whether k is split over workgroups.  Host code.
+// Which tile a product of the SwiGLU block is cut into, and whether k is split over workgroups.  Host code without a
+// HIP header: the test of which plans there are compiles it alone.
 #pragma once
 #include <stdint.h>
 
+#include <algorithm>
 #include <initializer_list>
 
 namespace mg {
@@ -96,5 +98,44 @@ inline void mlp_plan_pair(const MlpSize& p, const MlpSize& q, int cus, MlpPlan* 
             if (least < 0.0f || t < least) { least = t; *plan_p = a.plan; *plan_q = b.plan; }
         }
 }
+
+// The block's products: [gate | up] with the activation, the second projection; the activation's gradient, that of an input, that of
+// weights.
+enum class MlpWhat { gate_up, down, activation_bwd, input_grad, weight_grad };
+inline MlpSize mlp_size(MlpWhat what, int64_t M, int64_t N, int64_t K) {
+    const bool fused = what == MlpWhat::gate_up || what == MlpWhat::activation_bwd;   // the activation needs whole sums
+    return {M, what == MlpWhat::gate_up ? 2 * N : N, K, what == MlpWhat::weight_grad, !fused};
+}
+inline int64_t mlp_partial_bytes(MlpPlan p, int64_t M, int64_t N) { return p.splits > 1 ? p.splits * M * N * 4 : 0; }
+
+struct MlpForward {
+    MlpPlan gate_up, down;
+    int64_t workspace;
+    MlpForward(int64_t t, int64_t d, int64_t h, int cus)
+        : gate_up(mlp_plan(mlp_size(MlpWhat::gate_up, t, h, d), cus)), down(mlp_plan(mlp_size(MlpWhat::down, t, d, h), cus)),
+          workspace(mlp_partial_bytes(down, t, d)) {}
+};
+
+// Two launches: the gradients of w3 and, through the activation, of [gate | up]; then those of w12 and x.
+struct MlpBackward {
+    MlpPlan w3{-1, 1}, act{-1, 1}, w12{-1, 1}, x{-1, 1};
+    int64_t workspace[2], at[2];   // bytes of each launch, and where its second product's begin
+    MlpBackward(int64_t t, int64_t d, int64_t h, bool want_x, bool want_12, bool want_3, int cus) {
+        const MlpSize s3 = mlp_size(MlpWhat::weight_grad, d, h, t), sa = mlp_size(MlpWhat::activation_bwd, t, h, d);
+        const MlpSize s12 = mlp_size(MlpWhat::weight_grad, 2 * h, d, t), sx = mlp_size(MlpWhat::input_grad, t, d, 2 * h);
+        const bool want_a = want_x || want_12;
+        if (want_3 && want_a) mlp_plan_pair(s3, sa, cus, &w3, &act);
+        else if (want_3) w3 = mlp_plan(s3, cus);
+        else if (want_a) act = mlp_plan(sa, cus);
+        if (want_12 && want_x) mlp_plan_pair(s12, sx, cus, &w12, &x);
+        else if (want_12) w12 = mlp_plan(s12, cus);
+        else if (want_x) x = mlp_plan(sx, cus);
+        at[0] = mlp_partial_bytes(w3, d, h);
+        workspace[0] = at[0];
+        at[1] = mlp_partial_bytes(w12, 2 * h, d);
+        workspace[1] = at[1] + mlp_partial_bytes(x, t, d);
+    }
+    int64_t needs() const { return std::max(workspace[0], workspace[1]); }
+};
 
 }  // namespace mg

@@ -1,5 +1,10 @@
 """What of the block's own products can be checked without a GPU: the sizes and arguments the C entry points take,
 and the calls MegaGemmTriton hands to them."""
+import random
+import shutil
+import subprocess
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -89,3 +94,24 @@ def test_a_replaced_function_is_called(handed_over, monkeypatch, what):
     owner, name, value = REPLACED[what]
     monkeypatch.setattr(owner, name, value)
     assert handed_over(_module()) is None
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a C++ compiler")
+def test_every_planned_kernel_is_run_against_float64(lib, tmp_path):
+    """What the planner makes of the sizes the C entry points take, against the sizes of test_mlp_gpu.py."""
+    from test_mlp_gpu import SIZES
+
+    program = tmp_path / "mlp_plans"
+    subprocess.run(["g++", "-std=c++17", "-O2", str(Path(__file__).parent / "standalone" / "mlp_plans.cpp"), "-o", str(program)], check=True)
+
+    def plans(sizes):
+        text = "\n".join("%d %d %d" % s for s in sizes)
+        return set(subprocess.run([str(program)], input=text, text=True, capture_output=True, check=True).stdout.split())
+
+    rng = random.Random(0)
+    spread = lambda low, high: round(low * (high / low) ** rng.random())
+    sizes = [(spread(1, 1 << 20), 64 * spread(1, 1024), 64 * spread(1, 1024)) for _ in range(40000)]
+    sizes = [s for s in sizes if lib.mg_mlp_fits(*s, 2)]
+    assert len(sizes) > 20000
+    missing = plans(sizes) - plans(SIZES)
+    assert not missing

@@ -20,10 +20,10 @@ def _call(name, tensors, sizes, dtype):
     wanted = sum(1 << i for i, t in enumerate(tensors[:3]) if t is not None) if name == "mg_mlp_bwd" else 0
     U.check(U.lib().mg_mlp_workspace(*sizes, U.CODES[dtype], wanted, ctypes.byref(need)))
     size = need.value
-    work = torch.full((size + 1024,), 0x7F, device="cuda", dtype=torch.uint8)       # NaN where nothing is written
+    work = torch.full((size + 1024,), 0xFF, device="cuda", dtype=torch.uint8)       # NaN where nothing is written
     U.check(getattr(U.lib(), name)(*[t if t is None else t.data_ptr() for t in tensors], work.data_ptr() if size else None, size,
                                    *sizes, U.CODES[dtype], U.stream()))
-    assert (work[size:] == 0x7F).all()
+    assert (work[size:] == 0xFF).all()
 
 
 def _guarded(shape, dtype):
@@ -46,12 +46,18 @@ def _bounded(got, ref, terms, count, dtype, extra=0.0):
     assert worst <= 0.0, f"beyond the error bound by {worst}"
 
 
-@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
-@pytest.mark.parametrize("tokens,d_model,hidden", [
+# every product on every tile, k whole and in parts: tests/test_mlp_cpu.py asks the planner
+SIZES = [
     (1, 64, 64), (17, 1024, 1792), (64, 2048, 5504), (65, 64, 192), (127, 192, 64), (128, 128, 128), (129, 128, 256), (257, 320, 448), (300, 704, 1088),
     (1000, 512, 1344), (1024, 2048, 3584), (513, 1536, 4096), (2047, 1024, 2816), (96, 4096, 6912), (640, 3136, 8384),
     (127, 1024, 11008), (130, 3136, 8000), (70, 8192, 1088), (200, 704, 2752),   # k in 2 to 8 parts, of 43.5 and 9.5 steps
-])
+    (2048, 512, 512), (4099, 512, 1024), (4096, 2048, 3584), (10601, 64, 4416),  # weight gradients in parts, k ragged in two of them
+    (603, 3456, 9216), (1322, 3200, 5376), (1499, 2944, 5120), (18342, 6592, 192),   # second projection and gradient of x on the large tiles
+]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("tokens,d_model,hidden", SIZES)
 def test_products_against_float64(tokens, d_model, hidden, dtype):
     x, w12, w3 = _case(tokens, d_model, hidden, dtype)
     dy = torch.randn(tokens, d_model, device="cuda", generator=torch.Generator("cuda").manual_seed(5)).to(x.dtype)
@@ -97,6 +103,60 @@ def test_products_against_float64(tokens, d_model, hidden, dtype):
         dw = work.double() if i < 2 else None
         a = (dw if i == 0 else dw.t()) if i < 2 else a
         _bounded(alone[i], a @ b, a.abs() @ b.abs(), count, dtype)
+
+
+@pytest.mark.parametrize("tokens,d_model,hidden", [(1198371, 64, 448), (5, 65536, 8128)])
+def test_tensors_just_below_2_gib(tokens, d_model, hidden):
+    """On whole numbers, whose sums are exact: every result is the one in float64 rounded once."""
+    dt, sizes, g = torch.bfloat16, (tokens, d_model, hidden), torch.Generator("cuda").manual_seed(0)
+    ints = lambda *s: torch.randint(-1, 2, s, device="cuda", generator=g, dtype=torch.int8).to(dt)
+    x, w12, w3, dy, h2 = ints(tokens, d_model), ints(2 * hidden, d_model), ints(d_model, hidden), ints(tokens, d_model), ints(tokens, hidden)
+
+    def same(got, a, b, scale=1.0):
+        b = b.double()
+        for i in range(0, a.size(0), 1 << 16):
+            assert torch.equal(got[i:i + (1 << 16)], (a[i:i + (1 << 16)].double() @ b * scale).to(dt))
+
+    def same_over_tokens(got, a, b):
+        total = sum(a[i:i + (1 << 16)].double().t() @ b[i:i + (1 << 16)].double() for i in range(0, tokens, 1 << 16))
+        assert torch.equal(got, total.to(dt))
+
+    (out, c0), (h, c1), (gu, c2) = (_guarded(s, dt) for s in ((tokens, d_model), (tokens, hidden), (tokens, 2 * hidden)))
+    _call("mg_mlp_fwd", (out, h, gu, x, w12, w3), sizes, "bf16")
+    _intact(c0, c1, c2)
+    same(gu, x, w12.t())
+    for i in range(0, tokens, 1 << 16):
+        hd, bd = h[i:i + (1 << 16)].double(), w3.double()
+        _bounded(out[i:i + (1 << 16)], hd @ bd.t(), hd.abs() @ bd.abs().t(), hidden, "bf16")
+    del out, h, c0, c1
+    gu[:, :hidden], gu[:, hidden:] = 64, 1                   # where silu(g) is g and its slope 1
+    (dx, c3), (da, c4), (db, c5), (dgu, c6) = (_guarded(s, dt) for s in (
+        (tokens, d_model), (2 * hidden, d_model), (d_model, hidden), (tokens, 2 * hidden)))
+    _call("mg_mlp_bwd", (dx, da, db, dgu, dy, x, w12, w3, gu, h2), sizes, "bf16")
+    _intact(c2, c3, c4, c5, c6)
+    same(dgu[:, :hidden], dy, w3)
+    same(dgu[:, hidden:], dy, w3, 64.0)
+    same(dx, dgu, w12)
+    same_over_tokens(da, dgu, x)
+    same_over_tokens(db, dy, h2)
+
+
+def test_a_workspace_that_is_missing_or_too_small_is_refused():
+    """By the host, before anything is launched."""
+    sizes = t, d, h = 127, 1024, 11008
+    x, w12, w3 = _case(t, d, h, "bf16")
+    out, hid, gu = torch.zeros_like(x), x.new_empty(t, h), x.new_empty(t, 2 * h)
+    grads = [torch.zeros_like(v) for v in (x, w12, w3)]
+    for name, wanted, tensors in (("mg_mlp_fwd", 0, (out, hid, gu, x, w12, w3)), ("mg_mlp_bwd", 7, (*grads, torch.empty_like(gu), out, x, w12, w3, gu, hid))):
+        need = ctypes.c_int64(0)
+        U.check(U.lib().mg_mlp_workspace(*sizes, 2, wanted, ctypes.byref(need)))
+        assert need.value > 0
+        work = torch.empty(need.value, device="cuda", dtype=torch.uint8)
+        for p, n in ((None, 0), (None, need.value), (work.data_ptr(), need.value - 1), (work.data_ptr(), 0)):
+            assert getattr(U.lib(), name)(*(v.data_ptr() for v in tensors), p, n, *sizes, 2, U.stream()) == -1
+            assert "workspace must hold" in U.lib().mg_last_error().decode()
+    torch.cuda.synchronize()
+    assert not out.any() and not any(v.any() for v in grads)
 
 
 def test_what_is_not_finite_stays_in_its_row_and_column():
