@@ -778,14 +778,15 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
 //   4096 x 11008: 8 315 / 194, 320 530 / 422; 133 / 153, 1024 985 / 811; 312 / 288, 2048 1986 / 1443; 594 / 471
 //   beyond 128 MiB of weights and 2048 tokens: 4096 x 6912 3072 1414 / 1343; 404 / 442, 3072 x 8192 4095 1620 / 1629; 470 / 481
 //   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2, from there on: 1024 x 2816 48 23.0 / 19.3.
-// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162 / 44; 47 / 15.  Beyond the tokens of a decoding step
-// forward alone goes the same way, so that it gives the same bits; it loses up to 14 % where its tiles just miss a round of the
-// compute units.
+// Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162 / 44; 47 / 15.  Forward alone has a line of its own
+// (mlp_forward_wins).
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only) {
     if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
     const int64_t weights = 6 * d_model * hidden;
-    if (forward_only && tokens <= MG_BLOCK_MAX_TOKENS) return weights >= 16LL << 20;
-    return tokens <= 2048 || weights <= 128LL << 20;
+    if (tokens > 2048 && weights > 128LL << 20) return 0;
+    if (!forward_only) return 1;
+    if (tokens <= MG_BLOCK_MAX_TOKENS && weights < 16LL << 20) return 0;
+    return mlp_forward_wins(tokens, d_model, hidden);
 }
 
 namespace {

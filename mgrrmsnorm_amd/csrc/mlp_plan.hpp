@@ -46,7 +46,7 @@ inline bool mlp_way(const MlpSize& p, int i, int splits, MlpWay* way) {
 }
 constexpr int kMlpSplits[] = {1, 2, 3, 4, 6, 8};
 
-inline MlpPlan mlp_plan(const MlpSize& p, int cus) {
+inline MlpPlan mlp_plan(const MlpSize& p, int cus, float* us = nullptr) {
     MlpPlan best = {-1, 1};
     float least = 0.0f;
     for (int i = 0; i < 4; ++i)
@@ -56,6 +56,7 @@ inline MlpPlan mlp_plan(const MlpSize& p, int cus) {
             const float t = (float)((w.tiles + cus - 1) / cus) * w.tile_us + w.extra_us;
             if (best.shape < 0 || t < least) { best = w.plan; least = t; }
         }
+    if (us != nullptr) *us = least;
     return best;
 }
 
@@ -109,12 +110,32 @@ inline MlpSize mlp_size(MlpWhat what, int64_t M, int64_t N, int64_t K) {
 inline int64_t mlp_partial_bytes(MlpPlan p, int64_t M, int64_t N) { return p.splits > 1 ? p.splits * M * N * 4 : 0; }
 
 struct MlpForward {
+    float us[2];           // expected
     MlpPlan gate_up, down;
     int64_t workspace;
     MlpForward(int64_t t, int64_t d, int64_t h, int cus)
-        : gate_up(mlp_plan(mlp_size(MlpWhat::gate_up, t, h, d), cus)), down(mlp_plan(mlp_size(MlpWhat::down, t, d, h), cus)),
+        : gate_up(mlp_plan(mlp_size(MlpWhat::gate_up, t, h, d), cus, &us[0])), down(mlp_plan(mlp_size(MlpWhat::down, t, d, h), cus, &us[1])),
           workspace(mlp_partial_bytes(down, t, d)) {}
 };
+
+// Whether the two launches of a forward pass that no backward pass follows take no more time than the library's products
+// and the activation, on the 256 compute units that both sides were measured on (700 sizes: 20 to 65536 tokens, 3 to 425 MB of
+// weights, replayed graphs, bf16 and fp16).  The library's time scatters by 10 % around the line below, which lies where least
+// is lost on either side; up to the given weights these products win or are level at every number of tokens measured:
+//   below 24 MB: 512 x 1024 17.3 / 14.7 us at 65 tokens, 286 / 239 at 65536; 1024 x 2816 19.1 / 18.8, 1049 / 1005;
+//   below 60 MB and 5000 tokens: 2048 x 3584 1024 tokens 64.7 / 54.9, 4096 169 / 164, but 8192 299 / 309; 1664 x 4608 1800 tokens 120 / 106;
+//   beyond: 4096 x 11008 256 tokens 120 / 107, but 320 135 / 147 and 384 146 / 162 (row tiles that just miss), 448 169 / 160; 4096 x 6912 256
+//     86 / 75, 640 131 / 146, 768 141 / 163, 2048 294 / 301; 4096 x 5440 65536 tokens 6102 / 6767; 8192 x 2048 64 tokens 41 / 56.
+// Of the sizes taken 1 in 100 is more than 2 % slower (worst 4096 tokens, 4096 x 4096, 299 / 324).  Between 20 and 130 tokens sizes of less
+// than 40 us, where three operators take 47 us on the host, are taken although a replayed graph may lose 1 to 6 us (65 tokens, 1536 x 2560
+// 18.0 / 22.3, eager 48 / 22).  Wins given up: 5 to 20 % at some sizes beyond 60 MB and 640 tokens (2048, 4096 x 11008 592 / 468).
+inline bool mlp_forward_wins(int64_t t, int64_t d, int64_t h) {
+    const float mb = 6e-6f * (float)d * (float)h;
+    if (mb <= 24.0f || (mb <= 60.0f && t <= 5000)) return true;
+    const MlpForward pass(t, d, h, 256);
+    const float library_us = 20.0f + 30.0f * (float)std::min<int64_t>(t, 256) / 256.0f + 0.15f * mb + mb * (float)t / 2000.0f;
+    return pass.us[0] + pass.us[1] <= library_us;
+}
 
 // Two launches: the gradients of w3 and, through the activation, of [gate | up]; then those of w12 and x.
 struct MlpBackward {

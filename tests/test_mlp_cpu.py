@@ -28,7 +28,11 @@ def test_sizes(lib, tokens, d_model, hidden, dtype, fits):
 
 @pytest.mark.parametrize("tokens,d_model,hidden,training,alone", [
     (1, 64, 64, 1, 0), (16, 1024, 1792, 1, 0), (64, 1024, 1792, 1, 0), (65, 1024, 1792, 1, 1), (1, 1024, 2816, 1, 1),
-    (2048, 4096, 6912, 1, 1), (2049, 4096, 6912, 0, 0), (8192, 4096, 5440, 1, 1),
+    (2048, 4096, 6912, 1, 0), (2049, 4096, 6912, 0, 0), (8192, 4096, 5440, 1, 0),
+    # forward alone: faster and slower than the library's products, by the times beside the rule
+    (65536, 512, 1024, 1, 1), (1024, 2048, 3584, 1, 1), (8192, 2048, 3584, 1, 0), (256, 4096, 11008, 1, 1), (320, 4096, 11008, 1, 0),
+    (384, 4096, 11008, 1, 0), (448, 4096, 11008, 1, 1), (256, 4096, 6912, 1, 1), (640, 4096, 6912, 1, 0), (65536, 4096, 5440, 1, 0),
+    (64, 8192, 2048, 1, 0), (64, 4096, 6912, 1, 1),
 ])
 def test_where_they_are_taken(lib, tokens, d_model, hidden, training, alone):
     assert [lib.mg_mlp_preferred(tokens, d_model, hidden, 2, only) for only in (0, 1)] == [training, alone]
