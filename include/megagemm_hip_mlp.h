@@ -21,12 +21,17 @@ extern "C" {
  */
 int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
 
+/* What a call of the block consists of: forward and backward, forward alone, or forward and a backward pass for dx alone. */
+#define MG_MLP_ALL 0
+#define MG_MLP_FORWARD_ONLY 1
+#define MG_MLP_X_LEARNS 2
+
 /*
  * 1 where they are also taken rather than library products around mg_swiglu_fwd and mg_swiglu_bwd (0 for sizes they do not
- * take): for forward and backward, or for the forward pass that no backward pass follows.  A rule fitted to times of both sides, which
- * stand beside it: the few sizes it gets wrong lose up to 10 %.  Both bindings ask this.
+ * take) in such a call.  A rule fitted to times of both sides, which stand beside it: the few sizes it gets wrong lose up to 10 %.
+ * Both bindings ask this.
  */
-int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only);
+int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int call);
 
 /* What a workspace is for: the forward pass, or a backward pass that wants the sum of these. */
 #define MG_MLP_FORWARD 0

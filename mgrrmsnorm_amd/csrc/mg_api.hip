@@ -779,12 +779,19 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
 //   beyond 128 MiB of weights and 2048 tokens: 4096 x 6912 3072 1414 / 1343; 404 / 442, 3072 x 8192 4095 1620 / 1629; 470 / 481
 //   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2, from there on: 1024 x 2816 48 23.0 / 19.3.
 // Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162 / 44; 47 / 15.  Forward alone has a line of its own
-// (mlp_forward_wins).
-int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int forward_only) {
+// (mlp_forward_wins).  A step in which only x learns has no weight gradients, whose tiles win most:
+//   4096 x 6912: 700 tokens 328 / 305, 900 366 / 319, but 1300 479 / 508; 2048 x 3584: 4096 358 / 329, 8192 629 / 652, 16384 1249 / 1318
+//   1024 x 2816: 8192 342 / 300; 1024 x 1792: 8192 214 / 192, 16384 374 / 389; 512 x 1024 65536 tokens 617 / 585
+//   hidden not above d_model: 4096 x 4096 1024 tokens 244 / 210, 1100 (fp16) 274 / 288, 3072 524 / 572; 4096 x 2048 2500 249 / 280
+//   one token: 512 x 1024 27.3 / 30.9, 2048 x 2048 39.5 / 43.2, eager 3 times as fast
+// All others, at up to a million tokens: 0.97 (16000 tokens, 2048 x 6144) to 3.9 times as fast as the library's.
+int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int call) {
     if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
     const int64_t weights = 6 * d_model * hidden;
     if (tokens > 2048 && weights > 128LL << 20) return 0;
-    if (!forward_only) return 1;
+    if (call == MG_MLP_ALL) return 1;
+    if (call == MG_MLP_X_LEARNS)
+        return d_model <= 512 || (tokens <= 8192 && tokens * d_model * hidden <= (hidden > d_model ? 32000000000LL : 18000000000LL));
     if (tokens <= MG_BLOCK_MAX_TOKENS && weights < 16LL << 20) return 0;
     return mlp_forward_wins(tokens, d_model, hidden);
 }

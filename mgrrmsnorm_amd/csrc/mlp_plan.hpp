@@ -128,7 +128,7 @@ struct MlpForward {
 //     86 / 75, 640 131 / 146, 768 141 / 163, 2048 294 / 301; 4096 x 5440 65536 tokens 6102 / 6767; 8192 x 2048 64 tokens 41 / 56.
 // Of the sizes taken 1 in 100 is more than 2 % slower (worst 4096 tokens, 4096 x 4096, 299 / 324).  Between 20 and 130 tokens sizes of less
 // than 40 us, where three operators take 47 us on the host, are taken although a replayed graph may lose 1 to 6 us (65 tokens, 1536 x 2560
-// 18.0 / 22.3, eager 48 / 22).  Wins given up: 5 to 20 % at some sizes beyond 60 MB and 640 tokens (2048, 4096 x 11008 592 / 468).
+// 18.0 / 22.3, eager 46 / 20).  Wins given up: 5 to 20 % at some sizes beyond 60 MB and 640 tokens (2048, 4096 x 11008 592 / 468).
 inline bool mlp_forward_wins(int64_t t, int64_t d, int64_t h) {
     const float mb = 6e-6f * (float)d * (float)h;
     if (mb <= 24.0f || (mb <= 60.0f && t <= 5000)) return true;

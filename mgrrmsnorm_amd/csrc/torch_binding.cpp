@@ -473,7 +473,7 @@ struct MlpNode : public torch::autograd::Function<MlpNode> {
 bool swiglu_mlp_fits(const Tensor& x, int64_t hidden) {
     const auto type = x.scalar_type();
     if ((type != at::kHalf && type != at::kBFloat16) || !x.is_cuda() || x.dim() < 1 || x.size(-1) < 1) return false;
-    return mg_mlp_preferred(x.numel() / x.size(-1), x.size(-1), hidden, dtype_code(type), !torch::GradMode::is_enabled()) == 1;
+    return mg_mlp_preferred(x.numel() / x.size(-1), x.size(-1), hidden, dtype_code(type), torch::GradMode::is_enabled() ? MG_MLP_ALL : MG_MLP_FORWARD_ONLY) == 1;
 }
 
 // w3(silu(gate) * up) with [gate | up] = w12(x), differentiable, in this package's own products; an undefined tensor
@@ -488,8 +488,9 @@ Tensor swiglu_mlp(const Tensor& x, const Tensor& w12, const Tensor& w3) {
     if (w12.scalar_type() != type || w3.scalar_type() != type || w12.device() != x.device() || w3.device() != x.device() ||
         !w12.is_contiguous() || !w3.is_contiguous())
         return none;
-    const bool learns = torch::GradMode::is_enabled() && (x.requires_grad() || w12.requires_grad() || w3.requires_grad());
-    if (mg_mlp_preferred(x.numel() / d_model, d_model, hidden, dtype_code(type), !learns) != 1) return none;
+    const bool weights_learn = w12.requires_grad() || w3.requires_grad(), learns = torch::GradMode::is_enabled() && (x.requires_grad() || weights_learn);
+    const int call = !learns ? MG_MLP_FORWARD_ONLY : weights_learn ? MG_MLP_ALL : MG_MLP_X_LEARNS;
+    if (mg_mlp_preferred(x.numel() / d_model, d_model, hidden, dtype_code(type), call) != 1) return none;
     const auto off = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; };
     if (off(w12) || off(w3) || (x.is_contiguous() && off(x))) return none;   // a copy of x is aligned
     if (learns) {

@@ -217,15 +217,18 @@ def swiglu_backward(grad_out: torch.Tensor, gate_up: torch.Tensor, hidden_dim: i
 _MLP_CODES = {torch.float16: 1, torch.bfloat16: 2}
 
 
-def _preferred(x, hidden, forward_only):
+_MLP_ALL, _MLP_FORWARD_ONLY, _MLP_X_LEARNS = range(3)
+
+
+def _preferred(x, hidden, call):
     d_model = x.size(-1)
-    return _lib.load().mg_mlp_preferred(x.numel() // d_model, d_model, hidden, _MLP_CODES[x.dtype], int(forward_only)) == 1
+    return _lib.load().mg_mlp_preferred(x.numel() // d_model, d_model, hidden, _MLP_CODES[x.dtype], call) == 1
 
 
 def swiglu_mlp_fits(x: torch.Tensor, hidden_dim: int) -> bool:
     if x.dtype not in _MLP_CODES or not x.is_cuda or x.dim() < 1 or x.size(-1) < 1:
         return False
-    return _preferred(x, hidden_dim, not torch.is_grad_enabled())
+    return _preferred(x, hidden_dim, _MLP_ALL if torch.is_grad_enabled() else _MLP_FORWARD_ONLY)
 
 
 def _plain_dense(t: torch.Tensor) -> bool:
@@ -365,8 +368,10 @@ def swiglu_mlp(x: torch.Tensor, w12: torch.Tensor, w3: torch.Tensor):
         return None
     if any(w.dtype != x.dtype or w.device != x.device or not w.is_contiguous() or w.data_ptr() % 16 != 0 for w in (w12, w3)):
         return None
-    learns = torch.is_grad_enabled() and (x.requires_grad or w12.requires_grad or w3.requires_grad)
-    if not _preferred(x, hidden, not learns) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
+    weights_learn = w12.requires_grad or w3.requires_grad
+    learns = torch.is_grad_enabled() and (x.requires_grad or weights_learn)
+    call = _MLP_FORWARD_ONLY if not learns else _MLP_ALL if weights_learn else _MLP_X_LEARNS
+    if not _preferred(x, hidden, call) or (x.is_contiguous() and x.data_ptr() % 16 != 0):
         return None
     if learns:
         return _MlpFunction.apply(x.contiguous(), w12, w3)[0] if x.requires_grad or w12.requires_grad else None

@@ -38,6 +38,15 @@ def test_where_they_are_taken(lib, tokens, d_model, hidden, training, alone):
     assert [lib.mg_mlp_preferred(tokens, d_model, hidden, 2, only) for only in (0, 1)] == [training, alone]
 
 
+@pytest.mark.parametrize("tokens,d_model,hidden,taken", [
+    (1, 512, 1024, 1), (65536, 512, 1024, 1), (8192, 1024, 2816, 1), (8193, 1024, 1792, 0), (900, 4096, 6912, 1), (1300, 4096, 6912, 0), (4096, 2048, 3584, 1),
+    (8192, 2048, 3584, 0), (1024, 4096, 4096, 1), (1100, 4096, 4096, 0), (2500, 4096, 2048, 0), (3000, 4096, 6912, 0),
+])
+def test_where_they_are_taken_if_only_x_learns(lib, tokens, d_model, hidden, taken):
+    assert lib.mg_mlp_preferred(tokens, d_model, hidden, 1, 2) == taken
+    assert lib.mg_mlp_preferred(tokens, d_model, hidden, 1, 0) >= taken
+
+
 def test_bad_arguments_are_refused(lib):
     t, d, h = 100, 64, 128
     error = lambda: lib.mg_last_error().decode()

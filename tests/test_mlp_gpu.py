@@ -288,6 +288,12 @@ def test_what_goes_through_the_projections(binding, monkeypatch):
     w12.requires_grad_(False)
     assert not _takes(module, x) and _takes(module, x.clone().requires_grad_())   # only w3 learns
     w12.requires_grad_()
+    # frozen weights and more tokens than the gradient of x alone is taken for
+    wide = _module(1024, 1792).requires_grad_(False)
+    many = torch.randn(9000, 1024, device="cuda", dtype=torch.bfloat16)
+    assert not _takes(wide, many.requires_grad_()) and _takes(wide, many[:8000])
+    wide.w12.requires_grad_()
+    assert _takes(wide, many)
     # a checkpointed block, and a gradient of a gradient, which the activation refuses
     dy = torch.randn_like(x)
     got = _grads(module, x, dy, lambda t: torch.utils.checkpoint.checkpoint(module, t, use_reentrant=False))
