@@ -172,15 +172,16 @@ struct MlpProduct {
         read(f, first, 0);
         if constexpr (C::SUBSTEPS == 2) read(g, first, 1);
     }
-    // With one substep a step is one block of instructions: the next fragments' reads between the first half of the
-    // multiplications, the requests between all of them.  Left to itself the compiler issues the reads in a bunch, in front of
-    // the multiplications or behind them (1024 x 3584 outputs, k 2048: 18.9 / 18.5 us, 1024 x 2048, k 3584: 22.2 / 21.5; with two
-    // substeps its own order is as good or better).
-    static __device__ __forceinline__ void interleave() {
+    // The order of one fragment's worth of instructions, since the compiler, left to itself, issues the reads in a bunch.
+    // With one substep: the next fragments' reads between the first half of the multiplications, the requests between all of them
+    // (1024 x 3584 outputs, k 2048: 18.9 / 18.5 us, 1024 x 2048, k 3584: 22.2 / 21.5).  LATE, for the second of two substeps: the reads
+    // between the second half, no requests.
+    template <bool LATE> static __device__ __forceinline__ void interleave() {
         constexpr int M = C::FM * C::FN, H = M / 2, R = C::FM * (A_ALONG_K ? 1 : 2) + C::FN * (B_ALONG_K ? 1 : 2);
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            const int reads = i < H ? R * (i + 1) / H - R * i / H : 0, requests = PER_STEP * (i + 1) / M - PER_STEP * i / M;
+            const int at = LATE ? i - H : i, reads = at >= 0 && at < H ? R * (at + 1) / H - R * at / H : 0;
+            const int requests = LATE ? 0 : PER_STEP * (i + 1) / M - PER_STEP * i / M;
 #pragma unroll
             for (int k = 0; k < reads; ++k) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
 #pragma unroll
@@ -197,18 +198,22 @@ struct MlpProduct {
         read(next, cur, 0);
         request(refill);
         multiply(sums, f);
-        interleave();
+        interleave<false>();
     }
     // Two: `g` holds the second fragments of the stage before, and cur's on return; cur's first ones are multiplied in here.
+    // The halves are kept apart and the second one's reads late (forward + backward fp16, 2048 tokens, 4096 x 11008, and 1404,
+    // 2944 x 5120: 1453 and 384 us; reads where the compiler puts them 1468, 395; nothing kept apart 1552, 393 (bf16); every read early
+    // 1474, 382, but 128, 4096 x 11008 268 against 256).
     __device__ __forceinline__ void two_substeps(const char MG_LDS* __restrict__ cur, char MG_LDS* __restrict__ refill, MlpSums<C>& sums,
                                                  MlpFragments<C>& g) {
         MlpFragments<C> f;
         read(f, cur, 0);
         request(refill);
         multiply(sums, g);
-        __builtin_amdgcn_sched_barrier(0);   // else `g` is read between the multiplications that still need it: 2048 tokens,
-        read(g, cur, 1);                     // 4096 x 11008, forward + backward 1552 us against 1416
+        __builtin_amdgcn_sched_barrier(0);
+        read(g, cur, 1);
         multiply(sums, f);
+        interleave<true>();
     }
     // From one to the next: that has arrived for every wave, and every wave has read all of this one.
     __device__ __forceinline__ void next_stage(char MG_LDS* now, char MG_LDS* next) const {

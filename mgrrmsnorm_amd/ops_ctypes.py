@@ -338,6 +338,8 @@ def _mlp_backward_in_operations(grad_output, dh, want, x, w12, w3, gate_up, h):
     wanted, take the gradients those take and refuse what those refuse."""
     d_model, hidden = w3.shape
     out = [None, None, None]
+    if grad_output is None and dh is None:
+        return tuple(out)
     lead = (grad_output if dh is None else dh).shape[:-1]
     if dh is not None:
         dh = dh.reshape(-1, hidden)

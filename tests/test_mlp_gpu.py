@@ -402,6 +402,16 @@ def test_gradients_that_are_no_plain_tensors(binding):
             seen.append(func)
             return func(*args, **(kwargs or {}))
 
+    class Nothing(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t.sum()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    assert torch.autograd.grad(Nothing.apply(y), (module.w12.weight, w3), retain_graph=True, allow_unused=True) == (None, None)
     seen = []
     with Seen():
         got = torch.autograd.grad(y, (module.w12.weight, w3), dy[0], retain_graph=True)
