@@ -28,7 +28,7 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype);
 
 /*
  * 1 where they are also taken rather than library products around mg_swiglu_fwd and mg_swiglu_bwd (0 for sizes they do not
- * take) in such a call.  A rule fitted to times of both sides, which stand beside it: the few sizes it gets wrong lose up to 10 %.
+ * take) in such a call.  A rule fitted to times of both sides, which stand beside it: the few sizes it gets wrong lose a few per cent.
  * Both bindings ask this.
  */
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int call);
@@ -40,8 +40,8 @@ int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype,
 #define MG_MLP_DW3 4
 
 /*
- * Bytes of workspace a pass needs on the current device, 0 for none: where tokens are few, k is split over workgroups,
- * whose sums meet there in fp32.
+ * Bytes of workspace a pass needs on the current device, 0 for none: where a product has few tiles, its k is split over workgroups,
+ * whose sums meet there in fp32.  For sizes mg_mlp_preferred takes at most about 260 MiB, and less than the tensors the pass writes.
  */
 int mg_mlp_workspace(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int pass, int64_t* bytes);
 

@@ -772,19 +772,20 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
 
 // Where they take no more time than the library's products and the activation between them.  GPU time in
 // replayed graphs (library / these, us, bf16, d_model x hidden, forward + backward; forward):
-//   512 x 1024: 1 token 34.6 / 31.5, 320 59 / 37; 21.1 / 17.2, 1024 72 / 43; 24.9 / 19.8
-//   1024 x 1792: 8 46.1 / 39.3, 128 69 / 46; 20.9 / 21.5, 1024 99 / 65; 30.8 / 26.8
-//   2048 x 3584: 8 82 / 66, 128 100 / 65; 28.2 / 27.2, 1024 211 / 153; 64 / 57, 4095 562 / 480; 165 / 152
-//   4096 x 11008: 8 315 / 194, 320 530 / 422; 133 / 153, 1024 985 / 811; 312 / 288, 2048 1986 / 1443; 594 / 471
-//   beyond 128 MiB of weights and 2048 tokens: 4096 x 6912 3072 1414 / 1343; 404 / 442, 3072 x 8192 4095 1620 / 1629; 470 / 481
-//   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2, from there on: 1024 x 2816 48 23.0 / 19.3.
+//   512 x 1024: 1 token 36.3 / 30.7, 320 57 / 35; 20.6 / 15.9, 1024 70 / 41; 23.7 / 18.0
+//   1024 x 1792: 8 48.8 / 38.3, 128 67 / 44; 20.0 / 20.4, 1024 98 / 65; 28.5 / 24.6
+//   2048 x 3584: 8 89 / 70, 128 107 / 72; 29.9 / 31.9, 1024 215 / 154; 64.9 / 54.4, 4095 562 / 490; 168 / 160
+//   4096 x 11008: 8 324 / 199, 320 531 / 411; 134 / 146, 1024 980 / 784; 280 / 261, 2048 1975 / 1419; 588 / 462
+//   beyond 128 MiB of weights and 2048 tokens: 4096 x 6912 3072 1436 / 1311; 410 / 441, 3072 x 8192 4095 1635 / 1538; 481 / 497
+//   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2 and 18.5 / 17.9 (two boxes), from there on: 1024 x 2816 48 21.7 / 18.4.
 // Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162 / 44; 47 / 15.  Forward alone has a line of its own
 // (mlp_forward_wins).  A step in which only x learns has no weight gradients, whose tiles win most:
-//   4096 x 6912: 700 tokens 328 / 305, 900 366 / 319, but 1300 479 / 508; 2048 x 3584: 4096 358 / 329, 8192 629 / 652, 16384 1249 / 1318
-//   1024 x 2816: 8192 342 / 300; 1024 x 1792: 8192 214 / 192, 16384 374 / 389; 512 x 1024 65536 tokens 617 / 585
-//   hidden not above d_model: 4096 x 4096 1024 tokens 244 / 210, 1100 (fp16) 274 / 288, 3072 524 / 572; 4096 x 2048 2500 249 / 280
-//   one token: 512 x 1024 27.3 / 30.9, 2048 x 2048 39.5 / 43.2, eager 3 times as fast
-// All others, at up to a million tokens: 0.97 (16000 tokens, 2048 x 6144) to 3.9 times as fast as the library's.
+//   4096 x 6912: 700 tokens 329 / 300, 900 360 / 318, but 1300 470 / 512; 2048 x 3584: 4096 357 / 333, 8192 631 / 631, 16384 1227 / 1268
+//   1024 x 2816: 8192 354 / 301; 1024 x 1792: 8192 221 / 196, 16384 390 / 374 and (another box) 374 / 389; 512 x 1024 65536 tokens 611 / 569
+//   hidden not above d_model: 4096 x 4096 1024 tokens 239 / 208, 1100 (fp16) 272 / 289, 3072 526 / 575; 4096 x 2048 2500 253 / 275
+//   one token: 512 x 1024 27.1 / 30.6, 2048 x 2048 39.7 / 42.7, eager 3 times as fast
+// All others were measured at up to a million tokens: from about level (16000 tokens, 2048 x 6144 3146 / 3075) to 4 times as fast
+// (65536, 128 x 192 508 / 128).
 int mg_mlp_preferred(int64_t tokens, int64_t d_model, int64_t hidden, int dtype, int call) {
     if (!mg_mlp_fits(tokens, d_model, hidden, dtype)) return 0;
     const int64_t weights = 6 * d_model * hidden;

@@ -122,13 +122,13 @@ struct MlpForward {
 // and the activation, on the 256 compute units that both sides were measured on (700 sizes: 20 to 65536 tokens, 3 to 425 MB of
 // weights, replayed graphs, bf16 and fp16).  The library's time scatters by 10 % around the line below, which lies where least
 // is lost on either side; up to the given weights these products win or are level at every number of tokens measured:
-//   below 24 MB: 512 x 1024 17.3 / 14.7 us at 65 tokens, 286 / 239 at 65536; 1024 x 2816 19.1 / 18.8, 1049 / 1005;
-//   below 60 MB and 5000 tokens: 2048 x 3584 1024 tokens 64.7 / 54.9, 4096 169 / 164, but 8192 299 / 309; 1664 x 4608 1800 tokens 120 / 106;
-//   beyond: 4096 x 11008 256 tokens 120 / 107, but 320 135 / 147 and 384 146 / 162 (row tiles that just miss), 448 169 / 160; 4096 x 6912 256
-//     86 / 75, 640 131 / 146, 768 141 / 163, 2048 294 / 301; 4096 x 5440 65536 tokens 6102 / 6767; 8192 x 2048 64 tokens 41 / 56.
-// Of the sizes taken 1 in 100 is more than 2 % slower (worst 4096 tokens, 4096 x 4096, 299 / 324).  Between 20 and 130 tokens sizes of less
+//   below 24 MB: 512 x 1024 17.2 / 14.6 us at 65 tokens, 285 / 230 at 65536; 1024 x 2816 19.0 / 18.6, 1042 / 977;
+//   below 60 MB and 5000 tokens: 2048 x 3584 1024 tokens 64.9 / 54.4, 4096 168 / 160, but 8192 297 / 302; 1664 x 4608 1800 tokens 124 / 107;
+//   beyond: 4096 x 11008 256 tokens 118 / 109, but 320 134 / 146 and 384 145 / 158 (row tiles that just miss), 448 168 / 157; 4096 x 6912 256
+//     87 / 76, 640 131 / 146, 768 141 / 162, 2048 293 / 298; 4096 x 5440 65536 tokens 6090 / 6531; 8192 x 2048 64 tokens 41 / 56.
+// Of the sizes taken 1 in 100 is more than 2 % slower (worst 256 tokens, 8192 x 2048, 63 / 66).  Between 20 and 130 tokens sizes of less
 // than 40 us, where three operators take 47 us on the host, are taken although a replayed graph may lose 1 to 6 us (65 tokens, 1536 x 2560
-// 18.0 / 22.3, eager 46 / 20).  Wins given up: 5 to 20 % at some sizes beyond 60 MB and 640 tokens (2048, 4096 x 11008 592 / 468).
+// 18.6 / 22.6, eager 46 / 20).  Wins given up: 5 to 20 % at some sizes beyond 60 MB and 640 tokens (2048, 4096 x 11008 588 / 462).
 inline bool mlp_forward_wins(int64_t t, int64_t d, int64_t h) {
     const float mb = 6e-6f * (float)d * (float)h;
     if (mb <= 24.0f || (mb <= 60.0f && t <= 5000)) return true;

@@ -1,6 +1,7 @@
 """What of the block's own products can be checked without a GPU: the sizes and arguments the C entry points take,
 and the calls MegaGemmTriton hands to them."""
 import random
+import re
 import shutil
 import subprocess
 from pathlib import Path
@@ -15,6 +16,17 @@ from test_block_route_cpu import CHANGES, REPLACED, _module
 @pytest.fixture(scope="module")
 def lib():
     return _lib.load()
+
+
+def test_header_compiles_and_declares_what_the_library_exports(lib, tmp_path):
+    header = Path(__file__).resolve().parent.parent / "include" / "megagemm_hip_mlp.h"
+    text = re.sub(r"/\*.*?\*/", "", header.read_text(), flags=re.S)
+    assert sorted(re.findall(r"\b(mg_[a-z0-9_]+)\s*\(", text)) == sorted(_lib.MLP_SIGNATURES)
+    assert all(hasattr(lib, name) for name in _lib.MLP_SIGNATURES)
+    source = tmp_path / "t.c"
+    source.write_text('#include "megagemm_hip_mlp.h"\nint main(void){return MG_MLP_ALL + MG_MLP_FORWARD;}\n')
+    for compiler in (["gcc", "-std=c99"], ["g++", "-x", "c++"]):
+        subprocess.run([*compiler, "-Wall", "-Werror", f"-I{header.parent}", "-c", str(source), "-o", str(tmp_path / "t.o")], check=True)
 
 
 @pytest.mark.parametrize("tokens,d_model,hidden,dtype,fits", [
