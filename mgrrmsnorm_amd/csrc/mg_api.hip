@@ -777,11 +777,11 @@ int mg_mlp_fits(int64_t tokens, int64_t d_model, int64_t hidden, int dtype) {
 //   2048 x 3584: 8 89 / 70, 128 107 / 72; 29.9 / 31.9, 1024 215 / 154; 64.9 / 54.4, 4095 562 / 490; 168 / 160
 //   4096 x 11008: 8 324 / 199, 320 531 / 411; 134 / 146, 1024 980 / 784; 280 / 261, 2048 1975 / 1419; 588 / 462
 //   beyond 128 MiB of weights and 2048 tokens: 4096 x 6912 3072 1436 / 1311; 410 / 441, 3072 x 8192 4095 1635 / 1538; 481 / 497
-//   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2 and 18.5 / 17.9 (two boxes), from there on: 1024 x 2816 48 21.7 / 18.4.
+//   a decoding step of less than 16 MiB of weights: 1024 x 1792 48 tokens 17.4 / 20.2 and 18.5 / 17.9 (two sessions), from there on: 1024 x 2816 48 21.7 / 18.4.
 // Eager, the fewer launches win by more: 512 x 1024, 300 tokens 162 / 44; 47 / 15.  Forward alone has a line of its own
 // (mlp_forward_wins).  A step in which only x learns has no weight gradients, whose tiles win most:
 //   4096 x 6912: 700 tokens 329 / 300, 900 360 / 318, but 1300 470 / 512; 2048 x 3584: 4096 357 / 333, 8192 631 / 631, 16384 1227 / 1268
-//   1024 x 2816: 8192 354 / 301; 1024 x 1792: 8192 221 / 196, 16384 390 / 374 and (another box) 374 / 389; 512 x 1024 65536 tokens 611 / 569
+//   1024 x 2816: 8192 354 / 301; 1024 x 1792: 8192 221 / 196, 16384 390 / 374 and (another session) 374 / 389; 512 x 1024 65536 tokens 611 / 569
 //   hidden not above d_model: 4096 x 4096 1024 tokens 239 / 208, 1100 (fp16) 272 / 289, 3072 526 / 575; 4096 x 2048 2500 253 / 275
 //   one token: 512 x 1024 27.1 / 30.6, 2048 x 2048 39.7 / 42.7, eager 3 times as fast
 // All others were measured at up to a million tokens: from about level (16000 tokens, 2048 x 6144 3146 / 3075) to 4 times as fast
